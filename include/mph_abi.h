@@ -175,8 +175,9 @@ int mph_scene_run_phase(mph_scene* s, int phase);
  * R2g Swa Swg Swp Swv MaxRadius ParticleCount FluidCount PowerParticleCount
  * CellCount0..2 TotalCellCount NeighborIndCount NeighborIndCountP MultiGridDepth
  * CRIterations rr0 rr rs0 rs RefinementSteps ABlocks ASlots CBlocks, the timing
- * scalars of mph_scene_set_timing, TunedSpmv64 TunedSpmv32 TunedCac TunedFuse
- * TunedGalerkin (the variants the run-time tuner kept, -1 while still exploring),
+ * scalars of mph_scene_set_timing, TunedSpmv64 TunedSpmv32 TunedCac TunedGalerkin
+ * (the variants the run-time tuner kept, -1 while still exploring), TunedFuse (0: one
+ * variant of the fused coarse V-cycle),
  * and for the factored operator FactoredBytes and FactoredBytesF32 (algorithmic
  * bytes of one product with FP64 / FP32 scalars) and AssembledBlocks (1 when the
  * step assembled the 3x3 blocks: always for the assembled form; for the factored

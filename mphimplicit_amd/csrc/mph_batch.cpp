@@ -45,7 +45,6 @@ struct mph_batch {
     Autotune tune64, tune32;  // SpMV load-group depth of the scene-table launches
     std::vector<char> fac;      // per scene of the current solve: factored operator
     std::vector<char> cell;     // ... and its FP64 second pass cell-staged
-    Autotune tuneFuse;        // V-cycle levels fused into one workgroup per scene
     int* hctl = nullptr;      // [ns][kNCtl] coherent pinned mirrors of the scenes' CR control blocks
     size_t hctlCap = 0;
     hipEvent_t ev[2] = {nullptr, nullptr};  // the FP64 loop's last two iterations
@@ -130,7 +129,8 @@ int build_tables(mph_batch& B, const std::vector<mph_scene*>& sc, Tables& T, boo
         b.scal = B.scal.p + 8 * (size_t)s;
         b.mg = S.prm.multigrid ? 1 : 0;
         b.depth = b.mg ? S.depth : 0;
-        for (int v = 0; v < kFuseVariants; ++v) b.fuseOf[v] = b.mg ? S.fuseOf[v] : 0;
+        b.fuse = b.mg ? S.fuse : 0;
+        b.pack = S.pack;
         for (int l = 0; l < b.depth; ++l) b.lv[l] = S.lv[l].L;
         if (stop) {
             if ((rc = S.ctl.ensure(kNCtl))) return rc;
@@ -167,7 +167,6 @@ int read_scalars(mph_batch& B, int ns) {
     HIPCHK(hipStreamSynchronize(B.st));
     B.tune64.collect();
     B.tune32.collect();
-    B.tuneFuse.collect();
     return MPH_OK;
 }
 
@@ -222,58 +221,45 @@ struct VCycle {
     // precondition (main.cpp:4122-4266) of in -> out for the multigrid scenes in `on`
     void apply(const Set& on, int in, int out, bool part, bool f32) {
         if (on.empty()) return;
-        const int v = B.tuneFuse.pick();
-        B.tuneFuse.begin(T.st, v);
-        auto F = [&](int s) { return sc[s]->fuseOf[v]; };
-        int maxD = 0;
+        auto F = [&](int s) { return sc[s]->fuse; };  // levels F..depth-1: one workgroup
+        int maxF = 0;
         for (int s = 0; s < (int)sc.size(); ++s)
-            if (on.has(s)) maxD = std::max(maxD, sc[s]->depth);
-        mg_p2g_bu(T, on.m, in, curset(on, 0));  // P2G, S = 0, R = Q, S += invD R
-        ru(on, 0, f32);                          // pre-smooth x2
-        mg_residual(T, on.m, 0, curset(on, 0), f32);
-        for (int l = 1; l <= maxD - 1; ++l) {  // levels below each scene's fused part
-            Set inner, coarsest, both;
-            for (int s = 0; s < (int)sc.size(); ++s) {
-                if (!on.has(s) || l >= F(s)) continue;
-                const int D = sc[s]->depth;
-                if (D - 1 > l) inner.add(s), both.add(s);
-                else if (D - 1 == l) coarsest.add(s), both.add(s);
-            }
-            if (both.empty()) continue;
-            mg_restrict_bu(T, both.m, l, curset(both, l));
-            ru(both, l, f32);
-            ru(both, l, f32);
-            if (!inner.empty()) mg_residual(T, inner.m, l, curset(inner, l), f32);  // pre-smooth x3
-            ru(coarsest, l, f32);                                                  // coarsest: x4, then
-            ru(coarsest, l, f32);                                                  // the prolongation
-            if (!coarsest.empty()) mg_prolong(T, coarsest.m, l, curset(coarsest, l), curset(coarsest, l - 1));
-        }
-        Set fused;  // levels F..depth-1 of every scene in one launch
-        CurBits cb{};
-        for (int s = 0; s < (int)sc.size(); ++s)
-            if (on.has(s) && F(s) < sc[s]->depth) {
-                fused.add(s);
-                for (int l = F(s) - 1; l < sc[s]->depth; ++l)
-                    if (cur[s][l]) cb.lv[l].w[s >> 6] |= 1ull << (s & 63);
-            }
-        if (!fused.empty()) {
-            mg_coarse(T, fused.m, cb, v, f32);
-            for (int s = 0; s < (int)sc.size(); ++s)  // five sweeps per fused level, four at the coarsest
-                if (fused.has(s))
-                    for (int l = F(s); l < sc[s]->depth - 1; ++l) cur[s][l] ^= 1;
-        }
-        for (int l = maxD - 2; l >= 1; --l) {
-            Set up;
+            if (on.has(s)) maxF = std::max(maxF, F(s));
+        auto above = [&](int l) {  // the scenes whose level l has launches of its own
+            Set m;
             for (int s = 0; s < (int)sc.size(); ++s)
-                if (on.has(s) && sc[s]->depth - 2 >= l && l < F(s)) up.add(s);
-            if (up.empty()) continue;
-            for (int k = 0; k < 3; ++k) ru(up, l, f32);  // post-smooth x3
-            mg_prolong(T, up.m, l, curset(up, l), curset(up, l - 1));
+                if (on.has(s) && l < F(s)) m.add(s);
+            return m;
+        };
+        mg_p2g_bu(T, on.m, in, curset(on, 0));  // P2G, S = 0, R = Q, S += invD R
+        const Set top = above(0);
+        ru(top, 0, f32);  // pre-smooth x2
+        if (!top.empty()) mg_residual(T, top.m, 0, curset(top, 0), f32);
+        for (int l = 1; l < maxF; ++l) {
+            const Set m = above(l);
+            mg_restrict_bu(T, m.m, l, curset(m, l));  // pre-smooth x3
+            ru(m, l, f32);
+            ru(m, l, f32);
+            mg_residual(T, m.m, l, curset(m, l), f32);
         }
-        ru(on, 0, f32);  // post-smooth x2
-        ru(on, 0, f32);
+        for (int dim = 2; dim <= 3; ++dim) {  // levels F..depth-1 of every scene
+            Set m, cu;
+            for (int s = 0; s < (int)sc.size(); ++s)
+                if (on.has(s) && sc[s]->P.dim == dim) {
+                    m.add(s);
+                    if (cur[s][F(s) > 0 ? F(s) - 1 : 0]) cu.add(s);
+                    if (F(s) == 0) cur[s][0] ^= 1;
+                }
+            mg_coarse(T, m.m, cu.m, dim);
+        }
+        for (int l = maxF - 1; l >= 1; --l) {
+            const Set m = above(l);
+            for (int k = 0; k < 3; ++k) ru(m, l, f32);  // post-smooth x3
+            mg_prolong(T, m.m, l, curset(m, l), curset(m, l - 1));
+        }
+        ru(top, 0, f32);  // post-smooth x2
+        ru(top, 0, f32);
         mg_g2p(T, on.m, curset(on, 0), in, out, part);
-        B.tuneFuse.end(T.st);
     }
 };
 
@@ -364,8 +350,8 @@ int solve_fp64(mph_batch& B, const std::vector<mph_scene*>& sc, std::vector<char
     if (!active.empty()) {
         // the trials of the autotuners are read as their iterations complete (mark:
         // how many each had recorded at an iteration's event)
-        Autotune* tn[] = {&B.tune64, &B.tune32, &B.tuneFuse};
-        constexpr int kTn = 3;
+        Autotune* tn[] = {&B.tune64, &B.tune32};
+        constexpr int kTn = sizeof(tn) / sizeof(tn[0]);
         size_t mark[2][kTn];
         fp64_iteration(B, T, V, active, active);
         HIPCHK(hipEventRecord(B.ev[0], B.st));
@@ -565,7 +551,6 @@ int mph_batch_create(int device, mph_batch** out) {
     B->device = device;
     B->tune64.init(kSpmvVariants64, 3);
     B->tune32.init(kSpmvVariants32, 3);
-    B->tuneFuse.init(kFuseVariants, 3);
     if (hipStreamCreateWithFlags(&B->st, hipStreamNonBlocking) != hipSuccess) {
         delete B;
         return fail(MPH_E_DEVICE, "stream creation failed");
@@ -711,7 +696,6 @@ int mph_batch_destroy(mph_batch* B) {
         if (e) (void)hipEventDestroy(e);
     B->tune64.release();
     B->tune32.release();
-    B->tuneFuse.release();
     if (B->st) (void)hipStreamDestroy(B->st);
     delete B;
     return MPH_OK;

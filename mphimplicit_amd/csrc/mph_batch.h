@@ -40,10 +40,6 @@ __device__ inline int find_scene(const int* __restrict__ o, int ns, int b) {
     return lo;
 }
 
-struct CurBits {  // per level, the scenes whose ping-pong bit is set
-    SceneSet lv[kMaxLevels];
-};
-
 struct BScene {
     DevParams P;
     const int* nFluid;
@@ -62,7 +58,8 @@ struct BScene {
     double* scal;
     int depth;
     int mg;
-    int fuseOf[kFuseVariants];  // first level of the one-workgroup coarse cycle per variant
+    int fuse;                   // first level of the one-workgroup coarse cycle
+    CoarsePack pack;            // and its rows
     int factored;               // MPH_OPERATOR_FACTORED: products through fac, not val/val32
     FacOp fac[2];               // FP64 and FP32 scalars (FP32: mixed precision only)
     Level lv[kMaxLevels];  // .cur is ignored: it comes with each launch
@@ -130,8 +127,9 @@ void mg_residual_update(const Tables& T, const SceneSet& on, int l, const SceneS
 void mg_restrict(const Tables& T, const SceneSet& on, int l);  // level l-1 -> l
 void mg_prolong(const Tables& T, const SceneSet& on, int l, const SceneSet& curL, const SceneSet& curS);  // l -> l-1
 void mg_g2p(const Tables& T, const SceneSet& on, const SceneSet& cur0, int in, int out, bool part);
-// levels fuseOf[variant]..depth-1 of each scene in one workgroup
-void mg_coarse(const Tables& T, const SceneSet& on, const CurBits& cb, int variant, bool f32);
+// levels fuse..depth-1 of each scene in one workgroup; cur: the scenes whose level
+// fuse-1 (level 0 when fuse is 0) has its ping-pong bit set; dim: of the scenes in `on`
+void mg_coarse(const Tables& T, const SceneSet& on, const SceneSet& cur, int dim);
 
 }  // namespace batch
 }  // namespace mph

@@ -262,18 +262,20 @@ __global__ void __launch_bounds__(256) kb_mg_g2p(const BScene* tab, const int* o
     mg_g2p_chunk(B.P, L, B.cellIndex, B.invDiagA, B.vec[in], B.vec[out], part ? B.part : nullptr, lb, sh);
 }
 
-// levels fuse..depth-1 of each scene in its own workgroup; cur.lv[l] holds the
-// ping-pong bit of level l per scene
-__global__ void __launch_bounds__(kCoarseThreads) kb_mg_coarse(const BScene* tab, int ns, SceneSet on, CurBits cb, int variant,
-                                                    int f32) {
+// levels fuse..depth-1 of each scene in its own workgroup (mg_coarse_cycle; 2D and 3D
+// scenes take launches of their own)
+template <int N, int T, int XB>
+__global__ void __launch_bounds__(T) kb_mg_coarse(const BScene* tab, int ns, SceneSet on, SceneSet cur) {
     const int s = blockIdx.x;
     if (s >= ns || !in_set(on, s)) return;
     const BScene& B = tab[s];
-    if (halted(B)) return;
-    unsigned cur = 0;
-#pragma unroll
-    for (int l = 0; l < kMaxLevels; ++l) cur |= (in_set(cb.lv[l], s) ? 1u : 0u) << l;
-    mg_coarse_cycle(B.lv, B.fuseOf[variant], B.depth, cur, f32 != 0);
+    const CoarsePack K = B.pack;
+    if ((int)threadIdx.x >= K.stride) return;  // whole wavefronts without rows
+    __shared__ CoarseShared<T> sh;
+    const unsigned c = in_set(cur, s) ? 1u : 0u;
+    const Level& S = B.lv[B.fuse > 0 ? B.fuse - 1 : 0];
+    mg_coarse_cycle<N, T, XB>(K, B.fuse, B.depth, B.fuse > 0 ? S.R : S.Q, lv_s(S, B.fuse > 0 ? c : c ^ 1), S.nrow,
+                              B.ctl ? B.ctl + kCtlHalt : nullptr, sh);
 }
 
 #undef MPH_SCENE
@@ -397,9 +399,14 @@ void mg_g2p(const Tables& T, const SceneSet& on, const SceneSet& cur0, int in, i
     MPH_LAUNCH(kb_mg_g2p, kOffChunk, cur0, in, out, part ? 1 : 0);
 }
 
-void mg_coarse(const Tables& T, const SceneSet& on, const CurBits& cb, int variant, bool f32) {
-    if (T.ns > 0 && any(on))
-        hipLaunchKernelGGL(kb_mg_coarse, dim3(T.ns), dim3(kCoarseThreads), 0, T.st, T.tab, T.ns, on, cb, variant, f32 ? 1 : 0);
+void mg_coarse(const Tables& T, const SceneSet& on, const SceneSet& cur, int dim) {
+    if (T.ns <= 0 || !any(on)) return;
+    if (dim == 2)
+        hipLaunchKernelGGL((kb_mg_coarse<9, kCoarseRows2D, 4>), dim3(T.ns), dim3(kCoarseRows2D), 0, T.st, T.tab, T.ns,
+                           on, cur);
+    else
+        hipLaunchKernelGGL((kb_mg_coarse<27, kCoarseRows3D, 4>), dim3(T.ns), dim3(kCoarseRows3D), 0, T.st, T.tab, T.ns,
+                           on, cur);
 }
 
 #undef MPH_LAUNCH

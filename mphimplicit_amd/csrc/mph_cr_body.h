@@ -289,82 +289,249 @@ __device__ inline void mg_prolong_row(const Level& L, const Level& S, int row) {
     Sv[row] = y;
 }
 
-// Levels lc..D-1 of the V-cycle inside ONE workgroup: restriction into lc, the
-// down sweep (S = invD R, then two residual-update sweeps and a residual per
-// level), the coarsest level (S = invD R, then four residual-update sweeps), the
-// up sweep (three residual-update sweeps per level) and the prolongations back
-// into lc-1 -- the order of preconditionWithMultiGrid (4160-4255) for those levels.  Each step runs over the level's rows with a
-// stride of blockDim.x and ends at a workgroup barrier, so every row sees the
-// previous step complete.  `cur` holds the ping-pong state of each level (bit l)
-// on entry, lc-1 included; it advances as the separate launches would advance it
-// (afterwards every fused level but the coarsest has flipped).  f32: use a level's FP32
-// stencil where it has one.
-// The workgroup has kCoarseThreads threads: few enough that mg_row_sum's batches of
-// nine stencil cells (54 values in flight) fit in registers, so a sweep waits for
-// three rounds of loads per row.  (With 1024 threads and three cells per batch it
-// waited for nine: 68 us per cycle on the 1M-particle scene, levels 3 and 4.)
-constexpr int kCoarseThreads = 256;
+// Levels lc..D-1 of the V-cycle inside ONE workgroup, in the order of
+// preconditionWithMultiGrid (4160-4255) for those levels: restriction into lc, the
+// down sweep (S = invD R, then residual-update sweeps and a residual per level), the
+// coarsest level (S = invD R, then four residual-update sweeps), the up sweep and the
+// prolongations back into lc-1.  With lc = 0 the whole hierarchy is here: Q0 comes
+// from the P2G launch and S0 goes back for the G2P.
+//
+// Every row of every fused level is owned by one thread for the whole cycle, which
+// keeps the row's stencil values, its smoother weight, Q and S in registers; S and R
+// go through LDS, a workgroup barrier after every sweep.  The rows' values and places
+// are laid out per thread once per multigrid build (coarse_pack), so the cycle starts
+// with one round of coalesced loads, all in flight together (2.3-3.4 us), and a sweep
+// is 27 LDS reads and a chain of 81 ordered adds per row (9 and 27 in 2D).  The chain
+// bounds it: about 24 cycles per add, 0.9 us per 3D sweep.  Measured per cycle: 14.2 us
+// on the 64k-particle drop (105 rows), 18.8 us on the 1M-particle scene (216 rows),
+// 14.0 us on a 2D pool of 4,100 (372 rows).  Re-reading the stencils through L2 in
+// every sweep, three dependent rounds of loads each, took 47.7, 63.9 and 60.4 us.
+//
+// Invalid cells of a stencil narrower than 3 along an axis are padded with a zero
+// value and the row's own cell: they add a zero, which changes no bit of a sum that
+// starts at +0.  S*0.0 and Q*0.0 of the reference are zeros and are not formed.
 
-__device__ inline void mg_coarse_cycle(const Level* lvs, int lc, int D, unsigned cur, bool f32) {
-    auto lev = [&](int l) {
-        Level L = lvs[l];
-        L.cur = (cur >> l) & 1u;
-        return L;
+// The per-thread layout: value k of thread t at v[k*stride + t] (3N stencil values, then
+// invD; NaN-free zeros for threads without a row), int m of thread t at i[m*stride + t]:
+// (N+1)/2 pairs of 16-bit LDS places of the stencil cells, then the meta words below;
+// up[r] = the LDS place of the parent of row r of level lc-1.
+enum { kCmLevel = 0, kCmChild = 1, kCmSx = 2, kCmSy = 3, kCmParent = 4, kCmShape = 5, kCmWords = 6 };
+
+__device__ inline void coarse_pack(const Level* __restrict__ lvs, int lc, int D, bool f32, const CoarsePack& K) {
+    const int N = K.cells, NZ = N / 9, tid = threadIdx.x + blockIdx.x * blockDim.x;
+    if (lc > 0) {
+        const Level &L = lvs[lc], &F = lvs[lc - 1];
+        for (int r = tid; r < F.nrow; r += gridDim.x * blockDim.x) {
+            int fx, fy, fz;
+            grid_xyz(F, r / 3, fx, fy, fz);
+            K.up[r] = 3 * grid_id(L, ((fx + F.mn[0]) / 2) - L.mn[0], ((fy + F.mn[1]) / 2) - L.mn[1],
+                                  ((fz + F.mn[2]) / 2) - L.mn[2]) + r % 3;
+        }
+    }
+    if (tid >= K.stride) return;
+    int myl = -1, row = 0, base = 0, down = 0, upb = 0;  // first LDS places: own, finer, coarser level
+    for (int l = lc, b = 0, bp = 0; l < D; ++l) {
+        const int n = lvs[l].nrow;
+        if (tid >= b && tid < b + n) {
+            myl = l;
+            row = tid - b;
+            base = b;
+            down = l == lc ? 0 : bp;
+            upb = b + n;
+        }
+        bp = b;
+        b += n;
+    }
+    int* const im = K.i + (long long)((N + 1) / 2) * K.stride + tid;
+    im[kCmLevel * K.stride] = myl;
+    if (myl < 0) {
+        for (int k = 0; k <= 3 * N; ++k) K.v[(long long)k * K.stride + tid] = 0.0;
+        for (int m = 0; m < (N + 1) / 2; ++m) K.i[m * K.stride + tid] = 0;
+        for (int m = 1; m < kCmWords; ++m) im[m * K.stride] = 0;
+        return;
+    }
+    const Level& L = lvs[myl];
+    const int g = row / 3, rd = row % 3;
+    int gx, gy, gz;
+    grid_xyz(L, g, gx, gy, gz);
+    int lo = 0;
+    for (int k = 0; k < N; ++k) {
+        const int ex = k / (3 * NZ), ey = (k / NZ) % 3, ez = k % NZ;
+        const bool in = ex < L.cs[0] && ey < L.cs[1] && ez < L.cs[2];
+        const long long sh = in ? 3 * ((L.cs[1] * ex + ey) * L.cs[2] + ez) : 0;
+        for (int sd = 0; sd < 3; ++sd) {
+            const long long e = (sh + sd) * L.nrow + row;
+            K.v[(long long)(3 * k + sd) * K.stride + tid] = !in ? 0.0 : f32 && L.A32 ? (double)L.A32[e] : L.A[e];
+        }
+        const int jx = wrap3(gx + ex - 1 + L.cnt[0], L.cnt[0]), jy = wrap3(gy + ey - 1 + L.cnt[1], L.cnt[1]);
+        const int jz = NZ == 1 ? 0 : wrap3(gz + ez - 1 + L.cnt[2], L.cnt[2]);
+        const int pl = base + 3 * (in ? grid_id(L, jx, jy, jz) : g);
+        if (k & 1) K.i[(k / 2) * K.stride + tid] = lo | (pl << 16);
+        else lo = pl;
+    }
+    if (N & 1) K.i[(N / 2) * K.stride + tid] = lo;
+    K.v[(long long)(3 * N) * K.stride + tid] = L.invD[row];
+    int child = 0, sx = 0, sy = 0, shape = 0, parent = 0;
+    if (myl > 0) {  // the clipped 2x2x2 children (mg_restrict_row)
+        const Level& F = lvs[myl - 1];
+        const int x = gx + L.mn[0], y = gy + L.mn[1], z = gz + L.mn[2];
+        const int fmx = F.mn[0] > 2 * x, fmy = F.mn[1] > 2 * y, fmz = F.mn[2] > 2 * z;
+        const int nx = 2 - fmx - (F.mx[0] < 2 * (x + 1)), ny = 2 - fmy - (F.mx[1] < 2 * (y + 1));
+        const int nz = 2 - fmz - (F.mx[2] < 2 * (z + 1));
+        shape = nx | (ny << 2) | (nz << 4);
+        child = down + 3 * grid_id(F, (2 * x + fmx) - F.mn[0], (2 * y + fmy) - F.mn[1], (2 * z + fmz) - F.mn[2]) + rd;
+        sx = 3 * F.cnt[1] * F.cnt[2];
+        sy = 3 * F.cnt[2];
+    }
+    if (myl + 1 < D) {  // the parent (mg_prolong_row)
+        const Level& U = lvs[myl + 1];
+        parent = upb + 3 * grid_id(U, ((gx + L.mn[0]) / 2) - U.mn[0], ((gy + L.mn[1]) / 2) - U.mn[1],
+                                   ((gz + L.mn[2]) / 2) - U.mn[2]) + rd;
+    }
+    im[kCmChild * K.stride] = child;
+    im[kCmSx * K.stride] = sx;
+    im[kCmSy * K.stride] = sy;
+    im[kCmParent * K.stride] = parent;
+    im[kCmShape * K.stride] = shape;
+}
+
+template <int T>
+struct CoarseShared {
+    double S[2][T], R[T];
+};
+
+// K: the packed levels lc..D-1; in: R of level lc-1 (Q of level 0 when lc = 0); io: S of
+// level lc-1, which the prolongation updates (of level 0 when lc = 0, written); nio: its
+// rows.  XB: stencil cells whose LDS reads are in flight together.  halt: the CR stop
+// flag or null, tested once the loads are under way.
+template <int N, int T, int XB>
+__device__ inline void mg_coarse_cycle(const CoarsePack& K, int lc, int D, const double* __restrict__ in, double* io,
+                                       int nio, const int* halt, CoarseShared<T>& sh) {
+    const int tid = threadIdx.x, st = K.stride;
+    double a[3 * N], w, q = 0.0, s = 0.0;
+    int po[(N + 1) / 2];  // pairs of LDS places
+    // uniform bases and one lane offset
+    auto value = [&](int k) { return (K.v + (long long)k * st)[(unsigned)tid]; };
+    auto word = [&](int m) { return (K.i + (long long)m * st)[(unsigned)tid]; };
+    constexpr int M = (N + 1) / 2;
+    const int myl = word(M + kCmLevel), child = word(M + kCmChild), sx = word(M + kCmSx), sy = word(M + kCmSy);
+    const int parent = word(M + kCmParent), shape = word(M + kCmShape);
+    w = value(3 * N);
+#pragma unroll
+    for (int k = 0; k < M; ++k) po[k] = word(k);
+#pragma unroll
+    for (int k = 0; k < 3 * N; ++k) a[k] = value(k);
+    auto children = [&](const double* R) {  // mg_restrict_row
+        double v[8], sum = 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const bool on = (k >> 2) < (shape & 3) && ((k >> 1) & 1) < ((shape >> 2) & 3) && (k & 1) < (shape >> 4);
+            v[k] = on ? R[(k >> 2) * sx + ((k >> 1) & 1) * sy + (k & 1) * 3] : 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sum += 1.0 * 1.0 * v[k];
+        return sum;
     };
-    auto sweep = [&](const Level& L, int row, bool update) {  // mg_residual(_update)_row
-        const double* So = lv_s(L, L.cur);
-        const double sum = f32 && L.A32 ? mg_row_sum<float>(L, L.A32, So, row) : mg_row_sum<double>(L, L.A, So, row);
-        double y = L.Q[row];
-        y *= 1.0;
-        y += sum;
-        L.R[row] = y;
-        if (update) {
-            double s = So[row];
-            s *= 1.0;
-            s += 1.0 * L.invD[row] * y;
-            lv_s(L, L.cur ^ 1)[row] = s;
+    if (myl == lc) q = lc == 0 ? in[tid] : children(in + child);
+    if (cr_halted(halt)) return;
+    auto row_sum = [&](const double* x) {  // mg_row_sum
+        // XB cells' LDS reads are under way while the XB before them are added
+        double sum = 0.0, xv[2][3 * XB];
+        auto read = [&](int k0, double* v) {
+#pragma unroll
+            for (int u = 0; u < XB; ++u)
+                if (k0 + u < N) {
+                    const int k = k0 + u;
+                    unsigned pl = po[k / 2];
+                    asm volatile("" : "+v"(pl));  // unpacked here, not kept in 27 registers over the sweeps
+                    const double* xc = x + (k & 1 ? pl >> 16 : pl & 0xffff);
+#pragma unroll
+                    for (int sd = 0; sd < 3; ++sd) v[3 * u + sd] = xc[sd];
+                }
+        };
+        read(0, xv[0]);
+#pragma unroll
+        for (int k0 = 0; k0 < N; k0 += XB) {
+            const int h = (k0 / XB) & 1;
+            if (k0 + XB < N) read(k0 + XB, xv[h ^ 1]);
+            // reads stay above, then the terms, then the adds: a term formed right before
+            // its add would put the multiply's latency into the chain
+            asm volatile("" : : : "memory");
+#pragma unroll
+            for (int u = 0; u < 3 * XB; ++u)
+                if (3 * k0 + u < 3 * N) {
+                    xv[h][u] = -1.0 * a[3 * k0 + u] * xv[h][u];
+                    asm volatile("" : "+v"(xv[h][u]));
+                }
+#pragma unroll
+            for (int u = 0; u < 3 * XB; ++u)
+                if (3 * k0 + u < 3 * N) sum += xv[h][u];
+            asm volatile("" : "+v"(sum) : : "memory");
+        }
+        return sum;
+    };
+    unsigned pc = 0;  // the S buffer of the own level
+    auto sweeps = [&](int l, int n) {  // n residual-update sweeps of level l
+        for (int k = 0; k < n; ++k) {
+            if (myl == l) {
+                double y = q;
+                y *= 1.0;
+                y += row_sum(sh.S[pc]);
+                s *= 1.0;
+                s += 1.0 * w * y;
+                pc ^= 1;
+                sh.S[pc][tid] = s;
+            }
+            __syncthreads();
         }
     };
-    auto ru = [&](int l) {
-        const Level L = lev(l);
-        for (int row = threadIdx.x; row < L.nrow; row += blockDim.x) sweep(L, row, true);
+    for (int l = lc; l < D; ++l) {
+        if (myl == l) {  // restriction, then begin and update
+            if (l > lc) {
+                int c = child;
+                asm volatile("" : "+v"(c));  // the places are formed here, not kept over the sweeps
+                q = children(sh.R + c);
+            }
+            s += 1.0 * w * q;
+            sh.S[0][tid] = s;
+        }
         __syncthreads();
-        cur ^= 1u << l;
-    };
-    auto restrict_into = [&](int l) {
-        const Level L = lev(l);
-        for (int row = threadIdx.x; row < L.nrow; row += blockDim.x) mg_restrict_row(lvs[l - 1], L, row);
-        __syncthreads();
-    };
-    auto begin_update = [&](int l) {
-        const Level L = lev(l);
-        for (int row = threadIdx.x; row < L.nrow; row += blockDim.x) mg_begin_update_row(L, row);
-        __syncthreads();
-    };
-    auto prolong_from = [&](int l) {  // l -> l-1
-        const Level L = lev(l), S = lev(l - 1);
-        for (int row = threadIdx.x; row < S.nrow; row += blockDim.x) mg_prolong_row(L, S, row);
-        __syncthreads();
-    };
-    for (int l = lc; l < D - 1; ++l) {
-        restrict_into(l);
-        begin_update(l);
-        ru(l);
-        ru(l);
-        const Level L = lev(l);
-        for (int row = threadIdx.x; row < L.nrow; row += blockDim.x) sweep(L, row, false);
-        __syncthreads();
+        sweeps(l, l == D - 1 ? 4 : l == 0 ? 1 : 2);
+        if (l < D - 1) {
+            if (myl == l) {
+                double y = q;
+                y *= 1.0;
+                y += row_sum(sh.S[pc]);
+                sh.R[tid] = y;
+            }
+            __syncthreads();
+        }
     }
-    {
-        const int c = D - 1;
-        restrict_into(c);
-        begin_update(c);
-        for (int k = 0; k < 4; ++k) ru(c);
-        prolong_from(c);
-    }
+    // a level's S ends in buffer 0 after four sweeps (the coarsest), in 1 after five (or
+    // three, level 0)
     for (int l = D - 2; l >= lc; --l) {
-        for (int k = 0; k < 3; ++k) ru(l);
-        prolong_from(l);
+        if (myl == l) {
+            double sum = 0.0;
+            sum += 1.0 * 1.0 * sh.S[l + 1 == D - 1 ? 0 : 1][parent];
+            s *= 1.0;
+            s += sum;
+            sh.S[pc][tid] = s;
+        }
+        __syncthreads();
+        sweeps(l, l == 0 ? 2 : 3);
+    }
+    if (lc == 0) {
+        if (myl == 0) io[tid] = s;
+    } else {
+        const double* x = sh.S[lc == D - 1 ? 0 : 1];
+        for (int r = tid; r < nio; r += st) {
+            double sum = 0.0;
+            sum += 1.0 * 1.0 * x[K.up[r]];
+            double y = io[r];
+            y *= 1.0;
+            y += sum;
+            io[r] = y;
+        }
     }
 }
 

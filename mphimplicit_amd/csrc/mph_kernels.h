@@ -46,6 +46,22 @@ struct Level {  // geometry + storage of one multigrid level
     const int* halt;  // the CR stop flag, as DevParams::halt
 };
 
+// The V-cycle's small levels, one thread per row, laid out for the one-workgroup cycle
+// (body::mg_coarse_cycle) by launch_mg_coarse_pack: a longest run of levels up to the
+// coarsest whose rows fit one workgroup.  A 3D row's stencil takes 162 registers of the
+// 256 that 512 threads have, a 2D row's 54 of 128.  Depth bounds the coarsest level to
+// three cells per axis, so it always fits.
+constexpr int kCoarseRows3D = 512, kCoarseRows2D = 1024;
+struct CoarsePack {
+    double* v;   // [(3 cells + 1)][stride]: stencil values, then invD
+    int* i;      // [(cells + 1) / 2 + 6][stride]: LDS places of the stencil cells, meta words
+    int* up;     // [rows of level lc-1]: the LDS place of each row's parent
+    int stride;  // threads (rows rounded up to whole wavefronts)
+    int cells;   // 27, or 9 in 2D
+};
+inline size_t coarse_pack_values(int cells, int stride) { return (size_t)(3 * cells + 1) * stride; }
+inline size_t coarse_pack_ints(int cells, int stride) { return (size_t)((cells + 1) / 2 + 6) * stride; }
+
 // levels with fewer rows than this split their sweeps' rows over lanes by default
 constexpr int kLaneRowsDefault = 32768;
 
@@ -128,10 +144,6 @@ constexpr int kRuns = 28;     // run starts per fluid particle: 27 neighbour cel
 constexpr int kBlkRuns = kRuns - 1, kBlkStride = 6;
 constexpr int kMaxP = 40;     // P-neighbours staged in LDS per particle by the C Lambda C^T kernel
 constexpr int kMaxLevels = 20;   // multigrid depth = floor(log2(cells per axis)) + 1
-// the V-cycle levels with at most this many rows may run in the one-workgroup
-// coarse cycle; the choice among these thresholds is autotuned (0: none)
-constexpr int kFuseVariants = 3;
-constexpr int kFuseRowsOf[kFuseVariants] = {0, 256, 2048};
 
 // ---- cells (calculateCellParticle) ----
 void launch_hash(hipStream_t st, const DevParams& P, const double* pos, const int* type, uint64_t* keys);
@@ -219,11 +231,12 @@ void launch_mg_residual(hipStream_t st, Level& L);     // R = Q - A S
 void launch_mg_residual_update(hipStream_t st, Level& L);  // R = Q - A S; S += invD R
 void launch_mg_restrict(hipStream_t st, const Level& S, Level& L);
 void launch_mg_prolong(hipStream_t st, const Level& L, Level& S);
-// levels lc..D-1 of the V-cycle in one workgroup; lvs = device copy of the levels,
-// cur = their ping-pong bits (bit l, lc-1 included).  Afterwards every level in
-// lc..D-2 has flipped (5 sweeps) and the coarsest has not (4 sweeps).  halt: the CR
-// stop flag (DevParams::halt), or null.
-void launch_mg_coarse(hipStream_t st, const Level* lvs, int lc, int D, unsigned cur, bool f32, const int* halt);
+// levels lc..D-1 of the V-cycle in one workgroup, from their packed rows.  S is level
+// lc-1 (its R is restricted, its current S takes the prolongation), or level 0 itself
+// when lc = 0 (Q0 in, S0 out, three sweeps).  f32: pack the FP32 stencils where a level
+// has one.  lvs: device copy of the levels.
+void launch_mg_coarse_pack(hipStream_t st, const Level* lvs, int lc, int D, bool f32, const CoarsePack& K);
+void launch_mg_coarse(hipStream_t st, const DevParams& P, const CoarsePack& K, int lc, int D, const Level& S);
 void launch_mg_g2p(hipStream_t st, const DevParams& P, const Level& L0, const int* cellIndex,
                    const double* invDiagA, const double* q, double* u, double* part);
 // ---- conjugate residual ----

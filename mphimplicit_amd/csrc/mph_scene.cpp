@@ -408,6 +408,7 @@ int phase_multiply_c(mph_scene& S) {
 // calculateMultiGridDepth (2804-2850) on the bbox read back with the neighbour totals
 int phase_multigrid(mph_scene& S) {
     if (!S.prm.multigrid) return MPH_OK;
+    const DevParams& P = S.P;
     const int* bb = S.hbbox;  // max x,y,z then min x,y,z
     double mgc = 0.0;
     if ((bb[0] - bb[3]) > mgc) mgc = (bb[0] - bb[3] + 1);
@@ -452,16 +453,22 @@ int phase_multigrid(mph_scene& S) {
             L.A32 = H.A32.p;
         }
     }
-    // the small levels may run in one workgroup (launch_mg_coarse): first fused level
-    // per row threshold
-    for (int v = 0; v < kFuseVariants; ++v) {
-        S.fuseOf[v] = depth;
-        for (int l = 1; l < depth; ++l)
-            if (S.lv[l].L.nrow <= kFuseRowsOf[v]) {
-                S.fuseOf[v] = l;
-                break;
-            }
-    }
+    // the small levels run in one workgroup (launch_mg_coarse): the longest run of levels
+    // up to the coarsest whose rows fit it.  One launch takes the place of four to eight
+    // per level, at about 4.7 us each.
+    const int most = P.dim == 2 ? kCoarseRows2D : kCoarseRows3D;
+    int rows = 0;
+    S.fuse = depth;
+    while (S.fuse > 0 && rows + S.lv[S.fuse - 1].L.nrow <= most) rows += S.lv[--S.fuse].L.nrow;
+    if (S.fuse == depth) return fail(MPH_E_STATE, "the coarsest multigrid level exceeds one workgroup");
+    CoarsePack& K = S.pack;
+    K.cells = P.dim == 2 ? 9 : 27;
+    K.stride = (rows + 63) / 64 * 64;
+    const size_t ni = coarse_pack_ints(K.cells, K.stride), nu = S.fuse > 0 ? S.lv[S.fuse - 1].L.nrow : 0;
+    if ((rc = S.packV.ensure(coarse_pack_values(K.cells, K.stride))) || (rc = S.packI.ensure(ni + nu))) return rc;
+    K.v = S.packV.p;
+    K.i = S.packI.p;
+    K.up = S.packI.p + ni;
     S.hlv.resize(depth);
     for (int l = 0; l < depth; ++l) S.hlv[l] = S.lv[l].L;
     if ((rc = S.lvDev.ensure(kMaxLevels))) return rc;
@@ -487,6 +494,7 @@ int phase_multigrid(mph_scene& S) {
     if (mixed(S))
         for (int l = 0; l + 1 < depth; ++l)
             launch_convert_f32(S.st, S.lv[l].L.A, S.lv[l].L.A32, (long long)S.lv[l].L.nrow * S.lv[l].L.nshift);
+    launch_mg_coarse_pack(S.st, S.lvDev.p, S.fuse, depth, mixed(S), S.pack);  // the mixed solve's V-cycles are FP32
     return MPH_OK;
 }
 
@@ -495,40 +503,31 @@ int phase_multigrid(mph_scene& S) {
 // the P2G forms the CR update q = beta q + pqy (4364-4366) as it reads q
 void precondition(mph_scene& S, const double* in, double* out, double* part, const double* pqy = nullptr) {
     hipStream_t st = S.st;
-    const int v = S.tuneFuse.pick();
-    const int D = S.depth, F = S.fuseOf[v];  // levels F..D-1 run fused (F = D: none)
-    S.tuneFuse.begin(st, v);
+    const int D = S.depth, F = S.fuse;  // levels F..D-1 run in one workgroup
     Level& L0 = S.lv[0].L;
     if (pqy) launch_mg_p2g_bu_pq(st, S.P, L0, S.cellStart.p, S.q.p, pqy, S.scal.p);
     else launch_mg_p2g_bu(st, S.P, L0, S.cellStart.p, in);  // P2G, S = 0, R = Q, S += invD R
-    launch_mg_residual_update(st, L0);                  // pre-smooth x2
-    launch_mg_residual(st, L0);
-    for (int l = 1; l < D - 1 && l < F; ++l) {
+    if (F > 0) {
+        launch_mg_residual_update(st, L0);  // pre-smooth x2
+        launch_mg_residual(st, L0);
+    }
+    for (int l = 1; l < F; ++l) {
         Level& L = S.lv[l].L;
         launch_mg_restrict_bu(st, S.lv[l - 1].L, L);  // pre-smooth x3
         launch_mg_residual_update(st, L);
         launch_mg_residual_update(st, L);
         launch_mg_residual(st, L);
     }
-    if (F < D) {
-        unsigned cur = 0;
-        for (int l = F - 1; l < D; ++l) cur |= (unsigned)S.lv[l].L.cur << l;
-        launch_mg_coarse(st, S.lvDev.p, F, D, cur, S.lv[0].L.f32 != 0, S.P.halt);
-        for (int l = F; l < D - 1; ++l) S.lv[l].L.cur ^= 1;  // five sweeps each; the coarsest four
-    } else {
-        Level& L = S.lv[D - 1].L;
-        launch_mg_restrict_bu(st, S.lv[D - 2].L, L);  // S = invD R, then four sweeps
-        for (int k = 0; k < 4; ++k) launch_mg_residual_update(st, L);
-        launch_mg_prolong(st, L, S.lv[D - 2].L);
-    }
-    for (int l = (D - 2 < F - 1 ? D - 2 : F - 1); l > 0; --l) {
+    launch_mg_coarse(st, S.P, S.pack, F, D, S.lv[F > 0 ? F - 1 : 0].L);
+    if (F == 0) L0.cur ^= 1;
+    for (int l = F - 1; l > 0; --l) {
         Level& L = S.lv[l].L;
         for (int k = 0; k < 3; ++k) launch_mg_residual_update(st, L);  // post-smooth x3
         launch_mg_prolong(st, L, S.lv[l - 1].L);
     }
-    for (int k = 0; k < 2; ++k) launch_mg_residual_update(st, L0);  // post-smooth x2
+    if (F > 0)
+        for (int k = 0; k < 2; ++k) launch_mg_residual_update(st, L0);  // post-smooth x2
     launch_mg_g2p(st, S.P, L0, S.cellIndex.p, S.invDiagA.p, in, out, part);
-    S.tuneFuse.end(st);
 }
 
 // without MULTIGRID_SOLVER the preconditioner is a copy (main.cpp:4331, 4341, 4369)
@@ -565,7 +564,6 @@ void collect_tuning(mph_scene& S) {  // the stream is idle
     S.tuneSpmv64.collect();
     S.tuneSpmv32.collect();
     S.tuneCac.collect();
-    S.tuneFuse.collect();
     S.tuneGal.collect();
 }
 
@@ -800,8 +798,7 @@ hipError_t capture_iteration(mph_scene& S, int k, long long maxit) {
 
 // the graphs hold fixed launches: no variant exploration or per-launch timing
 bool graphs_allowed(const mph_scene& S) {
-    return S.crStop >= 2 && !S.spmvTiming && (!S.prm.multigrid || !S.tuneFuse.exploring()) &&
-           (factored(S) || !S.tuneSpmv64.exploring());
+    return S.crStop >= 2 && !S.spmvTiming && (factored(S) || !S.tuneSpmv64.exploring());
 }
 
 // The FP64 CR loop with the stop test on the device.  The prologue's stop test has
@@ -843,7 +840,7 @@ int cr_loop_device(mph_scene& S, long long maxit) {
     }
     // the variant trials of the eager iterations are read as their iterations complete
     // (mark: how many trials each autotuner had recorded at an iteration's event)
-    Autotune* tn[] = {&S.tuneSpmv64, &S.tuneSpmv32, &S.tuneCac, &S.tuneFuse, &S.tuneGal};
+    Autotune* tn[] = {&S.tuneSpmv64, &S.tuneSpmv32, &S.tuneCac, &S.tuneGal};
     constexpr int kTn = sizeof(tn) / sizeof(tn[0]);
     size_t mark[2][kTn];
     for (int t = 0; t < kTn; ++t) mark[0][t] = tn[t]->pend.size();
@@ -1168,10 +1165,11 @@ void destroy(mph_scene* S) {
     }
     S->aval32.release();
     S->lvDev.release();
+    S->packV.release();
+    S->packI.release();
     S->tuneSpmv64.release();
     S->tuneSpmv32.release();
     S->tuneCac.release();
-    S->tuneFuse.release();
     S->tuneGal.release();
     if (S->hpin) (void)hipHostFree(S->hpin);
     if (S->hrr) (void)hipHostFree(S->hrr);
@@ -1477,7 +1475,6 @@ int mph_scene_create(const mph_params* p, const mph_grid* g, int device, mph_sce
     S->tuneSpmv64.init(kSpmvVariants64, 3);
     S->tuneSpmv32.init(kSpmvVariants32, 3);
     S->tuneCac.init(kCacVariants, 1);
-    S->tuneFuse.init(kFuseVariants, 3);
     S->tuneGal.init(kGalVariants, 1);
     S->outputNext = S->time;
     S->vtkOutputNext = S->time;
@@ -1630,7 +1627,7 @@ int mph_scene_scalar(mph_scene* S, const char* name, double* v) {
     else if (n == "TunedSpmv64") *v = S->tuneSpmv64.best;
     else if (n == "TunedSpmv32") *v = S->tuneSpmv32.best;
     else if (n == "TunedCac") *v = S->tuneCac.best;
-    else if (n == "TunedFuse") *v = S->tuneFuse.best;
+    else if (n == "TunedFuse") *v = 0;  // one variant: the levels that fit one workgroup are fused
     else if (n == "TunedGalerkin") *v = S->tuneGal.best;
     else if (n == "FactoredCellsUsed") *v = factored(*S) && fac_cells(*S) ? 1.0 : 0.0;
     else if (n == "FactoredBytes" || n == "FactoredBytesF32") {
@@ -1831,6 +1828,7 @@ int mph_scene_device_bytes(mph_scene* S, unsigned long long* bytes) {
         n += H.A32.cap * sizeof(float);
     }
     n += S->aval32.cap * sizeof(float);
+    n += S->packV.cap * sizeof(double) + S->packI.cap * sizeof(int);
     *bytes = n;
     return MPH_OK;
 }

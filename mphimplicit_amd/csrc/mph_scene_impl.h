@@ -201,7 +201,10 @@ struct mph_scene {
     int hbbox[6] = {0, 0, 0, 0, 0, 0};
     int depth = 0;
     int laneRowsMax = mph::kLaneRowsDefault;  // levels with fewer rows take the lane-split sweeps
-    int fuseOf[mph::kFuseVariants] = {0, 0, 0};  // first level of the one-workgroup coarse cycle
+    int fuse = 0;             // first level of the one-workgroup coarse cycle
+    mph::CoarsePack pack{};   // its rows
+    mph::host::DBuf<double> packV;
+    mph::host::DBuf<int> packI;
     std::vector<mph::host::HostLevel> lv;
     std::vector<mph::Level> hlv;           // level records as uploaded to lvDev
     mph::host::DBuf<mph::Level> lvDev;
@@ -258,8 +261,8 @@ struct mph_scene {
     long long spmvLaunches = 0, spmvLaunches32 = 0;
     int spmvTimingErr = 0;
     // run-time variant choice (SpMV load groups per precision, C Lambda C^T schedule,
-    // V-cycle levels fused into one workgroup)
-    mph::host::Autotune tuneSpmv64, tuneSpmv32, tuneCac, tuneFuse, tuneGal;
+    // level-0 Galerkin)
+    mph::host::Autotune tuneSpmv64, tuneSpmv32, tuneCac, tuneGal;
     int batches = 0;  // batches holding this scene (it cannot be destroyed meanwhile)
 };
 

@@ -415,11 +415,16 @@ __global__ void k_mg_prolong(Level L, Level S) {
     if (row < S.nrow) mg_prolong_row(L, S, row);
 }
 
-// cur: ping-pong bits of levels lc-1..D-1 (bit l), tracked by the host
-__global__ void __launch_bounds__(kCoarseThreads) k_mg_coarse(const Level* __restrict__ lvs, int lc, int D, unsigned cur,
-                                                   int f32, const int* halt) {
-    if (cr_halted(halt)) return;
-    mg_coarse_cycle(lvs, lc, D, cur, f32 != 0);
+// levels lc..D-1 in one workgroup (mg_coarse_cycle)
+template <int N, int T, int XB>
+__global__ void __launch_bounds__(T) k_mg_coarse(CoarsePack K, int lc, int D, const double* __restrict__ in, double* io,
+                                                 int nio, const int* halt) {
+    __shared__ CoarseShared<T> sh;
+    mg_coarse_cycle<N, T, XB>(K, lc, D, in, io, nio, halt, sh);
+}
+
+__global__ void k_mg_coarse_pack(const Level* __restrict__ lvs, int lc, int D, int f32, CoarsePack K) {
+    coarse_pack(lvs, lc, D, f32 != 0, K);
 }
 
 __global__ void __launch_bounds__(256) k_mg_g2p(DevParams P, Level L, const int* __restrict__ cellIndex,
@@ -794,8 +799,18 @@ void launch_mg_restrict(hipStream_t st, const Level& S, Level& L) {
 void launch_mg_prolong(hipStream_t st, const Level& L, Level& S) {
     hipLaunchKernelGGL(k_mg_prolong, dim3(nblk(S.nrow, 256)), dim3(256), 0, st, L, S);
 }
-void launch_mg_coarse(hipStream_t st, const Level* lvs, int lc, int D, unsigned cur, bool f32, const int* halt) {
-    hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(kCoarseThreads), 0, st, lvs, lc, D, cur, f32 ? 1 : 0, halt);
+void launch_mg_coarse_pack(hipStream_t st, const Level* lvs, int lc, int D, bool f32, const CoarsePack& K) {
+    hipLaunchKernelGGL(k_mg_coarse_pack, dim3(kCoarseRows2D / 64), dim3(64), 0, st, lvs, lc, D, f32 ? 1 : 0, K);
+}
+void launch_mg_coarse(hipStream_t st, const DevParams& P, const CoarsePack& K, int lc, int D, const Level& S) {
+    const double* in = lc == 0 ? S.Q : S.R;
+    double* io = S.S[lc == 0 ? S.cur ^ 1 : S.cur];
+#define MPH_COARSE(N, T, XB) \
+    hipLaunchKernelGGL((k_mg_coarse<N, T, XB>), dim3(1), dim3(K.stride), 0, st, K, lc, D, in, io, S.nrow, P.halt)
+    if (K.cells == 9) MPH_COARSE(9, kCoarseRows2D, 4);
+    else if (K.stride <= 256) MPH_COARSE(27, 256, 9);
+    else MPH_COARSE(27, kCoarseRows3D, 4);
+#undef MPH_COARSE
 }
 void launch_mg_g2p(hipStream_t st, const DevParams& P, const Level& L0, const int* cellIndex,
                    const double* invDiagA, const double* q, double* u, double* part) {
