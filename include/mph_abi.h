@@ -236,10 +236,8 @@ int mph_scene_set_timing(mph_scene* s, int on);
  *   "FactoredCells"     1: the FP64 factored product's second pass runs one
  *                  workgroup per cell with the visited cells' records staged in
  *                  LDS; 0: the chunk kernel, every neighbour gathered through the
- *                  caches; 2 (default): the cells in 3D scenes and in scenes of at
- *                  most 16384 fluid particles, the chunk kernel otherwise (larger 2D
- *                  scenes, whose cells hold too few rows for a workgroup).  Alone
- *                  and in a batch; the same bits either way.
+ *                  caches; 2 (default): the faster one, which is the cells wherever
+ *                  they can be staged.  Alone and in a batch; the same bits either way.
  *   "FactoredCellsXcd"  1 (default): the cells of that pass are dealt to the XCDs in
  *                  contiguous ranges; 0: round robin.
  *   "CrStop"       where the FP64 CR loop tests rr/rr0 < tol (main.cpp:4344-4346):

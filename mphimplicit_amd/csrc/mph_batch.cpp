@@ -45,6 +45,7 @@ struct mph_batch {
     Autotune tune64, tune32;  // SpMV load-group depth of the scene-table launches
     std::vector<char> fac;      // per scene of the current solve: factored operator
     std::vector<char> cell;     // ... and its FP64 second pass cell-staged
+    std::vector<char> shape;    // ... in this launch shape (kFacCell*)
     int* hctl = nullptr;      // [ns][kNCtl] coherent pinned mirrors of the scenes' CR control blocks
     size_t hctlCap = 0;
     hipEvent_t ev[2] = {nullptr, nullptr};  // the FP64 loop's last two iterations
@@ -95,6 +96,7 @@ int build_tables(mph_batch& B, const std::vector<mph_scene*>& sc, Tables& T, boo
     B.htab.assign(ns, BScene{});
     B.fac.assign(ns, 0);
     B.cell.assign(ns, 0);
+    B.shape.assign(ns, 0);
     B.hoff.assign((size_t)kOffRows * (ns + 1), 0);
     for (int s = 0; s < ns; ++s) {
         mph_scene& S = *sc[s];
@@ -143,7 +145,8 @@ int build_tables(mph_batch& B, const std::vector<mph_scene*>& sc, Tables& T, boo
         // the cell-staged FP64 pass: one workgroup per cell of the fluid bounding box
         const FacOp& F = b.fac[0];
         const long long cells = (long long)F.cellCnt[0] * F.cellCnt[1] * F.cellCnt[2];
-        B.cell[s] = b.factored && F.cellStart && cells > 0 ? 1 : 0;
+        B.cell[s] = b.factored && F.slot && cells > 0 ? 1 : 0;
+        B.shape[s] = (char)F.cellShape;
         put(kOffCell, B.cell[s] ? (int)cells : 0);
         put(kOffChunk, (S.P.nf + 255) / 256);
         put(kOffElem, (int)((3LL * S.P.nf + 255) / 256));
@@ -193,7 +196,7 @@ void bspmv(mph_batch& B, const Tables& T, const SceneSet& on, const SceneSet& fi
         spmv(T, onA, first, f32, alpha, x, beta, yin, y, y2, p_copy, dot, v);
         A.end(B.st);
     }
-    if (anyF) spmv_fac(T, onF, first, cells, f32, alpha, x, beta, yin, y, y2, p_copy, dot);
+    if (anyF) spmv_fac(T, onF, first, cells, B.shape.data(), f32, alpha, x, beta, yin, y, y2, p_copy, dot);
 }
 
 // the V-cycle of every scene in `on`, level by level; cur[s][l] is the ping-pong

@@ -97,8 +97,8 @@ void spmv(const Tables& T, const SceneSet& on, const SceneSet& first, bool f32, 
 // the same product for scenes of the factored form; `cells`: the scenes whose FP64
 // second pass is the cell-staged one (spmv_fac_cells), the others take the chunk
 // kernel
-void spmv_fac(const Tables& T, const SceneSet& on, const SceneSet& first, const SceneSet& cells, bool f32,
-              double alpha, int x, double beta, int yin, int y, int y2, int p_copy, int dot);
+void spmv_fac(const Tables& T, const SceneSet& on, const SceneSet& first, const SceneSet& cells, const char* shapes,
+              bool f32, double alpha, int x, double beta, int yin, int y, int y2, int p_copy, int dot);
 // the cell-staged second pass of the FP64 factored product (after the first pass)
 // for the scenes of `on`, with no dot partials (mph_factored.hip).  Its grid covers
 // the cells of the scenes in `on` only: pre[s] is the first workgroup of scene s
@@ -106,8 +106,9 @@ void spmv_fac(const Tables& T, const SceneSet& on, const SceneSet& first, const 
 struct CellRanges {
     int pre[kMaxScenes + 1];
 };
-void spmv_fac_cells(const Tables& T, const SceneSet& on, const SceneSet& first, double alpha, int x, double beta,
-                    int yin, int y, int y2, int p_copy);
+// One launch per shape (shapes[s]: FacOp::cellShape of scene s).
+void spmv_fac_cells(const Tables& T, const SceneSet& on, const char* shapes, const SceneSet& first, double alpha,
+                    int x, double beta, int yin, int y, int y2, int p_copy);
 void dot_partial(const Tables& T, const SceneSet& on, int a, int b);
 void dot_final(const Tables& T, const SceneSet& on, int slot, int shift_slot);
 // r.r and the stop test per scene, as launch_dot_final_stop (BScene::ctl, tol, maxit)

@@ -91,11 +91,11 @@ __global__ void __launch_bounds__(256) kb_fac_y(const BScene* tab, const int* of
     double* pc = f && p_copy >= 0 ? B.vec[p_copy] : nullptr;
     const double* dx = dot >= 0 ? B.vec[dot] : nullptr;
     double* pt = dot >= 0 ? B.part : nullptr;
-    if constexpr (sizeof(VT) == 4)
+    if constexpr (sizeof(VT) == 4) {
         fac_y32_chunk<kNeg>(B.P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, dx, pt, lb, sh, rows);
-    else if (*F.wrap)
-        fac_y_chunk<kNeg, VT, true>(B.P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, dx, pt, lb, sh, rows);
-    else fac_y_chunk<kNeg, VT, false>(B.P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, dx, pt, lb, sh, rows);
+    } else {
+        fac_y_chunk_any<kNeg>(B.P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, dx, pt, lb, sh, rows);
+    }
 }
 
 __global__ void __launch_bounds__(256) kb_dot_partial(const BScene* tab, const int* off, int ns, SceneSet on,
@@ -324,14 +324,14 @@ void spmv(const Tables& T, const SceneSet& on, const SceneSet& first, bool f32, 
     }
 #undef MPH_SPMV
 }
-void spmv_fac(const Tables& T, const SceneSet& all, const SceneSet& first, const SceneSet& cells, bool f32,
-              double alpha, int x, double beta, int yin, int y, int y2, int p_copy, int dot) {
+void spmv_fac(const Tables& T, const SceneSet& all, const SceneSet& first, const SceneSet& cells, const char* shapes,
+              bool f32, double alpha, int x, double beta, int yin, int y, int y2, int p_copy, int dot) {
     SceneSet on = all, staged{};
     for (int k = 0; k < kMaxScenes / 64; ++k) staged.w[k] = f32 ? 0 : all.w[k] & cells.w[k];
     if (f32) MPH_LAUNCH(kb_fac_t<float>, kOffPart, x);
     else MPH_LAUNCH(kb_fac_t<double>, kOffPart, x);
     if (any(staged)) {  // the cell-staged pass, then its dot partials
-        spmv_fac_cells(T, staged, first, alpha, x, beta, yin, y, y2, p_copy);
+        spmv_fac_cells(T, staged, shapes, first, alpha, x, beta, yin, y, y2, p_copy);
         on = staged;
         if (dot >= 0) MPH_LAUNCH(kb_dot_partial, kOffChunk, dot, y);
         on = all;

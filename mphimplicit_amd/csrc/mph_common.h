@@ -41,6 +41,10 @@ struct DevParams {
     double cofA[4], cofK;
     double ai[4];        // CofA[t]*CofK*CofK
     double visc;         // 10.0 (3D) or 8.0 (2D), main.cpp:2285-2287
+    // the factored product recomputes a pair's scalars from its distance d:
+    // alpha = facV (1/d - invV) / d^2 for fluid pairs of viscosity mu0, inside RadiusV;
+    // beta = facP (1/d - invP) inside RadiusP
+    double facV, facP, invV, invP, mu0;
     double gravity[3];
     double density[4], bulk[4], bulkVisc[4], shear[4];
     double ratio[4][4];  // InteractionRatio

@@ -787,13 +787,43 @@ __device__ inline FacEntry32 fac_entry32(const float* __restrict__ base, long lo
     return {v[0], v[1], v[2], __float_as_int(v[3])};
 }
 
-// lanes per particle in both passes, and the list entries each lane has in flight
-// per batch (viscous entries FP64 and FP32; P entries)
-constexpr int kFacLanes = 8, kFacBatch = 4, kFacBatch32 = 8, kFacBatchP = 4;
+// 1/sqrt(v), v >= 1e-200, by the hardware's estimate (about 2^-24) and one step of third
+// order: within 2 ulp
+__device__ inline double rsqrt_ref(double v) {
+    const double y = __builtin_amdgcn_rsq(v);
+    const double e = __builtin_fma(-(v * y), y, 1.0);
+    return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+}
+
+// one fluid-neighbour entry of the second pass: adds (beta t - alpha r.x) r for the
+// displacement r.  The scalars come from the distance, alpha = facV (1/d - invV)+ / d^2
+// and beta = facP (1/d - invP)+ (DevParams; (.)+ clamps at 0, so the radii need no
+// test); their constants are in the operands: x is -facV x, t is facP t.  At r = 0 (the
+// row's own entry, the padding of a list, a coincident particle) everything is 0.
+// kVar: fluid pairs of several viscosities, alpha is the stored a and x is plain.
+// Written in explicit fused operations: every kernel that forms it gets the same bits.
+template <bool kVar>
+__device__ inline void fac_pair(const DevParams& P, double r0, double r1, double r2, double x0, double x1, double x2,
+                                double t, double a, double& s0, double& s1, double& s2) {
+    const double d2 = __builtin_fmax(__builtin_fma(r2, r2, __builtin_fma(r1, r1, r0 * r0)), 1.0e-200);
+    const double y = rsqrt_ref(d2);
+    const double dot = __builtin_fma(r2, x2, __builtin_fma(r1, x1, r0 * x0));
+    double f;
+    if (kVar) f = -(a * dot);
+    else f = (__builtin_fmax(y - P.invV, 0.0) * (y * y)) * dot;
+    f = __builtin_fma(__builtin_fmax(y - P.invP, 0.0), t, f);
+    s0 = __builtin_fma(f, r0, s0);
+    s1 = __builtin_fma(f, r1, s1);
+    s2 = __builtin_fma(f, r2, s2);
+}
+
+// list entries each lane of a second-pass row has in flight per batch; the FP32 form's
+// lanes per particle in both passes and entries in flight (viscous and P entries)
+constexpr int kFacBatch = 4, kFacLanes32 = 8, kFacBatch32 = 8, kFacBatchP = 4;
 // the first pass (k's P list up to its last fluid entry, about 20 entries): lanes per
-// particle and entries in flight per lane (198 us against 200 us with 8 x 4 on the 1M
-// scene)
-constexpr int kFacLanesT = 4, kFacBatchT = 8;
+// particle and entries in flight per lane, at six waves per SIMD (132 us on the 1M
+// scene, 160 us before beta was recomputed; 8 in flight at their three waves 140 us)
+constexpr int kFacLanesT = 4, kFacBatchT = 4;
 
 // the four planes of FacOp::rec
 struct FacPlanes {
@@ -810,8 +840,8 @@ __device__ inline FacPlanes fac_planes(const DevParams& P, double* rec) {
 // first pass over the 256 particles of `chunk` (fluid or wall):
 //   t_k = lambda_k (C_kk . x_k [k fluid] - sum_{j fluid, j != k} beta_kj r_kj . x_j),
 // written to k's record together with x_k (fluid k).  Every thread calls it.
-// (Streaming a stored v = beta r instead of gathering positions measured slower:
-// as many load instructions, more bytes.)
+// beta is recomputed from the distance, as in fac_pair.  (Streaming a stored v = beta r
+// instead of gathering positions measured slower: as many load instructions, more bytes.)
 template <bool kWrap>
 __device__ inline void fac_t_chunk(const DevParams& P, const FacOp& F, const double* __restrict__ x, int chunk) {
 #pragma clang fp contract(fast)
@@ -827,19 +857,15 @@ __device__ inline void fac_t_chunk(const DevParams& P, const FacOp& F, const dou
             const long long c0 = F.nPtrP[k];
             for (int jb = 0; jb < run; jb += G * U) {
                 int jx[U];
-                double bb[U];
+                bool use[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     // entries past the end load the run's last entry (run >= 1), so the
                     // list loads need no branches and issue together
                     const int jn = jb + g + u * G;
-                    const long long e = c0 + (jn < run ? jn : run - 1);
-                    const int je = F.nIndP[e];
-                    const double be = F.beta[e];
-                    const int j = jn < run ? je : k;
-                    const bool use = jn < run && j < P.nf && j != k;
-                    jx[u] = use ? j : 0;  // unused entries read particle 0 with weight 0
-                    bb[u] = use ? be : 0.0;
+                    const int je = F.nIndP[c0 + (jn < run ? jn : run - 1)];
+                    use[u] = jn < run && je < P.nf && je != k;
+                    jx[u] = use[u] ? je : 0;  // unused entries read particle 0 with weight 0
                 }
                 double v[U][6];
 #pragma unroll
@@ -857,9 +883,12 @@ __device__ inline void fac_t_chunk(const DevParams& P, const FacOp& F, const dou
                     const double r0 = fac_wrap<kWrap>(v[u][0] - pk0, W0, h0);
                     const double r1 = fac_wrap<kWrap>(v[u][1] - pk1, W1, h1);
                     const double r2 = fac_wrap<kWrap>(v[u][2] - pk2, W2, h2);
-                    acc -= bb[u] * ((r0 * v[u][3] + r1 * v[u][4]) + r2 * v[u][5]);
+                    const double d2 = __builtin_fmax((r0 * r0 + r1 * r1) + r2 * r2, 1.0e-200);
+                    const double b = use[u] ? __builtin_fmax(rsqrt_ref(d2) - P.invP, 0.0) : 0.0;
+                    acc -= b * ((r0 * v[u][3] + r1 * v[u][4]) + r2 * v[u][5]);
                 }
             }
+            acc *= P.facP;
         }
         acc = group_sum(acc, G);
         if (g == 0 && k < P.np) {
@@ -876,95 +905,97 @@ __device__ inline void fac_t_chunk(const DevParams& P, const FacOp& F, const dou
     }
 }
 
-// second pass over the 256 fluid rows of `chunk`:
-//   y_i = D_i x_i + C_ii t_i - sum_j alpha_ij r_ij (r_ij . x_j) + sum_{k != i} beta_ik r_ik t_k,
-// the row sums staged in rows[3*256] (LDS), then the tail of spmv_store.  Every
-// thread calls it.
-template <bool kNeg, class VT, bool kWrap>
-__device__ inline void fac_y_chunk(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
-                                   const double* yin, double* y, double* y2, double* p_copy,
-                                   const double* __restrict__ dotx, double* __restrict__ part, int chunk,
-                                   double* sh, double* rows) {
-#pragma clang fp contract(fast)
+// the C Lambda C^T terms of row i's wall neighbours (the P entries after the fluid
+// ones), one entry per lane and round; adds to the lane's sums
+template <bool kWrap>
+__device__ inline void fac_walls(const DevParams& P, const FacOp& F, const double* __restrict__ rt, int i, int g,
+                                 double pi0, double pi1, double pi2, double& s0, double& s1, double& s2) {
+    const double W0 = P.W[0], W1 = P.W[1], W2 = P.W[2], h0 = P.hW[0], h1 = P.hW[1], h2 = P.hW[2];
+    const long long c0 = F.nPtrP[i];
+    const int n = F.nCountP[i];
+    for (int jn = F.runP[i] + g; jn < n; jn += kFacLanes) {
+        const int k = F.nIndP[c0 + jn];
+        const double f = F.beta[c0 + jn] * rt[k];
+        const double r0 = fac_wrap<kWrap>(F.pos[3 * (long long)k] - pi0, W0, h0);
+        const double r1 = fac_wrap<kWrap>(F.pos[3 * (long long)k + 1] - pi1, W1, h1);
+        const double r2 = fac_wrap<kWrap>(F.pos[3 * (long long)k + 2] - pi2, W2, h2);
+        s0 = __builtin_fma(f, r0, s0);
+        s1 = __builtin_fma(f, r1, s1);
+        s2 = __builtin_fma(f, r2, s2);
+    }
+}
+
+// row i's sum over its fluid neighbours with every record gathered through the caches
+// (the chunk kernel, and cells with more records than the staging holds): lane g takes
+// entries g, g + 8, ... in order, as the staged walk does
+template <bool kWrap, bool kVar>
+__device__ inline void fac_row_gather(const DevParams& P, const FacOp& F, int i, int g, double pi0, double pi1,
+                                      double pi2, double& s0, double& s1, double& s2) {
     typedef double dv2 __attribute__((ext_vector_type(2)));
-    constexpr int G = kFacLanes;
-    const int g = threadIdx.x & (G - 1);
+    constexpr int G = kFacLanes, U = kFacBatch;
     const FacPlanes R = fac_planes(P, F.rec);
     const dv2* __restrict__ ra = (const dv2*)R.a;
     const dv2* __restrict__ rb = (const dv2*)R.b;
     const dv2* __restrict__ rc = (const dv2*)R.c;
     const double* __restrict__ rt = R.t;
-    const VT* __restrict__ alpha = (const VT*)F.alpha;
+    const double* __restrict__ alpha = (const double*)F.alpha;
     const double W0 = P.W[0], W1 = P.W[1], W2 = P.W[2], h0 = P.hW[0], h1 = P.hW[1], h2 = P.hW[2];
+    const double sx = kVar ? 1.0 : -P.facV;
+    const long long b0 = F.nPtr[i];
+    const int w = F.nFluid[i];
+    for (int jb = 0; jb < w; jb += G * U) {
+        int j[U];
+        double a[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int jn = jb + g + u * G;
+            const long long e = b0 + (jn < w ? jn : w - 1);
+            j[u] = F.nInd[e];
+            a[u] = kVar ? alpha[e] : 0.0;
+            if (jn >= w) {  // past the list: the row's own record adds nothing
+                j[u] = i;
+                a[u] = 0.0;
+            }
+        }
+        dv2 q0[U], q1[U], q2[U];
+        double q3[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            q0[u] = ra[j[u]];
+            q1[u] = rb[j[u]];
+            q2[u] = rc[j[u]];
+            q3[u] = rt[j[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const double r0 = fac_wrap<kWrap>(q1[u][1] - pi0, W0, h0);
+            const double r1 = fac_wrap<kWrap>(q2[u][0] - pi1, W1, h1);
+            const double r2 = fac_wrap<kWrap>(q2[u][1] - pi2, W2, h2);
+            fac_pair<kVar>(P, r0, r1, r2, sx * q0[u][0], sx * q0[u][1], sx * q1[u][0], P.facP * q3[u], a[u], s0, s1,
+                           s2);
+        }
+    }
+}
+
+// second pass over the 256 fluid rows of `chunk`:
+//   y_i = D_i x_i + C_ii t_i - sum_j alpha_ij r_ij (r_ij . x_j) + sum_{k != i} beta_ik r_ik t_k,
+// the row sums staged in rows[3*256] (LDS), then the tail of spmv_store.  A fluid
+// neighbour's alpha and beta terms are added together (fac_pair).  Every thread calls it.
+template <bool kNeg, bool kWrap, bool kVar>
+__device__ inline void fac_y_chunk(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
+                                   const double* yin, double* y, double* y2, double* p_copy,
+                                   const double* __restrict__ dotx, double* __restrict__ part, int chunk,
+                                   double* sh, double* rows) {
+    constexpr int G = kFacLanes;
+    const int g = threadIdx.x & (G - 1);
+    const double* __restrict__ rt = fac_planes(P, F.rec).t;
     for (int r = threadIdx.x / G; r < 256; r += 256 / G) {
         const int i = chunk * 256 + r;
         double s0 = 0.0, s1 = 0.0, s2 = 0.0;
         if (i < P.nf) {
             const double pi0 = F.pos[3 * i], pi1 = F.pos[3 * i + 1], pi2 = F.pos[3 * i + 2];
-            // viscous part over the fluid neighbours (alpha 0: self, beyond RadiusV);
-            // unused entries of a batch read i's own record with weight 0
-            const long long b0 = F.nPtr[i];
-            const int w = F.nFluid[i];
-            for (int jb = 0; jb < w; jb += G * kFacBatch) {
-                constexpr int U = kFacBatch;
-                int j[U];
-                double a[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int jn = jb + g + u * G;
-                    j[u] = jn < w ? F.nInd[b0 + jn] : i;
-                    a[u] = jn < w ? (double)alpha[b0 + jn] : 0.0;
-                }
-                dv2 q0[U], q1[U], q2[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    q0[u] = ra[j[u]];
-                    q1[u] = rb[j[u]];
-                    q2[u] = rc[j[u]];
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const double r0 = fac_wrap<kWrap>(q1[u][1] - pi0, W0, h0);
-                    const double r1 = fac_wrap<kWrap>(q2[u][0] - pi1, W1, h1);
-                    const double r2 = fac_wrap<kWrap>(q2[u][1] - pi2, W2, h2);
-                    const double f = a[u] * ((r0 * q0[u][0] + r1 * q0[u][1]) + r2 * q1[u][0]);
-                    s0 -= f * r0;
-                    s1 -= f * r1;
-                    s2 -= f * r2;
-                }
-            }
-            // C Lambda C^T part over the P neighbours (beta 0: self)
-            const long long c0 = F.nPtrP[i];
-            const int n = F.nCountP[i];
-            for (int jb = 0; jb < n; jb += G * kFacBatchP) {
-                constexpr int U = kFacBatchP;
-                int k[U];
-                double bb[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int jn = jb + g + u * G;
-                    k[u] = jn < n ? F.nIndP[c0 + jn] : i;
-                    bb[u] = jn < n ? F.beta[c0 + jn] : 0.0;
-                }
-                dv2 q1[U], q2[U];
-                double q3[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    q1[u] = rb[k[u]];
-                    q2[u] = rc[k[u]];
-                    q3[u] = rt[k[u]];
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const double r0 = fac_wrap<kWrap>(q1[u][1] - pi0, W0, h0);
-                    const double r1 = fac_wrap<kWrap>(q2[u][0] - pi1, W1, h1);
-                    const double r2 = fac_wrap<kWrap>(q2[u][1] - pi2, W2, h2);
-                    const double f = bb[u] * q3[u];
-                    s0 += f * r0;
-                    s1 += f * r1;
-                    s2 += f * r2;
-                }
-            }
+            fac_row_gather<kWrap, kVar>(P, F, i, g, pi0, pi1, pi2, s0, s1, s2);
+            fac_walls<kWrap>(P, F, rt, i, g, pi0, pi1, pi2, s0, s1, s2);
         }
         s0 = group_sum(s0, G);
         s1 = group_sum(s1, G);
@@ -993,13 +1024,28 @@ __device__ inline void fac_y_chunk(const DevParams& P, const FacOp& F, const dou
     spmv_store(P.nf, i, r0, r1, r2, x, beta, yin, y, y2, p_copy, dotx, part, chunk, sh);
 }
 
+// the variant of fac_y_chunk that the scene's flags ask for (uniform)
+template <bool kNeg>
+__device__ inline void fac_y_chunk_any(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
+                                       const double* yin, double* y, double* y2, double* p_copy,
+                                       const double* __restrict__ dotx, double* __restrict__ part, int chunk,
+                                       double* sh, double* rows) {
+#define MPH_Y(WRAP, VAR) \
+    fac_y_chunk<kNeg, WRAP, VAR>(P, F, x, beta, yin, y, y2, p_copy, dotx, part, chunk, sh, rows)
+    const int wrap = F.wrap[0], var = F.wrap[1];
+    if (!wrap && !var) MPH_Y(false, false);
+    else if (!var) MPH_Y(true, false);
+    else MPH_Y(true, true);  // the wrapped displacement of a pair inside the domain is the plain one
+#undef MPH_Y
+}
+
 // FP32 form of the two passes (mixed-precision inner solves): the displacements are
 // folded into the stored vectors (v_kj = beta_kj r_kj, u_ij = sqrt(alpha_ij) r_ij),
 // so a pass gathers only a neighbour's 16-byte record (x, t as floats).  Arithmetic
 // is FP64 on the FP32-stored values.
 __device__ inline void fac_t32_chunk(const DevParams& P, const FacOp& F, const double* __restrict__ x, int chunk) {
 #pragma clang fp contract(fast)
-    constexpr int G = kFacLanes, U = kFacBatchP;
+    constexpr int G = kFacLanes32, U = kFacBatchP;
     typedef float fv4 __attribute__((ext_vector_type(4)));
     const int g = threadIdx.x & (G - 1);
     for (int r = threadIdx.x / G; r < 256; r += 256 / G) {
@@ -1058,7 +1104,7 @@ __device__ inline void fac_y32_chunk(const DevParams& P, const FacOp& F, const d
                                      double* sh, double* rows) {
 #pragma clang fp contract(fast)
     typedef float fv4 __attribute__((ext_vector_type(4)));
-    constexpr int G = kFacLanes, U = kFacBatch32;
+    constexpr int G = kFacLanes32, U = kFacBatch32;
     const int g = threadIdx.x & (G - 1);
     const fv4* __restrict__ rec = (const fv4*)F.rec32;
     // the viscous loop is software-pipelined: the columns and u of the next batch

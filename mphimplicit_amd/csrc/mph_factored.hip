@@ -22,17 +22,13 @@
 // because the RadiusP relation is symmetric up to rounding in the distance.
 //
 // The product is the assembled one up to rounding: the same terms, associated
-// differently.  It reads about 12 bytes per block (a 4-byte column and an 8-byte
-// alpha) where the assembled product reads 76.  A neighbour's x, position and t are
-// gathered through the caches from planes of 16-byte pairs (FacOp::rec): three
-// 16-byte loads per entry, where separate arrays would take six or four 8-byte
-// gathers.  Each row is walked by a group of 8 lanes, each with 4 entries in flight,
-// so that the gathers of one load instruction fall on consecutive particles of the
-// cell-ordered list, and so on consecutive pairs of a plane.  Measured on a jittered
-// 100^3 lattice (172 entries per row), every arrangement of this pass with 64-byte
-// records per particle (one lane per row, groups of 8 to 64 lanes, with or without
-// an XCD-aware block order) landed between 0.94 and 1.3 ms; the planes take it to
-// 0.90 ms.  The cache traffic of the gathers, not HBM, bounds it.
+// differently.  alpha and beta are functions of the distance alone where one viscosity
+// fills the scene (FacOp::wrap[1] = 0), so the FP64 passes recompute them from the
+// positions with a few fused operations (body::fac_pair) and read 2 to 4 bytes per
+// neighbour where the assembled product reads 76.  A neighbour's x, position and t come
+// from planes of 16-byte pairs (FacOp::rec), staged per cell in LDS or gathered through
+// the caches.  Each row is walked by a group of 8 lanes, so that the reads of one load
+// instruction fall on consecutive particles of the cell-ordered list.
 //
 // Scenes whose multigrid levels allow it assemble no 3x3 blocks at all: level 0
 // and InvDiagA come from the same scalars (k_fac_g, k_fac_gal0, k_fac_invdiag).
@@ -480,7 +476,7 @@ __global__ void __launch_bounds__(256) k_fac_invdiag(DevParams P, FacOp F, doubl
 // the wrap flag is uniform, so the branch is taken by the whole launch; the FP32
 // form has no displacements to wrap
 template <class VT>
-__global__ void __launch_bounds__(256) k_fac_t(DevParams P, FacOp F, const double* __restrict__ x) {
+__global__ void __launch_bounds__(256, 6) k_fac_t(DevParams P, FacOp F, const double* __restrict__ x) {
     if (cr_halted(P.halt)) return;
     if constexpr (sizeof(VT) == 4) body::fac_t32_chunk(P, F, x, blockIdx.x);
     else if (*F.wrap) body::fac_t_chunk<true>(P, F, x, blockIdx.x);
@@ -494,28 +490,50 @@ __global__ void __launch_bounds__(256) k_fac_y(DevParams P, FacOp F, const doubl
     if (cr_halted(P.halt)) return;
     __shared__ double sh[256];
     __shared__ double rows[3 * 256];
-    if constexpr (sizeof(VT) == 4)
+    if constexpr (sizeof(VT) == 4) {
         body::fac_y32_chunk<kNeg>(P, F, x, beta, yin, y, y2, p_copy, dotx, part, blockIdx.x, sh, rows);
-    else if (*F.wrap)
-        body::fac_y_chunk<kNeg, VT, true>(P, F, x, beta, yin, y, y2, p_copy, dotx, part, blockIdx.x, sh, rows);
-    else body::fac_y_chunk<kNeg, VT, false>(P, F, x, beta, yin, y, y2, p_copy, dotx, part, blockIdx.x, sh, rows);
+    } else {
+        body::fac_y_chunk_any<kNeg>(P, F, x, beta, yin, y, y2, p_copy, dotx, part, blockIdx.x, sh, rows);
+    }
 }
 
 // ---------------------------------------------------------------------------
-// The FP64 second pass with the viscous gathers from LDS.
+// The FP64 second pass with its gathers from LDS.
 //
 // Every row of one cell visits the same 27 (9 in 2D) cells, so one workgroup per row
-// cell stages the records (x and position) of the fluid particles of those cells in
-// LDS once, and its rows read their fluid neighbours' records from there instead of
+// cell stages the records (x, position, t) of the fluid particles of those cells in LDS
+// once, and its rows read their fluid neighbours' records from there instead of
 // gathering them through L1 and L2 per entry (each gather instruction of the chunk
-// kernel touched about 21 cache lines).  The P part (about a tenth of the entries,
-// walls included) keeps the global gathers.  A row's entries, lanes and order of
-// summation are those of body::fac_y_chunk, so the results are the chunk kernel's.
-// The rows go straight to y; the dot partials of the fused epilogue come from a
-// dot-partial launch afterwards (the chunks of 256 rows do not follow cells).
-constexpr int kCellThreads = 512;  // 64 rows of kFacLanes lanes per pass
-constexpr int kCellSlots = 1536;   // staged records of 48 B: 72 KiB, two workgroups per CU
+// kernel touched about 21 cache lines).  An entry is a 2-byte place; alpha and beta are
+// recomputed from the distance (body::fac_pair), and as the RadiusP neighbours are among
+// the fluid neighbours, one walk forms both terms.  On the 1M-particle scene the pass
+// takes 428 us; it took 726 us when it streamed alpha beside the places and walked the P
+// lists on their own (10 bytes per entry at 4.3 TB/s, a dependent round of list loads
+// per 32 entries, and the P part's gathers).  The VALU issues 61% of the time, the rest
+// is a workgroup's waits for its loads at two workgroups per CU.
+// A row's entries, lanes and order of summation are those of body::fac_row_gather, so
+// the results are the chunk kernel's.  The rows go straight to y; the dot partials of
+// the fused epilogue come from a dot-partial launch afterwards (the chunks of 256 rows
+// do not follow cells).
+//
+// Everything a workgroup needs of its cell is in a descriptor built once per step
+// (k_fac_slots), so it waits for two rounds of loads before it computes: the
+// descriptor, then the staged records, the first places and the rows' diagonal terms
+// together.
 constexpr int kCellTable = 32;     // visited cells (27 in 3D) padded for the binary search
+
+// words of FacOp::cellDesc, per cell of the fluid bounding box
+enum {
+    kFdRow = 0,     // first fluid row
+    kFdRows = 1,    // rows (0: nothing to do)
+    kFdTotal = 2,   // staged records; -1: more than the staging holds
+    kFdBatches = 3, // batches of 4 entries per lane of the longest row
+    kFdOwn = 4,     // place of the first row's own record
+    kFdWalls = 5,   // some row has wall neighbours within RadiusP
+    kFdPieces = 6,  // pieces of up to 64 consecutive particles; (first place | count << 16, first particle) of each
+    kFdPiece0 = 8
+};
+static_assert(kFdPiece0 + 2 * (27 + kFacCellSlots[kFacCell3DWide] / 64) <= kFacDesc, "the pieces fit the descriptor");
 
 // element k of y (and y2) from the row's sum sm, as spmv_store: the separate
 // roundings of y = beta*yin + sum (this function is compiled without contraction);
@@ -535,44 +553,27 @@ __device__ inline void fac_cell_store1(int k, double sm, double yv, double y2v, 
 
 typedef double dv2c __attribute__((ext_vector_type(2)));
 
-// the visited cells of a row cell: fluid ranges in visiting order and LDS offsets
-struct FacCellTable {
-    int vlo[kCellTable], voff[kCellTable], vcnt[kCellTable];
-    int vex[kCellTable];  // first staged place of each visited cell (past the last: INT_MAX)
-    int total;            // staged records of the visited cells
-};
-struct FacCellShared {  // the product's LDS: the table and the records
-    FacCellTable tab;
-    dv2c rec[3 * kCellSlots];
-};
+// the cell of bounding-box index b (z fastest)
+__device__ inline void fac_cell_xyz(const FacOp& F, int b, int& cx, int& cy, int& cz) {
+    cz = F.cellLo[2] + b % F.cellCnt[2];
+    cy = F.cellLo[1] + (b / F.cellCnt[2]) % F.cellCnt[1];
+    cx = F.cellLo[0] + b / (F.cellCnt[2] * F.cellCnt[1]);
+}
 
-// Workgroup b's row cell (b counts the scene's workgroups of the launch; cell
-// (x, y, z) of the fluid bounding box, z fastest): its
-// fluid rows [rs, rs + nrows) and, in T, the visited cells in the neighbour search's
-// order (ascending CellId, so their fluid ranges ascend too) with their LDS offsets,
-// filled by wavefront 0.  False (for the whole workgroup) if the cell has no fluid.
-// Ends with a workgroup barrier when it returns true.
-__device__ inline bool fac_cell_table(const DevParams& P, const FacOp& F, FacCellTable& T, int& rs, int& nrows,
-                                      int& nv, int b) {
+// FacOp::cellDesc and the places of every row of bounding-box cell blockIdx.x
+__global__ void __launch_bounds__(256) k_fac_slots(DevParams P, FacOp F, int cap) {
+    __shared__ int vlo[kCellTable], voff[kCellTable], vex[kCellTable], total, most, walls;
     const int t = threadIdx.x;
-    if (F.cellXcd) {
-        // workgroups are dealt to the 8 XCDs in turn: XCD x = b mod 8 takes a contiguous
-        // range of cells instead, so that the cells running on one XCD at a time are
-        // neighbours and share their visited cells' records in that XCD's L2
-        const int nb = F.cellCnt[0] * F.cellCnt[1] * F.cellCnt[2], per = nb / 8, rem = nb % 8, x = b % 8;
-        b = x * per + (x < rem ? x : rem) + b / 8;
-    }
+    int cx, cy, cz;
+    fac_cell_xyz(F, blockIdx.x, cx, cy, cz);
+    int* const D = F.cellDesc + (long long)kFacDesc * blockIdx.x;
     const int* C = P.C;
-    const int cz = F.cellLo[2] + b % F.cellCnt[2];
-    const int cy = F.cellLo[1] + (b / F.cellCnt[2]) % F.cellCnt[1];
-    const int cx = F.cellLo[0] + b / (F.cellCnt[2] * F.cellCnt[1]);
     const int c = (cx * C[1] + cy) * C[2] + cz;
-    rs = F.cellStart[c];
-    nrows = F.cellStart[c + 1] - rs;
-    if (nrows <= 0) return false;
-    const int nx = 2 * P.range[0] + 1, ny = 2 * P.range[1] + 1, nz = 2 * P.range[2] + 1;
-    nv = nx * ny * nz;
-    if (t < 64) {
+    const int rs = F.cellStart[c], nrows = F.cellStart[c + 1] - rs;
+    if (t == 0) D[kFdRows] = nrows;
+    if (nrows <= 0) return;
+    const int nx = 2 * P.range[0] + 1, ny = 2 * P.range[1] + 1, nz = 2 * P.range[2] + 1, nv = nx * ny * nz;
+    if (t < 64) {  // the visited cells in the neighbour search's order (ascending CellId)
         int lo = 0x7fffffff, cnt = 0;
         if (t < nv) {
             const int bx = 2 * P.range[0] - (cx + P.range[0]) % C[0];
@@ -593,182 +594,185 @@ __device__ inline bool fac_cell_table(const DevParams& P, const FacOp& F, FacCel
             if (t >= d) incl += u;
         }
         if (t < kCellTable) {
-            T.vlo[t] = lo;
-            T.vcnt[t] = cnt;
-            T.voff[t] = (incl - cnt) - (t < nv ? lo : 0);
-            T.vex[t] = t < nv ? incl - cnt : 0x7fffffff;
+            vlo[t] = lo;
+            voff[t] = (incl - cnt) - (t < nv ? lo : 0);
+            vex[t] = t < nv ? incl - cnt : 0x7fffffff;
         }
-        if (t == 63) T.total = incl;
+        if (t == 63) {
+            total = incl;
+            most = 0;
+            walls = 0;
+        }
     }
     __syncthreads();
-    return true;
-}
-
-// the staged place of fluid particle j: j + voff of the last visited range starting at
-// or before j
-__device__ inline int fac_cell_slot(const FacCellTable& T, int j) {
-    int v = 0;
+    // the place of fluid particle j: j + voff of the last visited range starting at or
+    // before j
+    auto place = [&](int j) {
+        int v = 0;
 #pragma unroll
-    for (int step = kCellTable / 2; step >= 1; step >>= 1)
-        if (T.vlo[v + step] <= j) v += step;
-    return j + T.voff[v];
-}
-
-// FacOp::slot of every fluid-neighbour entry of the fluid rows of cells whose visited
-// cells fit the staging (the product gathers the others' records from global memory)
-__global__ void __launch_bounds__(kCellThreads) k_fac_slots(DevParams P, FacOp F) {
-    __shared__ FacCellTable T;
-    int rs, nrows, nv;
-    if (!fac_cell_table(P, F, T, rs, nrows, nv, blockIdx.x)) return;
-    if (T.total > kCellSlots) return;
-    constexpr int G = body::kFacLanes, U = 4;  // U entries per lane in flight
-    for (int r = threadIdx.x / G; r < nrows; r += kCellThreads / G) {
+        for (int step = kCellTable / 2; step >= 1; step >>= 1)
+            if (vlo[v + step] <= j) v += step;
+        return j + voff[v];
+    };
+    for (int r = t; r < nrows; r += 256) {
+        atomicMax(&most, F.nFluid[rs + r]);
+        if (F.nCountP[rs + r] > F.runP[rs + r]) atomicOr(&walls, 1);
+    }
+    __syncthreads();
+    constexpr int G = kFacLanes;
+    const int nb = (most + 4 * G - 1) / (4 * G);
+    if (t == 0) {
+        D[kFdRow] = rs;
+        D[kFdTotal] = total <= cap ? total : -1;
+        D[kFdBatches] = nb;
+        D[kFdOwn] = place(rs);
+        D[kFdWalls] = walls;
+        int m = 0;
+        for (int v = 0; v < nv && total <= cap;) {  // cells with consecutive particles share pieces
+            const int p0 = vex[v], j0 = vlo[v];
+            int p1 = p0;
+            do {
+                p1 = v + 1 < nv ? vex[v + 1] : total;
+                ++v;
+            } while (v < nv && vlo[v] == j0 + (p1 - p0));
+            for (int p = p0; p < p1; p += 64, ++m) {
+                D[kFdPiece0 + 2 * m] = p | (p1 - p < 64 ? p1 - p : 64) << 16;
+                D[kFdPiece0 + 2 * m + 1] = j0 + (p - p0);
+            }
+        }
+        D[kFdPieces] = m;
+    }
+    if (total > cap) return;  // that cell's rows gather from global memory
+    // 32 lanes write a row's places, two each
+    for (int r = t / 32; r < nrows; r += 8) {
         const int i = rs + r;
         const long long b0 = F.nPtr[i];
         const int w = F.nFluid[i];
-        for (int jb = threadIdx.x & (G - 1); jb < w; jb += G * U) {
-            int j[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) j[u] = jb + u * G < w ? F.nInd[b0 + jb + u * G] : 0;
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (jb + u * G < w) F.slot[b0 + jb + u * G] = (unsigned short)fac_cell_slot(T, j[u]);
+        unsigned* const sl = (unsigned*)(F.slot + (long long)i * F.slotRow);
+        const int own = place(i);
+        for (int q = 2 * (t & 31); q < 8 * G * ((nb + 1) / 2); q += 64) {
+            // places q and q + 1 of block q / 8G: lane (q / 8) mod G, entries q mod 8 and the next
+            const int e = q / (8 * G) * (8 * G) + (q & 7) * G + (q >> 3) % G;
+            const int a = e < w ? place(F.nInd[b0 + e]) : own, b = e + G < w ? place(F.nInd[b0 + e + G]) : own;
+            sl[q / 2] = (unsigned)a | (unsigned)b << 16;
         }
     }
 }
 
-// the viscous list entries of a batch: lane g takes entries jb + g + u*G (u < U).
-// kSlot: the staged places (FacOp::slot), else the columns.  Entries past the row's
-// end take i's own record (own) with weight 0; their loads read the row's last entry
-// (w >= 1), so that the loads need no branches and issue together
-template <int U, bool kSlot>
-__device__ inline void fac_cell_list(const FacOp& F, const double* __restrict__ alpha, long long b0, int w, int own,
-                                     int jb, int g, int* j, double* a) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int jn = jb + g + u * body::kFacLanes;
-        const long long e = b0 + (jn < w ? jn : w - 1);
-        const int jj = kSlot ? (int)F.slot[e] : F.nInd[e];
-        const double aa = alpha[e];
-        j[u] = jn < w ? jj : own;
-        a[u] = jn < w ? aa : 0.0;
-    }
-}
-
-// the P-list entries of a batch (branch-free loads as fac_cell_list; n >= 1: self):
-// lane g takes entries jb + g + u*G; entries past the list take i with weight 0
-template <int UP>
-__device__ inline void fac_cell_plist(const FacOp& F, long long c0, int n, int i, int jb, int g, int* k, double* bb) {
-#pragma unroll
-    for (int u = 0; u < UP; ++u) {
-        const int jn = jb + g + u * body::kFacLanes;
-        const long long e = c0 + (jn < n ? jn : n - 1);
-        const int kk = F.nIndP[e];
-        const double be = F.beta[e];
-        k[u] = jn < n ? kk : i;
-        bb[u] = jn < n ? be : 0.0;
-    }
-}
-
-// what a row's walk starts from: its position, list extents and staged place (the
-// loads that only depend on the row)
-struct FacRowHead {
-    double pi0, pi1, pi2;
-    long long b0, c0;
-    int w, n, own;
+// the staged records in four planes: t (facP t), x0 x1, x2 p0, p1 p2 (x scaled as
+// body::fac_pair takes it)
+template <int kCap>
+struct FacCellShared {
+    double t[kCap];
+    dv2c a[kCap], b[kCap], c[kCap];
 };
 
-template <bool kSlot>
-__device__ inline void fac_cell_row_head(const FacOp& F, const FacCellTable& T, int i, FacRowHead& S) {
-    S.pi0 = F.pos[3 * i];
-    S.pi1 = F.pos[3 * i + 1];
-    S.pi2 = F.pos[3 * i + 2];
-    S.b0 = F.nPtr[i];
-    S.w = F.nFluid[i];
-    S.c0 = F.nPtrP[i];
-    S.n = F.nCountP[i];
-    S.own = kSlot ? fac_cell_slot(T, i) : i;
+// one batch of a row's walk: the four entries whose places are in w0, w1
+template <bool kWrap, bool kVar, int kCap>
+__device__ inline void fac_cell_batch(const DevParams& P, const FacCellShared<kCap>& L, unsigned w0, unsigned w1,
+                                      const double* al, double pi0, double pi1, double pi2, double& s0, double& s1,
+                                      double& s2) {
+    const unsigned sl[4] = {w0 & 0xffffu, w0 >> 16, w1 & 0xffffu, w1 >> 16};
+    dv2c q0[4], q1[4], q2[4];
+    double q3[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        q0[u] = L.a[sl[u]];
+        q1[u] = L.b[sl[u]];
+        q2[u] = L.c[sl[u]];
+        q3[u] = L.t[sl[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const double r0 = body::fac_wrap<kWrap>(q1[u][1] - pi0, P.W[0], P.hW[0]);
+        const double r1 = body::fac_wrap<kWrap>(q2[u][0] - pi1, P.W[1], P.hW[1]);
+        const double r2 = body::fac_wrap<kWrap>(q2[u][1] - pi2, P.W[2], P.hW[2]);
+        body::fac_pair<kVar>(P, r0, r1, r2, q0[u][0], q0[u][1], q1[u][0], q3[u], kVar ? al[u] : 0.0, s0, s1, s2);
+    }
 }
 
-// The rows of one cell.  kStaged: the fluid records of the visited cells are in LDS
-// (L.rec), read through the precomputed places (FacOp::slot) if kSlot, else through
-// a search of the table; otherwise every record is gathered from global memory.
-// None of this changes which lane takes an entry or the order in which a lane adds
-// its terms.  (Loading the next batch's list entries before the current batch's
-// records, or 8 entries per batch instead of 4, measured slower: 151.7 and 169.8
-// against 125.9 ms per step on the 1M scene; loading them after the records, into a
-// second buffer, changed the product by 0.3%; loading the first row's start before
-// the staging took 14 more registers and, held to four waves per SIMD, spilled:
-// 1.41 against 0.93 ms per product.)
-template <bool kNeg, bool kWrap, bool kStaged, bool kSlot>
-__device__ inline void fac_y_cell_rows(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
+// workgroup b of the pass over scene (P, F); kThreads, kCap: kFacCell* of F.cellShape
+template <bool kNeg, bool kWrap, bool kVar, int kThreads, int kCap>
+__device__ inline void fac_y_cell_body(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
                                        const double* yin, double* y, double* y2, double* p_copy,
-                                       const FacCellShared& L, int rs, int nrows) {
-#pragma clang fp contract(fast)
-    typedef double dv2 __attribute__((ext_vector_type(2)));
-    constexpr int G = body::kFacLanes, U = body::kFacBatch, UP = body::kFacBatchP;
-    const int t = threadIdx.x;
+                                       FacCellShared<kCap>& L, int b) {
+    constexpr int G = kFacLanes, kRows = kThreads / G;
+    if (F.cellXcd) {
+        // workgroups are dealt to the 8 XCDs in turn: XCD x = b mod 8 takes a contiguous
+        // range of cells instead, so that the cells running on one XCD at a time are
+        // neighbours and share their visited cells' records in that XCD's L2
+        const int nb = F.cellCnt[0] * F.cellCnt[1] * F.cellCnt[2], per = nb / 8, rem = nb % 8, xc = b % 8;
+        b = xc * per + (xc < rem ? xc : rem) + b / 8;
+    }
+    const int* __restrict__ D = F.cellDesc + (long long)kFacDesc * b;
+    const int rs = D[kFdRow], nrows = D[kFdRows], total = D[kFdTotal], nb = D[kFdBatches], own = D[kFdOwn];
+    const int walls = D[kFdWalls], m = D[kFdPieces];
+    if (nrows <= 0) return;  // the whole workgroup
+    const int t = threadIdx.x, g = t & (G - 1);
     const body::FacPlanes R = body::fac_planes(P, F.rec);
-    const dv2* __restrict__ ra = (const dv2*)R.a;
-    const dv2* __restrict__ rb = (const dv2*)R.b;
-    const dv2* __restrict__ rc = (const dv2*)R.c;
     const double* __restrict__ rt = R.t;
-    const double* __restrict__ alpha = (const double*)F.alpha;
-    const double W0 = P.W[0], W1 = P.W[1], W2 = P.W[2], h0 = P.hW[0], h1 = P.hW[1], h2 = P.hW[2];
-    const int g = t & (G - 1);
-    const int passes = (nrows + kCellThreads / G - 1) / (kCellThreads / G);
+    const unsigned short* __restrict__ slot = F.slot;
+    const long long srow = F.slotRow;
+    auto places = [&](int i, int blk) {  // the lane's 8 entries of block blk of row i
+        return *(const uint4*)(slot + (long long)i * srow + 8 * G * blk + 8 * g);
+    };
+    uint4 pl = {0, 0, 0, 0};
+    const bool staged = total >= 0;
+    if (staged) {
+        if (t / G < nrows) pl = places(rs + t / G, 0);
+        // wavefront w stages pieces w, w + kWaves, ...: uniform bases, the records of a
+        // piece consecutive, and every load of a round of pieces issued before the first
+        // store
+        const dv2c* __restrict__ ra = (const dv2c*)R.a;
+        const dv2c* __restrict__ rb = (const dv2c*)R.b;
+        const dv2c* __restrict__ rc = (const dv2c*)R.c;
+        constexpr int kWaves = kThreads / 64, K = 3;
+        const int lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t / 64);
+        const double sx = kVar ? 1.0 : -P.facV;
+        for (int k0 = wv; k0 < m; k0 += kWaves * K) {
+            dv2c qa[K], qb[K], qc[K];
+            double qt[K];
+            int p0[K], n[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const int pc = k0 + k * kWaves;
+                const int h = pc < m ? D[kFdPiece0 + 2 * pc] : 0, j0 = pc < m ? D[kFdPiece0 + 2 * pc + 1] : 0;
+                p0[k] = h & 0xffff;
+                n[k] = h >> 16;
+                if (lane < n[k]) {
+                    qa[k] = (ra + j0)[(unsigned)lane];
+                    qb[k] = (rb + j0)[(unsigned)lane];
+                    qc[k] = (rc + j0)[(unsigned)lane];
+                    qt[k] = (rt + j0)[(unsigned)lane];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (lane < n[k]) {
+                    const int r = p0[k] + lane;
+                    L.a[r] = dv2c{sx * qa[k][0], sx * qa[k][1]};
+                    L.b[r] = dv2c{sx * qb[k][0], qb[k][1]};
+                    L.c[r] = qc[k];
+                    L.t[r] = P.facP * qt[k];
+                }
+        }
+        __syncthreads();
+    }
+    const int passes = (nrows + kRows - 1) / kRows;
     for (int ps = 0; ps < passes; ++ps) {  // uniform trip count: every lane reaches the group sums
-        const int r = ps * (kCellThreads / G) + t / G;
+        const int r = ps * kRows + t / G;
         const bool on = r < nrows;
         const int i = rs + (on ? r : 0);
         double s0 = 0.0, s1 = 0.0, s2 = 0.0;
         double dA = 0.0, dB = 0.0, dC = 0.0, xi0 = 0.0, xi1 = 0.0, xi2 = 0.0, ti = 0.0, sc = 0.0, yv = 0.0, y2v = 0.0;
         if (on) {
-            // the row's start; the first P batch stays in flight during the viscous part
-            FacRowHead S;
-            fac_cell_row_head<kStaged && kSlot>(F, L.tab, i, S);
-            const double pi0 = S.pi0, pi1 = S.pi1, pi2 = S.pi2;
-            const long long b0 = S.b0, c0 = S.c0;
-            const int w = S.w, n = S.n, own = S.own;
-            int j[U], k[UP];
-            double a[U], bb[UP];
-            fac_cell_list<U, kStaged && kSlot>(F, alpha, b0, w, own, 0, g, j, a);
-            fac_cell_plist<UP>(F, c0, n, i, 0, g, k, bb);
-            // viscous part over the fluid neighbours (alpha 0: self, beyond RadiusV)
-            for (int jb = 0; jb < w; jb += G * U) {
-                dv2 q0[U], q1[U], q2[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    if (kStaged) {
-                        const int sl = kSlot ? j[u] : fac_cell_slot(L.tab, j[u]);
-                        q0[u] = L.rec[3 * sl];
-                        q1[u] = L.rec[3 * sl + 1];
-                        q2[u] = L.rec[3 * sl + 2];
-                    } else {
-                        q0[u] = ra[j[u]];
-                        q1[u] = rb[j[u]];
-                        q2[u] = rc[j[u]];
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const double r0 = body::fac_wrap<kWrap>(q1[u][1] - pi0, W0, h0);
-                    const double r1 = body::fac_wrap<kWrap>(q2[u][0] - pi1, W1, h1);
-                    const double r2 = body::fac_wrap<kWrap>(q2[u][1] - pi2, W2, h2);
-                    const double f = a[u] * ((r0 * q0[u][0] + r1 * q0[u][1]) + r2 * q1[u][0]);
-                    s0 -= f * r0;
-                    s1 -= f * r1;
-                    s2 -= f * r2;
-                }
-                if (jb + G * U < w) fac_cell_list<U, kStaged && kSlot>(F, alpha, b0, w, own, jb + G * U, g, j, a);
-            }
             // lanes 0..2 of the row: the loads of their component of the diagonal term
-            // and of y, in flight during the P part
+            // and of y, in flight during the walk
             if (g < 3) {
-                const double* D = F.diag + 9 * i + 3 * g;
-                dA = D[0];
-                dB = D[1];
-                dC = D[2];
+                const double* Dg = F.diag + 9 * i + 3 * g;
+                dA = Dg[0];
+                dB = Dg[1];
+                dC = Dg[2];
                 xi0 = x[3 * i];
                 xi1 = x[3 * i + 1];
                 xi2 = x[3 * i + 2];
@@ -777,31 +781,44 @@ __device__ inline void fac_y_cell_rows(const DevParams& P, const FacOp& F, const
                 yv = yin[3 * i + g];
                 if (y2) y2v = y2[3 * i + g];
             }
-            // C Lambda C^T part over the P neighbours (beta 0: self)
-            for (int jb = 0; jb < n; jb += G * UP) {
-                if (jb > 0) fac_cell_plist<UP>(F, c0, n, i, jb, g, k, bb);
-                // the position from pos (24 contiguous bytes, mostly one cache line)
-                // rather than from the record planes (two lines), and t
-                double q0[UP][3], q3[UP];
-#pragma unroll
-                for (int u = 0; u < UP; ++u) {
-                    const long long k3 = 3 * (long long)k[u];
-                    q0[u][0] = F.pos[k3];
-                    q0[u][1] = F.pos[k3 + 1];
-                    q0[u][2] = F.pos[k3 + 2];
-                    q3[u] = rt[k[u]];
+            double pi0, pi1, pi2;
+            if (staged) {
+                if (ps > 0) pl = places(i, 0);
+                pi0 = L.b[own + r][1];
+                pi1 = L.c[own + r][0];
+                pi2 = L.c[own + r][1];
+                long long e0 = 0;
+                int w = 0;
+                if (kVar) {
+                    e0 = F.nPtr[i];
+                    w = F.nFluid[i];
                 }
+                const double* __restrict__ alpha = (const double*)F.alpha;
+                auto alphas = [&](int jb, double* al) {
 #pragma unroll
-                for (int u = 0; u < UP; ++u) {
-                    const double r0 = body::fac_wrap<kWrap>(q0[u][0] - pi0, W0, h0);
-                    const double r1 = body::fac_wrap<kWrap>(q0[u][1] - pi1, W1, h1);
-                    const double r2 = body::fac_wrap<kWrap>(q0[u][2] - pi2, W2, h2);
-                    const double f = bb[u] * q3[u];
-                    s0 += f * r0;
-                    s1 += f * r1;
-                    s2 += f * r2;
+                    for (int u = 0; u < 4; ++u) {
+                        const int jn = jb + g + u * G;
+                        al[u] = kVar && jn < w ? alpha[e0 + jn] : 0.0;
+                    }
+                };
+                for (int k = 0; k < nb; k += 2) {
+                    const uint4 cur = pl;
+                    if (k + 2 < nb) pl = places(i, k / 2 + 1);
+                    double al[4];
+                    alphas(4 * G * k, al);
+                    fac_cell_batch<kWrap, kVar>(P, L, cur.x, cur.y, al, pi0, pi1, pi2, s0, s1, s2);
+                    if (k + 1 < nb) {
+                        alphas(4 * G * (k + 1), al);
+                        fac_cell_batch<kWrap, kVar>(P, L, cur.z, cur.w, al, pi0, pi1, pi2, s0, s1, s2);
+                    }
                 }
+            } else {
+                pi0 = F.pos[3 * i];
+                pi1 = F.pos[3 * i + 1];
+                pi2 = F.pos[3 * i + 2];
+                body::fac_row_gather<kWrap, kVar>(P, F, i, g, pi0, pi1, pi2, s0, s1, s2);
             }
+            if (walls) body::fac_walls<kWrap>(P, F, rt, i, g, pi0, pi1, pi2, s0, s1, s2);
         }
         s0 = body::group_sum(s0, G);  // every lane of the group holds the sums
         s1 = body::group_sum(s1, G);
@@ -814,77 +831,39 @@ __device__ inline void fac_y_cell_rows(const DevParams& P, const FacOp& F, const
     }
 }
 
-template <bool kNeg, bool kWrap>
-__device__ inline void fac_y_cell_body(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
-                                       const double* yin, double* y, double* y2, double* p_copy, FacCellShared& L,
-                                       int b) {
-    int rs, nrows, nv;
-    if (!fac_cell_table(P, F, L.tab, rs, nrows, nv, b)) return;  // the whole workgroup: no fluid in this cell
-    if (L.tab.total > kCellSlots) {  // too many records to stage: gather them from global memory
-        fac_y_cell_rows<kNeg, kWrap, false, false>(P, F, x, beta, yin, y, y2, p_copy, L, rs, nrows);
-        return;
-    }
-    {
-        // thread t stages places t, t + kCellThreads, ...: every load is issued before
-        // the first store, so the staging waits for one round trip to memory.  Place r
-        // holds the record of particle vlo[v] + r - vex[v] of the last visited cell v
-        // with vex[v] <= r (empty cells share their successor's vex)
-        const body::FacPlanes R = body::fac_planes(P, F.rec);
-        const dv2c* __restrict__ ra = (const dv2c*)R.a;
-        const dv2c* __restrict__ rb = (const dv2c*)R.b;
-        const dv2c* __restrict__ rc = (const dv2c*)R.c;
-        constexpr int kRounds = kCellSlots / kCellThreads;
-        static_assert(kRounds * kCellThreads == kCellSlots, "the staging rounds cover the slots");
-        const int t = threadIdx.x, total = L.tab.total;
-        dv2c qa[kRounds], qb[kRounds], qc[kRounds];
-#pragma unroll
-        for (int k = 0; k < kRounds; ++k) {
-            const int r = t + k * kCellThreads;
-            if (r < total) {
-                int v = 0;
-#pragma unroll
-                for (int step = kCellTable / 2; step >= 1; step >>= 1)
-                    if (L.tab.vex[v + step] <= r) v += step;
-                const int j = L.tab.vlo[v] + (r - L.tab.vex[v]);
-                qa[k] = ra[j];
-                qb[k] = rb[j];
-                qc[k] = rc[j];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < kRounds; ++k) {
-            const int r = t + k * kCellThreads;
-            if (r < total) {
-                L.rec[3 * r] = qa[k];
-                L.rec[3 * r + 1] = qb[k];
-                L.rec[3 * r + 2] = qc[k];
-            }
-        }
-    }
-    __syncthreads();
-    if (F.slot) fac_y_cell_rows<kNeg, kWrap, true, true>(P, F, x, beta, yin, y, y2, p_copy, L, rs, nrows);
-    else fac_y_cell_rows<kNeg, kWrap, true, false>(P, F, x, beta, yin, y, y2, p_copy, L, rs, nrows);
+template <bool kNeg, int kThreads, int kCap>
+__device__ inline void fac_y_cell_any(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
+                                      const double* yin, double* y, double* y2, double* p_copy,
+                                      FacCellShared<kCap>& L, int b) {
+#define MPH_Y(WRAP, VAR) \
+    fac_y_cell_body<kNeg, WRAP, VAR, kThreads, kCap>(P, F, x, beta, yin, y, y2, p_copy, L, b)
+    const int wrap = F.wrap[0], var = F.wrap[1];  // uniform: the whole launch takes one branch
+    if (!wrap && !var) MPH_Y(false, false);
+    else if (!var) MPH_Y(true, false);
+    else MPH_Y(true, true);
+#undef MPH_Y
 }
 
-template <bool kNeg>
-__global__ void __launch_bounds__(kCellThreads) k_fac_y_cell(DevParams P, FacOp F, const double* __restrict__ x,
-                                                             double beta, const double* yin, double* y, double* y2,
-                                                             double* p_copy) {
+// four waves per SIMD: two workgroups of 512 threads on a CU
+template <bool kNeg, int kShape>
+__global__ void __launch_bounds__(kFacCellThreads[kShape], kShape == kFacCell3DWide ? 2 : 4)
+    k_fac_y_cell(DevParams P, FacOp F, const double* __restrict__ x, double beta, const double* yin, double* y,
+                 double* y2, double* p_copy) {
     if (cr_halted(P.halt)) return;
-    __shared__ FacCellShared L;
-    if (*F.wrap) fac_y_cell_body<kNeg, true>(P, F, x, beta, yin, y, y2, p_copy, L, blockIdx.x);
-    else fac_y_cell_body<kNeg, false>(P, F, x, beta, yin, y, y2, p_copy, L, blockIdx.x);
+    __shared__ FacCellShared<kFacCellSlots[kShape]> L;
+    fac_y_cell_any<kNeg, kFacCellThreads[kShape], kFacCellSlots[kShape]>(P, F, x, beta, yin, y, y2, p_copy, L,
+                                                                         blockIdx.x);
 }
 
 // The same pass for the scenes of a batch (the scene-table launches of mph_batch.hip):
 // workgroup b belongs to the scene s with R.pre[s] <= b < R.pre[s+1] and runs that
 // scene's cell b - R.pre[s] with its FP64 factored operator.  The grid covers the
-// scenes of the launch's set only (converged scenes have empty ranges).  The scenes
+// scenes of the launch's set and shape only (the others have empty ranges).  The scenes
 // of `first` also write y2 and p_copy.
-template <bool kNeg>
-__global__ void __launch_bounds__(kCellThreads) kb_fac_y_cell(const batch::BScene* __restrict__ tab, batch::CellRanges R, int ns,
-                                                              batch::SceneSet first, int x, double beta, int yin, int y,
-                                                              int y2, int p_copy) {
+template <bool kNeg, int kShape>
+__global__ void __launch_bounds__(kFacCellThreads[kShape], kShape == kFacCell3DWide ? 2 : 4)
+    kb_fac_y_cell(const batch::BScene* __restrict__ tab, batch::CellRanges R, int ns, batch::SceneSet first, int x,
+                  double beta, int yin, int y, int y2, int p_copy) {
     int lo = 0, hi = ns;  // the last s with R.pre[s] <= b
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -894,7 +873,7 @@ __global__ void __launch_bounds__(kCellThreads) kb_fac_y_cell(const batch::BScen
     const int s = lo, lb = (int)blockIdx.x - R.pre[lo];
     const batch::BScene& B = tab[s];
     if (batch::halted(B)) return;
-    __shared__ FacCellShared L;
+    __shared__ FacCellShared<kFacCellSlots[kShape]> L;
     // the scene's parameters as values: uniform loads into scalar registers (read
     // through the table, the compiler keeps them in vector registers and spills)
     const DevParams P = B.P;
@@ -902,8 +881,8 @@ __global__ void __launch_bounds__(kCellThreads) kb_fac_y_cell(const batch::BScen
     const bool f = batch::in_set(first, s);
     double* y2p = f && y2 >= 0 ? B.vec[y2] : nullptr;
     double* pc = f && p_copy >= 0 ? B.vec[p_copy] : nullptr;
-    if (*F.wrap) fac_y_cell_body<kNeg, true>(P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, L, lb);
-    else fac_y_cell_body<kNeg, false>(P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, L, lb);
+    fac_y_cell_any<kNeg, kFacCellThreads[kShape], kFacCellSlots[kShape]>(P, F, B.vec[x], beta, B.vec[yin], B.vec[y],
+                                                                         y2p, pc, L, lb);
 }
 
 template <bool kNeg, class VT>
@@ -912,9 +891,14 @@ void fac_launch(hipStream_t st, const DevParams& P, const FacOp& F, const double
     if (passes & 1) hipLaunchKernelGGL(k_fac_t<VT>, dim3(nblk(P.np, 256)), dim3(256), 0, st, P, F, x);
     if (!(passes & 2)) return;
     const long long cells = (long long)F.cellCnt[0] * F.cellCnt[1] * F.cellCnt[2];
-    if (sizeof(VT) == 8 && F.cellStart && cells > 0) {
-        hipLaunchKernelGGL((k_fac_y_cell<kNeg>), dim3((unsigned)cells), dim3(kCellThreads), 0, st, P, F, x, beta, yin,
-                           y, y2, p_copy);
+    if (sizeof(VT) == 8 && F.slot && cells > 0) {
+#define MPH_CELL(SHAPE)                                                                                           \
+    hipLaunchKernelGGL((k_fac_y_cell<kNeg, SHAPE>), dim3((unsigned)cells), dim3(kFacCellThreads[SHAPE]), 0, st, P, F, \
+                       x, beta, yin, y, y2, p_copy)
+        if (F.cellShape == kFacCell2D) MPH_CELL(kFacCell2D);
+        else if (F.cellShape == kFacCell3D) MPH_CELL(kFacCell3D);
+        else MPH_CELL(kFacCell3DWide);
+#undef MPH_CELL
         if (part) launch_dot_partial(st, P, dotx, y, part);
         return;
     }
@@ -965,28 +949,37 @@ void launch_fac_rec_positions(hipStream_t st, const DevParams& P, const double* 
 
 void launch_fac_slots(hipStream_t st, const DevParams& P, const FacOp& F) {
     const long long cells = (long long)F.cellCnt[0] * F.cellCnt[1] * F.cellCnt[2];
-    if (P.nf == 0 || !F.cellStart || !F.slot || cells <= 0) return;
-    hipLaunchKernelGGL(k_fac_slots, dim3((unsigned)cells), dim3(kCellThreads), 0, st, P, F);
+    if (P.nf == 0 || !F.slot || cells <= 0) return;
+    hipLaunchKernelGGL(k_fac_slots, dim3((unsigned)cells), dim3(256), 0, st, P, F, kFacCellSlots[F.cellShape]);
 }
 
 namespace batch {
-void spmv_fac_cells(const Tables& T, const SceneSet& on, const SceneSet& first, double alpha, int x, double beta,
-                    int yin, int y, int y2, int p_copy) {
-    CellRanges R;
+void spmv_fac_cells(const Tables& T, const SceneSet& on, const char* shapes, const SceneSet& first, double alpha,
+                    int x, double beta, int yin, int y, int y2, int p_copy) {
     const int* o = T.hoff + (size_t)kOffCell * (T.ns + 1);
-    int g = 0;
-    for (int s = 0; s < T.ns; ++s) {
-        R.pre[s] = g;
-        if ((on.w[s >> 6] >> (s & 63)) & 1ull) g += o[s + 1] - o[s];
+    for (int shape = 0; shape < kFacCellShapes; ++shape) {
+        CellRanges R;
+        int g = 0;
+        for (int s = 0; s < T.ns; ++s) {
+            R.pre[s] = g;
+            if (((on.w[s >> 6] >> (s & 63)) & 1ull) && shapes[s] == shape) g += o[s + 1] - o[s];
+        }
+        R.pre[T.ns] = g;
+        if (g <= 0) continue;
+#define MPH_CELL(NEG, SHAPE)                                                                                        \
+    hipLaunchKernelGGL((kb_fac_y_cell<NEG, SHAPE>), dim3(g), dim3(kFacCellThreads[SHAPE]), 0, T.st, T.tab, R, T.ns, \
+                       first, x, beta, yin, y, y2, p_copy)
+#define MPH_SIGN(SHAPE)                       \
+    do {                                      \
+        if (alpha < 0) MPH_CELL(true, SHAPE); \
+        else MPH_CELL(false, SHAPE);          \
+    } while (0)
+        if (shape == kFacCell2D) MPH_SIGN(kFacCell2D);
+        else if (shape == kFacCell3D) MPH_SIGN(kFacCell3D);
+        else MPH_SIGN(kFacCell3DWide);
+#undef MPH_SIGN
+#undef MPH_CELL
     }
-    R.pre[T.ns] = g;
-    if (g <= 0) return;
-    if (alpha < 0)
-        hipLaunchKernelGGL((kb_fac_y_cell<true>), dim3(g), dim3(kCellThreads), 0, T.st, T.tab, R, T.ns, first, x, beta,
-                           yin, y, y2, p_copy);
-    else
-        hipLaunchKernelGGL((kb_fac_y_cell<false>), dim3(g), dim3(kCellThreads), 0, T.st, T.tab, R, T.ns, first, x,
-                           beta, yin, y, y2, p_copy);
 }
 }  // namespace batch
 

@@ -100,8 +100,10 @@ struct FacOp {
     // consecutive particles of the cell-ordered list, read consecutive 16-byte
     // pairs.  Positions are written with the P slices; x and t by every first pass.
     double* rec;
-    // 1 when some neighbour pair interacts through the periodic boundary (then the
-    // displacements take the minimum image); set by the matrix-A launch
+    // flags set by the matrix-A launch.  [0]: some neighbour pair interacts through the
+    // periodic boundary (the displacements then take the minimum image).  [1]: some
+    // fluid pair's viscosity is not DevParams::mu0 (the second pass then reads alpha
+    // instead of recomputing it from the distance)
     const int* wrap;
     // FP32 form (the inner solves of mixed precision), which needs no positions:
     // u = sqrt(alpha) r per fluid-neighbour entry and v = beta r per P entry, each a
@@ -111,16 +113,36 @@ struct FacOp {
     const float* u32;
     const float* v32;
     float* rec32;
-    // cell-staged FP64 second pass (null cellStart: the chunk kernel): one workgroup
-    // per cell of the fluid bounding box cellLo + [0, cellCnt), which stages the
-    // records of the row cell's visited cells in LDS for the viscous gathers
+    // cell-staged FP64 second pass (null slot: the chunk kernel): one workgroup per cell
+    // of the fluid bounding box cellLo + [0, cellCnt), which stages the records of the
+    // row cell's visited cells in LDS for the gathers
     const int* cellStart;
     int cellLo[3], cellCnt[3];
     int cellXcd;  // 1: each XCD takes a contiguous range of cells (else round robin)
-    // [E] per fluid-neighbour entry of a fluid row: the neighbour's place in the row
-    // cell's staged records (launch_fac_slots), read instead of the column (or null)
+    int cellShape;  // kFacCell*: the launch shape
+    // built by launch_fac_slots.  cellDesc [cells][kFacDesc]: what a workgroup needs of
+    // its cell.  slot [nf][slotRow]: per fluid row its fluid neighbours' places among
+    // the staged records, in blocks of 8 G entries (G = kFacLanes lanes walk a row)
+    // of which lane g reads the 8 consecutive places that stand for entries g, g + G,
+    // ..., g + 7 G; padded with the row's own place
+    int* cellDesc;
     unsigned short* slot;
+    int slotRow;
 };
+constexpr int kFacDesc = 160;
+// lanes per row of the FP64 second pass.  A 3D row has about 170 fluid neighbours, a 2D
+// row about 37; a 3D cell about 41 rows, one pass of 512 threads.  (16 lanes in 3D, two
+// passes: 444 against 428 us per second pass on the 1M scene.)
+constexpr int kFacLanes = 8;
+// launch shapes of the cell-staged pass: threads per workgroup and staged records (56
+// bytes of LDS each).  3D: 1408 records let two workgroups share a CU (27 cells of 3.51
+// spacings hold at most 11^3 = 1331 lattice particles); domains of few cells have wider
+// ones and take 2816, one workgroup per CU.  2D: a cell holds about 12 rows and its 9
+// visited cells 110-144 records, so 128 threads and 256 records keep many workgroups on
+// a CU.
+enum { kFacCell3D = 0, kFacCell3DWide = 1, kFacCell2D = 2, kFacCellShapes = 3 };
+constexpr int kFacCellThreads[kFacCellShapes] = {512, 512, 128};
+constexpr int kFacCellSlots[kFacCellShapes] = {1408, 2816, 256};
 
 constexpr int kSlice = 64;    // particles per A slice (one wavefront)
 
@@ -184,8 +206,7 @@ void launch_forces(hipStream_t st, const DevParams& P, const int* type, const do
 // ---- implicit assembly ----
 // alpha/diag/wrap (each may be null): the factored form's viscous scalar per
 // fluid-neighbour entry (FacOp order), the diagonal block without C Lambda C^T, and
-// the flag set when a pair interacts through the periodic boundary (wrap must be 0
-// before the launch).  blk (with runStart; may be null): the level-0 run sums
+// the two flags of FacOp::wrap (0 before the launch).  blk (with runStart; may be null): the level-0 run sums
 // [nf][kBlkRuns][kBlkStride] of the factored form, each in list order
 void launch_matrix_a(hipStream_t st, const DevParams& P, const int* type, const double* pos, const double* vel,
                      const double* mass, const double* mu, const int* nCount, const int* nFluid,
@@ -270,7 +291,7 @@ void launch_fac_spmv(hipStream_t st, const DevParams& P, const FacOp& F, double 
 // the positions of the FP64 records (planes b odd and c of FacOp::rec, 7*np doubles)
 // copied from one record buffer into another; x and t are written by each product
 void launch_fac_rec_positions(hipStream_t st, const DevParams& P, const double* from, double* to);
-// FacOp::slot of the fluid-neighbour entries (after the lists; the cell-staged pass)
+// FacOp::cellDesc and slot (after the lists and runP; the cell-staged pass)
 void launch_fac_slots(hipStream_t st, const DevParams& P, const FacOp& F);
 
 void launch_convert_f32(hipStream_t st, const double* in, float* out, long long n);

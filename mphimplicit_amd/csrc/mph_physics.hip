@@ -407,7 +407,10 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
                     const double wdrij = -dwq_k(P.Kv, P.m2V, dij, P.radV);
                     const double e[3] = {q.x[0] / dij, q.x[1] / dij, q.x[2] / dij};
                     const double muij = 2.0 * (mui * muj) / (mui + muj);
-                    if (falpha) alpha = P.visc * muij * wdrij / (dij * dij * dij);
+                    if (falpha) {
+                        alpha = P.visc * muij * wdrij / (dij * dij * dij);
+                        if (jn < nfl && !(muij == P.mu0)) atomicOr(fwrap + 1, 1);
+                    }
                     for (int r = 0; r < 3; ++r)
                         for (int sdim = 0; sdim < 3; ++sdim)
                             t[3 * r + sdim] = +P.visc * muij * e[sdim] * e[r] * wdrij / dij;

@@ -109,6 +109,18 @@ int init_constants(mph_scene& S, const mph_grid& g) {
         for (int u = 0; u < 4; ++u) P.ratio[t][u] = p.interaction_ratio[t][u];
     }
     P.visc = dim == 2 ? 8.0 : 10.0;
+    // the viscosity of a fluid pair (main.cpp:2279) where one fluid fills the scene
+    double m0 = P.shear[1];
+    for (int i = 0; i < g.np; ++i)
+        if (g.type[i] == 0) {
+            m0 = P.shear[0];
+            break;
+        }
+    P.mu0 = 2.0 * (m0 * m0) / (m0 + m0);
+    P.facV = P.visc * P.mu0 * P.Kv * 2.0 / P.radV;
+    P.facP = P.Kp * 2.0 / P.radP;
+    P.invV = 1.0 / P.radV;
+    P.invP = 1.0 / P.radP;
     for (int d = 0; d < 3; ++d) P.gravity[d] = p.gravity[d];
     // initializeWall (1023-1062)
     for (int w = 2; w < 4; ++w) {
@@ -178,7 +190,14 @@ bool mixed(const mph_scene& S) { return S.prm.precision == MPH_PRECISION_MIXED; 
 bool factored(const mph_scene& S) { return S.prm.operator_form == MPH_OPERATOR_FACTORED; }
 
 bool fac_cells(const mph_scene& S) {
-    return S.facCells == 1 || (S.facCells == 2 && (S.P.dim == 3 || S.P.nf <= kFacCellsSmall));
+    return S.facCells != 0;
+}
+
+// cells of the fluid bounding box
+long long fac_bbox_cells(const mph_scene& S) {
+    long long n = 1;
+    for (int d = 0; d < 3; ++d) n *= S.hbbox[d] - S.hbbox[3 + d] + 1;
+    return n;
 }
 
 bool blocks_wanted(const mph_scene& S) {
@@ -334,9 +353,9 @@ int phase_matrix_a(mph_scene& S) {
         return rc;
     if (factored(S)) {
         const long long ne = S.E > 0 ? S.E : 1;
-        if ((rc = S.falpha.ensure(ne)) || (rc = S.fdiag.ensure(9 * (size_t)S.P.nf)) || (rc = S.fwrap.ensure(1)))
+        if ((rc = S.falpha.ensure(ne)) || (rc = S.fdiag.ensure(9 * (size_t)S.P.nf)) || (rc = S.fwrap.ensure(2)))
             return rc;
-        launch_fill_i32(S.st, S.fwrap.p, 1, 0);
+        launch_fill_i32(S.st, S.fwrap.p, 2, 0);
     }
     // the level-0 run sums, for a factored level 0 (the multigrid phase reads them)
     const bool runsums = factored(S) && !S.blocks && S.prm.multigrid;
@@ -371,10 +390,15 @@ int phase_matrix_c(mph_scene& S) {
                      S.runP.p, S.selfC.p, S.frec.p);
         if (mixed(S))  // alpha was written by the matrix-A phase
             launch_fac_u(S.st, S.P, S.nFluid.p, S.nPtr.p, S.nInd.p, S.falpha.p, S.pos.p, S.fu32.p);
-        // the staged places of the viscous entries for the cell-staged FP64 pass (a
-        // scene alone and in a batch)
-        if (fac_cells(S)) {
-            if ((rc = S.fslot.ensure(S.E > 0 ? S.E : 1))) return rc;
+        // the cells' descriptors and the rows' staged places for the cell-staged FP64 pass
+        // (a scene alone and in a batch).  A row's places take as many blocks as the
+        // longest row: where that is far above the mean (a clump of particles), the pass
+        // is left to the chunk kernel
+        const long long blk = 8 * kFacLanes, row = blk * ((S.hmaxW + blk - 1) / blk), cells = fac_bbox_cells(S);
+        if (fac_cells(S) && row * S.P.nf <= 4 * S.E + (64 << 20) && cells > 0) {
+            if ((rc = S.fslot.ensure((size_t)(row * S.P.nf))) || (rc = S.fdesc.ensure((size_t)(kFacDesc * cells))))
+                return rc;
+            S.fslotRow = (int)row;
             S.fslotValid = true;
             launch_fac_slots(S.st, S.P, fac_op(S, false));
         }
@@ -618,14 +642,20 @@ FacOp fac_op(mph_scene& S, bool f32) {
     F.v32 = f32 ? S.fv32.p : nullptr;
     F.rec32 = f32 ? S.frec32.p : nullptr;
     // the cell-staged second pass over the fluid bounding box (max x,y,z then min)
-    const bool cells = fac_cells(S);
-    F.cellStart = cells ? S.cellStart.p : nullptr;
-    F.slot = cells && S.fslot.p && S.fslotValid ? S.fslot.p : nullptr;
+    const bool cells = fac_cells(S) && S.fslotValid;
+    F.cellStart = S.cellStart.p;
+    F.slot = cells ? S.fslot.p : nullptr;
+    F.slotRow = S.fslotRow;
+    F.cellDesc = S.fdesc.p;
     F.cellXcd = S.facCellXcd ? 1 : 0;
     for (int d = 0; d < 3; ++d) {
         F.cellLo[d] = S.hbbox[3 + d];
         F.cellCnt[d] = cells ? S.hbbox[d] - S.hbbox[3 + d] + 1 : 0;
     }
+    // the records of 3x3x3 cells of a lattice decide how many are staged
+    double most = 1;
+    for (int d = 0; d < 3; ++d) most *= std::ceil(3.0 * S.P.cw[d] / S.P.l);
+    F.cellShape = S.P.dim == 2 ? kFacCell2D : most <= kFacCellSlots[kFacCell3D] ? kFacCell3D : kFacCell3DWide;
     return F;
 }
 
@@ -1149,6 +1179,7 @@ void destroy(mph_scene* S) {
     for (DBuf<double>* b : {&S->falpha, &S->fdiag, &S->selfC, &S->fbeta, &S->frec}) b->release();
     S->fu32.release();
     S->fslot.release();
+    S->fdesc.release();
     S->fv32.release();
     S->frec32.release();
     for (DBuf<double>* b : {&S->pos, &S->pos2, &S->vel, &S->vel2, &S->force, &S->mass, &S->kappa, &S->lambda,
@@ -1643,8 +1674,10 @@ int mph_scene_scalar(mph_scene* S, const char* name, double* v) {
         // in place of the 4-byte column.
         if (!factored(*S)) return fail(MPH_E_STATE, "the scene applies the assembled operator");
         const bool f64 = n == "FactoredBytes";
-        const double ab = f64 ? 8.0 : 12.0, vb = f64 ? 8.0 : 12.0, recb = f64 ? 32.0 : 16.0;
-        // the cell-staged FP64 pass reads the 2-byte place instead of the column
+        // FP64: alpha and beta are recomputed from the distances, so a fluid neighbour is a
+        // 2-byte staged place (cell-staged pass) or a 4-byte column, a P entry of the first
+        // pass a column; a wall neighbour of the second pass a column and beta
+        const double ab = f64 ? 0.0 : 12.0, vb = f64 ? 0.0 : 12.0, recb = f64 ? 32.0 : 16.0;
         const double colb = f64 && fac_cells(*S) && S->fslotValid ? 2.0 : 4.0;
         const double posb = f64 ? 24.0 : 0.0;
         std::vector<int> nfl, ncp, run;
@@ -1658,7 +1691,8 @@ int mph_scene_scalar(mph_scene* S, const char* name, double* v) {
             if (run[k] > 0) t += (4.0 + vb) * run[k] + 8.0 + posb;  // entries, lambda, position
         }
         for (int i = 0; i < P.nf; ++i)
-            t += (colb + ab) * nfl[i] + (4.0 + vb) * ncp[i] + 4.0 + 4.0 + 72.0 + 24.0 + 72.0;
+            t += (colb + ab) * nfl[i] + (f64 ? 12.0 * (ncp[i] - run[i]) : (4.0 + vb) * ncp[i]) + 4.0 + 4.0 + 72.0 +
+                 24.0 + 72.0;
         *v = t;
     }
     else if (n == "SpmvLaunchesF32") *v = (double)S->spmvLaunches32;
@@ -1813,7 +1847,7 @@ int mph_scene_device_bytes(mph_scene* S, unsigned long long* bytes) {
     n += (S->fgtab.cap + S->fblk.cap) * sizeof(double);
     for (DBuf<double>* b : {&S->falpha, &S->fdiag, &S->selfC, &S->fbeta, &S->frec}) n += b->cap * sizeof(double);
     n += (S->fu32.cap + S->fv32.cap + S->frec32.cap) * sizeof(float);
-    n += S->fslot.cap * sizeof(unsigned short);
+    n += S->fslot.cap * sizeof(unsigned short) + S->fdesc.cap * sizeof(int);
     n += S->runStart.cap * sizeof(unsigned short);
     for (DBuf<double>* b : {&S->pos, &S->pos2, &S->vel, &S->vel2, &S->force, &S->mass, &S->kappa, &S->lambda,
                             &S->mu, &S->densA, &S->gcen, &S->pressA, &S->volStrainP, &S->divP, &S->pressP,

@@ -187,16 +187,15 @@ struct mph_scene {
     bool blocks = true;  // this step assembles the 3x3 blocks (see blocks_wanted)
     mph::host::DBuf<double> falpha, fdiag, selfC, fbeta, frec;  // FacOp::alpha, diag, selfC, beta, rec
     mph::host::DBuf<float> fu32, fv32, frec32;  // FP32 form (mixed precision): FacOp::u32, v32, rec32
-    // FP64 second pass staged per cell in LDS: 1 always, 0 never (the chunk kernel),
-    // 2 (default) in 3D scenes and in scenes of at most kFacCellsSmall fluid
-    // particles.  Measured per product, 2D 130k-188k fluid: chunk 76-88 us, cells
-    // 174-241 us (a 2D cell holds ~12 rows, a 512-lane workgroup stages 9 cells for
-    // them); 3D 166k-176k: chunk 269-282 us, cells 189-207 us; 2.2k-2.8k fluid, 2D and
-    // 3D: chunk 41-68 us, cells 23-27 us.
+    // FP64 second pass staged per cell in LDS (0: the chunk kernel; 1, 2: the cells).
+    // Measured per second pass, chunk kernel against cells (with their dot partials): 2D
+    // 160k fluid 49 against 37 us; 3D 1M about 1150 against 438 us.
     int facCells = 2;
     bool facCellXcd = true;  // FacOp::cellXcd
-    mph::host::DBuf<unsigned short> fslot;  // FacOp::slot
-    bool fslotValid = false;                // fslot matches the current lists
+    mph::host::DBuf<unsigned short> fslot;  // FacOp::slot, rows of fslotRow places
+    mph::host::DBuf<int> fdesc;             // FacOp::cellDesc
+    int fslotRow = 0;
+    bool fslotValid = false;                // they match the current lists
     // multigrid
     int hbbox[6] = {0, 0, 0, 0, 0, 0};
     int depth = 0;
@@ -272,7 +271,6 @@ namespace host {
 
 bool mixed(const mph_scene& S);
 bool factored(const mph_scene& S);
-constexpr int kFacCellsSmall = 16384;
 // rows of the convergence record (16 bytes each): iterations past this are not kept
 constexpr long long kConvRowsMax = 1LL << 22;
 bool fac_cells(const mph_scene& S);  // the FP64 second pass is the cell-staged one (facCells)
