@@ -151,7 +151,11 @@ int build_tables(mph_batch& B, const std::vector<mph_scene*>& sc, Tables& T, boo
         put(kOffChunk, (S.P.nf + 255) / 256);
         put(kOffElem, (int)((3LL * S.P.nf + 255) / 256));
         put(kOffPart, (S.P.np + 255) / 256);
-        for (int l = 0; l < b.depth; ++l) put(kOffLevel + l, (b.lv[l].nrow + 255) / 256);
+        put(kOffP2g, b.mg ? (8 * b.lv[0].nrow + 255) / 256 : 0);
+        for (int l = 0; l < b.depth; ++l) {
+            put(kOffLevel + l, (b.lv[l].nrow + 255) / 256);
+            put(kOffSweep + l, ((b.lv[l].lanes ? 4 : 1) * b.lv[l].nrow + 255) / 256);
+        }
     }
     for (int row = 0; row < kOffRows; ++row)
         for (int s = 0; s < ns; ++s) B.hoff[(size_t)row * (ns + 1) + s + 1] += B.hoff[(size_t)row * (ns + 1) + s];
@@ -221,8 +225,9 @@ struct VCycle {
         for (int s = 0; s < (int)sc.size(); ++s)
             if (on.has(s)) cur[s][l] ^= 1;
     }
-    // precondition (main.cpp:4122-4266) of in -> out for the multigrid scenes in `on`
-    void apply(const Set& on, int in, int out, bool part, bool f32) {
+    // precondition (main.cpp:4122-4266) of in -> out for the multigrid scenes in `on`;
+    // the scenes of pq update q = beta q + y on the way (in = kQ)
+    void apply(const Set& on, const Set& pq, int in, int out, bool part, bool f32) {
         if (on.empty()) return;
         auto F = [&](int s) { return sc[s]->fuse; };  // levels F..depth-1: one workgroup
         int maxF = 0;
@@ -234,7 +239,7 @@ struct VCycle {
                 if (on.has(s) && l < F(s)) m.add(s);
             return m;
         };
-        mg_p2g_bu(T, on.m, in, curset(on, 0));  // P2G, S = 0, R = Q, S += invD R
+        mg_p2g_bu(T, on.m, pq.m, in, curset(on, 0));  // P2G, S = 0, R = Q, S += invD R
         const Set top = above(0);
         ru(top, 0, f32);  // pre-smooth x2
         if (!top.empty()) mg_residual(T, top.m, 0, curset(top, 0), f32);
@@ -267,7 +272,7 @@ struct VCycle {
 };
 
 // apply_m of mph_scene.cpp for a set of scenes: the V-cycle, or a copy without it
-void apply_m(VCycle& V, const Set& on, int in, int out, bool part, bool f32) {
+void apply_m(VCycle& V, const Set& on, int in, int out, bool part, bool f32, const Set& pq = Set{}) {
     Set mg, plain;
     for (int s = 0; s < (int)V.sc.size(); ++s)
         if (on.has(s)) (V.sc[s]->prm.multigrid ? mg : plain).add(s);
@@ -275,7 +280,7 @@ void apply_m(VCycle& V, const Set& on, int in, int out, bool part, bool f32) {
         copy(V.T, plain.m, in, out);
         if (part) dot_partial(V.T, plain.m, in, out);
     }
-    V.apply(mg, in, out, part, f32);
+    V.apply(mg, pq, in, out, part, f32);
 }
 
 void solve_prologue(const Tables& T, const std::vector<mph_scene*>& sc, const Set& all) {
@@ -306,15 +311,16 @@ bool nonfinite(double v) { return !std::isfinite(v); }
 // (the scenes of `first` also q = y, p = s; the others update p and q), rho = s.y,
 // u = M^-1 q, tmp = q.u, x, r and s updated, then r.r and the stop test on the device
 void fp64_iteration(mph_batch& B, const Tables& T, VCycle& V, const Set& on, const Set& first) {
-    Set rest;
+    // with the multigrid preconditioner the P2G updates q and the x update p
+    Set rest, pq;
     for (int s = 0; s < T.ns; ++s)
-        if (on.has(s) && !first.has(s)) rest.add(s);
+        if (on.has(s) && !first.has(s)) (V.sc[s]->prm.multigrid ? pq : rest).add(s);
     bspmv(B, T, on.m, first.m, false, 1.0, kS, 0.0, kY, kY, kQ, kP, kS);
     dot_final(T, on.m, kRHO, kRHOP);
     pq_update(T, rest.m);
-    apply_m(V, on, kQ, kU, true, false);
+    apply_m(V, on, kQ, kU, true, false, pq);
     dot_final(T, on.m, kTMP, -1);
-    xrs_update(T, on.m, kX);
+    xrs_update(T, on.m, pq.m, kX);
     dot_final_stop(T, on.m, 1);
 }
 
@@ -500,10 +506,13 @@ int solve_mixed(mph_batch& B, const std::vector<mph_scene*>& sc, std::vector<cha
         if (!inner.empty()) {
             bspmv(B, T, inner.m, restart.m, true, 1.0, kS, 0.0, kY, kY, kQ, kP, kS);
             dot_final(T, inner.m, kRHO, kRHOP);
-            pq_update(T, rest.m);
-            apply_m(V, inner, kQ, kU, true, true);
+            Set plain, pq;  // as fp64_iteration
+            for (int s = 0; s < ns; ++s)
+                if (rest.has(s)) (sc[s]->prm.multigrid ? pq : plain).add(s);
+            pq_update(T, plain.m);
+            apply_m(V, inner, kQ, kU, true, true, pq);
             dot_final(T, inner.m, kTMP, -1);
-            xrs_update(T, inner.m, kD);
+            xrs_update(T, inner.m, pq.m, kD);
             dot_final(T, inner.m, kRR, -1);
             for (int s = 0; s < ns; ++s)
                 if (inner.has(s)) z[s].it++, z[s].total++;

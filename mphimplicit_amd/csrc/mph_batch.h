@@ -20,8 +20,18 @@ enum { kX = 0, kR, kS, kY, kP, kQ, kU, kB, kROut, kD, kNVec };
 // rows of the block-offset table: 256-particle chunks of the fluid particles,
 // 256-element blocks of the 3*nf vectors, 256-particle blocks of all particles, the
 // fluid bounding box's cells (the cell-staged factored pass; 0 for the other
-// scenes), then 256-row blocks of each multigrid level
-enum { kOffChunk = 0, kOffElem = 1, kOffPart = 2, kOffCell = 3, kOffLevel = 4, kOffRows = kOffLevel + kMaxLevels };
+// scenes), the blocks of the P2G (8 lanes per level-0 row), then per multigrid level its
+// 256-row blocks and the blocks of its sweeps (4 lanes per row where Level::lanes)
+enum {
+    kOffChunk = 0,
+    kOffElem = 1,
+    kOffPart = 2,
+    kOffCell = 3,
+    kOffP2g = 4,
+    kOffLevel = 5,
+    kOffSweep = kOffLevel + kMaxLevels,
+    kOffRows = kOffSweep + kMaxLevels
+};
 
 struct SceneSet {
     unsigned long long w[kMaxScenes / 64];
@@ -116,10 +126,10 @@ void dot_final_stop(const Tables& T, const SceneSet& on, int step);
 void ctl_reset(const Tables& T, const SceneSet& on);    // ctl = 0 (before the solve's first kernel)
 void ctl_release(const Tables& T, const SceneSet& on);  // ctl[kCtlHalt] = 0 (kernels after the loop run)
 void pq_update(const Tables& T, const SceneSet& on);
-void xrs_update(const Tables& T, const SceneSet& on, int x);
+void xrs_update(const Tables& T, const SceneSet& on, const SceneSet& pq, int x);  // pq: p = beta p + s first
 void store_velocity(const Tables& T, const SceneSet& on);
-void mg_p2g(const Tables& T, const SceneSet& on, int in);
-void mg_p2g_bu(const Tables& T, const SceneSet& on, int in, const SceneSet& cur);  // P2G, begin, update
+// P2G, begin, update; the scenes of pq form q = beta q + y on the way (in = kQ)
+void mg_p2g_bu(const Tables& T, const SceneSet& on, const SceneSet& pq, int in, const SceneSet& cur);
 void mg_restrict_bu(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);  // l-1 -> l, begin, update
 void mg_begin(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);
 void mg_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);

@@ -157,10 +157,14 @@ __global__ void kb_pq_update(const BScene* tab, const int* off, int ns, SceneSet
 }
 
 __global__ void __launch_bounds__(256) kb_xrs_update(const BScene* tab, const int* off, int ns, SceneSet on,
-                                                     int x) {
+                                                     SceneSet pq, int x) {
     __shared__ double sh[256];
     MPH_SCENE(kOffChunk)
-    xrs_update_chunk(B.P.nf, B.scal, B.vec[kP], B.vec[kQ], B.vec[kU], B.vec[x], B.vec[kR], B.vec[kS], B.part, lb,
+    if (in_set(pq, s))
+        xrs_update_chunk<true>(B.P.nf, B.scal, B.vec[kP], B.vec[kQ], B.vec[kU], B.vec[x], B.vec[kR], B.vec[kS],
+                               B.part, lb, sh);
+    else
+        xrs_update_chunk<false>(B.P.nf, B.scal, B.vec[kP], B.vec[kQ], B.vec[kU], B.vec[x], B.vec[kR], B.vec[kS], B.part, lb,
                      sh);
 }
 
@@ -178,20 +182,21 @@ __device__ inline Level level(const BScene& B, int l, const SceneSet& cur, int s
     return L;
 }
 
-__global__ void kb_mg_p2g(const BScene* tab, const int* off, int ns, SceneSet on, int in) {
-    MPH_SCENE(kOffLevel)
-    const int row = lb * 256 + threadIdx.x;
-    const Level& L = B.lv[0];
-    if (row < L.nrow) mg_p2g_row(B.P, L, B.cellStart, B.vec[in], row);
-}
-
-__global__ void kb_mg_p2g_bu(const BScene* tab, const int* off, int ns, SceneSet on, int in, SceneSet cur) {
-    MPH_SCENE(kOffLevel)
-    const int row = lb * 256 + threadIdx.x;
+__global__ void __launch_bounds__(256) kb_mg_p2g_bu(const BScene* tab, const int* off, int ns, SceneSet on,
+                                                    SceneSet pq, int in, SceneSet cur) {
+    __shared__ double tb[256 * kP2gK];
+    MPH_SCENE(kOffP2g)
     const Level L = level(B, 0, cur, s);
-    if (row >= L.nrow) return;
-    mg_p2g_row(B.P, L, B.cellStart, B.vec[in], row);
-    mg_begin_update_row(L, row);
+    const bool f = in_set(pq, s);
+#define MPH_P2G(PQ, ORD) mg_p2g_lanes<PQ, ORD>(B.P, L, B.cellStart, B.vec[in], B.vec[kY], B.scal, lb, tb)
+    if (L.ordered) {
+        if (f) MPH_P2G(true, true);
+        else MPH_P2G(false, true);
+    } else {
+        if (f) MPH_P2G(true, false);
+        else MPH_P2G(false, false);
+    }
+#undef MPH_P2G
 }
 
 __global__ void kb_mg_restrict_bu(const BScene* tab, const int* off, int ns, SceneSet on, int l, SceneSet cur) {
@@ -199,8 +204,7 @@ __global__ void kb_mg_restrict_bu(const BScene* tab, const int* off, int ns, Sce
     const int row = lb * 256 + threadIdx.x;
     const Level L = level(B, l, cur, s);
     if (row >= L.nrow) return;
-    mg_restrict_row(B.lv[l - 1], L, row);
-    mg_begin_update_row(L, row);
+    mg_begin_update_row(L, row, mg_restrict_row(B.lv[l - 1], L, row));
 }
 
 __global__ void kb_mg_begin(const BScene* tab, const int* off, int ns, SceneSet on, int l, SceneSet cur) {
@@ -218,24 +222,35 @@ __global__ void kb_mg_update(const BScene* tab, const int* off, int ns, SceneSet
 }
 
 // FP32 stencil where the level has one and the launch asks for it (mixed inner solve)
-__global__ void kb_mg_residual(const BScene* tab, const int* off, int ns, SceneSet on, int l, SceneSet cur,
-                               int f32) {
-    MPH_SCENE(kOffLevel + l)
-    const int row = lb * 256 + threadIdx.x;
-    const Level L = level(B, l, cur, s);
-    if (row >= L.nrow) return;
-    if (f32 && L.A32) mg_residual_row<float>(L, row);
-    else mg_residual_row<double>(L, row);
+template <class VT, bool kUpdate, bool kOrd>
+__device__ inline void sweep(const Level& L, int lb, double* tb) {
+    if (!L.lanes) {
+        const int row = lb * 256 + threadIdx.x;
+        if (row >= L.nrow) return;
+        if constexpr (kUpdate) mg_residual_update_row<VT, kOrd>(L, row);
+        else mg_residual_row<VT, kOrd>(L, row);
+        return;
+    }
+    const long long t = (long long)lb * 256 + threadIdx.x;
+    const bool s3 = L.cs[0] == 3 && L.cs[1] == 3;
+    if (s3 && L.cs[2] == 3) mg_sweep_lanes<VT, kUpdate, kOrd, 3, 3, 3>(L, t, tb);
+    else if (s3 && L.cs[2] == 1) mg_sweep_lanes<VT, kUpdate, kOrd, 3, 3, 1>(L, t, tb);
+    else mg_sweep_lanes<VT, kUpdate, kOrd, 0, 0, 0>(L, t, tb);
 }
-
-__global__ void kb_mg_residual_update(const BScene* tab, const int* off, int ns, SceneSet on, int l, SceneSet cur,
-                                      int f32) {
-    MPH_SCENE(kOffLevel + l)
-    const int row = lb * 256 + threadIdx.x;
+template <bool kUpdate>
+__global__ void __launch_bounds__(256) kb_mg_sweep(const BScene* tab, const int* off, int ns, SceneSet on, int l,
+                                                   SceneSet cur, int f32) {
+    __shared__ double tb[256 * kRowTerms];
+    MPH_SCENE(kOffSweep + l)
     const Level L = level(B, l, cur, s);
-    if (row >= L.nrow) return;
-    if (f32 && L.A32) mg_residual_update_row<float>(L, row);
-    else mg_residual_update_row<double>(L, row);
+    const bool h = f32 && L.A32;
+    if (L.ordered) {
+        if (h) sweep<float, kUpdate, true>(L, lb, tb);
+        else sweep<double, kUpdate, true>(L, lb, tb);
+    } else {
+        if (h) sweep<float, kUpdate, false>(L, lb, tb);
+        else sweep<double, kUpdate, false>(L, lb, tb);
+    }
 }
 
 __global__ void kb_mg_restrict(const BScene* tab, const int* off, int ns, SceneSet on, int l) {
@@ -274,8 +289,11 @@ __global__ void __launch_bounds__(T) kb_mg_coarse(const BScene* tab, int ns, Sce
     __shared__ CoarseShared<T> sh;
     const unsigned c = in_set(cur, s) ? 1u : 0u;
     const Level& S = B.lv[B.fuse > 0 ? B.fuse - 1 : 0];
-    mg_coarse_cycle<N, T, XB>(K, B.fuse, B.depth, B.fuse > 0 ? S.R : S.Q, lv_s(S, B.fuse > 0 ? c : c ^ 1), S.nrow,
-                              B.ctl ? B.ctl + kCtlHalt : nullptr, sh);
+    const double* in = B.fuse > 0 ? S.R : S.Q;
+    double* io = lv_s(S, B.fuse > 0 ? c : c ^ 1);
+    const int* halt = B.ctl ? B.ctl + kCtlHalt : nullptr;
+    if (K.ordered) mg_coarse_cycle<N, T, XB, true>(K, B.fuse, B.depth, in, io, S.nrow, halt, sh);
+    else mg_coarse_cycle<N, T, XB, false>(K, B.fuse, B.depth, in, io, S.nrow, halt, sh);
 }
 
 #undef MPH_SCENE
@@ -366,15 +384,16 @@ void pq_update(const Tables& T, const SceneSet& on) {
     const int g = T.blocks(kOffElem);
     if (g > 0 && any(on)) hipLaunchKernelGGL(kb_pq_update, dim3(g), dim3(256), 0, T.st, T.tab, T.off, T.ns, on);
 }
-void xrs_update(const Tables& T, const SceneSet& on, int x) { MPH_LAUNCH(kb_xrs_update, kOffChunk, x); }
+void xrs_update(const Tables& T, const SceneSet& on, const SceneSet& pq, int x) {
+    MPH_LAUNCH(kb_xrs_update, kOffChunk, pq, x);
+}
 void store_velocity(const Tables& T, const SceneSet& on) {
     const int g = T.blocks(kOffElem);
     if (g > 0 && any(on))
         hipLaunchKernelGGL(kb_store_velocity, dim3(g), dim3(256), 0, T.st, T.tab, T.off, T.ns, on);
 }
-void mg_p2g(const Tables& T, const SceneSet& on, int in) { MPH_LAUNCH(kb_mg_p2g, kOffLevel, in); }
-void mg_p2g_bu(const Tables& T, const SceneSet& on, int in, const SceneSet& cur) {
-    MPH_LAUNCH(kb_mg_p2g_bu, kOffLevel, in, cur);
+void mg_p2g_bu(const Tables& T, const SceneSet& on, const SceneSet& pq, int in, const SceneSet& cur) {
+    MPH_LAUNCH(kb_mg_p2g_bu, kOffP2g, pq, in, cur);
 }
 void mg_restrict_bu(const Tables& T, const SceneSet& on, int l, const SceneSet& cur) {
     MPH_LAUNCH(kb_mg_restrict_bu, kOffLevel + l, l, cur);
@@ -386,10 +405,10 @@ void mg_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur) 
     MPH_LAUNCH(kb_mg_update, kOffLevel + l, l, cur);
 }
 void mg_residual(const Tables& T, const SceneSet& on, int l, const SceneSet& cur, bool f32) {
-    MPH_LAUNCH(kb_mg_residual, kOffLevel + l, l, cur, f32 ? 1 : 0);
+    MPH_LAUNCH(kb_mg_sweep<false>, kOffSweep + l, l, cur, f32 ? 1 : 0);
 }
 void mg_residual_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur, bool f32) {
-    MPH_LAUNCH(kb_mg_residual_update, kOffLevel + l, l, cur, f32 ? 1 : 0);
+    MPH_LAUNCH(kb_mg_sweep<true>, kOffSweep + l, l, cur, f32 ? 1 : 0);
 }
 void mg_restrict(const Tables& T, const SceneSet& on, int l) { MPH_LAUNCH(kb_mg_restrict, kOffLevel + l, l); }
 void mg_prolong(const Tables& T, const SceneSet& on, int l, const SceneSet& curL, const SceneSet& curS) {

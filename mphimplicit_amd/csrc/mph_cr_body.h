@@ -104,21 +104,6 @@ __device__ inline int galerkin_self(const DevParams& P, const Level& L, int g) {
 // ---------------------------------------------------------------------------
 // multigrid rows (preconditionWithMultiGrid)
 
-// P2G: Q0 = 0*Q0 + sum over the cell's fluid particles of q (2964-2997)
-__device__ inline void mg_p2g_row(const DevParams& P, const Level& L, const int* __restrict__ cellStart,
-                                  const double* __restrict__ q, int row) {
-    const int g = row / 3, rd = row % 3;
-    int gx, gy, gz;
-    grid_xyz(L, g, gx, gy, gz);
-    const int ic = cell_id(P, gx + L.mn[0], gy + L.mn[1], gz + L.mn[2]);
-    double sum = 0.0;
-    for (int ip = cellStart[ic]; ip < cellStart[ic + 1]; ++ip) sum += 1.0 * 1.0 * q[3 * ip + rd];
-    double y = L.Q[row];
-    y *= 0.0;
-    y += sum;
-    L.Q[row] = y;
-}
-
 __device__ inline void mg_begin_row(const Level& L, int row) {  // myDscal(0.0, S); myDcopy(Q, R)
     double* S = lv_s(L, L.cur);
     S[row] *= 0.0;
@@ -133,16 +118,13 @@ __device__ inline void mg_update_row(const Level& L, int row) {  // myDdmv(1.0, 
     S[row] = y;
 }
 
-// mg_begin_row then mg_update_row on the same row (both touch that row only)
-__device__ inline void mg_begin_update_row(const Level& L, int row) {
-    double* S = lv_s(L, L.cur);
-    double y = S[row];
-    y *= 0.0;
-    const double r = L.Q[row];
+// mg_begin_row then mg_update_row on the same row (both touch that row only).  S*0.0 is a
+// zero and Q is never -0 (a sum from +0), so S = invD Q is formed without the old S.
+__device__ inline void mg_begin_update_row(const Level& L, int row, double r) {
     L.R[row] = r;
-    y *= 1.0;
+    double y = 0.0;
     y += 1.0 * L.invD[row] * r;
-    S[row] = y;
+    lv_s(L, L.cur)[row] = y;
 }
 
 // (v mod n) for 0 <= v < 3n without a division
@@ -152,12 +134,41 @@ __device__ inline int wrap3(int v, int n) {
     return v;
 }
 
-// sum over the 27-point (9 in 2D) block stencil of -1.0*a*x in shift order; the
-// wrapped neighbour index (g + e - 1 + cnt) % cnt of the reference's periodic
+// The sum over the 27-point (9 in 2D) block stencil of -1.0*a*x.  Ordered: in shift
+// order, one chain of up to 81 dependent adds (about 24 cycles each).  Otherwise (the
+// factored form, which keeps no bits of the reference): four chains over the stencil
+// cells [uQ, (u+1)Q), Q = cells/4 rounded up, with fused multiply-adds, combined as
+// (c0 + c1) + (c2 + c3); the lane-split sweeps give each lane one chain, so every kernel
+// that takes such a sum gets the same bits.  Per sweep of a level of 5k rows 4.2 us
+// against 4.75 us ordered, of the one-workgroup cycle 12.8 against 14.4 us (64k drop).
+template <bool kOrd>
+struct RowSum {
+    double c[kOrd ? 1 : 4];
+    __device__ inline RowSum() {
+        for (double& v : c) v = 0.0;
+    }
+    // the three entries of stencil cell q of N
+    __device__ inline void add(int q, int Q, double a, double x) {
+        if constexpr (kOrd) c[0] += -1.0 * a * x;
+        else {
+            const int u = q / Q;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (u == k) c[k] = __builtin_fma(-a, x, c[k]);
+        }
+    }
+    __device__ inline double total() const {
+        if constexpr (kOrd) return c[0];
+        else return (c[0] + c[1]) + (c[2] + c[3]);
+    }
+};
+__host__ __device__ constexpr int row_chain(int cells) { return (cells + 3) / 4; }
+
+// The wrapped neighbour index (g + e - 1 + cnt) % cnt of the reference's periodic
 // stencil (main.cpp:3323-3325) is formed by subtraction (its argument is < 3 cnt).
 // Full stencils (3x3x3, 3x3x1) take an unrolled path that issues the loads of nine
-// cells at a time before summing them in order; smaller levels take the loop.
-template <class VT, int C0, int C1, int C2>
+// cells at a time before summing them; smaller levels take the loop.
+template <class VT, int C0, int C1, int C2, bool kOrd>
 __device__ inline double mg_row_sum_full(const Level& L, const VT* __restrict__ A, const double* __restrict__ x,
                                          int row, int gx, int gy, int gz) {
     constexpr int N = C0 * C1 * C2;
@@ -170,7 +181,7 @@ __device__ inline double mg_row_sum_full(const Level& L, const VT* __restrict__ 
     for (int e = 0; e < C1; ++e) jy[e] = wrap3(gy + e - 1 + c1, c1);
 #pragma unroll
     for (int e = 0; e < C2; ++e) jz[e] = wrap3(gz + e - 1 + c2, c2);
-    double sum = 0.0;
+    RowSum<kOrd> sum;
 #pragma unroll
     for (int q0 = 0; q0 < N; q0 += 9) {
         VT av[27];
@@ -192,42 +203,45 @@ __device__ inline double mg_row_sum_full(const Level& L, const VT* __restrict__ 
         for (int t = 0; t < 9; ++t)
             if (q0 + t < N)
 #pragma unroll
-                for (int sd = 0; sd < 3; ++sd) sum += -1.0 * (double)av[3 * t + sd] * xv[3 * t + sd];
+                for (int sd = 0; sd < 3; ++sd) sum.add(q0 + t, row_chain(N), (double)av[3 * t + sd], xv[3 * t + sd]);
     }
-    return sum;
+    return sum.total();
 }
 
-template <class VT>
+template <class VT, bool kOrd>
 __device__ inline double mg_row_sum(const Level& L, const VT* __restrict__ A, const double* __restrict__ x, int row) {
     const int g = row / 3;
     int gx, gy, gz;
     grid_xyz(L, g, gx, gy, gz);
-    if (L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 3) return mg_row_sum_full<VT, 3, 3, 3>(L, A, x, row, gx, gy, gz);
-    if (L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 1) return mg_row_sum_full<VT, 3, 3, 1>(L, A, x, row, gx, gy, gz);
+    if (L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 3)
+        return mg_row_sum_full<VT, 3, 3, 3, kOrd>(L, A, x, row, gx, gy, gz);
+    if (L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 1)
+        return mg_row_sum_full<VT, 3, 3, 1, kOrd>(L, A, x, row, gx, gy, gz);
     const int c0 = L.cnt[0], c1 = L.cnt[1], c2 = L.cnt[2];
-    const int nrow = L.nrow;
+    const int nrow = L.nrow, Q = row_chain(L.cs[0] * L.cs[1] * L.cs[2]);
     const VT* a = A + row;  // entry sh of the row at a[sh * nrow]
-    double sum = 0.0;
+    RowSum<kOrd> sum;
+    int q = 0;
     for (int ex = 0; ex < L.cs[0]; ++ex) {
         const int jx = wrap3(gx + ex - 1 + c0, c0);
         for (int ey = 0; ey < L.cs[1]; ++ey) {
             const int jy = wrap3(gy + ey - 1 + c1, c1);
             const int bxy = (c1 * c2) * jx + c2 * jy;
-            for (int ez = 0; ez < L.cs[2]; ++ez) {
+            for (int ez = 0; ez < L.cs[2]; ++ez, ++q) {
                 const int jz = wrap3(gz + ez - 1 + c2, c2);
                 const double* xc = x + 3 * (bxy + jz);
-                for (int sd = 0; sd < 3; ++sd, a += nrow) sum += -1.0 * (double)a[0] * xc[sd];
+                for (int sd = 0; sd < 3; ++sd, a += nrow) sum.add(q, Q, (double)a[0], xc[sd]);
             }
         }
     }
-    return sum;
+    return sum.total();
 }
 
 // myDcopy(Q, R); myDcsrmv(-1.0, A, S, 1.0, R)
-template <class VT>
+template <class VT, bool kOrd>
 __device__ inline void mg_residual_row(const Level& L, int row) {
     const VT* A = sizeof(VT) == 8 ? (const VT*)L.A : (const VT*)L.A32;
-    const double sum = mg_row_sum(L, A, lv_s(L, L.cur), row);
+    const double sum = mg_row_sum<VT, kOrd>(L, A, lv_s(L, L.cur), row);
     double y = L.Q[row];
     y *= 1.0;
     y += sum;
@@ -236,11 +250,11 @@ __device__ inline void mg_residual_row(const Level& L, int row) {
 
 // residual then smoother update of the same row; the new iterate goes to the other
 // S buffer so every thread still reads the old one
-template <class VT>
+template <class VT, bool kOrd>
 __device__ inline void mg_residual_update_row(const Level& L, int row) {
     const double* So = lv_s(L, L.cur);
     const VT* A = sizeof(VT) == 8 ? (const VT*)L.A : (const VT*)L.A32;
-    const double sum = mg_row_sum(L, A, So, row);
+    const double sum = mg_row_sum<VT, kOrd>(L, A, So, row);
     double y = L.Q[row];
     y *= 1.0;
     y += sum;
@@ -251,8 +265,91 @@ __device__ inline void mg_residual_update_row(const Level& L, int row) {
     lv_s(L, L.cur ^ 1)[row] = s;
 }
 
-// restriction (R of 3115-3175): Q_L = 0*Q_L + sum of the clipped 2x2x2 children of R_S
-__device__ inline void mg_restrict_row(const Level& S, const Level& L, int row) {
+// The same sweeps with kRowLanes lanes per row, for levels too small to fill the GPU
+// with one thread per row (a row's 81 loads are then latency-bound).  Lane u loads the
+// entries of stencil cells [uQ, (u+1)Q).  Ordered: it forms their terms -1.0 a x and the
+// row's first lane adds all terms in stencil order (the order of mg_row_sum), read back
+// through LDS.  Otherwise each lane sums its own, one of RowSum's four chains.  So the
+// sums are those of mg_residual_row and mg_residual_update_row either way.  Measured on
+// a level of 73k rows, one thread per row is faster (14.3 against 18.4 us per ordered
+// sweep, 14.5 against 15.6 us unordered); on levels of 10k rows and fewer the lanes take
+// 20-30% off.  C0 C1 C2 give the
+// stencil at compile time (3x3x3, 3x3x1); 0 0 0 reads it from the level (other shapes),
+// at the price of runtime index arithmetic.
+// t: the thread's number over the level's lanes; tb: kRowTerms doubles per thread of the
+// workgroup (ordered only)
+constexpr int kRowLanes = 4, kRowQ = 7;  // kRowQ: stencil cells per lane (27 / 4, rounded up)
+constexpr int kRowTerms = 3 * kRowQ;
+template <class VT, bool kUpdate, bool kOrd, int C0, int C1, int C2>
+__device__ inline void mg_sweep_lanes(const Level& L, long long t, double* tb) {
+    constexpr int T = kRowTerms;
+    const int u = threadIdx.x & (kRowLanes - 1);
+    const int row = (int)(t / kRowLanes);
+    const bool on = row < L.nrow;
+    const int cs1 = C0 ? C1 : L.cs[1], cs2 = C0 ? C2 : L.cs[2];
+    const int N = (C0 ? C0 : L.cs[0]) * cs1 * cs2, Q = row_chain(N);  // N <= 27
+    const VT* __restrict__ A = sizeof(VT) == 8 ? (const VT*)L.A : (const VT*)L.A32;
+    const double* __restrict__ x = lv_s(L, L.cur);
+    const long long nrow = L.nrow;
+    double a[T], xv[T];
+    if (on) {
+        int gx, gy, gz;
+        grid_xyz(L, row / 3, gx, gy, gz);
+        const int c0 = L.cnt[0], c1 = L.cnt[1], c2 = L.cnt[2];
+#pragma unroll
+        for (int k = 0; k < kRowQ; ++k) {
+            const int q = u * Q + k;
+            if (k < Q && q < N) {
+                const int ex = q / (cs1 * cs2), ey = (q / cs2) % cs1, ez = q % cs2;
+                const int jx = wrap3(gx + ex - 1 + c0, c0), jy = wrap3(gy + ey - 1 + c1, c1);
+                const int jz = wrap3(gz + ez - 1 + c2, c2);
+                const double* xc = x + 3 * ((c1 * c2) * jx + c2 * jy + jz);
+#pragma unroll
+                for (int sd = 0; sd < 3; ++sd) {
+                    a[3 * k + sd] = (double)A[(3 * q + sd) * nrow + row];
+                    xv[3 * k + sd] = xc[sd];
+                }
+            } else {
+#pragma unroll
+                for (int sd = 0; sd < 3; ++sd) a[3 * k + sd] = xv[3 * k + sd] = 0.0;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < T; ++e) a[e] = xv[e] = 0.0;
+    }
+    double sum = 0.0;
+    if constexpr (kOrd) {
+#pragma unroll
+        for (int e = 0; e < T; ++e) tb[T * threadIdx.x + e] = -1.0 * a[e] * xv[e];
+        wave_sync();
+        if (u != 0 || !on) return;
+        for (int v = 0; v < kRowLanes; ++v)
+            for (int k = 0; k < Q && v * Q + k < N; ++k)
+#pragma unroll
+                for (int sd = 0; sd < 3; ++sd) sum += tb[T * (threadIdx.x + v) + 3 * k + sd];
+    } else {
+#pragma unroll
+        for (int e = 0; e < T; ++e) sum = __builtin_fma(-a[e], xv[e], sum);
+        sum += __shfl_xor(sum, 1, 64);
+        sum += __shfl_xor(sum, 2, 64);
+        if (u != 0 || !on) return;
+    }
+    double y = L.Q[row];
+    y *= 1.0;
+    y += sum;
+    L.R[row] = y;
+    if (kUpdate) {
+        double sv = x[row];
+        sv *= 1.0;
+        sv += 1.0 * L.invD[row] * y;
+        lv_s(L, L.cur ^ 1)[row] = sv;
+    }
+}
+
+// restriction (R of 3115-3175): Q_L = 0*Q_L + sum of the clipped 2x2x2 children of R_S,
+// returned
+__device__ inline double mg_restrict_row(const Level& S, const Level& L, int row) {
     const int g = row / 3, rd = row % 3;
     int lx, ly, lz;
     grid_xyz(L, g, lx, ly, lz);
@@ -267,10 +364,8 @@ __device__ inline void mg_restrict_row(const Level& S, const Level& L, int row) 
                                        (2 * lcz + az + fmz) - S.mn[2]);
                 sum += 1.0 * 1.0 * S.R[3 * sg + rd];
             }
-    double y = L.Q[row];
-    y *= 0.0;
-    y += sum;
-    L.Q[row] = y;
+    L.Q[row] = sum;  // Q*0.0 is a zero, the sum never -0
+    return sum;
 }
 
 // prolongation (P of 3216-3241): S_S += injection of the parent's S_L
@@ -404,7 +499,7 @@ struct CoarseShared {
 // level lc-1, which the prolongation updates (of level 0 when lc = 0, written); nio: its
 // rows.  XB: stencil cells whose LDS reads are in flight together.  halt: the CR stop
 // flag or null, tested once the loads are under way.
-template <int N, int T, int XB>
+template <int N, int T, int XB, bool kOrd>
 __device__ inline void mg_coarse_cycle(const CoarsePack& K, int lc, int D, const double* __restrict__ in, double* io,
                                        int nio, const int* halt, CoarseShared<T>& sh) {
     const int tid = threadIdx.x, st = K.stride;
@@ -436,7 +531,8 @@ __device__ inline void mg_coarse_cycle(const CoarsePack& K, int lc, int D, const
     if (cr_halted(halt)) return;
     auto row_sum = [&](const double* x) {  // mg_row_sum
         // XB cells' LDS reads are under way while the XB before them are added
-        double sum = 0.0, xv[2][3 * XB];
+        RowSum<kOrd> sum;
+        double xv[2][3 * XB];
         auto read = [&](int k0, double* v) {
 #pragma unroll
             for (int u = 0; u < XB; ++u)
@@ -454,21 +550,16 @@ __device__ inline void mg_coarse_cycle(const CoarsePack& K, int lc, int D, const
         for (int k0 = 0; k0 < N; k0 += XB) {
             const int h = (k0 / XB) & 1;
             if (k0 + XB < N) read(k0 + XB, xv[h ^ 1]);
-            // reads stay above, then the terms, then the adds: a term formed right before
-            // its add would put the multiply's latency into the chain
-            asm volatile("" : : : "memory");
+            asm volatile("" : : : "memory");  // the reads stay above, the adds below
 #pragma unroll
-            for (int u = 0; u < 3 * XB; ++u)
-                if (3 * k0 + u < 3 * N) {
-                    xv[h][u] = -1.0 * a[3 * k0 + u] * xv[h][u];
-                    asm volatile("" : "+v"(xv[h][u]));
-                }
+            for (int u = 0; u < XB; ++u)
+                if (k0 + u < N)
 #pragma unroll
-            for (int u = 0; u < 3 * XB; ++u)
-                if (3 * k0 + u < 3 * N) sum += xv[h][u];
-            asm volatile("" : "+v"(sum) : : "memory");
+                    for (int sd = 0; sd < 3; ++sd) sum.add(k0 + u, row_chain(N), a[3 * (k0 + u) + sd], xv[h][3 * u + sd]);
+#pragma unroll
+            for (double& c : sum.c) asm volatile("" : "+v"(c) : : "memory");
         }
-        return sum;
+        return sum.total();
     };
     unsigned pc = 0;  // the S buffer of the own level
     auto sweeps = [&](int l, int n) {  // n residual-update sweeps of level l
@@ -546,14 +637,19 @@ __device__ inline void mg_g2p_chunk(const DevParams& P, const Level& L, const in
         const int cx = key / (P.C[1] * P.C[2]) % P.C[0], cy = key / (P.C[2]) % P.C[1], cz = key % P.C[2];
         const int g = grid_id(L, cx - L.mn[0], cy - L.mn[1], cz - L.mn[2]);
         const double* S0 = lv_s(L, L.cur);
-        double uu[3], qq[3];
+        double uu[3], qq[3], z[3], c[3];
         for (int r = 0; r < 3; ++r) {
             qq[r] = q[3 * i + r];
-            double y = u[3 * i + r];
-            y *= 0.0;
-            y += 1.0 * invDiagA[3 * i + r] * qq[r];
+            z[r] = 1.0 * invDiagA[3 * i + r] * qq[r];
+            c[r] = S0[3 * g + r];
+        }
+        // y = u*0.0 + D^-1 q: the zero only matters for the sign of a zero product
+        if (z[0] == 0.0 || z[1] == 0.0 || z[2] == 0.0)
+            for (int r = 0; r < 3; ++r) z[r] += u[3 * i + r] * 0.0;
+        for (int r = 0; r < 3; ++r) {
             double sum = 0.0;
-            sum += 1.0 * 1.0 * S0[3 * g + r];
+            sum += 1.0 * 1.0 * c[r];
+            double y = z[r];
             y *= 1.0;
             y += sum;
             uu[r] = y;
@@ -1263,6 +1359,72 @@ __device__ inline double pq_elem(double beta, double v, double w) {
     v *= beta;
     v += 1.0 * w;
     return v;
+}
+
+// P2G (2964-2997), then begin + update of level 0 on the same row, with kP2gLanes lanes
+// per row: level 0 has one row per cell and component, too few to fill the GPU with one
+// thread each.  Lane u loads q of the cell's particles p0 + u, p0 + u + kP2gLanes, ...
+// (kP2gK per pass).  Ordered: the row's first lane adds them in particle order from
+// LDS.  Otherwise each lane adds its own and a butterfly the lanes' sums.  kPq: the CR
+// loop's q = beta q + y (4364-4366) is formed here as q is loaded and written back
+// (every fluid particle lies in exactly one level-0 cell, so each element is updated
+// once); q is written only then.  tb: 256 * kP2gK doubles of LDS (ordered only).
+// Unordered, with the update, 19.0 us on the 1M scene (72 MB, 3.8 TB/s) and 5.6 us on
+// the 64k drop; ordered 25.2 and 9.8 us, bound by the first lane's chain of adds.
+constexpr int kP2gLanes = 8, kP2gK = 8;
+template <bool kPq, bool kOrd>
+__device__ inline void mg_p2g_lanes(const DevParams& P, const Level& L, const int* __restrict__ cellStart, double* q,
+                                    const double* __restrict__ yv, const double* __restrict__ scal, int block,
+                                    double* tb) {
+    const double beta = kPq ? scal[kRHO] / scal[kRHOP] : 0.0;
+    const int u = threadIdx.x & (kP2gLanes - 1);
+    const int row = (int)(((long long)block * 256 + threadIdx.x) / kP2gLanes);
+    const bool on = row < L.nrow;
+    int p0 = 0, p1 = 0;
+    const int rd = row % 3;
+    if (on) {
+        int gx, gy, gz;
+        grid_xyz(L, row / 3, gx, gy, gz);
+        const int ic = cell_id(P, gx + L.mn[0], gy + L.mn[1], gz + L.mn[2]);
+        p0 = cellStart[ic];
+        p1 = cellStart[ic + 1];
+    }
+    double sum = 0.0;
+    for (int base = p0; base < p1; base += kP2gLanes * kP2gK) {  // the same trips in every lane of the row
+        double t[kP2gK], yt[kP2gK];
+#pragma unroll
+        for (int k = 0; k < kP2gK; ++k) {
+            const int ip = base + u + kP2gLanes * k;
+            t[k] = ip < p1 ? q[3 * ip + rd] : 0.0;
+            yt[k] = kPq && ip < p1 ? yv[3 * ip + rd] : 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < kP2gK; ++k) {
+            const int ip = base + u + kP2gLanes * k;
+            if (kPq && ip < p1) {
+                t[k] = pq_elem(beta, t[k], yt[k]);
+                q[3 * ip + rd] = t[k];
+            }
+        }
+        if constexpr (kOrd) {
+#pragma unroll
+            for (int k = 0; k < kP2gK; ++k) tb[kP2gK * threadIdx.x + k] = t[k];
+            wave_sync();
+            if (u == 0)
+                for (int k = 0; k < kP2gK; ++k)
+                    for (int v = 0; v < kP2gLanes; ++v)
+                        if (base + v + kP2gLanes * k < p1) sum += 1.0 * 1.0 * tb[kP2gK * (threadIdx.x + v) + k];
+            wave_sync();
+        } else {
+#pragma unroll
+            for (int k = 0; k < kP2gK; ++k) sum += t[k];
+        }
+    }
+    if constexpr (!kOrd)
+        for (int m = 1; m < kP2gLanes; m <<= 1) sum += __shfl_xor(sum, m, 64);
+    if (u != 0 || !on) return;
+    L.Q[row] = sum;  // Q*0.0 is a zero, the sum never -0
+    mg_begin_update_row(L, row, sum);
 }
 
 __device__ inline void pq_update_elem(const double* __restrict__ scal, const double* __restrict__ s,

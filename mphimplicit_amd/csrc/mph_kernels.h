@@ -43,6 +43,8 @@ struct Level {  // geometry + storage of one multigrid level
     float* A32;    // FP32 copy of A for the mixed-precision inner solve (or null)
     int f32;       // smoothers read A32 instead of A
     int lanes;     // sweeps split each row over lanes (small levels; set by the host)
+    int ordered;   // sums run in the reference's order (the assembled form, bit for bit);
+                   // 0: in fixed shorter chains (the factored form)
     const int* halt;  // the CR stop flag, as DevParams::halt
 };
 
@@ -58,6 +60,7 @@ struct CoarsePack {
     int* up;     // [rows of level lc-1]: the LDS place of each row's parent
     int stride;  // threads (rows rounded up to whole wavefronts)
     int cells;   // 27, or 9 in 2D
+    int ordered; // Level::ordered
 };
 inline size_t coarse_pack_values(int cells, int stride) { return (size_t)(3 * cells + 1) * stride; }
 inline size_t coarse_pack_ints(int cells, int stride) { return (size_t)((cells + 1) / 2 + 6) * stride; }
@@ -240,7 +243,6 @@ void launch_mg_galerkinL(hipStream_t st, const Level& S, const Level& L);
 void launch_mg_invd(hipStream_t st, const Level& L);
 void launch_fill(hipStream_t st, double* x, long long n, double v);
 void launch_fill_i32(hipStream_t st, int* x, long long n, int v);  // a kernel, not a memset node
-void launch_mg_p2g(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, const double* q);
 void launch_mg_p2g_bu(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, const double* q);
 // the same after q = beta q + y (beta = rho / rho_prev from scal), written back to q
 void launch_mg_p2g_bu_pq(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, double* q,

@@ -471,6 +471,7 @@ int phase_multigrid(mph_scene& S) {
         L.cur = 0;
         L.f32 = 0;
         L.lanes = L.nrow < S.laneRowsMax ? 1 : 0;
+        L.ordered = factored(S) ? 0 : 1;
         L.A32 = nullptr;
         if (mixed(S) && l + 1 < depth) {  // the coarsest level stays FP64
             if ((rc = H.A32.ensure((size_t)L.nrow * L.nshift))) return rc;
@@ -487,6 +488,7 @@ int phase_multigrid(mph_scene& S) {
     if (S.fuse == depth) return fail(MPH_E_STATE, "the coarsest multigrid level exceeds one workgroup");
     CoarsePack& K = S.pack;
     K.cells = P.dim == 2 ? 9 : 27;
+    K.ordered = factored(S) ? 0 : 1;
     K.stride = (rows + 63) / 64 * 64;
     const size_t ni = coarse_pack_ints(K.cells, K.stride), nu = S.fuse > 0 ? S.lv[S.fuse - 1].L.nrow : 0;
     if ((rc = S.packV.ensure(coarse_pack_values(K.cells, K.stride))) || (rc = S.packI.ensure(ni + nu))) return rc;

@@ -223,66 +223,12 @@ __global__ void k_fill_i32(int* x, long long n, int v) {
 // myDcopy / myDscal of the reference: y = beta*y + sum_k (alpha*a_k)*x_k with the
 // sum formed first, y = beta*y + (alpha*d)*x.
 
-__global__ void k_mg_p2g(DevParams P, Level L, const int* __restrict__ cellStart, const double* __restrict__ q) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row < L.nrow) mg_p2g_row(P, L, cellStart, q, row);
-}
-
-// P2G, then begin + update of level 0 on the same row, with kP2gLanes lanes per
-// row: lane u loads q of the cell's particles p0 + u, p0 + u + kP2gLanes, ...
-// (kP2gK per pass), and the row's first lane adds them in particle order from LDS,
-// as mg_p2g_row does.  Level 0 has one row per
-// cell and component, too few to fill the GPU with one thread each.
-// kPq: the CR loop's q = beta q + y (4364-4366) is formed here as q is loaded and
-// written back (every fluid particle lies in exactly one level-0 cell, so each
-// element is updated once); q is written only then.
-constexpr int kP2gLanes = 8, kP2gK = 8;
-template <bool kPq>
-__global__ void __launch_bounds__(256) k_mg_p2g_bu_lanes(DevParams P, Level L, const int* __restrict__ cellStart,
-                                                         double* q, const double* __restrict__ yv,
-                                                         const double* __restrict__ scal) {
+template <bool kPq, bool kOrd>
+__global__ void __launch_bounds__(256) k_mg_p2g_bu(DevParams P, Level L, const int* __restrict__ cellStart, double* q,
+                                                   const double* __restrict__ yv, const double* __restrict__ scal) {
     if (cr_halted(L.halt)) return;
-    __shared__ double tb[256 * kP2gK];
-    const double beta = kPq ? scal[kRHO] / scal[kRHOP] : 0.0;
-    const int u = threadIdx.x & (kP2gLanes - 1);
-    const int row = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / kP2gLanes);
-    const bool on = row < L.nrow;
-    int p0 = 0, p1 = 0;
-    const int rd = row % 3;
-    if (on) {
-        int gx, gy, gz;
-        grid_xyz(L, row / 3, gx, gy, gz);
-        const int ic = cell_id(P, gx + L.mn[0], gy + L.mn[1], gz + L.mn[2]);
-        p0 = cellStart[ic];
-        p1 = cellStart[ic + 1];
-    }
-    double sum = 0.0;
-    for (int base = p0; base < p1; base += kP2gLanes * kP2gK) {  // the same trips in every lane of the row
-        double t[kP2gK];
-#pragma unroll
-        for (int k = 0; k < kP2gK; ++k) {
-            const int ip = base + u + kP2gLanes * k;
-            t[k] = ip < p1 ? q[3 * ip + rd] : 0.0;
-            if (kPq && ip < p1) {
-                t[k] = pq_elem(beta, t[k], yv[3 * ip + rd]);
-                q[3 * ip + rd] = t[k];
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < kP2gK; ++k) tb[kP2gK * threadIdx.x + k] = t[k];
-        wave_sync();
-        if (u == 0)
-            for (int k = 0; k < kP2gK; ++k)
-                for (int v = 0; v < kP2gLanes; ++v)
-                    if (base + v + kP2gLanes * k < p1) sum += 1.0 * 1.0 * tb[kP2gK * (threadIdx.x + v) + k];
-        wave_sync();
-    }
-    if (u != 0 || !on) return;
-    double y = L.Q[row];
-    y *= 0.0;
-    y += sum;
-    L.Q[row] = y;
-    mg_begin_update_row(L, row);
+    __shared__ double tb[kOrd ? 256 * kP2gK : 1];
+    mg_p2g_lanes<kPq, kOrd>(P, L, cellStart, q, yv, scal, blockIdx.x, tb);
 }
 
 // restriction into L, then begin + update of L on the same row
@@ -290,8 +236,7 @@ __global__ void k_mg_restrict_bu(Level S, Level L) {
     if (cr_halted(L.halt)) return;
     const int row = blockIdx.x * blockDim.x + threadIdx.x;
     if (row >= L.nrow) return;
-    mg_restrict_row(S, L, row);
-    mg_begin_update_row(L, row);
+    mg_begin_update_row(L, row, mg_restrict_row(S, L, row));
 }
 
 __global__ void k_mg_begin(Level L) {
@@ -304,84 +249,26 @@ __global__ void k_mg_update(Level L) {
     if (row < L.nrow) mg_update_row(L, row);
 }
 
-template <class VT>
-__global__ void k_mg_residual(Level L) {
+template <class VT, bool kOrd>
+__global__ void __launch_bounds__(256) k_mg_residual(Level L) {
     if (cr_halted(L.halt)) return;
     const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row < L.nrow) mg_residual_row<VT>(L, row);
+    if (row < L.nrow) mg_residual_row<VT, kOrd>(L, row);
 }
 
-template <class VT>
-__global__ void k_mg_residual_update(Level L) {
+template <class VT, bool kOrd>
+__global__ void __launch_bounds__(256) k_mg_residual_update(Level L) {
     if (cr_halted(L.halt)) return;
     const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row < L.nrow) mg_residual_update_row<VT>(L, row);
+    if (row < L.nrow) mg_residual_update_row<VT, kOrd>(L, row);
 }
 
-// The same sweeps with kRowLanes lanes per row, for levels too small to fill the
-// GPU with one thread per row (a row's 81 loads are then latency-bound).  Lane u
-// loads the entries of stencil cells [uQ, (u+1)Q) and forms their terms -1.0 a x;
-// the row's first lane adds all terms in stencil order (the order of mg_row_sum),
-// read back through LDS, so the sums are those of mg_residual_row and
-// mg_residual_update_row.  Measured on a level of 73k rows, one thread per row is
-// faster (14.3 against 18.4 us per sweep); on levels of 10k rows and fewer the lanes
-// take 20-30% off.  C0 C1 C2 give the stencil at compile time (3x3x3, 3x3x1); 0 0 0
-// reads it from the level (other shapes), at the price of runtime index arithmetic.
-constexpr int kRowLanes = 4, kRowBlock = 128, kRowQ = 7;  // kRowQ: stencil cells per lane (27 / 4, rounded up)
-
-template <class VT, bool kUpdate, int C0, int C1, int C2>
+constexpr int kRowBlock = 128;
+template <class VT, bool kUpdate, bool kOrd, int C0, int C1, int C2>
 __global__ void __launch_bounds__(kRowBlock) k_mg_sweep_lanes(Level L) {
     if (cr_halted(L.halt)) return;
-    constexpr int T = 3 * kRowQ;
-    __shared__ double tb[kRowBlock * T];
-    const int u = threadIdx.x & (kRowLanes - 1);
-    const int row = (int)(((long long)blockIdx.x * kRowBlock + threadIdx.x) / kRowLanes);
-    const bool on = row < L.nrow;
-    const int cs1 = C0 ? C1 : L.cs[1], cs2 = C0 ? C2 : L.cs[2];
-    const int N = (C0 ? C0 : L.cs[0]) * cs1 * cs2, Q = (N + kRowLanes - 1) / kRowLanes;  // N <= 27
-    const VT* __restrict__ A = sizeof(VT) == 8 ? (const VT*)L.A : (const VT*)L.A32;
-    const double* __restrict__ x = L.S[L.cur];
-    const long long nrow = L.nrow;
-    double t[T];
-    if (on) {
-        int gx, gy, gz;
-        grid_xyz(L, row / 3, gx, gy, gz);
-        const int c0 = L.cnt[0], c1 = L.cnt[1], c2 = L.cnt[2];
-#pragma unroll
-        for (int k = 0; k < kRowQ; ++k) {
-            const int q = u * Q + k;
-            if (k < Q && q < N) {
-                const int ex = q / (cs1 * cs2), ey = (q / cs2) % cs1, ez = q % cs2;
-                const int jx = wrap3(gx + ex - 1 + c0, c0), jy = wrap3(gy + ey - 1 + c1, c1);
-                const int jz = wrap3(gz + ez - 1 + c2, c2);
-                const double* xc = x + 3 * ((c1 * c2) * jx + c2 * jy + jz);
-#pragma unroll
-                for (int sd = 0; sd < 3; ++sd) t[3 * k + sd] = -1.0 * (double)A[(3 * q + sd) * nrow + row] * xc[sd];
-            } else {
-#pragma unroll
-                for (int sd = 0; sd < 3; ++sd) t[3 * k + sd] = 0.0;
-            }
-        }
-    }
-#pragma unroll
-    for (int e = 0; e < T; ++e) tb[T * threadIdx.x + e] = on ? t[e] : 0.0;
-    wave_sync();
-    if (u != 0 || !on) return;
-    double sum = 0.0;
-    for (int v = 0; v < kRowLanes; ++v)
-        for (int k = 0; k < Q && v * Q + k < N; ++k)
-#pragma unroll
-            for (int sd = 0; sd < 3; ++sd) sum += tb[T * (threadIdx.x + v) + 3 * k + sd];
-    double y = L.Q[row];
-    y *= 1.0;
-    y += sum;
-    L.R[row] = y;
-    if (kUpdate) {
-        double sv = x[row];
-        sv *= 1.0;
-        sv += 1.0 * L.invD[row] * y;
-        L.S[L.cur ^ 1][row] = sv;
-    }
+    __shared__ double tb[kOrd ? kRowBlock * kRowTerms : 1];
+    mg_sweep_lanes<VT, kUpdate, kOrd, C0, C1, C2>(L, (long long)blockIdx.x * kRowBlock + threadIdx.x, tb);
 }
 
 // launches the lane-split sweep on a small level; false for a large one
@@ -390,7 +277,11 @@ bool launch_sweep_lanes(hipStream_t st, const Level& L) {
     if (!L.lanes || L.cs[0] * L.cs[1] * L.cs[2] > kRowLanes * kRowQ) return false;
     const int nb = nblk((long long)kRowLanes * L.nrow, kRowBlock);
     const bool s3 = L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 3, s2 = L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 1;
-#define MPH_SWEEP(VT, A, B, C) hipLaunchKernelGGL((k_mg_sweep_lanes<VT, kUpdate, A, B, C>), dim3(nb), dim3(kRowBlock), 0, st, L)
+#define MPH_SWEEP(VT, A, B, C)                                                                                       \
+    do {                                                                                                             \
+        if (L.ordered) hipLaunchKernelGGL((k_mg_sweep_lanes<VT, kUpdate, true, A, B, C>), dim3(nb), dim3(kRowBlock), 0, st, L); \
+        else hipLaunchKernelGGL((k_mg_sweep_lanes<VT, kUpdate, false, A, B, C>), dim3(nb), dim3(kRowBlock), 0, st, L);          \
+    } while (0)
     if (L.f32) {
         if (s3) MPH_SWEEP(float, 3, 3, 3);
         else if (s2) MPH_SWEEP(float, 3, 3, 1);
@@ -416,11 +307,11 @@ __global__ void k_mg_prolong(Level L, Level S) {
 }
 
 // levels lc..D-1 in one workgroup (mg_coarse_cycle)
-template <int N, int T, int XB>
+template <int N, int T, int XB, bool kOrd>
 __global__ void __launch_bounds__(T) k_mg_coarse(CoarsePack K, int lc, int D, const double* __restrict__ in, double* io,
                                                  int nio, const int* halt) {
     __shared__ CoarseShared<T> sh;
-    mg_coarse_cycle<N, T, XB>(K, lc, D, in, io, nio, halt, sh);
+    mg_coarse_cycle<N, T, XB, kOrd>(K, lc, D, in, io, nio, halt, sh);
 }
 
 __global__ void k_mg_coarse_pack(const Level* __restrict__ lvs, int lc, int D, int f32, CoarsePack K) {
@@ -759,18 +650,22 @@ void launch_fill(hipStream_t st, double* x, long long n, double v) {
 void launch_fill_i32(hipStream_t st, int* x, long long n, int v) {
     if (n > 0) hipLaunchKernelGGL(k_fill_i32, dim3(nblk(n, 256)), dim3(256), 0, st, x, n, v);
 }
-void launch_mg_p2g(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, const double* q) {
-    hipLaunchKernelGGL(k_mg_p2g, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, P, L, cellStart, q);
-}
+static int p2g_blocks(const Level& L) { return nblk((long long)kP2gLanes * L.nrow, 256); }
 void launch_mg_p2g_bu(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, const double* q) {
-    // not written without kPq
-    hipLaunchKernelGGL(k_mg_p2g_bu_lanes<false>, dim3(nblk((long long)kP2gLanes * L.nrow, 256)), dim3(256), 0, st, P,
-                       L, cellStart, const_cast<double*>(q), nullptr, nullptr);
+    double* qw = const_cast<double*>(q);  // not written without kPq
+    if (L.ordered)
+        hipLaunchKernelGGL((k_mg_p2g_bu<false, true>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, qw,
+                           nullptr, nullptr);
+    else
+        hipLaunchKernelGGL((k_mg_p2g_bu<false, false>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, qw,
+                           nullptr, nullptr);
 }
 void launch_mg_p2g_bu_pq(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, double* q,
                          const double* y, const double* scal) {
-    hipLaunchKernelGGL(k_mg_p2g_bu_lanes<true>, dim3(nblk((long long)kP2gLanes * L.nrow, 256)), dim3(256), 0, st, P,
-                       L, cellStart, q, y, scal);
+    if (L.ordered)
+        hipLaunchKernelGGL((k_mg_p2g_bu<true, true>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, q, y, scal);
+    else
+        hipLaunchKernelGGL((k_mg_p2g_bu<true, false>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, q, y, scal);
 }
 void launch_mg_restrict_bu(hipStream_t st, const Level& S, Level& L) {
     hipLaunchKernelGGL(k_mg_restrict_bu, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, S, L);
@@ -781,18 +676,22 @@ void launch_mg_begin(hipStream_t st, Level& L) {
 void launch_mg_update(hipStream_t st, Level& L) {
     hipLaunchKernelGGL(k_mg_update, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
 }
+#define MPH_ROWS(KERNEL)                                                                                           \
+    do {                                                                                                           \
+        const int nb = nblk(L.nrow, 256);                                                                          \
+        if (L.f32 && L.ordered) hipLaunchKernelGGL((KERNEL<float, true>), dim3(nb), dim3(256), 0, st, L);          \
+        else if (L.f32) hipLaunchKernelGGL((KERNEL<float, false>), dim3(nb), dim3(256), 0, st, L);                 \
+        else if (L.ordered) hipLaunchKernelGGL((KERNEL<double, true>), dim3(nb), dim3(256), 0, st, L);             \
+        else hipLaunchKernelGGL((KERNEL<double, false>), dim3(nb), dim3(256), 0, st, L);                           \
+    } while (0)
 void launch_mg_residual(hipStream_t st, Level& L) {
-    if (launch_sweep_lanes<false>(st, L)) return;
-    if (L.f32) hipLaunchKernelGGL(k_mg_residual<float>, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
-    else hipLaunchKernelGGL(k_mg_residual<double>, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
+    if (!launch_sweep_lanes<false>(st, L)) MPH_ROWS(k_mg_residual);
 }
 void launch_mg_residual_update(hipStream_t st, Level& L) {
-    if (!launch_sweep_lanes<true>(st, L)) {
-        if (L.f32) hipLaunchKernelGGL(k_mg_residual_update<float>, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
-        else hipLaunchKernelGGL(k_mg_residual_update<double>, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
-    }
+    if (!launch_sweep_lanes<true>(st, L)) MPH_ROWS(k_mg_residual_update);
     L.cur ^= 1;
 }
+#undef MPH_ROWS
 void launch_mg_restrict(hipStream_t st, const Level& S, Level& L) {
     hipLaunchKernelGGL(k_mg_restrict, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, S, L);
 }
@@ -805,8 +704,13 @@ void launch_mg_coarse_pack(hipStream_t st, const Level* lvs, int lc, int D, bool
 void launch_mg_coarse(hipStream_t st, const DevParams& P, const CoarsePack& K, int lc, int D, const Level& S) {
     const double* in = lc == 0 ? S.Q : S.R;
     double* io = S.S[lc == 0 ? S.cur ^ 1 : S.cur];
-#define MPH_COARSE(N, T, XB) \
-    hipLaunchKernelGGL((k_mg_coarse<N, T, XB>), dim3(1), dim3(K.stride), 0, st, K, lc, D, in, io, S.nrow, P.halt)
+#define MPH_COARSE(N, T, XB)                                                                                         \
+    do {                                                                                                             \
+        if (K.ordered)                                                                                               \
+            hipLaunchKernelGGL((k_mg_coarse<N, T, XB, true>), dim3(1), dim3(K.stride), 0, st, K, lc, D, in, io, S.nrow, P.halt); \
+        else                                                                                                         \
+            hipLaunchKernelGGL((k_mg_coarse<N, T, XB, false>), dim3(1), dim3(K.stride), 0, st, K, lc, D, in, io, S.nrow, P.halt); \
+    } while (0)
     if (K.cells == 9) MPH_COARSE(9, kCoarseRows2D, 4);
     else if (K.stride <= 256) MPH_COARSE(27, 256, 9);
     else MPH_COARSE(27, kCoarseRows3D, 4);
