@@ -14,6 +14,7 @@ namespace {
 
 constexpr int kSortBlock = 2048;  // keys per LDS block (16 KiB)
 constexpr int kSortThreads = 256;
+constexpr int kScanShare = 32768;  // particles from which four share a wavefront of the neighbour search
 
 __device__ inline int cell_id(const DevParams& P, int cx, int cy, int cz) {  // CellId, main.cpp:109-113
     const int* C = P.C;
@@ -139,122 +140,195 @@ __global__ void k_reorder(DevParams P, const uint64_t* __restrict__ keys, const 
     }
 }
 
-// The neighbour cells of particle i in the reference's visiting order
-// (main.cpp:1410-1445): ascending CellId.  `visit(lo, hi)` receives particle ranges.
-template <bool kFluid, class F>
-__device__ inline void for_cells(const DevParams& P, const int* __restrict__ cellStart, int key, F&& visit) {
-    const int* C = P.C;
-    const int rx = P.range[0], ry = P.range[1], rz = P.range[2];
-    const int icx = (key / (C[1] * C[2])) % P.T;
-    const int icy = (key / C[2]) % C[1];
-    const int icz = key % C[2];
-    int jx[3], jy[3], jz[3];
-    for (int k = 0; k < 2 * rx + 1; ++k) jx[k] = ((icx - rx + k) % C[0] + C[0]) % C[0];
-    for (int k = 0; k < 2 * ry + 1; ++k) jy[k] = ((icy - ry + k) % C[1] + C[1]) % C[1];
-    for (int k = 0; k < 2 * rz + 1; ++k) jz[k] = ((icz - rz + k) % C[2] + C[2]) % C[2];
-    const int bx = (2 * rx) - (icx + rx) % C[0], by = (2 * ry) - (icy + ry) % C[1], bz = (2 * rz) - (icz + rz) % C[2];
-    const int x0 = bx > 0 ? bx : 0, y0 = by > 0 ? by : 0, z0 = bz > 0 ? bz : 0;
-    for (int a = x0; a < x0 + (2 * rx + 1); ++a)
-        for (int b = y0; b < y0 + (2 * ry + 1); ++b)
-            for (int c = z0; c < z0 + (2 * rz + 1); ++c) {
-                const int jc = cell_id(P, jx[a % (2 * rx + 1)], jy[b % (2 * ry + 1)], jz[c % (2 * rz + 1)]);
-                const int off = kFluid ? 0 : P.T;
-                visit(cellStart[off + jc], cellStart[off + jc + 1]);
-            }
-}
+// what the neighbour search writes (main.cpp:1406-1511, 1567-1666).  Count pass: the
+// counts, `most` and, with lists, the lists themselves in
+// per-particle scratch of capM / capP entries; a particle with more raises *overflow,
+// which sends the search to the fill pass.  Fill pass: the lists at ptrM / ptrP.
+// runStart: for fluid particles where the fluid neighbours of each visited cell start in
+// the list (runStart[i][q], q in visiting order, runStart[i][ncells] = fluid count); the
+// multigrid level-0 build reads these runs directly.
+struct NeighborOut {
+    int *nCount, *nFluid, *nCountP;
+    int* most;  // [0], [1]: largest P and fluid count of a fluid particle (they size the LDS staging of
+                // the C Lambda C^T kernel and the A rows); [2], [3]: largest count and P count of any
+    int *listM, *listP;
+    int capM, capP;
+    const long long *ptrM, *ptrP;
+    unsigned short* runStart;
+    int* overflow;
+};
 
-// visit(j, q2) with q2 the squared minimum-image distance of candidate j to
-// (xi, yi, zi), for j = lo..hi-1 in ascending order.  The coordinates of eight
-// candidates are loaded together before the first min_image: its branch (the division
-// of the wrapped case) would otherwise hold each load back until the previous
-// coordinate is done.  Past hi the loads repeat candidate hi-1, which is not visited.
-// (Per step on the 1M scene: 3.56 ms with two candidates, 3.35 with four, 3.21 with
-// eight, at four waves per SIMD in each case.)
-template <class V>
-__device__ inline void scan_range(const DevParams& P, const double* __restrict__ pos, double xi, double yi, double zi,
-                                  int lo, int hi, V&& visit) {
-    constexpr int U = 8;
-    for (int j0 = lo; j0 < hi; j0 += U) {
-        double c[U][3];
+// One wavefront scans the candidates of U consecutive particles, 64 at a time: the hits'
+// ballot gives every lane its place in the list, so the lists come out in the visiting
+// order (ascending CellId, main.cpp:1410-1445) with coalesced stores.  Visited cells that
+// hold consecutive particles (the three along z) are scanned as one range of about 120
+// candidates; U particles of one cell share its ranges and the candidates' coordinates.
+// A particle per thread walked its 1100 candidates in series: 460 us for the smallest
+// scene, 17 us now; at 1.3M particles its strided list stores also cost, 2.60 ms
+// against 2.15 ms (U = 4).
+template <int U, bool kFill>
+__global__ void __launch_bounds__(256) k_neighbors(DevParams P, const double* __restrict__ pos,
+                                                   const int* __restrict__ cellIndex,
+                                                   const int* __restrict__ cellStart, NeighborOut O) {
+    const int lane = threadIdx.x & 63;
+    const int i0 = __builtin_amdgcn_readfirstlane((int)(((long long)blockIdx.x * 256 + threadIdx.x) >> 6) * U);
+    if (i0 >= P.np) return;
+    const int left = P.np - i0 < U ? P.np - i0 : U;
+    double xi[U][3];
+    int key[U], n[U], nfl[U], npp[U], rc[U];
+    int *lm[U], *lp[U];
+    const bool lists = O.listM != nullptr;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int j = j0 + u < hi ? j0 + u : hi - 1;
-            c[u][0] = pos[3 * j];
-            c[u][1] = pos[3 * j + 1];
-            c[u][2] = pos[3 * j + 2];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (j0 + u >= hi) break;
-            const double q0 = min_image(c[u][0], xi, P.W[0], P.hW[0]);
-            const double q1 = min_image(c[u][1], yi, P.W[1], P.hW[1]);
-            const double q2 = min_image(c[u][2], zi, P.W[2], P.hW[2]);
-            visit(j0 + u, q0 * q0 + q1 * q1 + q2 * q2);
-        }
+    for (int u = 0; u < U; ++u) {
+        const int i = i0 + (u < left ? u : 0);
+        for (int d = 0; d < 3; ++d) xi[u][d] = pos[3 * (long long)i + d];
+        key[u] = cellIndex[i];
+        lm[u] = O.listM + (kFill ? O.ptrM[i] : (long long)i * O.capM);
+        lp[u] = O.listP + (kFill ? O.ptrP[i] : (long long)i * O.capP);
+        n[u] = nfl[u] = npp[u] = rc[u] = 0;
     }
-}
-
-// count pass, main.cpp:1406-1511; also the largest P-neighbour count of a fluid
-// particle (it sizes the LDS staging of the C Lambda C^T kernel), the largest counts
-// of any particle (they size the scratch lists of the next search), and, when scrM is
-// set, the lists themselves: the hits go in visiting order into per-particle scratch
-// of capM / capP entries (runStart as the fill pass writes it), and a particle with
-// more raises *overflow, which sends the search to the fill pass.
-__global__ void k_neighbor_count(DevParams P, const double* __restrict__ pos, const int* __restrict__ cellIndex,
-                                 const int* __restrict__ cellStart, int* __restrict__ nCount,
-                                 int* __restrict__ nFluid, int* __restrict__ nCountP, int* __restrict__ maxFluidP,
-                                 int* __restrict__ scrM, int capM, int* __restrict__ scrP, int capP,
-                                 unsigned short* __restrict__ runStart, int* __restrict__ overflow) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= P.np) return;
-    const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-    const int key = cellIndex[i];
-    int n = 0, nfl = 0, npp = 0;
-    int* sm = scrM ? scrM + (long long)i * capM : nullptr;
-    int* sp = scrM ? scrP + (long long)i * capP : nullptr;
-    unsigned short* rs = scrM && i < P.nf ? runStart + (long long)i * kRuns : nullptr;
-    int q = 0;
-    for_cells<true>(P, cellStart, key, [&](int lo, int hi) {
-        if (rs) rs[q] = (unsigned short)n;
-        q++;
-        scan_range(P, pos, xi, yi, zi, lo, hi, [&](int j, double q2) {
-            if (q2 <= P.maxR2) {
-                if (sm && n < capM) sm[n] = j;
-                n++;
-                nfl++;
-                if (q2 <= P.radP2) {
-                    if (sp && npp < capP) sp[npp] = j;
-                    npp++;
+    const int* C = P.C;
+    const int nx = 2 * P.range[0] + 1, ny = 2 * P.range[1] + 1, nz = 2 * P.range[2] + 1, nv = nx * ny * nz;
+    const double in0 = 0.4 * P.hW[0], in1 = 0.4 * P.hW[1], in2 = 0.4 * P.hW[2];
+    unsigned todo = (1u << left) - 1;
+    while (todo) {  // the particles of one cell at a time
+        int k = key[0];
+#pragma unroll
+        for (int u = U - 1; u >= 0; --u)
+            if (todo >> u & 1) k = key[u];
+        unsigned set = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if ((todo >> u & 1) && key[u] == k) set |= 1u << u;
+        todo &= ~set;
+        // lane q < nv: the particle ranges of visited cell q, fluid and wall
+        int lo[2] = {0, 0}, hi[2] = {0, 0};
+        if (lane < nv) {
+            const int cx = (k / (C[1] * C[2])) % P.T, cy = (k / C[2]) % C[1], cz = k % C[2];
+            const int bx = 2 * P.range[0] - (cx + P.range[0]) % C[0], by = 2 * P.range[1] - (cy + P.range[1]) % C[1];
+            const int bz = 2 * P.range[2] - (cz + P.range[2]) % C[2];
+            const int a = ((bx > 0 ? bx : 0) + lane / (ny * nz)) % nx, b = ((by > 0 ? by : 0) + (lane / nz) % ny) % ny;
+            const int c = ((bz > 0 ? bz : 0) + lane % nz) % nz;
+            const int jc = cell_id(P, cx - P.range[0] + a, cy - P.range[1] + b, cz - P.range[2] + c);
+            lo[0] = cellStart[jc];
+            hi[0] = cellStart[jc + 1];
+            lo[1] = cellStart[P.T + jc];
+            hi[1] = cellStart[P.T + jc + 1];
+        }
+        int off = hi[0] - lo[0];  // fluid candidates before cell `lane`
+        for (int d = 1; d < 32; d <<= 1) {
+            const int v = __shfl_up(off, d, 64);
+            if (lane >= d) off += v;
+        }
+        off = lane < nv ? off - (hi[0] - lo[0]) : 0x7fffffff;
+#pragma unroll
+        for (int wall = 0; wall < 2; ++wall) {
+            if (wall) {
+                // walls without fluid neighbours skip the wall scan (main.cpp:1474); walls
+                // occupy [nf, np) after every sort
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (!(set >> u & 1)) continue;
+                    nfl[u] = n[u];
+                    if (i0 + u >= P.nf && n[u] == 0) set &= ~(1u << u);
                 }
+                if (!set) break;
             }
-        });
-    });
-    if (rs) rs[q] = (unsigned short)n;
-    // walls without fluid neighbours skip the wall scan (main.cpp:1474); walls
-    // occupy [nf, np) after every sort
-    if (!(i >= P.nf && n == 0))
-        for_cells<false>(P, cellStart, key, [&](int lo, int hi) {
-            scan_range(P, pos, xi, yi, zi, lo, hi, [&](int j, double q2) {
-                if (q2 <= P.maxR2) {
-                    if (sm && n < capM) sm[n] = j;
-                    n++;
-                    if (q2 <= P.radP2) {
-                        if (sp && npp < capP) sp[npp] = j;
-                        npp++;
+            const int before = __shfl_up(hi[wall], 1, 64);
+            unsigned long long starts = __ballot(lane < nv && (lane == 0 || lo[wall] != before));
+            int flat = 0;
+            while (starts) {
+                const int s = __builtin_ctzll(starts);
+                starts &= starts - 1;
+                const int e = starts ? __builtin_ctzll(starts) : nv;
+                const int jlo = __builtin_amdgcn_readlane(lo[wall], s);
+                const int jhi = __builtin_amdgcn_readlane(hi[wall], e - 1);
+                for (int j0 = jlo; j0 < jhi; j0 += 128) {
+                    double c[2][3];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {  // past the end: candidate jhi - 1, not taken
+                        const int j = j0 + 64 * h + lane < jhi ? j0 + 64 * h + lane : jhi - 1;
+                        for (int d = 0; d < 3; ++d) c[h][d] = pos[3 * (long long)j + d];
+                    }
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int j = j0 + 64 * h + lane;
+                        if (h && j0 + 64 >= jhi) break;
+                        unsigned long long below = 0;  // the chunk's candidates before cell `lane`
+                        if (!wall) {
+                            const int b = off - flat;
+                            below = b <= 0 ? 0 : b >= 64 ? ~0ull : (1ull << b) - 1;
+                            flat += 64;  // only the last chunk of a range is shorter
+                            if (j0 + 64 * (h + 1) > jhi) flat -= j0 + 64 * (h + 1) - jhi;
+                        }
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            if (!(set >> u & 1)) continue;
+                            // min_image of a difference well inside the box is (e + hw) - hw; one
+                            // branch for the wavefront instead of one per coordinate
+                            double q0 = c[h][0] - xi[u][0], q1 = c[h][1] - xi[u][1], q2 = c[h][2] - xi[u][2];
+                            const bool near = fabs(q0) <= in0 && fabs(q1) <= in1 && fabs(q2) <= in2;
+                            if (__ballot(!near) == 0) {
+                                q0 = q0 + P.hW[0] - P.hW[0];
+                                q1 = q1 + P.hW[1] - P.hW[1];
+                                q2 = q2 + P.hW[2] - P.hW[2];
+                            } else {
+                                q0 = min_image(c[h][0], xi[u][0], P.W[0], P.hW[0]);
+                                q1 = min_image(c[h][1], xi[u][1], P.W[1], P.hW[1]);
+                                q2 = min_image(c[h][2], xi[u][2], P.W[2], P.hW[2]);
+                            }
+                            const double r2 = q0 * q0 + q1 * q1 + q2 * q2;
+                            const bool hit = j < jhi && r2 <= P.maxR2, hitP = hit && r2 <= P.radP2;
+                            const unsigned long long M = __ballot(hit), MP = __ballot(hitP);
+                            if (kFill || lists) {
+                                const int at = n[u] + __builtin_amdgcn_mbcnt_hi((unsigned)(M >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo((unsigned)M, 0));
+                                const int atP = npp[u] + __builtin_amdgcn_mbcnt_hi((unsigned)(MP >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((unsigned)MP, 0));
+                                if (hit && (kFill || at < O.capM)) lm[u][at] = j;
+                                if (hitP && (kFill || atP < O.capP)) lp[u][atP] = j;
+                                if (!wall) rc[u] += __popcll(M & below);
+                            }
+                            n[u] += __popcll(M);
+                            npp[u] += __popcll(MP);
+                        }
                     }
                 }
-            });
-        });
-    nCount[i] = n;
-    nFluid[i] = nfl;
-    nCountP[i] = npp;
-    if (i < P.nf) {
-        atomicMax(maxFluidP, npp);      // [0]: largest P-neighbour count of a fluid particle
-        atomicMax(maxFluidP + 1, nfl);  // [1]: largest fluid-neighbour count (A row length)
+            }
+        }
     }
-    atomicMax(maxFluidP + 2, n);    // [2]: largest neighbour count
-    atomicMax(maxFluidP + 3, npp);  // [3]: largest P-neighbour count
-    if (sm && (n > capM || npp > capP)) atomicOr(overflow, 1);
+    if (kFill || lists)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < left && i0 + u < P.nf && lane <= nv) O.runStart[(long long)(i0 + u) * kRuns + lane] = (unsigned short)rc[u];
+    if (kFill) return;
+    int m[4] = {0, 0, 0, 0}, vn = 0, vf = 0, vp = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (u >= left) continue;
+        if (i0 + u < P.nf) {
+            m[0] = npp[u] > m[0] ? npp[u] : m[0];
+            m[1] = nfl[u] > m[1] ? nfl[u] : m[1];
+        }
+        m[2] = n[u] > m[2] ? n[u] : m[2];
+        m[3] = npp[u] > m[3] ? npp[u] : m[3];
+        if (lane == u) {
+            vn = n[u];
+            vf = nfl[u];
+            vp = npp[u];
+        }
+    }
+    if (lane < left) {
+        O.nCount[i0 + lane] = vn;
+        O.nFluid[i0 + lane] = vf;
+        O.nCountP[i0 + lane] = vp;
+    }
+    if (lane < 4) {  // few wavefronts raise a maximum: look before the atomic
+        const int v = lane == 0 ? m[0] : lane == 1 ? m[1] : lane == 2 ? m[2] : m[3];
+        if (v > __hip_atomic_load(&O.most[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(&O.most[lane], v);
+    }
+    if (lists && lane == 0 && (m[2] > O.capM || m[3] > O.capP)) atomicOr(O.overflow, 1);
 }
 
 // the lists from the scratch of the count pass, 32 lanes per particle (coalesced)
@@ -275,40 +349,6 @@ __global__ void __launch_bounds__(256) k_neighbor_compact(DevParams P, const int
     const int* sp = scrP + (long long)i * capP;
     for (int k = g; k < n; k += G) nInd[b + k] = sm[k];
     for (int k = g; k < npp; k += G) nIndP[bp + k] = sp[k];
-}
-
-// fill pass, main.cpp:1567-1666.  For fluid particles it also records where the
-// fluid neighbours of each visited cell start in the list (runStart[i][q], q in
-// visiting order, runStart[i][ncells] = fluid count): the multigrid level-0 build
-// reads these runs directly.
-__global__ void k_neighbor_fill(DevParams P, const double* __restrict__ pos, const int* __restrict__ cellIndex,
-                                const int* __restrict__ cellStart, const int* __restrict__ nCount,
-                                const long long* __restrict__ nPtr, const long long* __restrict__ nPtrP,
-                                int* __restrict__ nInd, int* __restrict__ nIndP,
-                                unsigned short* __restrict__ runStart) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= P.np) return;
-    const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-    const int key = cellIndex[i];
-    long long k = nPtr[i], kp = nPtrP[i];
-    auto put = [&](int lo, int hi) {
-        scan_range(P, pos, xi, yi, zi, lo, hi, [&](int j, double q2) {
-            if (q2 <= P.maxR2) {
-                nInd[k++] = j;
-                if (q2 <= P.radP2) nIndP[kp++] = j;
-            }
-        });
-    };
-    unsigned short* rs = i < P.nf ? runStart + (long long)i * kRuns : nullptr;
-    int q = 0;
-    const long long k0 = k;
-    for_cells<true>(P, cellStart, key, [&](int lo, int hi) {
-        if (rs) rs[q] = (unsigned short)(k - k0);
-        q++;
-        put(lo, hi);
-    });
-    if (rs) rs[q] = (unsigned short)(k - k0);
-    if (!(i >= P.nf && nCount[i] == 0)) for_cells<false>(P, cellStart, key, put);
 }
 
 // ---- exclusive scan of int counts into int64 offsets (out[0]=0, out[n]=total) ----
@@ -424,11 +464,28 @@ void launch_reorder(hipStream_t st, const DevParams& P, const uint64_t* keys, co
                        perm2, pos2, vel2, cellIndex);
 }
 
+namespace {
+
+// particles per wavefront: four share their cell's candidates where the scene fills the
+// GPU's 8192 wavefronts several times over all the same, one otherwise
+template <bool kFill>
+void neighbors(hipStream_t st, const DevParams& P, const double* pos, const int* cellIndex, const int* cellStart,
+               const NeighborOut& O) {
+    if (P.np >= kScanShare)
+        hipLaunchKernelGGL((k_neighbors<4, kFill>), dim3(nblk(64LL * ((P.np + 3) / 4), 256)), dim3(256), 0, st, P, pos,
+                           cellIndex, cellStart, O);
+    else
+        hipLaunchKernelGGL((k_neighbors<1, kFill>), dim3(nblk(64LL * P.np, 256)), dim3(256), 0, st, P, pos, cellIndex,
+                           cellStart, O);
+}
+
+}  // namespace
+
 void launch_neighbor_count(hipStream_t st, const DevParams& P, const double* pos, const int* cellIndex,
                            const int* cellStart, int* nCount, int* nFluid, int* nCountP, int* maxFluidP, int* scrM,
                            int capM, int* scrP, int capP, unsigned short* runStart, int* overflow) {
-    hipLaunchKernelGGL(k_neighbor_count, dim3(nblk(P.np, 128)), dim3(128), 0, st, P, pos, cellIndex, cellStart,
-                       nCount, nFluid, nCountP, maxFluidP, scrM, capM, scrP, capP, runStart, overflow);
+    neighbors<false>(st, P, pos, cellIndex, cellStart,
+                     {nCount, nFluid, nCountP, maxFluidP, scrM, scrP, capM, capP, nullptr, nullptr, runStart, overflow});
 }
 
 void launch_neighbor_compact(hipStream_t st, const DevParams& P, const int* nCount, const int* nCountP,
@@ -439,10 +496,10 @@ void launch_neighbor_compact(hipStream_t st, const DevParams& P, const int* nCou
 }
 
 void launch_neighbor_fill(hipStream_t st, const DevParams& P, const double* pos, const int* cellIndex,
-                          const int* cellStart, const int* nCount, const long long* nPtr, const long long* nPtrP,
-                          int* nInd, int* nIndP, unsigned short* runStart) {
-    hipLaunchKernelGGL(k_neighbor_fill, dim3(nblk(P.np, 128)), dim3(128), 0, st, P, pos, cellIndex, cellStart,
-                       nCount, nPtr, nPtrP, nInd, nIndP, runStart);
+                          const int* cellStart, const long long* nPtr, const long long* nPtrP, int* nInd, int* nIndP,
+                          unsigned short* runStart) {
+    neighbors<true>(st, P, pos, cellIndex, cellStart,
+                    {nullptr, nullptr, nullptr, nullptr, nInd, nIndP, 0, 0, nPtr, nPtrP, runStart, nullptr});
 }
 
 int scan_scratch_len(int n) { return nblk(n > 0 ? n : 1, kScanTile); }

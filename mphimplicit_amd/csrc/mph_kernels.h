@@ -192,8 +192,8 @@ void launch_neighbor_compact(hipStream_t st, const DevParams& P, const int* nCou
 void launch_scan_i64(hipStream_t st, const int* in, long long* out, int n, long long* scratch, int scratch_len);
 int scan_scratch_len(int n);
 void launch_neighbor_fill(hipStream_t st, const DevParams& P, const double* pos, const int* cellIndex,
-                          const int* cellStart, const int* nCount, const long long* nPtr, const long long* nPtrP,
-                          int* nInd, int* nIndP, unsigned short* runStart);
+                          const int* cellStart, const long long* nPtr, const long long* nPtrP, int* nInd, int* nIndP,
+                          unsigned short* runStart);
 void launch_slice_width(hipStream_t st, int nf, int nslices, const int* nFluid, int* width);
 // ---- kinematics and explicit forces ----
 void launch_kinematics(hipStream_t st, const DevParams& P, const WallKin& wk, const int* type, double* pos,

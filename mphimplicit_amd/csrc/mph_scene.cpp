@@ -324,8 +324,8 @@ int phase_neighbor_finish(mph_scene& S) {
         launch_neighbor_compact(S.st, P, S.nCount.p, S.nCountP.p, S.nPtr.p, S.nPtrP.p, S.scrM.p, S.searchCapM,
                                 S.scrP.p, S.searchCapP, S.nInd.p, S.nIndP.p);
     else
-        launch_neighbor_fill(S.st, P, S.pos.p, S.cellIndex.p, S.cellStart.p, S.nCount.p, S.nPtr.p, S.nPtrP.p,
-                             S.nInd.p, S.nIndP.p, S.runStart.p);
+        launch_neighbor_fill(S.st, P, S.pos.p, S.cellIndex.p, S.cellStart.p, S.nPtr.p, S.nPtrP.p, S.nInd.p,
+                             S.nIndP.p, S.runStart.p);
     return MPH_OK;
 }
 
