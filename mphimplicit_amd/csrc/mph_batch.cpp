@@ -150,7 +150,9 @@ int build_tables(mph_batch& B, const std::vector<mph_scene*>& sc, Tables& T, boo
         put(kOffCell, B.cell[s] ? (int)cells : 0);
         put(kOffChunk, (S.P.nf + 255) / 256);
         put(kOffElem, (int)((3LL * S.P.nf + 255) / 256));
-        put(kOffPart, (S.P.np + 255) / 256);
+        put(kOffRowsT, (S.P.np + kFacRowsT - 1) / kFacRowsT);
+        put(kOffRowsT32, (S.P.np + kFacRowsY - 1) / kFacRowsY);
+        put(kOffRowsY, (S.P.nf + kFacRowsY - 1) / kFacRowsY);
         put(kOffP2g, b.mg ? (8 * b.lv[0].nrow + 255) / 256 : 0);
         for (int l = 0; l < b.depth; ++l) {
             put(kOffLevel + l, (b.lv[l].nrow + 255) / 256);

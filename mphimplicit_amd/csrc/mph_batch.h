@@ -18,17 +18,20 @@ constexpr int kMaxScenes = 256;  // bits of a SceneSet
 enum { kX = 0, kR, kS, kY, kP, kQ, kU, kB, kROut, kD, kNVec };
 
 // rows of the block-offset table: 256-particle chunks of the fluid particles,
-// 256-element blocks of the 3*nf vectors, 256-particle blocks of all particles, the
-// fluid bounding box's cells (the cell-staged factored pass; 0 for the other
-// scenes), the blocks of the P2G (8 lanes per level-0 row), then per multigrid level its
-// 256-row blocks and the blocks of its sweeps (4 lanes per row where Level::lanes)
+// 256-element blocks of the 3*nf vectors, the fluid bounding box's cells (the
+// cell-staged factored pass; 0 for the other scenes), the workgroups of the factored
+// first pass (FP64, FP32) and of its second pass over rows, the blocks of the P2G (8
+// lanes per level-0 row), then per multigrid level its 256-row blocks and the blocks of
+// its sweeps (4 lanes per row where Level::lanes)
 enum {
     kOffChunk = 0,
     kOffElem = 1,
-    kOffPart = 2,
-    kOffCell = 3,
-    kOffP2g = 4,
-    kOffLevel = 5,
+    kOffCell = 2,
+    kOffRowsT = 3,
+    kOffRowsT32 = 4,
+    kOffRowsY = 5,
+    kOffP2g = 6,
+    kOffLevel = 7,
     kOffSweep = kOffLevel + kMaxLevels,
     kOffRows = kOffSweep + kMaxLevels
 };

@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(256) kb_spmv(const BScene* tab, const int* off
 
 template <class VT>
 __global__ void __launch_bounds__(256) kb_fac_t(const BScene* tab, const int* off, int ns, SceneSet on, int x) {
-    MPH_SCENE(kOffPart)
+    MPH_SCENE(sizeof(VT) == 4 ? kOffRowsT32 : kOffRowsT)
     const FacOp& F = B.fac[sizeof(VT) == 4 ? 1 : 0];
     if constexpr (sizeof(VT) == 4) fac_t32_chunk(B.P, F, B.vec[x], lb);
     else if (*F.wrap) fac_t_chunk<true>(B.P, F, B.vec[x], lb);
@@ -81,21 +81,14 @@ __global__ void __launch_bounds__(256) kb_fac_t(const BScene* tab, const int* of
 template <bool kNeg, class VT>
 __global__ void __launch_bounds__(256) kb_fac_y(const BScene* tab, const int* off, int ns, SceneSet on,
                                                 SceneSet first, int x, double beta, int yin, int y, int y2,
-                                                int p_copy, int dot) {
-    __shared__ double sh[256];
-    __shared__ double rows[3 * 256];
-    MPH_SCENE(kOffChunk)
+                                                int p_copy) {
+    MPH_SCENE(kOffRowsY)
     const bool f = in_set(first, s);
     const FacOp& F = B.fac[sizeof(VT) == 4 ? 1 : 0];
     double* y2p = f && y2 >= 0 ? B.vec[y2] : nullptr;
     double* pc = f && p_copy >= 0 ? B.vec[p_copy] : nullptr;
-    const double* dx = dot >= 0 ? B.vec[dot] : nullptr;
-    double* pt = dot >= 0 ? B.part : nullptr;
-    if constexpr (sizeof(VT) == 4) {
-        fac_y32_chunk<kNeg>(B.P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, dx, pt, lb, sh, rows);
-    } else {
-        fac_y_chunk_any<kNeg>(B.P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, dx, pt, lb, sh, rows);
-    }
+    if constexpr (sizeof(VT) == 4) fac_y32_chunk<kNeg>(B.P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, lb);
+    else fac_y_chunk_any<kNeg>(B.P, F, B.vec[x], beta, B.vec[yin], B.vec[y], y2p, pc, lb);
 }
 
 __global__ void __launch_bounds__(256) kb_dot_partial(const BScene* tab, const int* off, int ns, SceneSet on,
@@ -346,16 +339,14 @@ void spmv_fac(const Tables& T, const SceneSet& all, const SceneSet& first, const
               bool f32, double alpha, int x, double beta, int yin, int y, int y2, int p_copy, int dot) {
     SceneSet on = all, staged{};
     for (int k = 0; k < kMaxScenes / 64; ++k) staged.w[k] = f32 ? 0 : all.w[k] & cells.w[k];
-    if (f32) MPH_LAUNCH(kb_fac_t<float>, kOffPart, x);
-    else MPH_LAUNCH(kb_fac_t<double>, kOffPart, x);
-    if (any(staged)) {  // the cell-staged pass, then its dot partials
+    if (f32) MPH_LAUNCH(kb_fac_t<float>, kOffRowsT32, x);
+    else MPH_LAUNCH(kb_fac_t<double>, kOffRowsT, x);
+    if (any(staged)) {
         spmv_fac_cells(T, staged, shapes, first, alpha, x, beta, yin, y, y2, p_copy);
-        on = staged;
-        if (dot >= 0) MPH_LAUNCH(kb_dot_partial, kOffChunk, dot, y);
-        on = all;
         for (int k = 0; k < kMaxScenes / 64; ++k) on.w[k] &= ~staged.w[k];
     }
-#define MPH_FAC(NEG, VT) MPH_LAUNCH((kb_fac_y<NEG, VT>), kOffChunk, first, x, beta, yin, y, y2, p_copy, dot)
+#define MPH_FAC(NEG, VT) \
+    MPH_LAUNCH((kb_fac_y<NEG, VT>), kOffRowsY, first, x, beta, yin, y, y2, p_copy)
     if (f32) {
         if (alpha < 0) MPH_FAC(true, float);
         else MPH_FAC(false, float);
@@ -364,6 +355,8 @@ void spmv_fac(const Tables& T, const SceneSet& all, const SceneSet& first, const
         else MPH_FAC(false, double);
     }
 #undef MPH_FAC
+    on = all;
+    if (dot >= 0) MPH_LAUNCH(kb_dot_partial, kOffChunk, dot, y);
 }
 void dot_partial(const Tables& T, const SceneSet& on, int a, int b) { MPH_LAUNCH(kb_dot_partial, kOffChunk, a, b); }
 void dot_final(const Tables& T, const SceneSet& on, int slot, int shift_slot) {

@@ -917,9 +917,11 @@ __device__ inline void fac_pair(const DevParams& P, double r0, double r1, double
 // lanes per particle in both passes and entries in flight (viscous and P entries)
 constexpr int kFacBatch = 4, kFacLanes32 = 8, kFacBatch32 = 8, kFacBatchP = 4;
 // the first pass (k's P list up to its last fluid entry, about 20 entries): lanes per
-// particle and entries in flight per lane, at six waves per SIMD (132 us on the 1M
-// scene, 160 us before beta was recomputed; 8 in flight at their three waves 140 us)
+// particle and entries in flight per lane, at six waves per SIMD (126 us on the 1M
+// scene; 160 us before beta was recomputed and, with rows in series, 132 us where 8 in
+// flight at their three waves took 140 us)
 constexpr int kFacLanesT = 4, kFacBatchT = 4;
+static_assert(kFacRowsT == 256 / kFacLanesT && kFacRowsY == 256 / kFacLanes && kFacRowsY == 256 / kFacLanes32, "");
 
 // the four planes of FacOp::rec
 struct FacPlanes {
@@ -944,60 +946,58 @@ __device__ inline void fac_t_chunk(const DevParams& P, const FacOp& F, const dou
     constexpr int G = kFacLanesT, U = kFacBatchT;
     const int g = threadIdx.x & (G - 1);
     const double W0 = P.W[0], W1 = P.W[1], W2 = P.W[2], h0 = P.hW[0], h1 = P.hW[1], h2 = P.hW[2];
-    for (int r = threadIdx.x / G; r < 256; r += 256 / G) {
-        const int k = chunk * 256 + r;
-        double acc = 0.0;
-        const int run = k < P.np ? F.runP[k] : 0;
-        if (run > 0) {
-            const double pk0 = F.pos[3 * k], pk1 = F.pos[3 * k + 1], pk2 = F.pos[3 * k + 2];
-            const long long c0 = F.nPtrP[k];
-            for (int jb = 0; jb < run; jb += G * U) {
-                int jx[U];
-                bool use[U];
+    const int k = chunk * kFacRowsT + threadIdx.x / G;
+    double acc = 0.0;
+    const int run = k < P.np ? F.runP[k] : 0;
+    if (run > 0) {
+        const double pk0 = F.pos[3 * k], pk1 = F.pos[3 * k + 1], pk2 = F.pos[3 * k + 2];
+        const long long c0 = F.nPtrP[k];
+        for (int jb = 0; jb < run; jb += G * U) {
+            int jx[U];
+            bool use[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    // entries past the end load the run's last entry (run >= 1), so the
-                    // list loads need no branches and issue together
-                    const int jn = jb + g + u * G;
-                    const int je = F.nIndP[c0 + (jn < run ? jn : run - 1)];
-                    use[u] = jn < run && je < P.nf && je != k;
-                    jx[u] = use[u] ? je : 0;  // unused entries read particle 0 with weight 0
-                }
-                double v[U][6];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const long long j3 = 3 * (long long)jx[u];
-                    v[u][0] = F.pos[j3];
-                    v[u][1] = F.pos[j3 + 1];
-                    v[u][2] = F.pos[j3 + 2];
-                    v[u][3] = x[j3];
-                    v[u][4] = x[j3 + 1];
-                    v[u][5] = x[j3 + 2];
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const double r0 = fac_wrap<kWrap>(v[u][0] - pk0, W0, h0);
-                    const double r1 = fac_wrap<kWrap>(v[u][1] - pk1, W1, h1);
-                    const double r2 = fac_wrap<kWrap>(v[u][2] - pk2, W2, h2);
-                    const double d2 = __builtin_fmax((r0 * r0 + r1 * r1) + r2 * r2, 1.0e-200);
-                    const double b = use[u] ? __builtin_fmax(rsqrt_ref(d2) - P.invP, 0.0) : 0.0;
-                    acc -= b * ((r0 * v[u][3] + r1 * v[u][4]) + r2 * v[u][5]);
-                }
+            for (int u = 0; u < U; ++u) {
+                // entries past the end load the run's last entry (run >= 1), so the
+                // list loads need no branches and issue together
+                const int jn = jb + g + u * G;
+                const int je = F.nIndP[c0 + (jn < run ? jn : run - 1)];
+                use[u] = jn < run && je < P.nf && je != k;
+                jx[u] = use[u] ? je : 0;  // unused entries read particle 0 with weight 0
             }
-            acc *= P.facP;
-        }
-        acc = group_sum(acc, G);
-        if (g == 0 && k < P.np) {
-            const FacPlanes R = fac_planes(P, F.rec);
-            if (k < P.nf) {
-                const double x0 = x[3 * k], x1 = x[3 * k + 1], x2 = x[3 * k + 2];
-                acc += (F.selfC[3 * k] * x0 + F.selfC[3 * k + 1] * x1) + F.selfC[3 * k + 2] * x2;
-                R.a[2 * k] = x0;
-                R.a[2 * k + 1] = x1;
-                R.b[2 * k] = x2;
+            double v[U][6];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const long long j3 = 3 * (long long)jx[u];
+                v[u][0] = F.pos[j3];
+                v[u][1] = F.pos[j3 + 1];
+                v[u][2] = F.pos[j3 + 2];
+                v[u][3] = x[j3];
+                v[u][4] = x[j3 + 1];
+                v[u][5] = x[j3 + 2];
             }
-            R.t[k] = run > 0 ? acc * F.lambda[k] : 0.0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const double r0 = fac_wrap<kWrap>(v[u][0] - pk0, W0, h0);
+                const double r1 = fac_wrap<kWrap>(v[u][1] - pk1, W1, h1);
+                const double r2 = fac_wrap<kWrap>(v[u][2] - pk2, W2, h2);
+                const double d2 = __builtin_fmax((r0 * r0 + r1 * r1) + r2 * r2, 1.0e-200);
+                const double b = use[u] ? __builtin_fmax(rsqrt_ref(d2) - P.invP, 0.0) : 0.0;
+                acc -= b * ((r0 * v[u][3] + r1 * v[u][4]) + r2 * v[u][5]);
+            }
         }
+        acc *= P.facP;
+    }
+    acc = group_sum(acc, G);
+    if (g == 0 && k < P.np) {
+        const FacPlanes R = fac_planes(P, F.rec);
+        if (k < P.nf) {
+            const double x0 = x[3 * k], x1 = x[3 * k + 1], x2 = x[3 * k + 2];
+            acc += (F.selfC[3 * k] * x0 + F.selfC[3 * k + 1] * x1) + F.selfC[3 * k + 2] * x2;
+            R.a[2 * k] = x0;
+            R.a[2 * k + 1] = x1;
+            R.b[2 * k] = x2;
+        }
+        R.t[k] = run > 0 ? acc * F.lambda[k] : 0.0;
     }
 }
 
@@ -1073,61 +1073,57 @@ __device__ inline void fac_row_gather(const DevParams& P, const FacOp& F, int i,
     }
 }
 
-// second pass over the 256 fluid rows of `chunk`:
+// element k of y (and y2) from the row's sum sm, as spmv_store: the separate
+// roundings of y = beta*yin + sum (compiled without contraction); yv and y2v are yin[k]
+// and y2[k], read before
+__device__ inline void fac_store1(int k, double sm, double yv, double y2v, double beta, double* y, double* y2) {
+    double yy = yv;
+    yy *= beta;
+    yy += sm;
+    if (y2) {
+        double zz = y2v;
+        zz *= beta;
+        zz += sm;
+        y2[k] = zz;
+    }
+    y[k] = yy;
+}
+
+// second pass over the kFacRowsY fluid rows of `chunk`, eight lanes a row:
 //   y_i = D_i x_i + C_ii t_i - sum_j alpha_ij r_ij (r_ij . x_j) + sum_{k != i} beta_ik r_ik t_k,
-// the row sums staged in rows[3*256] (LDS), then the tail of spmv_store.  A fluid
-// neighbour's alpha and beta terms are added together (fac_pair).  Every thread calls it.
+// a fluid neighbour's alpha and beta terms added together (fac_pair); then the tail of
+// spmv_store, one component to each of three lanes.
 template <bool kNeg, bool kWrap, bool kVar>
 __device__ inline void fac_y_chunk(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
-                                   const double* yin, double* y, double* y2, double* p_copy,
-                                   const double* __restrict__ dotx, double* __restrict__ part, int chunk,
-                                   double* sh, double* rows) {
+                                   const double* yin, double* y, double* y2, double* p_copy, int chunk) {
     constexpr int G = kFacLanes;
     const int g = threadIdx.x & (G - 1);
     const double* __restrict__ rt = fac_planes(P, F.rec).t;
-    for (int r = threadIdx.x / G; r < 256; r += 256 / G) {
-        const int i = chunk * 256 + r;
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-        if (i < P.nf) {
-            const double pi0 = F.pos[3 * i], pi1 = F.pos[3 * i + 1], pi2 = F.pos[3 * i + 2];
-            fac_row_gather<kWrap, kVar>(P, F, i, g, pi0, pi1, pi2, s0, s1, s2);
-            fac_walls<kWrap>(P, F, rt, i, g, pi0, pi1, pi2, s0, s1, s2);
-        }
-        s0 = group_sum(s0, G);
-        s1 = group_sum(s1, G);
-        s2 = group_sum(s2, G);
-        if (g == 0 && i < P.nf) {
-            const double* D = F.diag + 9 * i;
-            const double xi0 = x[3 * i], xi1 = x[3 * i + 1], xi2 = x[3 * i + 2];
-            const double ti = rt[i];
-            s0 = fac_diag_add(s0, D[0], D[1], D[2], xi0, xi1, xi2, F.selfC[3 * i], ti);
-            s1 = fac_diag_add(s1, D[3], D[4], D[5], xi0, xi1, xi2, F.selfC[3 * i + 1], ti);
-            s2 = fac_diag_add(s2, D[6], D[7], D[8], xi0, xi1, xi2, F.selfC[3 * i + 2], ti);
-            rows[3 * r] = kNeg ? -s0 : s0;
-            rows[3 * r + 1] = kNeg ? -s1 : s1;
-            rows[3 * r + 2] = kNeg ? -s2 : s2;
-        }
-    }
-    __syncthreads();
-    const int i = chunk * 256 + threadIdx.x;
-    const int t = threadIdx.x;
-    double r0 = 0.0, r1 = 0.0, r2 = 0.0;
+    const int i = chunk * kFacRowsY + threadIdx.x / G;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
     if (i < P.nf) {
-        r0 = rows[3 * t];
-        r1 = rows[3 * t + 1];
-        r2 = rows[3 * t + 2];
+        const double pi0 = F.pos[3 * i], pi1 = F.pos[3 * i + 1], pi2 = F.pos[3 * i + 2];
+        fac_row_gather<kWrap, kVar>(P, F, i, g, pi0, pi1, pi2, s0, s1, s2);
+        fac_walls<kWrap>(P, F, rt, i, g, pi0, pi1, pi2, s0, s1, s2);
     }
-    spmv_store(P.nf, i, r0, r1, r2, x, beta, yin, y, y2, p_copy, dotx, part, chunk, sh);
+    s0 = group_sum(s0, G);
+    s1 = group_sum(s1, G);
+    s2 = group_sum(s2, G);
+    if (g < 3 && i < P.nf) {
+        const int k = 3 * i + g;
+        const double* D = F.diag + 9 * i + 3 * g;
+        const double sg = fac_diag_add(g == 0 ? s0 : g == 1 ? s1 : s2, D[0], D[1], D[2], x[3 * i], x[3 * i + 1],
+                                       x[3 * i + 2], F.selfC[k], rt[i]);
+        fac_store1(k, kNeg ? -sg : sg, yin[k], y2 ? y2[k] : 0.0, beta, y, y2);
+        if (p_copy) p_copy[k] = x[k];
+    }
 }
 
 // the variant of fac_y_chunk that the scene's flags ask for (uniform)
 template <bool kNeg>
 __device__ inline void fac_y_chunk_any(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
-                                       const double* yin, double* y, double* y2, double* p_copy,
-                                       const double* __restrict__ dotx, double* __restrict__ part, int chunk,
-                                       double* sh, double* rows) {
-#define MPH_Y(WRAP, VAR) \
-    fac_y_chunk<kNeg, WRAP, VAR>(P, F, x, beta, yin, y, y2, p_copy, dotx, part, chunk, sh, rows)
+                                       const double* yin, double* y, double* y2, double* p_copy, int chunk) {
+#define MPH_Y(WRAP, VAR) fac_y_chunk<kNeg, WRAP, VAR>(P, F, x, beta, yin, y, y2, p_copy, chunk)
     const int wrap = F.wrap[0], var = F.wrap[1];
     if (!wrap && !var) MPH_Y(false, false);
     else if (!var) MPH_Y(true, false);
@@ -1144,179 +1140,142 @@ __device__ inline void fac_t32_chunk(const DevParams& P, const FacOp& F, const d
     constexpr int G = kFacLanes32, U = kFacBatchP;
     typedef float fv4 __attribute__((ext_vector_type(4)));
     const int g = threadIdx.x & (G - 1);
-    for (int r = threadIdx.x / G; r < 256; r += 256 / G) {
-        const int k = chunk * 256 + r;
-        double acc = 0.0;
-        const int run = k < P.np ? F.runP[k] : 0;
-        if (run > 0) {
-            const long long c0 = F.nPtrP[k];
-            for (int jb = 0; jb < run; jb += G * U) {
-                int jx[U];
-                float v[U][3];
+    const int k = chunk * kFacRowsY + threadIdx.x / G;
+    double acc = 0.0;
+    const int run = k < P.np ? F.runP[k] : 0;
+    if (run > 0) {
+        const long long c0 = F.nPtrP[k];
+        for (int jb = 0; jb < run; jb += G * U) {
+            int jx[U];
+            float v[U][3];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int jn = jb + g + u * G;
-                    const FacEntry32 en = fac_entry32(F.v32, c0 + (jn < run ? jn : 0));
-                    const int j = jn < run ? en.col : k;
-                    const bool use = jn < run && j < P.nf && j != k;
-                    jx[u] = use ? j : 0;  // unused entries read particle 0 with weight 0
-                    v[u][0] = use ? en.a0 : 0.0f;
-                    v[u][1] = use ? en.a1 : 0.0f;
-                    v[u][2] = use ? en.a2 : 0.0f;
-                }
-                double xv[U][3];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const long long j3 = 3 * (long long)jx[u];
-                    xv[u][0] = x[j3];
-                    xv[u][1] = x[j3 + 1];
-                    xv[u][2] = x[j3 + 2];
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    acc -= ((double)v[u][0] * xv[u][0] + (double)v[u][1] * xv[u][1]) + (double)v[u][2] * xv[u][2];
+            for (int u = 0; u < U; ++u) {
+                const int jn = jb + g + u * G;
+                const FacEntry32 en = fac_entry32(F.v32, c0 + (jn < run ? jn : 0));
+                const int j = jn < run ? en.col : k;
+                const bool use = jn < run && j < P.nf && j != k;
+                jx[u] = use ? j : 0;  // unused entries read particle 0 with weight 0
+                v[u][0] = use ? en.a0 : 0.0f;
+                v[u][1] = use ? en.a1 : 0.0f;
+                v[u][2] = use ? en.a2 : 0.0f;
             }
-        }
-        acc = group_sum(acc, G);
-        if (g == 0 && k < P.np) {
-            fv4 rk = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (k < P.nf) {
-                const double x0 = x[3 * k], x1 = x[3 * k + 1], x2 = x[3 * k + 2];
-                acc += (F.selfC[3 * k] * x0 + F.selfC[3 * k + 1] * x1) + F.selfC[3 * k + 2] * x2;
-                rk[0] = (float)x0;
-                rk[1] = (float)x1;
-                rk[2] = (float)x2;
+            double xv[U][3];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const long long j3 = 3 * (long long)jx[u];
+                xv[u][0] = x[j3];
+                xv[u][1] = x[j3 + 1];
+                xv[u][2] = x[j3 + 2];
             }
-            rk[3] = run > 0 ? (float)(acc * F.lambda[k]) : 0.0f;
-            ((fv4*)F.rec32)[k] = rk;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                acc -= ((double)v[u][0] * xv[u][0] + (double)v[u][1] * xv[u][1]) + (double)v[u][2] * xv[u][2];
         }
+    }
+    acc = group_sum(acc, G);
+    if (g == 0 && k < P.np) {
+        fv4 rk = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (k < P.nf) {
+            const double x0 = x[3 * k], x1 = x[3 * k + 1], x2 = x[3 * k + 2];
+            acc += (F.selfC[3 * k] * x0 + F.selfC[3 * k + 1] * x1) + F.selfC[3 * k + 2] * x2;
+            rk[0] = (float)x0;
+            rk[1] = (float)x1;
+            rk[2] = (float)x2;
+        }
+        rk[3] = run > 0 ? (float)(acc * F.lambda[k]) : 0.0f;
+        ((fv4*)F.rec32)[k] = rk;
     }
 }
 
 template <bool kNeg>
 __device__ inline void fac_y32_chunk(const DevParams& P, const FacOp& F, const double* __restrict__ x, double beta,
-                                     const double* yin, double* y, double* y2, double* p_copy,
-                                     const double* __restrict__ dotx, double* __restrict__ part, int chunk,
-                                     double* sh, double* rows) {
+                                     const double* yin, double* y, double* y2, double* p_copy, int chunk) {
 #pragma clang fp contract(fast)
     typedef float fv4 __attribute__((ext_vector_type(4)));
     constexpr int G = kFacLanes32, U = kFacBatch32;
     const int g = threadIdx.x & (G - 1);
     const fv4* __restrict__ rec = (const fv4*)F.rec32;
-    // the viscous loop is software-pipelined: the columns and u of the next batch
-    // (or of the next row's first batch) load while the current batch's records are
-    // gathered, so the two dependent round trips of a batch overlap
-    struct Batch {
-        int j[U];
-        float a[U][3];
-    };
-    auto vload = [&](int i, int w, long long b0, int jb, Batch& b) {
+    const int i = chunk * kFacRowsY + threadIdx.x / G;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    if (i < P.nf) {
+        // viscous part: -u (u . x_j).  Software-pipelined: the columns and u of the next
+        // batch load while the current batch's records are gathered
+        struct Batch {
+            int j[U];
+            float a[U][3];
+        };
+        const long long b0 = F.nPtr[i];
+        const int w = F.nFluid[i];
+        auto vload = [&](int jb, Batch& b) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int jn = jb + g + u * G;
-            const bool in = jn < w;
-            const FacEntry32 en = fac_entry32(F.u32, b0 + (in ? jn : 0));
-            b.j[u] = in ? en.col : i;  // unused entries: i's own record, u = 0
-            b.a[u][0] = in ? en.a0 : 0.0f;
-            b.a[u][1] = in ? en.a1 : 0.0f;
-            b.a[u][2] = in ? en.a2 : 0.0f;
-        }
-    };
-    Batch nb;
-    {
-        const int i0 = chunk * 256 + threadIdx.x / G;
-        if (i0 < P.nf) vload(i0, F.nFluid[i0], F.nPtr[i0], 0, nb);
-    }
-    for (int r = threadIdx.x / G; r < 256; r += 256 / G) {
-        const int i = chunk * 256 + r;
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-        if (i < P.nf) {
-            // viscous part: -u (u . x_j)
-            const long long b0 = F.nPtr[i];
-            const int w = F.nFluid[i];
-            Batch cb = nb;
+            for (int u = 0; u < U; ++u) {
+                const int jn = jb + g + u * G;
+                const bool in = jn < w;
+                const FacEntry32 en = fac_entry32(F.u32, b0 + (in ? jn : 0));
+                b.j[u] = in ? en.col : i;  // unused entries: i's own record, u = 0
+                b.a[u][0] = in ? en.a0 : 0.0f;
+                b.a[u][1] = in ? en.a1 : 0.0f;
+                b.a[u][2] = in ? en.a2 : 0.0f;
+            }
+        };
+        Batch nb;
+        vload(0, nb);
+        for (int jb = 0; jb < w; jb += G * U) {
+            const Batch cb = nb;
             fv4 q[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) q[u] = rec[cb.j[u]];
-            for (int jb = 0; jb < w; jb += G * U) {
-                const bool more = jb + G * U < w;
-                const int rn = r + 256 / G, in_ = chunk * 256 + rn;
-                if (more) vload(i, w, b0, jb + G * U, nb);
-                else if (rn < 256 && in_ < P.nf) vload(in_, F.nFluid[in_], F.nPtr[in_], 0, nb);
+            if (jb + G * U < w) vload(jb + G * U, nb);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const double a0 = cb.a[u][0], a1 = cb.a[u][1], a2 = cb.a[u][2];
-                    const double f = (a0 * (double)q[u][0] + a1 * (double)q[u][1]) + a2 * (double)q[u][2];
-                    s0 -= f * a0;
-                    s1 -= f * a1;
-                    s2 -= f * a2;
-                }
-                if (more) {
-                    cb = nb;
-#pragma unroll
-                    for (int u = 0; u < U; ++u) q[u] = rec[cb.j[u]];
-                }
-            }
-            // C Lambda C^T part: v_ik t_k
-            const long long c0 = F.nPtrP[i];
-            const int n = F.nCountP[i];
-            for (int jb = 0; jb < n; jb += G * kFacBatchP) {
-                constexpr int U = kFacBatchP;
-                int k[U];
-                float vv[U][3];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int jn = jb + g + u * G;
-                    const bool in = jn < n;
-                    const FacEntry32 en = fac_entry32(F.v32, c0 + (in ? jn : 0));
-                    k[u] = in ? en.col : i;
-                    vv[u][0] = in ? en.a0 : 0.0f;
-                    vv[u][1] = in ? en.a1 : 0.0f;
-                    vv[u][2] = in ? en.a2 : 0.0f;
-                }
-                fv4 q[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) q[u] = rec[k[u]];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const double t = q[u][3];
-                    s0 += (double)vv[u][0] * t;
-                    s1 += (double)vv[u][1] * t;
-                    s2 += (double)vv[u][2] * t;
-                }
+            for (int u = 0; u < U; ++u) {
+                const double a0 = cb.a[u][0], a1 = cb.a[u][1], a2 = cb.a[u][2];
+                const double f = (a0 * (double)q[u][0] + a1 * (double)q[u][1]) + a2 * (double)q[u][2];
+                s0 -= f * a0;
+                s1 -= f * a1;
+                s2 -= f * a2;
             }
         }
-        s0 = group_sum(s0, G);
-        s1 = group_sum(s1, G);
-        s2 = group_sum(s2, G);
-        if (g == 0 && i < P.nf) {
-            const double* D = F.diag + 9 * i;
-            const double xi0 = x[3 * i], xi1 = x[3 * i + 1], xi2 = x[3 * i + 2];
-            const double ti = rec[i][3];
-            double d0 = (D[0] * xi0 + D[1] * xi1) + D[2] * xi2;
-            double d1 = (D[3] * xi0 + D[4] * xi1) + D[5] * xi2;
-            double d2 = (D[6] * xi0 + D[7] * xi1) + D[8] * xi2;
-            d0 += F.selfC[3 * i] * ti;
-            d1 += F.selfC[3 * i + 1] * ti;
-            d2 += F.selfC[3 * i + 2] * ti;
-            s0 += d0;
-            s1 += d1;
-            s2 += d2;
-            rows[3 * r] = kNeg ? -s0 : s0;
-            rows[3 * r + 1] = kNeg ? -s1 : s1;
-            rows[3 * r + 2] = kNeg ? -s2 : s2;
+        // C Lambda C^T part: v_ik t_k
+        const long long c0 = F.nPtrP[i];
+        const int n = F.nCountP[i];
+        for (int jb = 0; jb < n; jb += G * kFacBatchP) {
+            constexpr int U = kFacBatchP;
+            int k[U];
+            float vv[U][3];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int jn = jb + g + u * G;
+                const bool in = jn < n;
+                const FacEntry32 en = fac_entry32(F.v32, c0 + (in ? jn : 0));
+                k[u] = in ? en.col : i;
+                vv[u][0] = in ? en.a0 : 0.0f;
+                vv[u][1] = in ? en.a1 : 0.0f;
+                vv[u][2] = in ? en.a2 : 0.0f;
+            }
+            fv4 q[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) q[u] = rec[k[u]];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const double t = q[u][3];
+                s0 += (double)vv[u][0] * t;
+                s1 += (double)vv[u][1] * t;
+                s2 += (double)vv[u][2] * t;
+            }
         }
     }
-    __syncthreads();
-    const int i = chunk * 256 + threadIdx.x;
-    const int t = threadIdx.x;
-    double r0 = 0.0, r1 = 0.0, r2 = 0.0;
-    if (i < P.nf) {
-        r0 = rows[3 * t];
-        r1 = rows[3 * t + 1];
-        r2 = rows[3 * t + 2];
+    s0 = group_sum(s0, G);
+    s1 = group_sum(s1, G);
+    s2 = group_sum(s2, G);
+    if (g < 3 && i < P.nf) {
+        const int k = 3 * i + g;
+        const double* D = F.diag + 9 * i + 3 * g;
+        double d = (D[0] * x[3 * i] + D[1] * x[3 * i + 1]) + D[2] * x[3 * i + 2];
+        d += F.selfC[k] * (double)rec[i][3];
+        const double sg = (g == 0 ? s0 : g == 1 ? s1 : s2) + d;
+        fac_store1(k, kNeg ? -sg : sg, yin[k], y2 ? y2[k] : 0.0, beta, y, y2);
+        if (p_copy) p_copy[k] = x[k];
     }
-    spmv_store(P.nf, i, r0, r1, r2, x, beta, yin, y, y2, p_copy, dotx, part, chunk, sh);
 }
 
 // chunk partial of x.y: per particle (x0 y0 + x1 y1) + x2 y2, then the chunk tree

@@ -484,17 +484,11 @@ __global__ void __launch_bounds__(256, 6) k_fac_t(DevParams P, FacOp F, const do
 }
 
 template <bool kNeg, class VT>
-__global__ void __launch_bounds__(256) k_fac_y(DevParams P, FacOp F, const double* __restrict__ x, double beta,
-                                               const double* yin, double* y, double* y2, double* p_copy,
-                                               const double* __restrict__ dotx, double* __restrict__ part) {
+__global__ void __launch_bounds__(256, 4) k_fac_y(DevParams P, FacOp F, const double* __restrict__ x, double beta,
+                                               const double* yin, double* y, double* y2, double* p_copy) {
     if (cr_halted(P.halt)) return;
-    __shared__ double sh[256];
-    __shared__ double rows[3 * 256];
-    if constexpr (sizeof(VT) == 4) {
-        body::fac_y32_chunk<kNeg>(P, F, x, beta, yin, y, y2, p_copy, dotx, part, blockIdx.x, sh, rows);
-    } else {
-        body::fac_y_chunk_any<kNeg>(P, F, x, beta, yin, y, y2, p_copy, dotx, part, blockIdx.x, sh, rows);
-    }
+    if constexpr (sizeof(VT) == 4) body::fac_y32_chunk<kNeg>(P, F, x, beta, yin, y, y2, p_copy, blockIdx.x);
+    else body::fac_y_chunk_any<kNeg>(P, F, x, beta, yin, y, y2, p_copy, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -534,22 +528,6 @@ enum {
     kFdPiece0 = 8
 };
 static_assert(kFdPiece0 + 2 * (27 + kFacCellSlots[kFacCell3DWide] / 64) <= kFacDesc, "the pieces fit the descriptor");
-
-// element k of y (and y2) from the row's sum sm, as spmv_store: the separate
-// roundings of y = beta*yin + sum (this function is compiled without contraction);
-// yv and y2v are yin[k] and y2[k], read before
-__device__ inline void fac_cell_store1(int k, double sm, double yv, double y2v, double beta, double* y, double* y2) {
-    double yy = yv;
-    yy *= beta;
-    yy += sm;
-    if (y2) {
-        double zz = y2v;
-        zz *= beta;
-        zz += sm;
-        y2[k] = zz;
-    }
-    y[k] = yy;
-}
 
 typedef double dv2c __attribute__((ext_vector_type(2)));
 
@@ -825,7 +803,7 @@ __device__ inline void fac_y_cell_body(const DevParams& P, const FacOp& F, const
         s2 = body::group_sum(s2, G);
         if (g < 3 && on) {  // lane g: component g, as body::fac_y_chunk computes it
             const double sg = body::fac_diag_add(g == 0 ? s0 : g == 1 ? s1 : s2, dA, dB, dC, xi0, xi1, xi2, sc, ti);
-            fac_cell_store1(3 * i + g, kNeg ? -sg : sg, yv, y2v, beta, y, y2);
+            body::fac_store1(3 * i + g, kNeg ? -sg : sg, yv, y2v, beta, y, y2);
             if (p_copy) p_copy[3 * i + g] = g == 0 ? xi0 : g == 1 ? xi1 : xi2;
         }
     }
@@ -888,10 +866,13 @@ __global__ void __launch_bounds__(kFacCellThreads[kShape], kShape == kFacCell3DW
 template <bool kNeg, class VT>
 void fac_launch(hipStream_t st, const DevParams& P, const FacOp& F, const double* x, double beta, const double* yin,
                 double* y, double* y2, double* p_copy, const double* dotx, double* part, int passes) {
-    if (passes & 1) hipLaunchKernelGGL(k_fac_t<VT>, dim3(nblk(P.np, 256)), dim3(256), 0, st, P, F, x);
+    constexpr bool f32 = sizeof(VT) == 4;
+    if (passes & 1)
+        hipLaunchKernelGGL(k_fac_t<VT>, dim3(nblk(P.np, f32 ? kFacRowsY : kFacRowsT)), dim3(256), 0, st,
+                           P, F, x);
     if (!(passes & 2)) return;
     const long long cells = (long long)F.cellCnt[0] * F.cellCnt[1] * F.cellCnt[2];
-    if (sizeof(VT) == 8 && F.slot && cells > 0) {
+    if (!f32 && F.slot && cells > 0) {
 #define MPH_CELL(SHAPE)                                                                                           \
     hipLaunchKernelGGL((k_fac_y_cell<kNeg, SHAPE>), dim3((unsigned)cells), dim3(kFacCellThreads[SHAPE]), 0, st, P, F, \
                        x, beta, yin, y, y2, p_copy)
@@ -899,11 +880,11 @@ void fac_launch(hipStream_t st, const DevParams& P, const FacOp& F, const double
         else if (F.cellShape == kFacCell3D) MPH_CELL(kFacCell3D);
         else MPH_CELL(kFacCell3DWide);
 #undef MPH_CELL
-        if (part) launch_dot_partial(st, P, dotx, y, part);
-        return;
+    } else {
+        hipLaunchKernelGGL((k_fac_y<kNeg, VT>), dim3(nblk(P.nf, kFacRowsY)), dim3(256), 0,
+                           st, P, F, x, beta, yin, y, y2, p_copy);
     }
-    hipLaunchKernelGGL((k_fac_y<kNeg, VT>), dim3(nblk(P.nf, kChunk)), dim3(kChunk), 0, st, P, F, x, beta, yin, y, y2,
-                       p_copy, dotx, part);
+    if (part) launch_dot_partial(st, P, dotx, y, part);
 }
 
 }  // namespace

@@ -137,6 +137,12 @@ constexpr int kFacDesc = 160;
 // row about 37; a 3D cell about 41 rows, one pass of 512 threads.  (16 lanes in 3D, two
 // passes: 444 against 428 us per second pass on the 1M scene.)
 constexpr int kFacLanes = 8;
+// rows of a 256-thread workgroup, one per group of lanes, of the FP64 first pass and of
+// the second (FP32: both).  (Workgroups of 256 rows, each group of lanes walking four or
+// eight in series, left most wavefront slots empty in scenes of less than about a million
+// particles: first pass 9.6 us at 2.9k particles, 18.4 at 182k, 132 at 1.3M, now 4.7, 11.8
+// and 126; FP32 second pass 62.9 us at 64k fluid particles, now 39 at 5 TB/s of entries.)
+constexpr int kFacRowsT = 64, kFacRowsY = 32;
 // launch shapes of the cell-staged pass: threads per workgroup and staged records (56
 // bytes of LDS each).  3D: 1408 records let two workgroups share a CU (27 cells of 3.51
 // spacings hold at most 11^3 = 1331 lattice particles); domains of few cells have wider
