@@ -803,7 +803,7 @@ __device__ inline void fac_y_cell_body(const DevParams& P, const FacOp& F, const
         s2 = body::group_sum(s2, G);
         if (g < 3 && on) {  // lane g: component g, as body::fac_y_chunk computes it
             const double sg = body::fac_diag_add(g == 0 ? s0 : g == 1 ? s1 : s2, dA, dB, dC, xi0, xi1, xi2, sc, ti);
-            body::fac_store1(3 * i + g, kNeg ? -sg : sg, yv, y2v, beta, y, y2);
+            body::store1(3 * i + g, kNeg ? -sg : sg, yv, y2v, beta, y, y2);
             if (p_copy) p_copy[3 * i + g] = g == 0 ? xi0 : g == 1 ? xi1 : xi2;
         }
     }

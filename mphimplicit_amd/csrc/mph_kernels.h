@@ -274,6 +274,13 @@ void launch_cr_init(hipStream_t st, const DevParams& P, const double* vel, const
 // SpMV variants differ only in how many block pairs are loaded per group (same
 // bits): FP64 2, 3 or 4 block pairs; FP32 1 or 2 block quads
 constexpr int kSpmvVariants64 = 3, kSpmvVariants32 = 2;
+// up to this many slices of 64 rows a wavefront takes one component of a slice's rows
+// (spmv_split in mph_cr_body.h), beyond it all three: the split reads x and the columns
+// three times and reaches 4.2 TB/s, the other 6.3 TB/s once enough wavefronts are there.
+// Split against whole, us per FP64 product with the 4.5 us of the dot partials that the
+// split launches on their own: 2D 65 slices 13.3/19.1, 223: 15.7/20.3, 438: 21.9/22.3;
+// 3D 144 slices 36.5/89.1, 216: 39.3/91.4, 436: 94.8/98.0, 631: 161/107, 1000: 196/129
+constexpr int kSpmvSplit = 400;
 void launch_spmv(hipStream_t st, const DevParams& P, ASlices A, const int* nFluid, double alpha, const double* x,
                  double beta, const double* yin, double* y, double* y2, double* p_copy, const double* dotx,
                  double* part, bool f32 = false, int variant = 0);

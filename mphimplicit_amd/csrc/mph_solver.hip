@@ -724,10 +724,26 @@ void launch_cr_init(hipStream_t st, const DevParams& P, const double* vel, const
                     const double* mass, double* x) {
     hipLaunchKernelGGL(k_cr_init, dim3(nblk(P.nf, 256)), dim3(256), 0, st, P, vel, force, mass, x);
 }
+template <bool kNeg, class VT>
+__global__ void __launch_bounds__(192, 2) k_spmv_split(int nf, const int* __restrict__ nFluid,
+                                                       const long long* __restrict__ start,
+                                                       const int* __restrict__ col, const VT* __restrict__ val,
+                                                       const double* __restrict__ x, double beta, const double* yin,
+                                                       double* y, double* y2, double* p_copy, const int* halt) {
+    if (cr_halted(halt)) return;
+    spmv_split<kNeg, VT>(nf, nFluid, start, col, val, x, beta, yin, y, y2, p_copy, blockIdx.x);
+}
+
 template <bool kNeg, class VT, int kUn>
 static void spmv_launch(hipStream_t st, const DevParams& P, const ASlices& A, const int* nFluid, const VT* val,
                         const double* x, double beta, const double* yin, double* y, double* y2, double* p_copy,
                         const double* dotx, double* part) {
+    if (A.nslices <= kSpmvSplit) {
+        hipLaunchKernelGGL((k_spmv_split<kNeg, VT>), dim3(A.nslices), dim3(192), 0, st, P.nf, nFluid, A.start, A.col, val,
+                           x, beta, yin, y, y2, p_copy, P.halt);
+        if (part) launch_dot_partial(st, P, dotx, y, part);
+        return;
+    }
     hipLaunchKernelGGL((k_spmv<kNeg, VT, kUn>), dim3(nblk(P.nf, kChunk)), dim3(kChunk), 0, st, P.nf, nFluid, A.start,
                        A.col, val, x, beta, yin, y, y2, p_copy, dotx, part, P.halt);
 }
