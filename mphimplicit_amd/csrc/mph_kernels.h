@@ -173,7 +173,6 @@ constexpr int kRuns = 28;     // run starts per fluid particle: 27 neighbour cel
 // of -alpha r r^T over that cell's run of fluid entries, a symmetric block kept as its
 // upper triangle (xx xy xz yy yz zz) in records of kBlkStride doubles
 constexpr int kBlkRuns = kRuns - 1, kBlkStride = 6;
-constexpr int kMaxP = 40;     // P-neighbours staged in LDS per particle by the C Lambda C^T kernel
 constexpr int kMaxLevels = 20;   // multigrid depth = floor(log2(cells per axis)) + 1
 
 // ---- cells (calculateCellParticle) ----
@@ -229,14 +228,12 @@ void launch_vector_p(hipStream_t st, const DevParams& P, const int* type, const 
                      const long long* nPtrP, const int* nIndP, double* vecP);
 void launch_b_minus_cp(hipStream_t st, const DevParams& P, const int* nCountP, const long long* nPtrP,
                        const int* nIndP, const double* cval, const double* vecP, double* b);
-// kernel modes: 0 P lists from global memory; 2 both lists staged in LDS; 3 staged,
-// and the merge records the matches before any arithmetic.  The tuner chooses
-// between modes 3 and 2 (variants 0, 1); mode 0 runs when a fluid particle has more
-// than kMaxP P-neighbours.  Same bits in every mode.
-constexpr int kCacVariants = 2;
-constexpr int kCacModeOf[kCacVariants] = {3, 2};
+// maxP: the largest P-neighbour count of a fluid particle; above 64 the lists are merged
+// instead of hashed (the same bits).  Also writes A.val32 when it is non-null
+// (nIndP is read up to kListSpare entries past its lists)
+constexpr int kListSpare = 3;
 void launch_cac(hipStream_t st, const DevParams& P, const int* nFluid, const int* nCountP, const long long* nPtrP,
-                const int* nIndP, const double* cval, const double* dval, ASlices A, int mode);  // also writes A.val32 when it is non-null
+                const int* nIndP, const double* cval, const double* dval, ASlices A, int maxP);
 // ---- multigrid ----
 void launch_fluid_bbox(hipStream_t st, const DevParams& P, const int* cellStart, int* bbox);
 void launch_inv_diag(hipStream_t st, const DevParams& P, const int* selfIdx, ASlices A, double* invDiagA);

@@ -638,45 +638,160 @@ __global__ void __launch_bounds__(256) k_b_minus_cp(DevParams P, const int* __re
 }
 
 // A += C Lambda C^T (multiplyMatrixC, 2586-2642): for each fluid i and each of its
-// fluid neighbours j, merge the sorted P-neighbour lists of i and j and sum
-// D_ik (x) C_jk over the shared k (D = C*Lambda, left to right as the reference),
-// then add the 3x3 sum to block (i, j).  Workgroup = one slice: lane = particle,
-// wave w takes the blocks k = w, w+4, ...  kMode >= 2: the slice's own index lists
-// are staged in LDS (odd row stride, no bank conflicts) and each thread copies j's
-// index list into LDS before merging (its loads all in flight at once instead of
-// one per merge step); with kMode 0 both are read from global memory;
-// kMode 3 in addition first merges without arithmetic, recording the matches, and
-// then adds them (the merge's three-way branch no longer carries the 9 products).
-// All give the same bits; the fastest is picked at run time.
-// The FP32 copy of the finished block is written when aval32 is non-null.
-template <int kMode>
+// fluid neighbours j, the sum of D_ik (x) C_jk over the k in both P-neighbour lists
+// (D = C*Lambda, left to right as the reference) in ascending order of k, added to the
+// 3x3 block (i, j).  Workgroup = one slice of 64 particles, lane = particle; the
+// wavefronts of gridDim.y workgroups share its block pairs.  The FP32 copy of the
+// finished block is written when aval32 is non-null.
+//
+// i's list is a hash table in LDS, entry k << 6 | place, four to a bucket of one 16-byte
+// read (a bucket is full before its successor takes entries).  A thread looks up the
+// entries of j's list, four under way at a time; both lists ascend, so the t-th hit of
+// one is the t-th of the other and the hits are two bit masks, from which the products
+// are added without a search.  A lookup replaces two steps of a merge, and the lists
+// need no copy in LDS: the merge kernel's copies (52 KB per workgroup of four
+// wavefronts) left it waiting at three workgroups per CU.
+// The values (0.8 GB read and written at 64k particles) go by pairs of blocks, whole lines:
+// a block at a time moved 4.0 GB and took 1.22 ms.  0.90 ms at 64k particles (the merge
+// kernel 1.67), 2.78 at 198k (3.84); with up to 16 workgroups to a slice 32 us at 216
+// (367) and 100 us at 9k (516).  The gathers of the lists and of C and D, a cache line per
+// lane, bound it next.
+constexpr int kCacBuckets = 32;
+__device__ inline unsigned cac_bucket(int k) { return ((unsigned)k * 0x9E3779B1u) >> 27; }
+
 __global__ void __launch_bounds__(256) k_cac(DevParams P, const int* __restrict__ nFluid,
                                              const int* __restrict__ nCountP, const long long* __restrict__ nPtrP,
                                              const int* __restrict__ nIndP, const double* __restrict__ cval,
                                              const double* __restrict__ dval, const long long* __restrict__ start,
                                              const int* __restrict__ acol, double* __restrict__ aval,
                                              float* __restrict__ aval32) {
-    constexpr int kStride = kMaxP + 1;
-    constexpr bool kLdsI = kMode >= 2, kLdsJ = kMode >= 2;  // mode 3: both + two-phase merge
-    __shared__ int sk[kLdsI ? kSlice * kStride : 1];
-    __shared__ int sj[kLdsJ ? 256 * kStride : 1];
-    const int slice = blockIdx.x;
-    const int base = slice * kSlice;
-    if (kLdsI) {
-        for (int t = threadIdx.x; t < kSlice * kMaxP; t += blockDim.x) {
-            const int l = t / kMaxP, a = t % kMaxP, i = base + l;
-            if (i < P.nf && a < nCountP[i]) sk[l * kStride + a] = nIndP[nPtrP[i] + a];
+    typedef double dv2 __attribute__((ext_vector_type(2)));
+    constexpr unsigned kEmpty = 0xffffffffu;
+    __shared__ uint4 tab[kSlice][kCacBuckets];
+    const int slice = blockIdx.x, base = slice * kSlice, t = threadIdx.x;
+    for (int e = t; e < kSlice * kCacBuckets; e += 256) (&tab[0][0])[e] = uint4{kEmpty, kEmpty, kEmpty, kEmpty};
+    __syncthreads();
+    {  // four threads per list
+        const int l = t / 4, i = base + l;
+        if (i < P.nf) {
+            const long long p = nPtrP[i];
+            const int n = nCountP[i];
+            for (int a = t & 3; a < n; a += 4) {
+                const int k = nIndP[p + a];
+                unsigned* const T = (unsigned*)tab[l];
+                unsigned s = 4 * cac_bucket(k);  // at most 64 entries in 128 slots: ends
+                while (atomicCAS(&T[s], kEmpty, (unsigned)k << 6 | a) != kEmpty) s = (s + 1) & (4 * kCacBuckets - 1);
+            }
         }
-        __syncthreads();
     }
-    const int lane = threadIdx.x % kSlice, wave = threadIdx.x / kSlice;
+    __syncthreads();
+    const int lane = t % kSlice, wave = t / kSlice;
     const int i = base + lane;
+    if (i >= P.nf) return;
+    const int nfl = nFluid[i];
+    const double* di = dval + 3 * nPtrP[i];
+    const long long sb = start[slice];
+    const uint4* const ti = tab[lane];
+    for (int k = 2 * (wave + 4 * blockIdx.y); k < nfl; k += 8 * gridDim.y) {
+        int j[2], nj[2];
+        long long pj[2];
+        const int hn = k + 1 < nfl ? 2 : 1;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            j[h] = acol[a_col_index(sb, k + (h < hn ? h : 0), lane)];
+            pj[h] = nPtrP[j[h]];
+            nj[h] = h < hn ? nCountP[j[h]] : 0;
+        }
+        // both blocks of a pair of values are written together: 16 bytes a lane, whole lines
+        dv2 v[9];
+        double sum[2][9];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const long long p = pj[h];
+            const int n = nj[h];
+            unsigned long long mi = 0, mj = 0;  // hits: places in i's and in j's list
+            for (int c0 = 0; c0 < n; c0 += 4) {
+                unsigned q[4], b[4];
+                uint4 w[4];
+                __builtin_memcpy(q, nIndP + p + c0, 16);  // past the end: not taken (kListSpare)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    b[u] = cac_bucket((int)q[u]);
+                    w[u] = ti[b[u]];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    auto hit = [&](const uint4& x) {  // the place, or 64 and more
+                        const unsigned y = q[u] << 6;
+                        const unsigned m0 = min(x.x ^ y, x.y ^ y), m1 = min(x.z ^ y, x.w ^ y);
+                        return min(m0, m1);
+                    };
+                    unsigned a = hit(w[u]);
+                    while (a >= 64 && w[u].w != kEmpty) {  // 64 entries leave a bucket that isn't full
+                        b[u] = (b[u] + 1) & (kCacBuckets - 1);
+                        w[u] = ti[b[u]];
+                        a = hit(w[u]);
+                    }
+                    if (a < 64 && c0 + u < n) {
+                        mi |= 1ull << a;
+                        mj |= 1ull << (c0 + u);
+                    }
+                }
+            }
+            if (h == 1)
+#pragma unroll
+                for (int e = 0; e < 9; ++e) v[e] = *(const dv2*)(aval + a_val_index(sb, k, e, lane));
+#pragma unroll
+            for (int e = 0; e < 9; ++e) sum[h][e] = 0.0;
+            double c[3], d[3];
+            auto load = [&]() {
+                const double* cj = cval + (mj ? 3 * (p + __builtin_ctzll(mj)) : 0);
+                const double* da = mi ? di + 3 * __builtin_ctzll(mi) : dval;
+#pragma unroll
+                for (int e = 0; e < 3; ++e) {
+                    c[e] = cj[e];
+                    d[e] = da[e];
+                }
+            };
+            load();
+            while (mj) {
+                const double c0 = c[0], c1 = c[1], c2 = c[2], d0 = d[0], d1 = d[1], d2 = d[2];
+                mi &= mi - 1;
+                mj &= mj - 1;
+                load();  // the next hit's
+                sum[h][0] += d0 * c0; sum[h][1] += d0 * c1; sum[h][2] += d0 * c2;
+                sum[h][3] += d1 * c0; sum[h][4] += d1 * c1; sum[h][5] += d1 * c2;
+                sum[h][6] += d2 * c0; sum[h][7] += d2 * c1; sum[h][8] += d2 * c2;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 9; ++e) {
+            v[e][0] += sum[0][e];
+            v[e][1] += sum[1][e];  // past the row's last block: a value that is never read
+            *(dv2*)(aval + a_val_index(sb, k, e, lane)) = v[e];
+            if (aval32)
+                for (int h = 0; h < hn; ++h) aval32[a_val32_index(sb, k + h, e, lane)] = (float)v[e][h];
+        }
+    }
+}
+
+// the same by merging the lists, for lists of more than 64 entries
+__global__ void __launch_bounds__(256) k_cac_merge(DevParams P, const int* __restrict__ nFluid,
+                                                   const int* __restrict__ nCountP,
+                                                   const long long* __restrict__ nPtrP,
+                                                   const int* __restrict__ nIndP, const double* __restrict__ cval,
+                                                   const double* __restrict__ dval,
+                                                   const long long* __restrict__ start,
+                                                   const int* __restrict__ acol, double* __restrict__ aval,
+                                                   float* __restrict__ aval32) {
+    const int slice = blockIdx.x;
+    const int lane = threadIdx.x % kSlice, wave = threadIdx.x / kSlice;
+    const int i = slice * kSlice + lane;
     if (i >= P.nf) return;
     const int nfl = nFluid[i];
     const long long pi = nPtrP[i];
     const int ni = nCountP[i];
-    const int* ki = kLdsI ? sk + lane * kStride : nIndP + pi;
-    int* kjs = sj + threadIdx.x * kStride;  // this thread's copy of j's list (kLdsJ)
+    const int* ki = nIndP + pi;
     const double* di = dval + 3 * pi;
     const long long sb = start[slice];
     for (int k = wave; k < nfl; k += 4) {
@@ -684,52 +799,28 @@ __global__ void __launch_bounds__(256) k_cac(DevParams P, const int* __restrict_
         const long long pj = nPtrP[j];
         const int nj = nCountP[j];
         const int* kj = nIndP + pj;
-        if (kLdsJ) {  // all loads of j's list in flight at once, then merge from LDS
-            for (int t = 0; t < nj; ++t) kjs[t] = kj[t];
-            kj = kjs;
-        }
         double sum[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        auto add = [&](int a, int c) {  // sum += D_i,k (x) C_j,k for the shared k
-            const double* cj = &cval[3 * (pj + c)];
-            const double c0 = cj[0], c1 = cj[1], c2 = cj[2];
-            const double d0 = di[3 * a], d1 = di[3 * a + 1], d2 = di[3 * a + 2];
-            sum[0] += d0 * c0; sum[1] += d0 * c1; sum[2] += d0 * c2;
-            sum[3] += d1 * c0; sum[4] += d1 * c1; sum[5] += d1 * c2;
-            sum[6] += d2 * c0; sum[7] += d2 * c1; sum[8] += d2 * c2;
-        };
-        if (kMode == 3) {
-            // merge without work in the loop: the matches (a, c), ascending, go over
-            // the already consumed front of j's list in LDS; then add them in order
-            int a = 0, c = 0, n = 0;
-            int ka = ni > 0 ? ki[0] : 0;
-            int kc = nj > 0 ? kjs[0] : 0;
-            while (a < ni && c < nj) {
-                const bool eq = ka == kc, le = ka <= kc, ge = ka >= kc;
-                if (eq) kjs[n++] = a | (c << 16);
-                a += le;
-                c += ge;
-                if (le && a < ni) ka = ki[a];
-                if (ge && c < nj) kc = kjs[c];
-            }
-            for (int t = 0; t < n; ++t) add(kjs[t] & 0xffff, kjs[t] >> 16);
-        } else {
-            int a = 0, c = 0;
-            int ka = ni > 0 ? ki[0] : 0;
-            int kc = nj > 0 ? kj[0] : 0;
-            while (a < ni && c < nj) {
-                if (ka == kc) {
-                    add(a, c);
-                    a++;
-                    c++;
-                    if (a < ni) ka = ki[a];
-                    if (c < nj) kc = kj[c];
-                } else if (ka < kc) {
-                    a++;
-                    if (a < ni) ka = ki[a];
-                } else {
-                    c++;
-                    if (c < nj) kc = kj[c];
-                }
+        int a = 0, c = 0;
+        int ka = ni > 0 ? ki[0] : 0;
+        int kc = nj > 0 ? kj[0] : 0;
+        while (a < ni && c < nj) {
+            if (ka == kc) {
+                const double* cj = &cval[3 * (pj + c)];
+                const double c0 = cj[0], c1 = cj[1], c2 = cj[2];
+                const double d0 = di[3 * a], d1 = di[3 * a + 1], d2 = di[3 * a + 2];
+                sum[0] += d0 * c0; sum[1] += d0 * c1; sum[2] += d0 * c2;
+                sum[3] += d1 * c0; sum[4] += d1 * c1; sum[5] += d1 * c2;
+                sum[6] += d2 * c0; sum[7] += d2 * c1; sum[8] += d2 * c2;
+                a++;
+                c++;
+                if (a < ni) ka = ki[a];
+                if (c < nj) kc = kj[c];
+            } else if (ka < kc) {
+                a++;
+                if (a < ni) ka = ki[a];
+            } else {
+                c++;
+                if (c < nj) kc = kj[c];
             }
         }
         for (int e9 = 0; e9 < 9; ++e9) {
@@ -740,7 +831,6 @@ __global__ void __launch_bounds__(256) k_cac(DevParams P, const int* __restrict_
         }
     }
 }
-
 
 }  // namespace
 
@@ -807,15 +897,19 @@ void launch_b_minus_cp(hipStream_t st, const DevParams& P, const int* nCountP, c
 }
 
 void launch_cac(hipStream_t st, const DevParams& P, const int* nFluid, const int* nCountP, const long long* nPtrP,
-                const int* nIndP, const double* cval, const double* dval, ASlices A, int mode) {
+                const int* nIndP, const double* cval, const double* dval, ASlices A, int maxP) {
     if (A.nslices == 0) return;
-#define MPH_CAC(M)                                                                                            \
-    hipLaunchKernelGGL(k_cac<M>, dim3(A.nslices), dim3(256), 0, st, P, nFluid, nCountP, nPtrP, nIndP, cval, dval, \
-                       A.start, A.col, A.val, A.val32)
-    if (mode == 3) MPH_CAC(3);
-    else if (mode == 2) MPH_CAC(2);
-    else MPH_CAC(0);
-#undef MPH_CAC
+    // a hash entry has 6 bits for the place in the list and 26 for the particle (the last
+    // number marks an empty one)
+    if (maxP > 64 || P.np >= (1 << 26) - 1) {
+        hipLaunchKernelGGL(k_cac_merge, dim3(A.nslices), dim3(256), 0, st, P, nFluid, nCountP, nPtrP, nIndP, cval, dval,
+                           A.start, A.col, A.val, A.val32);
+        return;
+    }
+    // few slices: up to 16 workgroups share one, towards 16 workgroups per CU
+    const int want = (4096 + A.nslices - 1) / A.nslices, y = want > 16 ? 16 : want;
+    hipLaunchKernelGGL(k_cac, dim3(A.nslices, y), dim3(256), 0, st, P, nFluid, nCountP, nPtrP, nIndP, cval, dval,
+                       A.start, A.col, A.val, A.val32);
 }
 
 }  // namespace mph

@@ -318,7 +318,7 @@ int phase_neighbor_finish(mph_scene& S) {
     S.blocks = blocks_wanted(S);
     S.fslotValid = false;  // the staged places follow the new lists (matrix-C phase)
     int rc;
-    if ((rc = S.nInd.ensure(S.E > 0 ? S.E : 1)) || (rc = S.nIndP.ensure(S.EP > 0 ? S.EP : 1))) return rc;
+    if ((rc = S.nInd.ensure(S.E > 0 ? S.E : 1)) || (rc = S.nIndP.ensure(S.EP + kListSpare))) return rc;
     S.oneScan = scanned;
     if (scanned)
         launch_neighbor_compact(S.st, P, S.nCount.p, S.nCountP.p, S.nPtr.p, S.nPtrP.p, S.scrM.p, S.searchCapM,
@@ -416,15 +416,7 @@ int phase_multiply_c(mph_scene& S) {
     }
     // C Lambda C^T also writes the FP32 copy of A in mixed precision (aval32) unless
     // the solve applies the factored form
-    if (S.hmaxP > kMaxP) {  // P lists too long for the LDS modes
-        launch_cac(S.st, S.P, S.nFluid.p, S.nCountP.p, S.nPtrP.p, S.nIndP.p, S.cval.p, S.dval.p, aslices(S), 0);
-    } else {
-        const int v = S.tuneCac.pick();
-        S.tuneCac.begin(S.st, v);
-        launch_cac(S.st, S.P, S.nFluid.p, S.nCountP.p, S.nPtrP.p, S.nIndP.p, S.cval.p, S.dval.p, aslices(S),
-                   kCacModeOf[v]);
-        S.tuneCac.end(S.st);
-    }
+    launch_cac(S.st, S.P, S.nFluid.p, S.nCountP.p, S.nPtrP.p, S.nIndP.p, S.cval.p, S.dval.p, aslices(S), S.hmaxP);
     S.assembled = true;
     return MPH_OK;
 }
@@ -589,7 +581,6 @@ int cr_tail(mph_scene& S, bool first, double* xv) {
 void collect_tuning(mph_scene& S) {  // the stream is idle
     S.tuneSpmv64.collect();
     S.tuneSpmv32.collect();
-    S.tuneCac.collect();
     S.tuneGal.collect();
 }
 
@@ -872,7 +863,7 @@ int cr_loop_device(mph_scene& S, long long maxit) {
     }
     // the variant trials of the eager iterations are read as their iterations complete
     // (mark: how many trials each autotuner had recorded at an iteration's event)
-    Autotune* tn[] = {&S.tuneSpmv64, &S.tuneSpmv32, &S.tuneCac, &S.tuneGal};
+    Autotune* tn[] = {&S.tuneSpmv64, &S.tuneSpmv32, &S.tuneGal};
     constexpr int kTn = sizeof(tn) / sizeof(tn[0]);
     size_t mark[2][kTn];
     for (int t = 0; t < kTn; ++t) mark[0][t] = tn[t]->pend.size();
@@ -1202,7 +1193,6 @@ void destroy(mph_scene* S) {
     S->packI.release();
     S->tuneSpmv64.release();
     S->tuneSpmv32.release();
-    S->tuneCac.release();
     S->tuneGal.release();
     if (S->hpin) (void)hipHostFree(S->hpin);
     if (S->hrr) (void)hipHostFree(S->hrr);
@@ -1507,7 +1497,6 @@ int mph_scene_create(const mph_params* p, const mph_grid* g, int device, mph_sce
     S->iStep = (int)(S->time / S->P.dt);
     S->tuneSpmv64.init(kSpmvVariants64, 3);
     S->tuneSpmv32.init(kSpmvVariants32, 3);
-    S->tuneCac.init(kCacVariants, 1);
     S->tuneGal.init(kGalVariants, 1);
     S->outputNext = S->time;
     S->vtkOutputNext = S->time;
@@ -1659,7 +1648,7 @@ int mph_scene_scalar(mph_scene* S, const char* name, double* v) {
     else if (n == "SpmvMsF32") *v = S->spmvMs32;
     else if (n == "TunedSpmv64") *v = S->tuneSpmv64.best;
     else if (n == "TunedSpmv32") *v = S->tuneSpmv32.best;
-    else if (n == "TunedCac") *v = S->tuneCac.best;
+    else if (n == "TunedCac") *v = 0;  // one variant
     else if (n == "TunedFuse") *v = 0;  // one variant: the levels that fit one workgroup are fused
     else if (n == "TunedGalerkin") *v = S->tuneGal.best;
     else if (n == "FactoredCellsUsed") *v = factored(*S) && fac_cells(*S) ? 1.0 : 0.0;

@@ -261,7 +261,7 @@ struct mph_scene {
     int spmvTimingErr = 0;
     // run-time variant choice (SpMV load groups per precision, C Lambda C^T schedule,
     // level-0 Galerkin)
-    mph::host::Autotune tuneSpmv64, tuneSpmv32, tuneCac, tuneGal;
+    mph::host::Autotune tuneSpmv64, tuneSpmv32, tuneGal;
     int batches = 0;  // batches holding this scene (it cannot be destroyed meanwhile)
 };
 
