@@ -6,8 +6,8 @@
 // 4494-4738).  Each of a particle's sums runs over the neighbour list in list
 // order, so every value is bit-identical to the reference.  The list walks of the
 // densities, forces and matrix A are entry-parallel: a group of kLanes lanes owns
-// the particle, lane g computes the terms of entries g, g + kLanes, ..., and the
-// group's first lane adds them, read back through LDS, in list order.
+// the particle, lane g computes the terms of entries g, g + kLanes, ..., and a lane per
+// component adds them, read back through LDS, in list order.
 #include "mph_kernels.h"
 
 namespace mph {
@@ -37,9 +37,35 @@ __device__ inline Rel rel(const DevParams& P, const double* __restrict__ pos, in
 
 // lanes per particle of the entry-parallel list walks (a workgroup is 256 lanes):
 // kLanes for the MaxRadius lists (about 180 entries in 3D), kLanesP for the RadiusP
-// lists (about 20).  Measured on the 1M scene: 4 lanes beat 2, 8 and 16 on the long
-// lists (k_forces 3.50 against 3.71 / 4.04 / 5.40 ms), 8 beat 4 on the short ones.
-constexpr int kLanes = 4, kLanesP = 8;
+// lists (about 20).  32 lanes on the long lists: matrix A 48 against 58 us at 4.9k
+// particles, but 4.26 against 3.76 ms at 1M (fewer particles to a wavefront share an
+// addition)
+constexpr int kLanes = 16, kLanesP = 8;
+
+// The terms of a round of kLanes entries, a row per component: the lane that owns a
+// component adds its row in list order, two terms to a read.  A term that the entry does
+// not have is +0: a sum starts at +0 and so is never -0, and adding it changes nothing.
+// One lane adding every component of its particle's entries, four lanes to a particle,
+// spent most of the walk there, one dependent LDS read after the other, in 45 rounds of
+// loads for a list of 180.  Densities, forces, matrix A at 4.9k particles: 71, 47, 160 us
+// then, 26, 23, 58 now; at 64k 130, 115, 285 and 83, 77, 253; at 1M 1.57, 1.34, 3.97 ms
+// and 1.18, 1.19, 3.76, of which matrix A's divisions and stores are most.
+template <int K>
+struct TermRows {
+    double v[256 / kLanes][K][kLanes + 2];
+    __device__ inline double add(int row, double s) const {  // s + the row's terms
+        typedef double dv2 __attribute__((ext_vector_type(2)));
+        const dv2* t = (const dv2*)v[threadIdx.x / kLanes][row];
+#pragma unroll
+        for (int o = 0; o < kLanes / 2; ++o) {
+            const dv2 w = t[o];
+            s += w[0];
+            s += w[1];
+        }
+        return s;
+    }
+    __device__ inline double& at(int row) { return v[threadIdx.x / kLanes][row][threadIdx.x % kLanes]; }
+};
 
 // calculateConvection, calculateWall, calculatePeriodicBoundary, resetForce
 __global__ void k_kinematics(DevParams P, WallKin wk, const int* __restrict__ type, double* __restrict__ pos,
@@ -79,96 +105,49 @@ __global__ void __launch_bounds__(256) k_densities(DevParams P, const int* __res
                                                    const long long* __restrict__ nPtr, const int* __restrict__ nInd,
                                                    double* __restrict__ densA, double* __restrict__ gcen,
                                                    double* __restrict__ volStrainP) {
-    // terms: DensityA, the three GravityCenter ones, DensityP.  Each lane takes U
-    // entries per round (entries base + u*G + g), whose loads are in flight together;
-    // the group's first lane adds the round's terms in list order
-    constexpr int G = kLanes, K = 5, U = 2;
-    __shared__ double tb[256 * U * K];
-    __shared__ int tf[256 * U];
+    // terms: DensityA, the three GravityCenter ones, DensityP
+    constexpr int G = kLanes, K = 5;
+    __shared__ TermRows<K> T;
     const int g = threadIdx.x & (G - 1);
     const int i = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) / G);
-    const bool own = i < P.np;
-    const int ti = own ? type[i] : 0;
-    double pi[3] = {0.0, 0.0, 0.0};
-    if (own)
-        for (int d = 0; d < 3; ++d) pi[d] = pos[3 * i + d];
-    double sa = 0.0, sg0 = 0.0, sg1 = 0.0, sg2 = 0.0, sp = 0.0;
-    const long long b = own ? nPtr[i] : 0;
-    const int n = own ? nCount[i] : 0;
-    int jnext[U];  // each lane's next entries load one round ahead
-    for (int u = 0; u < U; ++u) jnext[u] = g + u * G < n ? nInd[b + g + u * G] : 0;
-    for (int base = 0; base < n; base += G * U) {
-        int jcur[U];
-        for (int u = 0; u < U; ++u) {
-            const int jn = base + u * G + g;
-            jcur[u] = jnext[u];
-            jnext[u] = jn + G * U < n ? nInd[b + jn + G * U] : 0;
-        }
-        // the round's loads, before any branch (entries past the list read particle 0)
-        int tj[U];
-        double pj[U][3];
-        for (int u = 0; u < U; ++u) {
-            tj[u] = type[jcur[u]];
-            for (int d = 0; d < 3; ++d) pj[u][d] = pos[3 * jcur[u] + d];
-        }
-        for (int u = 0; u < U; ++u) {
-            const int jn = base + u * G + g;
-            int f = 0;
-            double t[K] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            if (jn < n) {
-                const int j = jcur[u];
-                if (i != j) {
-                    const double ratio = P.ratio[ti][tj[u]];
-                    Rel q;  // rel() on the loaded positions
-                    for (int d = 0; d < 3; ++d) q.x[d] = min_image(pj[u][d], pi[d], P.W[d], P.hW[d]);
-                    q.r2 = (q.x[0] * q.x[0] + q.x[1] * q.x[1] + q.x[2] * q.x[2]);
-                    if (P.radA2 - q.r2 >= 0) {
-                        const double r = sqrt(q.r2);
-                        t[0] = ratio * wa_k(P.Ka, r, P.radA);
-                        f |= 1;
-                    }
-                    if (P.radG2 - q.r2 >= 0) {
-                        const double r = sqrt(q.r2);
-                        const double weight = ratio * wq_k(P.Kg, r, P.radG);
-                        t[1] = q.x[0] * weight / P.R2g * P.radG;
-                        t[2] = q.x[1] * weight / P.R2g * P.radG;
-                        t[3] = q.x[2] * weight / P.R2g * P.radG;
-                        f |= 2;
-                    }
-                    if (P.radP2 - q.r2 >= 0) {
-                        const double r = sqrt(q.r2);
-                        t[4] = wq_k(P.Kp, r, P.radP);
-                        f |= 4;
-                    }
-                }
+    if (i >= P.np) return;  // the whole group
+    const int ti = type[i];
+    double pi[3];
+    for (int d = 0; d < 3; ++d) pi[d] = pos[3 * i + d];
+    double s = 0.0;
+    const long long b = nPtr[i];
+    const int n = nCount[i];
+    int jnext = g < n ? nInd[b + g] : 0;  // each lane's next entry loads one round ahead
+    for (int base = 0; base < n; base += G) {
+        const int jn = base + g, j = jnext;
+        jnext = jn + G < n ? nInd[b + jn + G] : 0;
+        double t[K] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        const int tj = type[j];  // before any branch (entries past the list read particle 0)
+        double pj[3];
+        for (int d = 0; d < 3; ++d) pj[d] = pos[3 * j + d];
+        if (jn < n && i != j) {
+            const double ratio = P.ratio[ti][tj];
+            Rel q;  // rel() on the loaded positions
+            for (int d = 0; d < 3; ++d) q.x[d] = min_image(pj[d], pi[d], P.W[d], P.hW[d]);
+            q.r2 = (q.x[0] * q.x[0] + q.x[1] * q.x[1] + q.x[2] * q.x[2]);
+            const double r = sqrt(q.r2);
+            if (P.radA2 - q.r2 >= 0) t[0] = ratio * wa_k(P.Ka, r, P.radA);
+            if (P.radG2 - q.r2 >= 0) {
+                const double weight = ratio * wq_k(P.Kg, r, P.radG);
+                t[1] = q.x[0] * weight / P.R2g * P.radG;
+                t[2] = q.x[1] * weight / P.R2g * P.radG;
+                t[3] = q.x[2] * weight / P.R2g * P.radG;
             }
-            for (int e = 0; e < K; ++e) tb[K * (U * threadIdx.x + u) + e] = t[e];
-            tf[U * threadIdx.x + u] = f;
+            if (P.radP2 - q.r2 >= 0) t[4] = wq_k(P.Kp, r, P.radP);
         }
+        for (int e = 0; e < K; ++e) T.at(e) = t[e];
         wave_sync();
-        if (g == 0)
-            for (int u = 0; u < U; ++u)
-                for (int v = 0; v < G && base + u * G + v < n; ++v) {
-                    const int sl = U * (threadIdx.x + v) + u;
-                    const int fu = tf[sl];
-                    const double* tu = tb + K * sl;
-                    if (fu & 1) sa += tu[0];
-                    if (fu & 2) {
-                        sg0 += tu[1];
-                        sg1 += tu[2];
-                        sg2 += tu[3];
-                    }
-                    if (fu & 4) sp += tu[4];
-                }
+        if (g < K) s = T.add(g, s);
         wave_sync();
     }
-    if (g == 0 && own) {
-        densA[i] = sa;
-        gcen[3 * i + 0] = sg0;
-        gcen[3 * i + 1] = sg1;
-        gcen[3 * i + 2] = sg2;
-        volStrainP[i] = (sp - P.N0p);
-    }
+    if (g == 0) densA[i] = s;
+    else if (g < 4) gcen[3 * i + g - 1] = s;
+    else if (g == 4) volStrainP[i] = (s - P.N0p);
 }
 
 // calculatePhysicalCoefficients (1704-1735) and the PressureA values (1807-1812)
@@ -201,125 +180,92 @@ __global__ void __launch_bounds__(256) k_forces(DevParams P, const int* __restri
                                                 const double* __restrict__ mass, double* __restrict__ force,
                                                 double* __restrict__ vel) {
     // terms: PressureA force, the two DiffuseInterface ones (3 each)
-    constexpr int G = kLanes, K = kSurf ? 9 : 3, U = 2;
-    __shared__ double tb[256 * U * K];
-    __shared__ int tf[256 * U];
+    constexpr int G = kLanes, K = kSurf ? 9 : 3;
+    __shared__ TermRows<K> T;
     const int g = threadIdx.x & (G - 1);
     const int i = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) / G);
-    const bool own = i < P.np;
-    const int ti = own ? type[i] : 0;
+    if (i >= P.np) return;  // the whole group
+    const int ti = type[i];
     const double ai = P.ai[ti];
     const double aj = P.ai[ti];  // the reference uses i's type for aj (main.cpp:1863)
     const double VoL = P.V / P.l;
-    const double pai = own ? pressA[i] : 0.0;
-    const double gi0 = own ? gcen[3 * i] : 0.0, gi1 = own ? gcen[3 * i + 1] : 0.0, gi2 = own ? gcen[3 * i + 2] : 0.0;
-    double fa[3] = {0.0, 0.0, 0.0}, fd[3] = {0.0, 0.0, 0.0};
-    const long long b = own ? nPtr[i] : 0;
-    const int n = own ? nCount[i] : 0;
-    double pi[3] = {0.0, 0.0, 0.0};
-    if (own)
-        for (int d = 0; d < 3; ++d) pi[d] = pos[3 * i + d];
-    // each lane takes U entries per round (base + u*G + g), their loads in flight
-    // together and issued one round ahead for the columns; the group's first lane
-    // adds the round's terms in list order
-    int jnext[U];
-    for (int u = 0; u < U; ++u) jnext[u] = g + u * G < n ? nInd[b + g + u * G] : 0;
-    for (int base = 0; base < n; base += G * U) {
-        int jcur[U], tjs[U];
-        double pajs[U], pj[U][3], gjs[U][3];
-        for (int u = 0; u < U; ++u) {
-            const int jn = base + u * G + g;
-            jcur[u] = jnext[u];
-            jnext[u] = jn + G * U < n ? nInd[b + jn + G * U] : 0;
+    const double pai = pressA[i];
+    const double gi[3] = {gcen[3 * i], gcen[3 * i + 1], gcen[3 * i + 2]};
+    double s = 0.0;  // lanes 0-2: the PressureA force, lanes 3-5: the DiffuseInterface force
+    const long long b = nPtr[i];
+    const int n = nCount[i];
+    double pi[3];
+    for (int d = 0; d < 3; ++d) pi[d] = pos[3 * i + d];
+    int jnext = g < n ? nInd[b + g] : 0;  // each lane's next entry loads one round ahead
+    for (int base = 0; base < n; base += G) {
+        const int jn = base + g, j = jnext;
+        jnext = jn + G < n ? nInd[b + jn + G] : 0;
+        const int tj = type[j];  // j's values load with its position (past the list: particle 0)
+        const double paj = pressA[j];
+        double pj[3], gj[3];
+        for (int d = 0; d < 3; ++d) {
+            pj[d] = pos[3 * j + d];
+            gj[d] = kSurf ? gcen[3 * j + d] : 0.0;
         }
-        for (int u = 0; u < U; ++u) {  // j's values load with its position (past the list: particle 0)
-            const int j = jcur[u];
-            tjs[u] = type[j];
-            pajs[u] = pressA[j];
-            for (int d = 0; d < 3; ++d) {
-                pj[u][d] = pos[3 * j + d];
-                gjs[u][d] = kSurf ? gcen[3 * j + d] : 0.0;
-            }
-        }
-        for (int u = 0; u < U; ++u) {
-            const int jn = base + u * G + g;
-            int f = 0;
-            double t[K];
-            for (int e = 0; e < K; ++e) t[e] = 0.0;
-            if (jn < n) {
-                const int j = jcur[u];
-                const int tj = tjs[u];
-                const double paj = pajs[u];
-                const double gj[3] = {gjs[u][0], gjs[u][1], gjs[u][2]};
-                Rel q;  // rel() on the loaded positions
-                for (int d = 0; d < 3; ++d) q.x[d] = min_image(pj[u][d], pi[d], P.W[d], P.hW[d]);
-                q.r2 = (q.x[0] * q.x[0] + q.x[1] * q.x[1] + q.x[2] * q.x[2]);
-                if (i != j && q.r2 != 0.0) {
-                    const double rij_ = P.ratio[ti][tj], rji_ = P.ratio[tj][ti];
-                    if (P.radA2 - q.r2 > 0) {
-                        const double r = sqrt(q.r2);
-                        const double dwij = rij_ * dwadr_k(P.Ka, P.invA, r, P.radA);
-                        const double dwji = rji_ * dwadr_k(P.Ka, P.invA, r, P.radA);
-                        for (int d = 0; d < 3; ++d) t[d] = (pai * dwij + paj * dwji) * (q.x[d] / r) * P.V;
-                        f |= 1;
-                    }
-                    if (kSurf && P.radG2 - q.r2 > 0) {
-                        const double r = sqrt(q.r2);
-                        const double wij = rij_ * wq_k(P.Kg, r, P.radG);
-                        const double wji = rji_ * wq_k(P.Kg, r, P.radG);
-                        const double gi[3] = {gi0, gi1, gi2};
-                        for (int d = 0; d < 3; ++d)
-                            t[3 + d] = (aj * gj[d] * wji - ai * gi[d] * wij) / P.R2g * P.radG * VoL;
-                        const double dwij = rij_ * dwq_k(P.Kg, P.m2G, r, P.radG);
-                        const double dwji = rji_ * dwq_k(P.Kg, P.m2G, r, P.radG);
-                        double gr = 0.0;
-                        for (int d = 0; d < 3; ++d) gr += (aj * gj[d] * dwji - ai * gi[d] * dwij) * q.x[d];
-                        for (int d = 0; d < 3; ++d) t[6 + d] = (gr) * (q.x[d] / r) / P.R2g * P.radG * VoL;
-                        f |= 2;
-                    }
+        double t[K];
+        for (int e = 0; e < K; ++e) t[e] = 0.0;
+        if (jn < n) {
+            Rel q;  // rel() on the loaded positions
+            for (int d = 0; d < 3; ++d) q.x[d] = min_image(pj[d], pi[d], P.W[d], P.hW[d]);
+            q.r2 = (q.x[0] * q.x[0] + q.x[1] * q.x[1] + q.x[2] * q.x[2]);
+            if (i != j && q.r2 != 0.0) {
+                const double rij_ = P.ratio[ti][tj], rji_ = P.ratio[tj][ti];
+                if (P.radA2 - q.r2 > 0) {
+                    const double r = sqrt(q.r2);
+                    const double dwij = rij_ * dwadr_k(P.Ka, P.invA, r, P.radA);
+                    const double dwji = rji_ * dwadr_k(P.Ka, P.invA, r, P.radA);
+                    for (int d = 0; d < 3; ++d) t[d] = (pai * dwij + paj * dwji) * (q.x[d] / r) * P.V;
+                }
+                if (kSurf && P.radG2 - q.r2 > 0) {
+                    const double r = sqrt(q.r2);
+                    const double wij = rij_ * wq_k(P.Kg, r, P.radG);
+                    const double wji = rji_ * wq_k(P.Kg, r, P.radG);
+                    for (int d = 0; d < 3; ++d)
+                        t[3 + d] = (aj * gj[d] * wji - ai * gi[d] * wij) / P.R2g * P.radG * VoL;
+                    const double dwij = rij_ * dwq_k(P.Kg, P.m2G, r, P.radG);
+                    const double dwji = rji_ * dwq_k(P.Kg, P.m2G, r, P.radG);
+                    double gr = 0.0;
+                    for (int d = 0; d < 3; ++d) gr += (aj * gj[d] * dwji - ai * gi[d] * dwij) * q.x[d];
+                    for (int d = 0; d < 3; ++d) t[6 + d] = (gr) * (q.x[d] / r) / P.R2g * P.radG * VoL;
                 }
             }
-            for (int e = 0; e < K; ++e) tb[K * (U * threadIdx.x + u) + e] = t[e];
-            tf[U * threadIdx.x + u] = f;
+        }
+        for (int e = 0; e < K; ++e) T.at(e) = t[e];
+        wave_sync();
+        if (g < 3) s = T.add(g, s);
+        if (kSurf && g >= 3 && g < 6) {  // both terms of an entry, then the next entry's
+            const double* t1 = T.v[threadIdx.x / G][g];
+            const double* t2 = T.v[threadIdx.x / G][g + 3];
+#pragma unroll 8
+            for (int o = 0; o < G; ++o) {
+                s -= t1[o];
+                s -= t2[o];
+            }
         }
         wave_sync();
-        if (g == 0)
-            for (int u = 0; u < U; ++u)
-                for (int v = 0; v < G && base + u * G + v < n; ++v) {
-                    const int sl = U * (threadIdx.x + v) + u;
-                    const int fu = tf[sl];
-                    const double* tu = tb + K * sl;
-                    if (fu & 1)
-                        for (int d = 0; d < 3; ++d) fa[d] += tu[d];
-                    if (kSurf && (fu & 2)) {
-                        for (int d = 0; d < 3; ++d) fd[d] -= tu[3 + d];
-                        for (int d = 0; d < 3; ++d) fd[d] -= tu[6 + d];
-                    }
-                }
-        wave_sync();
     }
-    if (g != 0 || !own) return;
-    double F[3];
-    for (int d = 0; d < 3; ++d) {
-        F[d] = force[3 * i + d];
-        F[d] += fa[d];
-        F[d] += fd[d];
-    }
+    const double fd = __shfl_down(s, 3, G);
+    if (g >= 3) return;
+    double F = force[3 * i + g];
+    F += s;
+    F += kSurf ? fd : 0.0;
     if (i < P.nf) {
         const double m = mass[i];
-        for (int d = 0; d < 3; ++d) {
-            F[d] += m * P.gravity[d];
-            vel[3 * i + d] += F[d] / m * P.dt;
-        }
+        F += m * P.gravity[g];
+        vel[3 * i + g] += F / m * P.dt;
     }
-    for (int d = 0; d < 3; ++d) force[3 * i + d] = F[d];
+    force[3 * i + g] = F;
 }
 
 // calculateMatrixA values (2251-2335): viscous blocks, inertia, wall terms of b.
-// kBlk: also the factored form's level-0 run sums (blk, from the run starts): while
-// the group's first lane adds every entry's block in list order, its second lane adds
-// the same fluid entries' -alpha r r^T (the negated block; 0 beyond RadiusV and for
-// the self entry) per visited cell, and stores each cell's sum when its run ends
+// kBlk: also the factored form's level-0 run sums (blk, from the run starts): lane q sums
+// the -alpha r r^T (the negated blocks; 0 beyond RadiusV and for the self entry) of the
+// fluid entries in visited cell q's run, all cells at a time
 template <bool kBlk>
 __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __restrict__ type,
                                                   const double* __restrict__ pos, const double* __restrict__ vel,
@@ -333,20 +279,21 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
                                                   const unsigned short* __restrict__ runStart,
                                                   double* __restrict__ blk) {
     constexpr int G = kLanes, K = 12;  // terms: the 3x3 coefficients, then a wall neighbour's velocity
-    __shared__ double tb[256 * K];
-    __shared__ int tf[256];  // bit 0: the self entry, bit 1: inside RadiusV, bit 2: and a wall neighbour
-    const int g = threadIdx.x & (G - 1);
+    __shared__ TermRows<K> T;
+    __shared__ int wall[256];  // a wall neighbour inside RadiusV
+    const int g = threadIdx.x & (G - 1), grp = threadIdx.x / G;
     const int i = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) / G);
-    const bool own = i < P.nf;
-    int iN = 0;
-    // s9: the group's first lane sums the diagonal block in it; with kBlk its second
-    // lane sums the current visited cell's run of -alpha r r^T (one register array)
-    double s9[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double sv0 = 0.0, sv1 = 0.0, sv2 = 0.0;
-    const double mui = own ? mu[i] : 0.0;
-    const long long b0 = own ? nPtr[i] : 0;
-    const int nfl = own ? nFluid[i] : 0, nc = own ? nCount[i] : 0;
-    const long long sb = own ? start[i / kSlice] : 0;
+    if (i >= P.nf) return;  // the whole group
+    double s = 0.0, sv = 0.0;  // lanes 0-8: the diagonal block; lanes 0-2: the wall terms of b
+    // lane g: the runs (upper triangles) of cells g, g + G
+    constexpr int R = kBlk ? (kBlkRuns + G - 1) / G : 1;
+    double run[R][6];
+    for (int c = 0; c < R; ++c)
+        for (int e = 0; e < 6; ++e) run[c][e] = 0.0;
+    const double mui = mu[i];
+    const long long b0 = nPtr[i];
+    const int nfl = nFluid[i], nc = nCount[i];
+    const long long sb = start[i / kSlice];
     const int lane = i % kSlice;
     // factored form: alpha_ij = visc mu_ij (-w_v'(d)) / d^3, the viscous block being
     // -alpha_ij r r^T (beside the neighbour list; 0 for self and beyond RadiusV)
@@ -356,39 +303,24 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
     // the 3x3 blocks are stored unless aval is null (a factored scene that builds its
     // multigrid level 0 from the factored form needs none)
     const bool blocks = aval != nullptr;
-    // the run sums: visited cell qr's run of fluid entries is [rsp[qr], rsp[qr+1])
-    typedef double dv2 __attribute__((ext_vector_type(2)));
-    const bool runner = kBlk && g == 1 && own;
-    // the group's run starts, staged in LDS by its four lanes (a flush then reads the
-    // next run's end there, not from global memory in the serial loop)
-    __shared__ unsigned short rsl[256 / G][kRuns];
-    unsigned short* const rsp = rsl[threadIdx.x / G];
-    if (kBlk && own)
-        for (int k = g; k < kRuns; k += G) rsp[k] = runStart[(long long)i * kRuns + k];
-    if (kBlk) wave_sync();
-    double* const bk = kBlk ? blk + (long long)(own ? i : 0) * kBlkRuns * kBlkStride : nullptr;
     const int nv = (2 * P.range[0] + 1) * (2 * P.range[1] + 1) * (2 * P.range[2] + 1);
-    int qr = 0, qend = runner ? rsp[1] : 0;
-    auto flush = [&]() {  // cell qr's sums (upper triangle), then the next cell
-        dv2* o = (dv2*)(bk + qr * kBlkStride);
-        o[0] = dv2{s9[0], s9[1]};
-        o[1] = dv2{s9[2], s9[4]};
-        o[2] = dv2{s9[5], s9[8]};
-        for (int e9 = 0; e9 < 9; ++e9) s9[e9] = 0.0;
-        ++qr;
-        qend = qr < nv ? rsp[qr + 1] : 0x7fffffff;
-    };
+    int q0[R], q1[R];
+    for (int c = 0; c < R; ++c) {
+        const bool in = kBlk && g + c * G < nv;
+        q0[c] = in ? runStart[(long long)i * kRuns + g + c * G] : 0;
+        q1[c] = in ? runStart[(long long)i * kRuns + g + c * G + 1] : 0;
+    }
+    int iN = 0;
     int jnext = g < nc ? nInd[b0 + g] : 0;  // each lane's next entry loads one round ahead
     for (int base = 0; base < nc; base += G) {
         const int jn = base + g;
-        const int jcur = jnext;
+        const int j = jnext;
         jnext = jn + G < nc ? nInd[b0 + jn + G] : 0;
         int f = 0;
         double t[K] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (jn < nc) {
-            const int j = jcur;
             if (i == j) {
-                f = 1;
+                iN = jn;
                 if (blocks) acol[a_col_index(sb, jn, lane)] = j;
                 if (jn < nfl) store_alpha(jn, 0.0);
             } else {
@@ -414,12 +346,11 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
                     for (int r = 0; r < 3; ++r)
                         for (int sdim = 0; sdim < 3; ++sdim)
                             t[3 * r + sdim] = +P.visc * muij * e[sdim] * e[r] * wdrij / dij;
-                    f = 2;
                     if (is_wall(tj)) {
                         t[9] = vel[3 * j];
                         t[10] = vel[3 * j + 1];
                         t[11] = vel[3 * j + 2];
-                        f |= 4;
+                        f = 1;
                     }
                 }
                 if (jn < nfl) {
@@ -431,50 +362,63 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
                 }
             }
         }
-        for (int e = 0; e < K; ++e) tb[K * threadIdx.x + e] = t[e];
-        tf[threadIdx.x] = f;
+        const bool walls = __ballot(f) != 0;
+        for (int e = 0; e < 9; ++e) T.at(e) = t[e];
+        if (walls) {
+            for (int e = 9; e < K; ++e) T.at(e) = t[e];
+            wall[threadIdx.x] = f;
+        }
         wave_sync();
-        // lanes 0 and 1 walk the same entries together: lane 0 adds each block, lane 1
-        // (runner) adds its negation, exactly -1.0 times it, per visited cell
-        if (g == 0 || runner) {
-            const double sgn = g == 0 ? 1.0 : -1.0;
-            for (int u = 0; u < G && base + u < nc; ++u) {
-                const int sl = threadIdx.x - g + u;
-                const int fu = tf[sl];
-                const double* c9 = tb + K * sl;
-                if (g != 0) {
-                    if (base + u >= nfl) break;  // the runs cover the fluid entries
-                    while (base + u >= qend) flush();
+        if (g < 9) s = T.add(g, s);
+        if (walls && g < 3) {
+            const double(&c)[K][G + 2] = T.v[grp];
+            for (int o = 0; o < G; ++o)
+                if (wall[grp * G + o]) {
+                    sv += c[3 * g][o] * c[9][o];
+                    sv += c[3 * g + 1][o] * c[10][o];
+                    sv += c[3 * g + 2][o] * c[11][o];
                 }
-                if (fu & 2)
-                    for (int e9 = 0; e9 < 9; ++e9) s9[e9] += sgn * c9[e9];
-                if (g == 0) {
-                    if (fu & 1) iN = base + u;
-                    if (fu & 4) {
-                        const double v0 = c9[9], v1 = c9[10], v2 = c9[11];
-                        sv0 += c9[0] * v0; sv0 += c9[1] * v1; sv0 += c9[2] * v2;
-                        sv1 += c9[3] * v0; sv1 += c9[4] * v1; sv1 += c9[5] * v2;
-                        sv2 += c9[6] * v0; sv2 += c9[7] * v1; sv2 += c9[8] * v2;
-                    }
+        }
+        if (kBlk) {
+            const double(&c)[K][G + 2] = T.v[grp];
+#pragma unroll
+            for (int h = 0; h < R; ++h) {
+                const int lo = q0[h] > base ? q0[h] - base : 0, hi = q1[h] < base + G ? q1[h] - base : G;
+                for (int o = lo; o < hi; ++o) {
+                    run[h][0] += -c[0][o];
+                    run[h][1] += -c[1][o];
+                    run[h][2] += -c[2][o];
+                    run[h][3] += -c[4][o];
+                    run[h][4] += -c[5][o];
+                    run[h][5] += -c[8][o];
                 }
             }
         }
         wave_sync();
     }
-    if (runner)
-        while (qr < nv) flush();  // the cells after the last fluid entry's run
-    if (g != 0 || !own) return;
+    for (int d = 1; d < G; d <<= 1) {  // the lane that met the self entry tells the others
+        const int o = __shfl_xor(iN, d, G);
+        iN = o > iN ? o : iN;
+    }
+    for (int h = 0; h < R; ++h)
+        if (kBlk && g + h * G < nv) {
+            typedef double dv2 __attribute__((ext_vector_type(2)));
+            dv2* o = (dv2*)(blk + ((long long)i * kBlkRuns + g + h * G) * kBlkStride);
+            o[0] = dv2{run[h][0], run[h][1]};
+            o[1] = dv2{run[h][2], run[h][3]};
+            o[2] = dv2{run[h][4], run[h][5]};
+        }
     const double coef = mass[i] / P.V / P.dt;
-    s9[0] += coef;
-    s9[4] += coef;
-    s9[8] += coef;
-    if (blocks)
-        for (int e9 = 0; e9 < 9; ++e9) aval[a_val_index(sb, iN, e9, lane)] = s9[e9];
-    if (fdiag)
-        for (int e9 = 0; e9 < 9; ++e9) fdiag[9 * i + e9] = s9[e9];
-    selfIdx[i] = iN;
-    const double bv[3] = {0.0 + sv0, 0.0 + sv1, 0.0 + sv2};
-    for (int d = 0; d < 3; ++d) b[3 * i + d] = bv[d] + coef * vel[3 * i + d];
+    if (g < 9) {
+        if (g % 4 == 0) s += coef;
+        if (blocks) aval[a_val_index(sb, iN, g, lane)] = s;
+        if (fdiag) fdiag[9 * (long long)i + g] = s;
+    }
+    if (g == 0) selfIdx[i] = iN;
+    if (g < 3) {
+        const double bv = 0.0 + sv;
+        b[3 * i + g] = bv + coef * vel[3 * i + g];
+    }
 }
 
 // calculateMatrixC values (2463-2507): C[3i+r][k] = e_r * (-w'_p).  Also
