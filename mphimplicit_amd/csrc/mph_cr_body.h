@@ -63,25 +63,29 @@ __device__ inline unsigned galerkin_mask(const DevParams& P, const Level& L, con
     unsigned mask = 0;
     const int* C = P.C;
     const int rx = P.range[0], ry = P.range[1], rz = P.range[2];
-    int jx[3], jy[3], jz[3];
-    for (int k = 0; k < 2 * rx + 1; ++k) jx[k] = ((cx - rx + k) % C[0] + C[0]) % C[0];
-    for (int k = 0; k < 2 * ry + 1; ++k) jy[k] = ((cy - ry + k) % C[1] + C[1]) % C[1];
-    for (int k = 0; k < 2 * rz + 1; ++k) jz[k] = ((cz - rz + k) % C[2] + C[2]) % C[2];
-    const int bx = (2 * rx) - (cx + rx) % C[0], by = (2 * ry) - (cy + ry) % C[1], bz = (2 * rz) - (cz + rz) % C[2];
+    // cells lie in [0, C), so their neighbours wrap without a division; so does the offset
+    // on the level grid, unless the domain's wrap takes it further than one cell
+    auto wrap = [](int v, int n) { return v < 0 ? v + n : v >= n ? v - n : v; };
+    auto slot = [](int d, int n) { return d >= -1 && d <= 1 && n >= 3 ? d + 1 : (d + 1 + n) % n; };
+    const int bx = (2 * rx) - wrap(cx + rx, C[0]), by = (2 * ry) - wrap(cy + ry, C[1]), bz = (2 * rz) - wrap(cz + rz, C[2]);
     const int x0 = bx > 0 ? bx : 0, y0 = by > 0 ? by : 0, z0 = bz > 0 ? bz : 0;
+    const int nx = 2 * rx + 1, ny = 2 * ry + 1, nz = 2 * rz + 1;
     int q = 0;
-    for (int a = x0; a < x0 + (2 * rx + 1); ++a)
-        for (int b = y0; b < y0 + (2 * ry + 1); ++b)
-            for (int cc = z0; cc < z0 + (2 * rz + 1); ++cc, ++q) {
-                const int ax = jx[a % (2 * rx + 1)], ay = jy[b % (2 * ry + 1)], az = jz[cc % (2 * rz + 1)];
-                const int jc = cell_id(P, ax, ay, az);
+    for (int a = x0; a < x0 + nx; ++a) {
+        const int ax = wrap(cx - rx + (a >= nx ? a - nx : a), C[0]);
+        const int ix = slot((ax - L.mn[0]) - gx, L.cnt[0]);
+        for (int b = y0; b < y0 + ny; ++b) {
+            const int ay = wrap(cy - ry + (b >= ny ? b - ny : b), C[1]);
+            const int iy = slot((ay - L.mn[1]) - gy, L.cnt[1]);
+            for (int cc = z0; cc < z0 + nz; ++cc, ++q) {
+                const int az = wrap(cz - rz + (cc >= nz ? cc - nz : cc), C[2]);
+                const int iz = slot((az - L.mn[2]) - gz, L.cnt[2]);
+                const int jc = (ax * C[1] + ay) * C[2] + az;
                 if (cellStart[jc] == cellStart[jc + 1]) continue;  // no fluid there
-                const int dx = (ax - L.mn[0]) - gx, dy = (ay - L.mn[1]) - gy, dz = (az - L.mn[2]) - gz;
-                const int ix = (dx + 1 + L.cnt[0]) % L.cnt[0];
-                const int iy = (dy + 1 + L.cnt[1]) % L.cnt[1];
-                const int iz = (dz + 1 + L.cnt[2]) % L.cnt[2];
                 if (L.cs[2] * L.cs[1] * ix + L.cs[2] * iy + iz == c) mask |= 1u << q;
             }
+        }
+    }
     return mask;
 }
 
@@ -450,19 +454,32 @@ __device__ inline void coarse_pack(const Level* __restrict__ lvs, int lc, int D,
     int gx, gy, gz;
     grid_xyz(L, g, gx, gy, gz);
     int lo = 0;
-    for (int k = 0; k < N; ++k) {
-        const int ex = k / (3 * NZ), ey = (k / NZ) % 3, ez = k % NZ;
-        const bool in = ex < L.cs[0] && ey < L.cs[1] && ez < L.cs[2];
-        const long long sh = in ? 3 * ((L.cs[1] * ex + ey) * L.cs[2] + ez) : 0;
-        for (int sd = 0; sd < 3; ++sd) {
-            const long long e = (sh + sd) * L.nrow + row;
-            K.v[(long long)(3 * k + sd) * K.stride + tid] = !in ? 0.0 : f32 && L.A32 ? (double)L.A32[e] : L.A[e];
+    const bool half = f32 && L.A32;
+    for (int k0 = 0; k0 < N; k0 += 9) {  // nine cells' values in flight
+        double v[27];
+        long long at[27];
+        bool in[9];
+#pragma unroll
+        for (int u = 0; u < 9; ++u) {
+            const int k = k0 + u, ex = k / (3 * NZ), ey = (k / NZ) % 3, ez = k % NZ;
+            in[u] = ex < L.cs[0] && ey < L.cs[1] && ez < L.cs[2];
+            const long long sh = in[u] ? 3 * ((L.cs[1] * ex + ey) * L.cs[2] + ez) : 0;
+            for (int sd = 0; sd < 3; ++sd) at[3 * u + sd] = (sh + sd) * L.nrow + row;
+            const int jx = wrap3(gx + ex - 1 + L.cnt[0], L.cnt[0]), jy = wrap3(gy + ey - 1 + L.cnt[1], L.cnt[1]);
+            const int jz = NZ == 1 ? 0 : wrap3(gz + ez - 1 + L.cnt[2], L.cnt[2]);
+            const int pl = base + 3 * (in[u] ? grid_id(L, jx, jy, jz) : g);
+            if (k & 1) K.i[(k / 2) * K.stride + tid] = lo | (pl << 16);
+            else lo = pl;
         }
-        const int jx = wrap3(gx + ex - 1 + L.cnt[0], L.cnt[0]), jy = wrap3(gy + ey - 1 + L.cnt[1], L.cnt[1]);
-        const int jz = NZ == 1 ? 0 : wrap3(gz + ez - 1 + L.cnt[2], L.cnt[2]);
-        const int pl = base + 3 * (in ? grid_id(L, jx, jy, jz) : g);
-        if (k & 1) K.i[(k / 2) * K.stride + tid] = lo | (pl << 16);
-        else lo = pl;
+        if (half) {
+#pragma unroll
+            for (int e = 0; e < 27; ++e) v[e] = (double)L.A32[at[e]];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 27; ++e) v[e] = L.A[at[e]];
+        }
+#pragma unroll
+        for (int e = 0; e < 27; ++e) K.v[(long long)(3 * k0 + e) * K.stride + tid] = in[e / 3] ? v[e] : 0.0;
     }
     if (N & 1) K.i[(N / 2) * K.stride + tid] = lo;
     K.v[(long long)(3 * N) * K.stride + tid] = L.invD[row];

@@ -260,38 +260,90 @@ __global__ void k_fac_g(DevParams P, const int* __restrict__ cellIndex, const in
     gmask[k] = (int)mask;
 }
 
-// level-0 row cell g (workgroup = one wavefront): the 3x3 blocks A0(g, c) of its
-// ncs stencil cells.  Lane l works on stencil cell c = l % ncs in partition
-// l / ncs; the 64 / ncs partitions split the row cell's particles (viscous part)
-// and the candidate list (C Lambda C^T part) round robin, and their sums are added
-// in partition order at the end.  The viscous part and the diagonal blocks come
-// from the run sums of the matrix-A pass (blk): a particle's record of each visited
-// cell that falls in stencil cell c.  (Walking the runs entry by entry here took
-// 3.95 ms of 4.7 on the 1M scene: a lane's particles and entries one after another,
-// with the centre cell's runs the longest.)  The candidates are the particles of the
-// cells around g whose G table holds g, filtered 64 at a time into an ordered list in
-// LDS (flushed when full).  The list and the partition sums share one LDS buffer.
-constexpr int kGal0List = 288;
-__global__ void __launch_bounds__(64) k_fac_gal0(DevParams P, Level L, FacOp F, const int* __restrict__ cellStart,
-                                                 const double* __restrict__ blk, const double* __restrict__ gtab,
-                                                 const int* __restrict__ gmask) {
+// level-0 row cell g (workgroup): the 3x3 blocks A0(g, c) of its ncs stencil cells.
+// Thread t works on stencil cell c = t % ncs in partition t / ncs; the partitions split
+// the row cell's particles (viscous part) and the candidate list (C Lambda C^T part)
+// round robin, and their sums are added in partition order at the end.  The viscous part
+// and the diagonal blocks come from the run sums of the matrix-A pass (blk): a particle's
+// record of each visited cell that falls in stencil cell c.  (Walking the runs entry by
+// entry here took 3.95 ms of 4.7 on the 1M scene.)  The candidates are the particles of
+// the cells around g whose G table holds g, compacted in order into a list in LDS
+// (flushed when full).  The list and the partition sums share one LDS buffer.  A walk is
+// a chain of loads, so many short ones: 145 us at 4.9k particles, 168 at 64k and 799 at 1M
+// (22k cells) with one wavefront and two partitions per cell, now 22, 62 and 636.
+// T threads: 64 in 2D (12 rows a cell and few candidates; 160k particles 67 us, 85 with
+// 128), 512 in 3D up to kGal0Cells cells, beyond it 256 (1M: 636 us, 831 with 512): enough
+// workgroups are there to wait for one another.
+constexpr int kGal0Cells = 4096;
+template <int T>
+__global__ void __launch_bounds__(T) k_fac_gal0(DevParams P, Level L, FacOp F, const int* __restrict__ cellStart,
+                                                const double* __restrict__ blk, const double* __restrict__ gtab,
+                                                const int* __restrict__ gmask) {
     typedef double dv2 __attribute__((ext_vector_type(2)));
-    __shared__ double sbuf[64 * 9];   // 4608 B: the list, then the partition sums
-    static_assert(4 * kGal0List * sizeof(int) <= sizeof(sbuf), "list exceeds the shared buffer");
-    int* lk = (int*)sbuf;             // candidate particle
-    int* lc = lk + kGal0List;         // its cell's offset from g, (dx+1) + 3 (dy+1) + 9 (dz+1)
-    int* lm = lc + kGal0List;         // its G mask
-    unsigned* lh = (unsigned*)(lm + kGal0List);  // the stencil cells its G mask reaches (a superset)
+    constexpr int kRanges = 54, kGal0List = 6 * T;  // ranges: fluid, then wall particles of 27 cells
+    __shared__ double sbuf[T * 9];    // the list, then the partition sums
+    static_assert(3 * kGal0List * sizeof(int) <= sizeof(sbuf), "list exceeds the shared buffer");
+    int* const lk = (int*)sbuf;       // candidate particle
+    int* const lc = lk + kGal0List;   // its cell's offset from g, (dx+1) + 3 (dy+1) + 9 (dz+1)
+    int* const lm = lc + kGal0List;   // its G mask
+    __shared__ signed char slots[27][27];  // [stencil cell][offset]: the G slot, -1 none
+    __shared__ int rlo[64], roff[64], rsg[64], hits[T / 64];  // roff: candidates before the range
+    __shared__ unsigned char rcell[64];
     const int ncs = L.cs[0] * L.cs[1] * L.cs[2];
-    const int nparts = 64 / ncs;
-    const int g = blockIdx.x, lane = threadIdx.x;
-    const int c = lane % ncs, part = lane / ncs;
+    const int nparts = T / ncs;
+    const int g = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t / 64;
+    const int c = t % ncs, part = t / ncs;
     const bool active = part < nparts;
     int gx, gy, gz;
     body::grid_xyz(L, g, gx, gy, gz);
     const int ax = gx + L.mn[0], ay = gy + L.mn[1], az = gz + L.mn[2];
     const int ic = body::cell_id(P, ax, ay, az);
     const int p0 = cellStart[ic], p1 = cellStart[ic + 1];
+    const int* C = P.C;
+    const int wx = ((ax % C[0]) + C[0]) % C[0], wy = ((ay % C[1]) + C[1]) % C[1], wz = ((az % C[2]) + C[2]) % C[2];
+    auto wrapc = [](int v, int cnt) { return v < 0 ? v + cnt : (v >= cnt ? v - cnt : v); };
+    auto inside = [&](int o) {  // offset within the neighbour range (2D: no z offsets)
+        const int dx = o % 3 - 1, dy = (o / 3) % 3 - 1, dz = o / 9 - 1;
+        return abs(dx) <= P.range[0] && abs(dy) <= P.range[1] && abs(dz) <= P.range[2];
+    };
+    // slot, in the G table of a particle at offset o, of stencil cell h (level-0 counts of
+    // at least 3 per axis: the caller checks)
+    for (int e = t; e < 27 * ncs; e += T) {
+        const int h = e / 27, o = e % 27;
+        const int iX = h / (L.cs[1] * L.cs[2]), iY = (h / L.cs[2]) % L.cs[1], iZ = h % L.cs[2];
+        const int hx = (((L.mn[0] + (gx + (L.cs[0] == 3 ? iX - 1 : 0) + L.cnt[0]) % L.cnt[0]) % C[0]) + C[0]) % C[0];
+        const int hy = (((L.mn[1] + (gy + (L.cs[1] == 3 ? iY - 1 : 0) + L.cnt[1]) % L.cnt[1]) % C[1]) + C[1]) % C[1];
+        const int hz = (((L.mn[2] + (gz + (L.cs[2] == 3 ? iZ - 1 : 0) + L.cnt[2]) % L.cnt[2]) % C[2]) + C[2]) % C[2];
+        slots[h][o] = !inside(o) ? -1
+                                 : (signed char)fac_slot(P, hx, hy, hz, wrapc(wx + o % 3 - 1, C[0]),
+                                                         wrapc(wy + (o / 3) % 3 - 1, C[1]), wrapc(wz + o / 9 - 1, C[2]));
+    }
+    if (wave == 0) {  // the candidates' ranges, cells by x, y, z offset
+        int cnt = 0, lo = 0, sg = -1, o = 0;
+        if (lane < kRanges) {
+            const int q = lane / 2, half = lane % 2;
+            o = q / 9 + 3 * ((q / 3) % 3) + 9 * (q % 3);
+            if (inside(o)) {
+                const int kx = wrapc(wx + o % 3 - 1, C[0]), ky = wrapc(wy + (o / 3) % 3 - 1, C[1]);
+                const int kz = wrapc(wz + o / 9 - 1, C[2]);
+                sg = fac_slot(P, wx, wy, wz, kx, ky, kz);
+                const int kc = half * P.T + body::cell_id(P, kx, ky, kz);
+                if (sg >= 0) {
+                    lo = cellStart[kc];
+                    cnt = cellStart[kc + 1] - lo;
+                }
+            }
+        }
+        int incl = cnt;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += v;
+        }
+        rlo[lane] = lo;
+        roff[lane] = incl - cnt;  // lanes past the ranges: the total
+        rsg[lane] = sg;
+        rcell[lane] = (unsigned char)o;
+    }
     double acc[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     // viscous part and the diagonal blocks: the run sums of the row cell's particles
     // in the visited cells that fall in stencil cell c, then the particle's diagonal
@@ -315,110 +367,80 @@ __global__ void __launch_bounds__(64) k_fac_gal0(DevParams P, Level L, FacOp F, 
                 acc[8] += v2.y;
             }
             if (dself)
-                for (int e = 0; e < 9; ++e) acc[e] += F.diag[9 * ip + e];
+                for (int e = 0; e < 9; ++e) acc[e] += F.diag[9 * (long long)ip + e];
         }
-    // C Lambda C^T part: lambda_k G_gk G_hk^T; h is stencil cell c (level-0 counts
-    // of at least 3 per axis: the caller checks)
-    const int iX = c / (L.cs[1] * L.cs[2]), iY = (c / L.cs[2]) % L.cs[1], iZ = c % L.cs[2];
-    const int* C = P.C;
-    const int hx = (((L.mn[0] + (gx + (L.cs[0] == 3 ? iX - 1 : 0) + L.cnt[0]) % L.cnt[0]) % C[0]) + C[0]) % C[0];
-    const int hy = (((L.mn[1] + (gy + (L.cs[1] == 3 ? iY - 1 : 0) + L.cnt[1]) % L.cnt[1]) % C[1]) + C[1]) % C[1];
-    const int hz = (((L.mn[2] + (gz + (L.cs[2] == 3 ? iZ - 1 : 0) + L.cnt[2]) % L.cnt[2]) % C[2]) + C[2]) % C[2];
-    const int wx = ((ax % C[0]) + C[0]) % C[0], wy = ((ay % C[1]) + C[1]) % C[1], wz = ((az % C[2]) + C[2]) % C[2];
+    __syncthreads();
+    // C Lambda C^T part: lambda_k G_gk G_hk^T for the listed k; h is stencil cell c
     int n = 0;  // entries in the list (uniform)
-    auto wrapc = [](int v, int cnt) { return v < 0 ? v + cnt : (v >= cnt ? v - cnt : v); };
     auto consume = [&]() {
-        // stencil bits of each entry: for every slot s of k's mask, the stencil
-        // offset of cell(k) + s from g, wrapped as the stencil wraps the level grid
-        // (a superset of the stencil cells whose exact slot test below passes)
-        for (int t = lane; t < n; t += 64) {
-            const int o = lc[t];
-            const int ko[3] = {o % 3 - 1, (o / 3) % 3 - 1, o / 9 - 1};
-            unsigned hb = 0;
-            for (unsigned m = (unsigned)lm[t]; m; m &= m - 1) {
-                const int sl = __builtin_ctz(m);
-                const int so[3] = {sl / 9 - 1, (sl / 3) % 3 - 1, sl % 3 - 1};
-                int idx = 0;
-                bool ok = true;
-                for (int a = 0; a < 3; ++a) {
-                    int v = ko[a] + so[a];
-                    if (L.cs[a] == 3) {
-                        if (v > 1) v -= L.cnt[a];
-                        else if (v < -1) v += L.cnt[a];
-                        ok = ok && v >= -1 && v <= 1;
-                        idx = 3 * idx + v + 1;
-                    } else {
-                        ok = ok && v == 0;
+        if (active)
+            for (int e0 = part; e0 < n; e0 += 2 * nparts) {  // two entries' loads under way
+                bool ok[2];
+                double lv[2], gg[2][3], gh[2][3];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int e = e0 + u * nparts < n ? e0 + u * nparts : e0;
+                    const int o = lc[e], sh = slots[c][o], k = lk[e];
+                    ok[u] = e0 + u * nparts < n && sh >= 0 && ((unsigned)lm[e] >> sh & 1u);
+                    const int sg = rsg[2 * (9 * (o % 3) + 3 * ((o / 3) % 3) + o / 9)];
+                    const double* G = gtab + 81 * (long long)k;
+                    lv[u] = F.lambda[k];
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        gg[u][d] = G[3 * sg + d];
+                        gh[u][d] = G[(ok[u] ? 3 * sh : 3 * sg) + d];
                     }
                 }
-                if (ok) hb |= 1u << idx;
-            }
-            lh[t] = hb;
-        }
-        __syncthreads();
-        if (active)
-            for (int t = part; t < n; t += nparts) {
-                if (!((lh[t] >> c) & 1u)) continue;
-                const int o = lc[t];
-                const int kx = wrapc(wx + o % 3 - 1, C[0]);
-                const int ky = wrapc(wy + (o / 3) % 3 - 1, C[1]);
-                const int kz = wrapc(wz + o / 9 - 1, C[2]);
-                const int sh = fac_slot(P, hx, hy, hz, kx, ky, kz);
-                if (sh < 0 || !(((unsigned)lm[t] >> sh) & 1u)) continue;
-                const int sg = fac_slot(P, wx, wy, wz, kx, ky, kz);
-                const int k = lk[t];
-                const double* G = gtab + 81 * (long long)k;
-                const double lv = F.lambda[k];
-                const double gg0 = G[3 * sg], gg1 = G[3 * sg + 1], gg2 = G[3 * sg + 2];
-                const double gh0 = G[3 * sh], gh1 = G[3 * sh + 1], gh2 = G[3 * sh + 2];
-                const double lg[3] = {lv * gg0, lv * gg1, lv * gg2};
-                for (int rr = 0; rr < 3; ++rr) {
-                    acc[3 * rr] += lg[rr] * gh0;
-                    acc[3 * rr + 1] += lg[rr] * gh1;
-                    acc[3 * rr + 2] += lg[rr] * gh2;
-                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    if (ok[u]) {
+                        const double lg[3] = {lv[u] * gg[u][0], lv[u] * gg[u][1], lv[u] * gg[u][2]};
+                        for (int rr = 0; rr < 3; ++rr) {
+                            acc[3 * rr] += lg[rr] * gh[u][0];
+                            acc[3 * rr + 1] += lg[rr] * gh[u][1];
+                            acc[3 * rr + 2] += lg[rr] * gh[u][2];
+                        }
+                    }
             }
         __syncthreads();
         n = 0;
     };
-    for (int dx = -P.range[0]; dx <= P.range[0]; ++dx)
-        for (int dy = -P.range[1]; dy <= P.range[1]; ++dy)
-            for (int dz = -P.range[2]; dz <= P.range[2]; ++dz) {
-                const int kx = ((ax + dx) % C[0] + C[0]) % C[0];
-                const int ky = ((ay + dy) % C[1] + C[1]) % C[1];
-                const int kz = ((az + dz) % C[2] + C[2]) % C[2];
-                const int sg = fac_slot(P, wx, wy, wz, kx, ky, kz);
-                if (sg < 0) continue;
-                const int kc = body::cell_id(P, kx, ky, kz);
-                for (int half = 0; half < 2; ++half) {  // fluid, then wall particles of the cell
-                    const int q0 = cellStart[half * P.T + kc], q1 = cellStart[half * P.T + kc + 1];
-                    for (int base = q0; base < q1; base += 64) {
-                        const int k = base + lane;
-                        const unsigned km = k < q1 ? (unsigned)gmask[k] : 0u;
-                        const bool hit = (km >> sg) & 1u;
-                        const unsigned long long bal = __ballot(hit);
-                        const int before = __popcll(bal & ((1ull << lane) - 1ull));
-                        const int cnt = __popcll(bal);
-                        if (n + cnt > kGal0List) consume();
-                        if (hit) {
-                            lk[n + before] = k;
-                            lc[n + before] = (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1);
-                            lm[n + before] = (int)km;
-                        }
-                        n += cnt;
-                        __syncthreads();
-                    }
-                }
-            }
+    const int total = roff[63];
+    for (int base = 0; base < total; base += T) {
+        const int idx = base + t;
+        int q = 0;  // the last range starting at or before the candidate
+#pragma unroll
+        for (int step = 32; step >= 1; step >>= 1)
+            if (q + step < kRanges && roff[q + step] <= idx) q += step;
+        const int k = rlo[q] + idx - roff[q];
+        const unsigned km = idx < total ? (unsigned)gmask[k] : 0u;
+        const bool hit = idx < total && (km >> rsg[q] & 1u);
+        const unsigned long long bal = __ballot(hit);
+        if (lane == 0) hits[wave] = __popcll(bal);
+        __syncthreads();
+        int before = __popcll(bal & ((1ull << lane) - 1ull)), cnt = 0;
+        for (int w = 0; w < T / 64; ++w) {
+            before += w < wave ? hits[w] : 0;
+            cnt += hits[w];
+        }
+        if (n + cnt > kGal0List) consume();
+        if (hit) {
+            lk[n + before] = k;
+            lc[n + before] = rcell[q];
+            lm[n + before] = (int)km;
+        }
+        n += cnt;
+        __syncthreads();
+    }
     consume();  // ends with a barrier: the list is dead, sbuf takes the partition sums
     if (active)
-        for (int e = 0; e < 9; ++e) sbuf[9 * lane + e] = acc[e];
+        for (int e = 0; e < 9; ++e) sbuf[9 * t + e] = acc[e];
     __syncthreads();
-    if (part == 0) {
-        for (int q = 1; q < nparts; ++q)
-            for (int e = 0; e < 9; ++e) acc[e] += sbuf[9 * (q * ncs + c) + e];
-        for (int rr = 0; rr < 3; ++rr)
-            for (int ss = 0; ss < 3; ++ss) L.A[(long long)(3 * c + ss) * L.nrow + 3 * g + rr] = acc[3 * rr + ss];
+    for (int h9 = t; h9 < 9 * ncs; h9 += T) {  // (stencil cell, entry)
+        double v = sbuf[h9];
+        for (int q = 1; q < nparts; ++q) v += sbuf[9 * ncs * q + h9];
+        const int h = h9 / 9, e = h9 % 9;
+        L.A[(long long)(3 * h + e % 3) * L.nrow + 3 * g + e / 3] = v;
     }
 }
 
@@ -902,8 +924,13 @@ void launch_fac_level0(hipStream_t st, const DevParams& P, const Level& L0, cons
     hipLaunchKernelGGL(k_fac_g, dim3(nblk(P.np, 128)), dim3(128), 0, st, P, cellIndex, F.runP, F.nPtrP, F.nIndP,
                        F.beta, F.pos, F.selfC, gtab, gmask);
     hipLaunchKernelGGL(k_fac_invdiag, dim3(nblk(8LL * P.nf, 256)), dim3(256), 0, st, P, F, invDiagA);
-    if (L0.cells > 0)
-        hipLaunchKernelGGL(k_fac_gal0, dim3(L0.cells), dim3(64), 0, st, P, L0, F, cellStart, blk, gtab, gmask);
+    if (L0.cells <= 0) return;
+#define MPH_GAL0(T) \
+    hipLaunchKernelGGL(k_fac_gal0<T>, dim3(L0.cells), dim3(T), 0, st, P, L0, F, cellStart, blk, gtab, gmask)
+    if (P.dim == 2) MPH_GAL0(64);
+    else if (L0.cells < kGal0Cells) MPH_GAL0(512);
+    else MPH_GAL0(256);
+#undef MPH_GAL0
 }
 
 void launch_fac_u(hipStream_t st, const DevParams& P, const int* nFluid, const long long* nPtr, const int* nInd,

@@ -100,7 +100,10 @@ __global__ void __launch_bounds__(256) k_mg_galerkin0(DevParams P, Level L, cons
 // loading the group's rows together (one coalesced 64-byte piece per entry pair)
 // fetches each line at most twice, where walking one particle at a time across
 // thousands of resident workgroups re-fetched it up to eight times.  Every (c, e)
-// thread then adds its runs particle by particle from LDS, in the same order.
+// thread then adds its runs particle by particle from LDS, in the same order, eight reads
+// in flight.  The next group's rows and run starts load while a group is added: 0.39 ms at
+// 64k particles and 0.98 at 198k, 0.68 and 1.80 when the run starts were read from global
+// memory one by one and every group was waited for.
 // Rows longer than kGalRow blocks are not supported (the caller checks).
 constexpr int kGalGroup = 4, kGalRow = 216;
 __global__ void __launch_bounds__(256) k_mg_galerkin0_lds(DevParams P, Level L, const int* __restrict__ cellStart,
@@ -109,41 +112,70 @@ __global__ void __launch_bounds__(256) k_mg_galerkin0_lds(DevParams P, Level L, 
                                                           const long long* __restrict__ start,
                                                           const double* __restrict__ aval) {
     typedef double d2 __attribute__((ext_vector_type(2)));
+    constexpr int kTask = (kGalRow / 2 * 9 * kGalGroup + 255) / 256;  // block pairs' entries per thread
     __shared__ double row[kGalGroup * kGalRow * 9];
+    __shared__ unsigned short rs[kGalGroup * kRuns];
     const int ncs = L.cs[0] * L.cs[1] * L.cs[2];
-    const int g = blockIdx.x;
-    const bool active = (int)threadIdx.x < 9 * ncs;
-    const int c = threadIdx.x / 9, e = threadIdx.x % 9;
+    const int g = blockIdx.x, t = threadIdx.x;
+    const bool active = t < 9 * ncs;
+    const int c = t / 9, e = t % 9;
     int gx, gy, gz;
     grid_xyz(L, g, gx, gy, gz);
     const int ic = cell_id(P, gx + L.mn[0], gy + L.mn[1], gz + L.mn[2]);
     const int p0 = cellStart[ic], p1 = cellStart[ic + 1];
     const unsigned mask = active ? galerkin_mask(P, L, cellStart, g, c) : 0u;
     double acc = 0.0;
-    for (int ip0 = p0; ip0 < p1;) {
+    // the group from particle ip: its rows' pairs and run starts, all loads in flight
+    // (past the rows' ends the last pair again, not stored)
+    d2 v[kTask];
+    unsigned short r1 = 0;
+    int n1 = 0;  // tasks of the group: pairs * 9 * particles
+    auto load = [&](int ip) {
         // groups aligned to kGalGroup particles never straddle a 64-particle slice
-        const int gend = min(p1, (ip0 / kGalGroup + 1) * kGalGroup);
-        const int G = gend - ip0;
-        const long long sb = start[ip0 / kSlice];
-        const int lane0 = ip0 % kSlice;
+        const int gend = min(p1, (ip / kGalGroup + 1) * kGalGroup), G = gend - ip;
+        const long long sb = start[ip / kSlice];
+        const int lane0 = ip % kSlice;
         int npair = 0;
-        for (int p = 0; p < G; ++p) npair = max(npair, (nFluid[ip0 + p] + 1) / 2);
+        for (int p = 0; p < G; ++p) npair = max(npair, (nFluid[ip + p] + 1) / 2);
+        n1 = npair * 9 * kGalGroup;
+        r1 = runStart[(long long)ip * kRuns + (t < G * kRuns ? t : 0)];
+        if (n1 == 0) return;  // empty rows
+#pragma unroll
+        for (int k = 0; k < kTask; ++k) {
+            const int task = t + 256 * k < n1 ? t + 256 * k : n1 - 1;
+            const int p = min(task % kGalGroup, G - 1), ee = (task / kGalGroup) % 9, m = task / (kGalGroup * 9);
+            v[k] = *(const d2*)&aval[a_val_index(sb, 2 * m, ee, lane0 + p)];
+        }
+    };
+    if (p0 < p1) load(p0);
+    for (int ip0 = p0; ip0 < p1;) {
+        const int gend = min(p1, (ip0 / kGalGroup + 1) * kGalGroup), G = gend - ip0;
         __syncthreads();  // the previous group has been used
-        for (int t = threadIdx.x; t < npair * 9 * G; t += blockDim.x) {
-            const int p = t % G, ee = (t / G) % 9, m = t / (G * 9);
-            const d2 v = *(const d2*)&aval[a_val_index(sb, 2 * m, ee, lane0 + p)];
-            row[(p * kGalRow + 2 * m) * 9 + ee] = v.x;
-            row[(p * kGalRow + 2 * m + 1) * 9 + ee] = v.y;
+        if (t < kGalGroup * kRuns) rs[t] = r1;
+#pragma unroll
+        for (int k = 0; k < kTask; ++k) {
+            const int task = t + 256 * k;
+            if (task >= n1) break;
+            const int p = task % kGalGroup, ee = (task / kGalGroup) % 9, m = task / (kGalGroup * 9);
+            row[(p * kGalRow + 2 * m) * 9 + ee] = v[k].x;
+            row[(p * kGalRow + 2 * m + 1) * 9 + ee] = v[k].y;
         }
         __syncthreads();
+        if (gend < p1) load(gend);  // on its way while this group is added
         if (mask)
             for (int p = 0; p < G; ++p) {
-                const unsigned short* rs = runStart + (long long)(ip0 + p) * kRuns;
                 const double* rp = row + p * kGalRow * 9 + e;
                 for (unsigned m = mask; m; m &= m - 1) {
                     const int q = __builtin_ctz(m);
-                    const int k1 = rs[q + 1];
-                    for (int k = rs[q]; k < k1; ++k) acc += rp[k * 9];
+                    const int k1 = rs[p * kRuns + q + 1];
+                    for (int k = rs[p * kRuns + q]; k < k1; k += 8) {  // eight reads in flight, added in order
+                        double w[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) w[u] = rp[min(k + u, kGalRow - 1) * 9];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            if (k + u < k1) acc += w[u];
+                    }
                 }
             }
         ip0 = gend;
@@ -154,49 +186,77 @@ __global__ void __launch_bounds__(256) k_mg_galerkin0_lds(DevParams P, Level L, 
     }
 }
 
-// coarse level = R A_fine P by summation (3414-3507): thread = (coarse cell, stencil
-// cell); children in R order, then fine stencil entries in shift order.
-__global__ void k_mg_galerkinL(Level S, Level L) {
-    const int ncs = L.cs[0] * L.cs[1] * L.cs[2];
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)L.cells * ncs) return;
-    const int g = (int)(t / ncs), c = (int)(t % ncs);
-    int lx, ly, lz;
-    grid_xyz(L, g, lx, ly, lz);
-    const int lcx = lx + L.mn[0], lcy = ly + L.mn[1], lcz = lz + L.mn[2];
-    const int fmx = S.mn[0] > 2 * lcx, fmy = S.mn[1] > 2 * lcy, fmz = S.mn[2] > 2 * lcz;
-    const int fMx = S.mx[0] < 2 * (lcx + 1), fMy = S.mx[1] < 2 * (lcy + 1), fMz = S.mx[2] < 2 * (lcz + 1);
-    double acc[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int ax = 0; ax < 2 - fmx - fMx; ++ax)
-        for (int ay = 0; ay < 2 - fmy - fMy; ++ay)
-            for (int az = 0; az < 2 - fmz - fMz; ++az) {
-                const int sgx = (2 * lcx + ax + fmx) - S.mn[0];
-                const int sgy = (2 * lcy + ay + fmy) - S.mn[1];
-                const int sgz = (2 * lcz + az + fmz) - S.mn[2];
-                const int srow0 = 3 * grid_id(S, sgx, sgy, sgz);
-                // the wraps take arguments in [0, 3 cnt): sg + e - 1 + cnt with sg < cnt,
-                // e < 3; jl - l + 1 + cnt with jl, l < cnt (wrap3, no division)
-                for (int ex = 0; ex < S.cs[0]; ++ex)
-                    for (int ey = 0; ey < S.cs[1]; ++ey)
-                        for (int ez = 0; ez < S.cs[2]; ++ez) {
-                            const int jsx = wrap3(sgx + ex - 1 + S.cnt[0], S.cnt[0]);
-                            const int jsy = wrap3(sgy + ey - 1 + S.cnt[1], S.cnt[1]);
-                            const int jsz = wrap3(sgz + ez - 1 + S.cnt[2], S.cnt[2]);
-                            const int jlx = ((jsx + S.mn[0]) / 2) - L.mn[0];
-                            const int jly = ((jsy + S.mn[1]) / 2) - L.mn[1];
-                            const int jlz = ((jsz + S.mn[2]) / 2) - L.mn[2];
-                            const int ix = wrap3((jlx - lx) + 1 + L.cnt[0], L.cnt[0]);
-                            const int iy = wrap3((jly - ly) + 1 + L.cnt[1], L.cnt[1]);
-                            const int iz = wrap3((jlz - lz) + 1 + L.cnt[2], L.cnt[2]);
-                            if (L.cs[2] * L.cs[1] * ix + L.cs[2] * iy + iz != c) continue;
-                            const int cS = S.cs[2] * S.cs[1] * ex + S.cs[2] * ey + ez;
-                            for (int r = 0; r < 3; ++r)
-                                for (int sd = 0; sd < 3; ++sd)
-                                    acc[3 * r + sd] += S.A[(long long)(3 * cS + sd) * S.nrow + srow0 + r];
-                        }
+// coarse level = R A_fine P by summation (3414-3507): workgroup = coarse cell, its
+// children's rows (8 x 27 blocks) staged in LDS in one round of loads; thread = (stencil
+// cell, block entry); children in R order, then fine stencil entries in shift order.
+// (A thread per stencil cell that tested every entry and loaded the matching blocks one
+// after the other took 118 us per level at 64k particles, 20 in 2D; now 10 and 7.)
+__global__ void __launch_bounds__(256) k_mg_galerkinL(Level S, Level L) {
+    __shared__ double sA[8 * 27 * 9];
+    const int g = blockIdx.x, t = threadIdx.x;
+    const int ncs = L.cs[0] * L.cs[1] * L.cs[2], scs = S.cs[0] * S.cs[1] * S.cs[2];
+    int l[3];
+    grid_xyz(L, g, l[0], l[1], l[2]);
+    int f0[3], fn[3];  // first child and children per axis
+    for (int d = 0; d < 3; ++d) {
+        const int lc = l[d] + L.mn[d];
+        const int lo = S.mn[d] > 2 * lc, hi = S.mx[d] < 2 * (lc + 1);
+        f0[d] = (2 * lc + lo) - S.mn[d];
+        fn[d] = 2 - lo - hi;
+    }
+    const int nch = fn[0] * fn[1] * fn[2];
+    {
+        constexpr int K = (8 * 27 * 9 + 255) / 256;
+        double v[K];
+        const int n = nch * scs * 9;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {  // entry (shift 3 cS + sd, child, r): r, then the child fastest
+            const int e = t + 256 * k < n ? t + 256 * k : n - 1;
+            const int r = e % 3, ch = (e / 3) % nch, sh = e / (3 * nch);
+            const int az = ch % fn[2], ay = (ch / fn[2]) % fn[1], ax = ch / (fn[2] * fn[1]);
+            v[k] = S.A[(long long)sh * S.nrow + 3 * grid_id(S, f0[0] + ax, f0[1] + ay, f0[2] + az) + r];
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int e = t + 256 * k;
+            if (e >= n) break;
+            const int r = e % 3, ch = (e / 3) % nch, sh = e / (3 * nch);
+            sA[(ch * 27 + sh / 3) * 9 + 3 * r + sh % 3] = v[k];
+        }
+    }
+    __syncthreads();
+    if (t >= 9 * ncs) return;
+    const int c = t / 9, e9 = t % 9;
+    const int ci[3] = {c / (L.cs[1] * L.cs[2]), (c / L.cs[2]) % L.cs[1], c % L.cs[2]};
+    // fine stencil offsets of child a along axis d that fall in stencil cell c: bits of m[d][a].
+    // The wraps take arguments in [0, 3 cnt): sg + e - 1 + cnt with sg < cnt, e < 3;
+    // jl - l + 1 + cnt with jl, l < cnt (wrap3, no division)
+    unsigned m[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+            for (int x = 0; x < S.cs[d]; ++x) {
+                const int js = wrap3(f0[d] + a + x - 1 + S.cnt[d], S.cnt[d]);
+                const int jl = ((js + S.mn[d]) / 2) - L.mn[d];
+                if (a < fn[d] && wrap3((jl - l[d]) + 1 + L.cnt[d], L.cnt[d]) == ci[d]) m[d][a] |= 1u << x;
             }
-    for (int r = 0; r < 3; ++r)
-        for (int sd = 0; sd < 3; ++sd) L.A[(long long)(3 * c + sd) * L.nrow + 3 * g + r] = acc[3 * r + sd];
+    double acc = 0.0;
+    for (int ax = 0; ax < fn[0]; ++ax)
+        for (int ay = 0; ay < fn[1]; ++ay)
+            for (int az = 0; az < fn[2]; ++az) {
+                const double* ch = sA + ((ax * fn[1] + ay) * fn[2] + az) * 243 + e9;
+                const unsigned my = ay ? m[1][1] : m[1][0], mz = az ? m[2][1] : m[2][0];
+                for (unsigned bx = ax ? m[0][1] : m[0][0]; bx; bx &= bx - 1)
+                    for (unsigned by = my; by; by &= by - 1) {
+                        const double* r = ch + (S.cs[1] * __builtin_ctz(bx) + __builtin_ctz(by)) * S.cs[2] * 9;
+                        double w[3];
+                        for (int z = 0; z < 3; ++z) w[z] = r[9 * z];  // past a narrow stencil: not taken
+                        for (int z = 0; z < 3; ++z)
+                            if (mz >> z & 1) acc += w[z];
+                    }
+            }
+    L.A[(long long)(3 * c + e9 % 3) * L.nrow + 3 * g + e9 / 3] = acc;
 }
 
 // invD = 2 / sum |a| per row (calculateMultiGridInvDiagA, 3510-3546)
@@ -204,7 +264,15 @@ __global__ void k_mg_invd(Level L) {
     const int row = blockIdx.x * blockDim.x + threadIdx.x;
     if (row >= L.nrow) return;
     double sum = 0.0;
-    for (int sh = 0; sh < L.nshift; ++sh) sum += fabs(L.A[(long long)sh * L.nrow + row]);
+    int sh = 0;
+    for (; sh + 27 <= L.nshift; sh += 27) {  // 27 loads in flight, added in order
+        double v[27];
+#pragma unroll
+        for (int u = 0; u < 27; ++u) v[u] = L.A[(long long)(sh + u) * L.nrow + row];
+#pragma unroll
+        for (int u = 0; u < 27; ++u) sum += fabs(v[u]);
+    }
+    for (; sh < L.nshift; ++sh) sum += fabs(L.A[(long long)sh * L.nrow + row]);  // narrow levels
     L.invD[row] = sum != 0.0 ? 2.0 / sum : 0.0;
 }
 
@@ -314,7 +382,7 @@ __global__ void __launch_bounds__(T) k_mg_coarse(CoarsePack K, int lc, int D, co
     mg_coarse_cycle<N, T, XB, kOrd>(K, lc, D, in, io, nio, halt, sh);
 }
 
-__global__ void k_mg_coarse_pack(const Level* __restrict__ lvs, int lc, int D, int f32, CoarsePack K) {
+__global__ void __launch_bounds__(64) k_mg_coarse_pack(const Level* __restrict__ lvs, int lc, int D, int f32, CoarsePack K) {
     coarse_pack(lvs, lc, D, f32 != 0, K);
 }
 
@@ -638,8 +706,7 @@ void launch_mg_galerkin0(hipStream_t st, const DevParams& P, const Level& L, con
                            runStart, A.start, A.val);
 }
 void launch_mg_galerkinL(hipStream_t st, const Level& S, const Level& L) {
-    const long long n = (long long)L.cells * L.cs[0] * L.cs[1] * L.cs[2];
-    hipLaunchKernelGGL(k_mg_galerkinL, dim3(nblk(n, 128)), dim3(128), 0, st, S, L);
+    hipLaunchKernelGGL(k_mg_galerkinL, dim3(L.cells), dim3(256), 0, st, S, L);
 }
 void launch_mg_invd(hipStream_t st, const Level& L) {
     hipLaunchKernelGGL(k_mg_invd, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
