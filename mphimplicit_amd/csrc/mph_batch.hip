@@ -153,11 +153,15 @@ __global__ void __launch_bounds__(256) kb_xrs_update(const BScene* tab, const in
                                                      SceneSet pq, int x) {
     __shared__ double sh[256];
     MPH_SCENE(kOffChunk)
+    auto coef = [&](double& alpha, double& beta) {
+        alpha = B.scal[kRHO] / B.scal[kTMP];
+        beta = in_set(pq, s) ? B.scal[kRHO] / B.scal[kRHOP] : 0.0;
+    };
     if (in_set(pq, s))
-        xrs_update_chunk<true>(B.P.nf, B.scal, B.vec[kP], B.vec[kQ], B.vec[kU], B.vec[x], B.vec[kR], B.vec[kS],
+        xrs_update_chunk<true>(B.P.nf, coef, B.vec[kP], B.vec[kQ], B.vec[kU], B.vec[x], B.vec[kR], B.vec[kS],
                                B.part, lb, sh);
     else
-        xrs_update_chunk<false>(B.P.nf, B.scal, B.vec[kP], B.vec[kQ], B.vec[kU], B.vec[x], B.vec[kR], B.vec[kS], B.part, lb,
+        xrs_update_chunk<false>(B.P.nf, coef, B.vec[kP], B.vec[kQ], B.vec[kU], B.vec[x], B.vec[kR], B.vec[kS], B.part, lb,
                      sh);
 }
 
@@ -181,7 +185,8 @@ __global__ void __launch_bounds__(256) kb_mg_p2g_bu(const BScene* tab, const int
     MPH_SCENE(kOffP2g)
     const Level L = level(B, 0, cur, s);
     const bool f = in_set(pq, s);
-#define MPH_P2G(PQ, ORD) mg_p2g_lanes<PQ, ORD>(B.P, L, B.cellStart, B.vec[in], B.vec[kY], B.scal, lb, tb)
+    auto beta = [&] { return B.scal[kRHO] / B.scal[kRHOP]; };
+#define MPH_P2G(PQ, ORD) mg_p2g_lanes<PQ, ORD>(B.P, L, B.cellStart, B.vec[in], B.vec[kY], beta, lb, tb)
     if (L.ordered) {
         if (f) MPH_P2G(true, true);
         else MPH_P2G(false, true);

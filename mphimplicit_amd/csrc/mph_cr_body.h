@@ -16,7 +16,8 @@ namespace body {
 __host__ __device__ inline int nblk(long long n, int bs) { return (int)((n + bs - 1) / bs); }
 
 // CR scalars: rr0, rs0, rr, rho, rho_prev, tmp (= q.u), rs
-enum { kRR0 = 0, kRS0 = 1, kRR = 2, kRHO = 3, kRHOP = 4, kTMP = 5, kRS = 6, kRSIter = 7, kNScal = 8 };
+enum { kRR0 = 0, kRS0 = 1, kRR = 2, kRHO = 3, kRHOP = 4, kTMP = 5, kRS = 6, kRSIter = 7, kNScal = 8,
+       kRHON = 10 };
 
 __device__ inline int cell_id(const DevParams& P, int cx, int cy, int cz) {
     const int* C = P.C;
@@ -1387,12 +1388,9 @@ __device__ inline void dot_partial_chunk(int nf, const double* __restrict__ x, c
     if (threadIdx.x == 0) part[chunk] = v;
 }
 
-// fold the chunk partials: lane l sums chunks l, l+256, ... from 0.0, then the tree.
-// scal[shift_slot] receives the previous scal[slot] first (rho -> rho_prev).
-__device__ inline void dot_final_body(const double* __restrict__ part, int nchunks, double* scal, int slot,
-                                      int shift_slot, double* sh, double* host = nullptr) {
-    // lane l adds chunks l, l + 256, ... in that order; eight loads are issued
-    // before their adds so the lane does not wait on each in turn
+// lane l's sum of the chunk partials l, l + 256, ... from 0.0 in that order; eight loads
+// are issued before their adds so the lane does not wait on each in turn
+__device__ inline double dot_lane_sum(const double* __restrict__ part, int nchunks) {
     double acc = 0.0;
     for (int c0 = threadIdx.x; c0 < nchunks; c0 += 256 * 8) {
         double v[8];
@@ -1402,12 +1400,35 @@ __device__ inline void dot_final_body(const double* __restrict__ part, int nchun
         for (int u = 0; u < 8; ++u)
             if (c0 + 256 * u < nchunks) acc = acc + v[u];
     }
-    const double v = block_tree_sum(acc, sh);
+    return acc;
+}
+
+// fold the chunk partials: the lanes' sums, then the tree.
+// scal[shift_slot] receives the previous scal[slot] first (rho -> rho_prev).
+__device__ inline void dot_final_body(const double* __restrict__ part, int nchunks, double* scal, int slot,
+                                      int shift_slot, double* sh, double* host = nullptr) {
+    const double v = block_tree_sum(dot_lane_sum(part, nchunks), sh);
     if (threadIdx.x == 0) {
         if (shift_slot >= 0) scal[shift_slot] = scal[slot];
         scal[slot] = v;
         if (host) *host = v;  // coherent pinned host memory: the CR stop test reads it
     }
+}
+
+// The same dot product in every thread of a workgroup that needs it (sh: 257 doubles), so
+// that a later iteration of a scene of up to kFoldChunks chunks launches no reduction of
+// rho and tmp: the P2G folds rho's partials and keeps it in scal[kRHON] beside the previous
+// rho in scal[kRHO], the x update folds tmp's, and the reduction of rr, which comes after
+// both, moves scal[kRHON] to scal[kRHO].
+__device__ inline double dot_fold(const double* __restrict__ part, int nchunks, double* sh) {
+    const double v = block_tree_sum(dot_lane_sum(part, nchunks), sh);
+    if (threadIdx.x == 0) sh[256] = v;
+    __syncthreads();
+    return sh[256];
+}
+__device__ inline void dot_shift_rho(double* scal) {
+    scal[kRHOP] = scal[kRHO];
+    scal[kRHO] = scal[kRHON];
 }
 
 // p = beta*p + 1.0*s, q = beta*q + 1.0*y with beta = rho/rho_prev (4360-4364)
@@ -1430,11 +1451,10 @@ __device__ inline double pq_elem(double beta, double v, double w) {
 // Unordered, with the update, 19.0 us on the 1M scene (72 MB, 3.8 TB/s) and 5.6 us on
 // the 64k drop; ordered 25.2 and 9.8 us, bound by the first lane's chain of adds.
 constexpr int kP2gLanes = 8, kP2gK = 8;
-template <bool kPq, bool kOrd>
+// coef(): beta, called by every thread of the workgroup (kPq only)
+template <bool kPq, bool kOrd, class F>
 __device__ inline void mg_p2g_lanes(const DevParams& P, const Level& L, const int* __restrict__ cellStart, double* q,
-                                    const double* __restrict__ yv, const double* __restrict__ scal, int block,
-                                    double* tb) {
-    const double beta = kPq ? scal[kRHO] / scal[kRHOP] : 0.0;
+                                    const double* __restrict__ yv, F coef, int block, double* tb) {
     const int u = threadIdx.x & (kP2gLanes - 1);
     const int row = (int)(((long long)block * 256 + threadIdx.x) / kP2gLanes);
     const bool on = row < L.nrow;
@@ -1447,6 +1467,7 @@ __device__ inline void mg_p2g_lanes(const DevParams& P, const Level& L, const in
         p0 = cellStart[ic];
         p1 = cellStart[ic + 1];
     }
+    const double beta = kPq ? coef() : 0.0;
     double sum = 0.0;
     for (int base = p0; base < p1; base += kP2gLanes * kP2gK) {  // the same trips in every lane of the row
         double t[kP2gK], yt[kP2gK];
@@ -1496,29 +1517,39 @@ __device__ inline void pq_update_elem(const double* __restrict__ scal, const dou
 // alpha = rho/tmp; x += alpha p; r -= alpha q; s -= alpha u (4372-4375) + r.r partial.
 // kPq: p = beta p + s first (with s before its update), written back; the CR loop's
 // p update is then this kernel's, not a launch of its own
-template <bool kPq = false>
-__device__ inline void xrs_update_chunk(int nf, const double* __restrict__ scal, double* __restrict__ p,
+// coef(alpha, beta): called by every thread of the workgroup, the vectors' loads under way
+template <bool kPq, class F>
+__device__ inline void xrs_update_chunk(int nf, F coef, double* __restrict__ p,
                                         const double* __restrict__ q, const double* __restrict__ u,
                                         double* __restrict__ x, double* __restrict__ r, double* __restrict__ s,
                                         double* __restrict__ part, int chunk, double* sh) {
     const int i = chunk * 256 + threadIdx.x;
     double t = 0.0;
+    double pv[3], qv[3], uv[3], xv[3], rv[3], sv[3], alpha, beta;
+    if (i < nf)
+        for (int d = 0; d < 3; ++d) {
+            const int k = 3 * i + d;
+            pv[d] = p[k];
+            sv[d] = s[k];
+            xv[d] = x[k];
+            rv[d] = r[k];
+            qv[d] = q[k];
+            uv[d] = u[k];
+        }
+    coef(alpha, beta);
     if (i < nf) {
-        const double alpha = scal[kRHO] / scal[kTMP];
         const double ma = -alpha;
-        const double beta = kPq ? scal[kRHO] / scal[kRHOP] : 0.0;
         double rr[3];
         for (int d = 0; d < 3; ++d) {
             const int k = 3 * i + d;
-            double pk = p[k];
             if (kPq) {
-                pk = pq_elem(beta, pk, s[k]);
-                p[k] = pk;
+                pv[d] = pq_elem(beta, pv[d], sv[d]);
+                p[k] = pv[d];
             }
-            x[k] += alpha * pk;
-            rr[d] = r[k] + ma * q[k];
+            x[k] = xv[d] + alpha * pv[d];
+            rr[d] = rv[d] + ma * qv[d];
             r[k] = rr[d];
-            s[k] += ma * u[k];
+            s[k] = sv[d] + ma * uv[d];
         }
         t = (rr[0] * rr[0] + rr[1] * rr[1]) + rr[2] * rr[2];
     }

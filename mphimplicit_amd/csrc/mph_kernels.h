@@ -167,6 +167,8 @@ __host__ __device__ inline long long a_val_index(long long sb, int k, int e, int
 __host__ __device__ inline long long a_val32_index(long long sb, int k, int e, int lane) {
     return (((sb / 4 + k / 4) * 9 + e) * 64 + lane) * 4 + (k & 3);
 }
+// scenes of up to this many chunks fold rho and tmp where they are read (body::dot_fold)
+constexpr int kFoldChunks = 1024;
 constexpr int kChunk = 256;   // particles per dot-product chunk / CR workgroup
 constexpr int kRuns = 28;     // run starts per fluid particle: 27 neighbour cells + end
 // the factored form's level-0 run sums: per fluid particle and visited cell, the sums
@@ -249,7 +251,7 @@ void launch_fill_i32(hipStream_t st, int* x, long long n, int v);  // a kernel, 
 void launch_mg_p2g_bu(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, const double* q);
 // the same after q = beta q + y (beta = rho / rho_prev from scal), written back to q
 void launch_mg_p2g_bu_pq(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, double* q,
-                         const double* y, const double* scal);
+                         const double* y, double* scal, const double* rho);  // rho: its partials, folded here, or null
 void launch_mg_restrict_bu(hipStream_t st, const Level& S, Level& L);  // restriction, begin, update
 void launch_mg_begin(hipStream_t st, Level& L);        // S *= 0; R = Q
 void launch_mg_update(hipStream_t st, Level& L);       // S += invD R
@@ -311,7 +313,7 @@ void launch_axpy(hipStream_t st, long long n, const double* x, double* y);  // y
 void launch_dot_partial(hipStream_t st, const DevParams& P, const double* x, const double* y, double* part);
 // host: optional coherent pinned host memory that also receives the value
 void launch_dot_final(hipStream_t st, const DevParams& P, const double* part, double* scal, int slot, int shift_slot,
-                      double* host = nullptr);
+                      double* host = nullptr, bool shiftRho = false);
 // The CR loop's control block int[kNCtl] in device memory: the stop flag the
 // iteration kernels test (DevParams::halt points at ctl[kCtlHalt]), the iterations
 // done and a non-finite flag.
@@ -323,7 +325,7 @@ enum { kCtlHalt = 0, kCtlIter = 1, kCtlBad = 2, kNCtl = 4 };
 // no-op once halted.  hctl and hrr: optional coherent pinned host memory that also
 // receives ctl[0..2] and rr.
 void launch_dot_final_stop(hipStream_t st, const DevParams& P, const double* part, double* scal, int* ctl, int step,
-                           double tol, long long maxit, int* hctl, double* hrr);
+                           double tol, long long maxit, int* hctl, double* hrr, bool shiftRho);
 // The convergence record of a CR iteration (main.cpp:4348-4351): the partials' sum
 // r.s into scal[kRSIter], then rec[2 it] = rr (scal[kRR]) and rec[2 it + 1] = r.s
 // for it = ctl[kCtlIter] (ctl null: the host's `it`), rows it >= cap skipped.  A
@@ -334,7 +336,8 @@ void launch_pq_update(hipStream_t st, const DevParams& P, const double* scal, co
                       double* p, double* q);
 // pq: p = beta p + s first, written back
 void launch_xrs_update(hipStream_t st, const DevParams& P, const double* scal, double* p, const double* q,
-                       const double* u, double* x, double* r, double* s, double* part, bool pq = false);
+                       const double* u, double* x, double* r, double* s, double* part, bool pq = false,
+                       const double* tmp = nullptr);  // tmp: its partials, folded here (pq only)
 void launch_store_velocity(hipStream_t st, const DevParams& P, const double* x, double* vel);
 // ---- output-step diagnostics ----
 void launch_diagnostics(hipStream_t st, const DevParams& P, const int* type, const double* pos, const double* vel,

@@ -519,11 +519,13 @@ int phase_multigrid(mph_scene& S) {
 // preconditionWithMultiGrid (4122-4266): out = D^-1 in + G2P V(P2G in); `part`
 // receives the chunk partials of in.out when non-null.  pqy non-null: in is S.q, and
 // the P2G forms the CR update q = beta q + pqy (4364-4366) as it reads q
-void precondition(mph_scene& S, const double* in, double* out, double* part, const double* pqy = nullptr) {
+// (rho: its partials when the P2G is to fold them, kFoldChunks)
+void precondition(mph_scene& S, const double* in, double* out, double* part, const double* pqy = nullptr,
+                  const double* rho = nullptr) {
     hipStream_t st = S.st;
     const int D = S.depth, F = S.fuse;  // levels F..D-1 run in one workgroup
     Level& L0 = S.lv[0].L;
-    if (pqy) launch_mg_p2g_bu_pq(st, S.P, L0, S.cellStart.p, S.q.p, pqy, S.scal.p);
+    if (pqy) launch_mg_p2g_bu_pq(st, S.P, L0, S.cellStart.p, S.q.p, pqy, S.scal.p, rho);
     else launch_mg_p2g_bu(st, S.P, L0, S.cellStart.p, in);  // P2G, S = 0, R = Q, S += invD R
     if (F > 0) {
         launch_mg_residual_update(st, L0);  // pre-smooth x2
@@ -559,6 +561,13 @@ int apply_m(mph_scene& S, const double* in, double* out, double* part) {
     return MPH_OK;
 }
 
+// a later CR iteration launches no reduction of rho and tmp: the kernels that read them
+// fold their partials (body::dot_fold).  Per iteration two launches of 1.7-4.6 us fewer; a
+// workgroup's fold costs under 1 us.  Larger scenes reduce them once.
+bool fold_dots(const mph_scene& S, bool first) {
+    return !first && S.prm.multigrid && (S.P.nf + kChunk - 1) / kChunk <= kFoldChunks;
+}
+
 // The rest of a CR iteration once rho = s.y is reduced (4362-4377): later iterations
 // p = beta p + s and q = beta q + y; u = M^-1 q, tmp = q.u; then xv += alpha p,
 // r -= alpha q, s -= alpha u with the r.r partials in S.part.  With the multigrid
@@ -571,10 +580,12 @@ int cr_tail(mph_scene& S, bool first, double* xv) {
     const bool fuse = !first && S.prm.multigrid;
     int rc;
     if (!first && !fuse) launch_pq_update(st, P, S.scal.p, S.s.p, S.y.p, S.p.p, S.q.p);
-    if (fuse) precondition(S, S.q.p, S.u.p, S.part.p, S.y.p);  // u = M^-1 q; tmp = q.u
-    else if ((rc = apply_m(S, S.q.p, S.u.p, S.part.p))) return rc;
-    launch_dot_final(st, P, S.part.p, S.scal.p, kTMP, -1);
-    launch_xrs_update(st, P, S.scal.p, S.p.p, S.q.p, S.u.p, xv, S.r.p, S.s.p, S.part.p, fuse);
+    const bool fold = fold_dots(S, first);
+    double* const tmp = fold ? S.part.p + P.nf / kChunk + 2 : S.part.p;  // beside rho's
+    if (fuse) precondition(S, S.q.p, S.u.p, tmp, S.y.p, fold ? S.part.p : nullptr);  // u = M^-1 q; tmp = q.u
+    else if ((rc = apply_m(S, S.q.p, S.u.p, tmp))) return rc;
+    if (!fold) launch_dot_final(st, P, tmp, S.scal.p, kTMP, -1);
+    launch_xrs_update(st, P, S.scal.p, S.p.p, S.q.p, S.u.p, xv, S.r.p, S.s.p, S.part.p, fuse, fold ? tmp : nullptr);
     return MPH_OK;
 }
 
@@ -782,11 +793,12 @@ int cr_iteration(mph_scene& S, bool first, bool dev, long long maxit, long long 
         launch_dot_final(st, P, S.part.p, S.scal.p, kRHO, kRHOP);
     } else {
         spmv(S, 1.0, S.s.p, 0.0, S.y.p, S.y.p, nullptr, nullptr, S.s.p, S.part.p);
-        launch_dot_final(st, P, S.part.p, S.scal.p, kRHO, kRHOP);
+        if (!fold_dots(S, first)) launch_dot_final(st, P, S.part.p, S.scal.p, kRHO, kRHOP);
     }
     if ((rc = cr_tail(S, first, S.x.p))) return rc;
-    if (dev) launch_dot_final_stop(st, P, S.part.p, S.scal.p, S.ctl.p, 1, S.prm.cr_tolerance, maxit, S.hctl, S.hrr);
-    else launch_dot_final(st, P, S.part.p, S.scal.p, kRR, -1, rr_host(S));
+    const bool fold = fold_dots(S, first);
+    if (dev) launch_dot_final_stop(st, P, S.part.p, S.scal.p, S.ctl.p, 1, S.prm.cr_tolerance, maxit, S.hctl, S.hrr, fold);
+    else launch_dot_final(st, P, S.part.p, S.scal.p, kRR, -1, rr_host(S), fold);
     return MPH_OK;
 }
 
@@ -924,7 +936,7 @@ int phase_solve(mph_scene& S) {
     const long long maxit = S.prm.max_iterations > 0 ? S.prm.max_iterations : n;
     S.convRows = 0;
     if (S.convCheck && (rc = S.convRec.ensure(2 * (size_t)std::min(std::max(maxit, 1LL), kConvRowsMax)))) return rc;
-    if (dev) launch_dot_final_stop(st, P, S.part.p, S.scal.p, S.ctl.p, 0, S.prm.cr_tolerance, maxit, S.hctl, S.hrr);
+    if (dev) launch_dot_final_stop(st, P, S.part.p, S.scal.p, S.ctl.p, 0, S.prm.cr_tolerance, maxit, S.hctl, S.hrr, false);
     else launch_dot_final(st, P, S.part.p, S.scal.p, kRR, -1, rr_host(S));
     if ((rc = read_scalar(S, kRR0, &S.rr0))) return rc;
     if (!std::isfinite(S.rr0)) return solve_nonfinite(S, "b.b", S.rr0);
@@ -1041,10 +1053,10 @@ int phase_solve_mixed(mph_scene& S) {
                 launch_dot_final(st, P, S.part.p, S.scal.p, kRHO, kRHOP);
             } else {
                 spmv(S, 1.0, S.s.p, 0.0, S.y.p, S.y.p, nullptr, nullptr, S.s.p, S.part.p, true);
-                launch_dot_final(st, P, S.part.p, S.scal.p, kRHO, kRHOP);
+                if (!fold_dots(S, false)) launch_dot_final(st, P, S.part.p, S.scal.p, kRHO, kRHOP);
             }
             if ((rc = cr_tail(S, it == 0, S.dvec.p))) return rc;
-            launch_dot_final(st, P, S.part.p, S.scal.p, kRR, -1, rr_host(S));
+            launch_dot_final(st, P, S.part.p, S.scal.p, kRR, -1, rr_host(S), fold_dots(S, it == 0));
         }
         S.facPref = nullptr;  // a first pass enqueued ahead of the inner stop is not used
         S.facPrefEv = -1;
@@ -1141,7 +1153,7 @@ int allocate(mph_scene& S) {
     ENS(S.width, (size_t)S.nslices); ENS(S.sliceStart, (size_t)S.nslices + 1); ENS(S.selfIdx, nf);
     ENS(S.b, 3 * nf); ENS(S.vecP, np); ENS(S.invDiagA, 3 * nf);
     ENS(S.x, 3 * nf); ENS(S.r, 3 * nf); ENS(S.s, 3 * nf); ENS(S.y, 3 * nf); ENS(S.p, 3 * nf); ENS(S.q, 3 * nf);
-    ENS(S.u, 3 * nf); ENS(S.part, nf / kChunk + 2); ENS(S.scal, 16);
+    ENS(S.u, 3 * nf); ENS(S.part, 2 * (nf / kChunk + 2)); ENS(S.scal, 16);
 #undef ENS
     HIPCHK(hipHostMalloc((void**)&S.hpin, 64 * sizeof(double), hipHostMallocDefault));
     HIPCHK(hipHostMalloc((void**)&S.hrr, 8 * sizeof(double), hipHostMallocCoherent));

@@ -54,7 +54,7 @@ struct HostLevel {
     DBuf<float> A32;
 };
 
-enum { kRR0 = 0, kRS0 = 1, kRR = 2, kRHO = 3, kRHOP = 4, kTMP = 5, kRS = 6, kRSIter = 7, kCheckRR = 8, kCheckRS = 9 };
+enum { kRR0 = 0, kRS0 = 1, kRR = 2, kRHO = 3, kRHOP = 4, kTMP = 5, kRS = 6, kRSIter = 7, kCheckRR = 8, kCheckRS = 9 };  // 10: rho of the iteration under way (kRHON)
 
 // Run-time choice among kernel variants that compute identical bits: while
 // exploring, launches cycle through the variants with HIP events around them;

@@ -293,10 +293,17 @@ __global__ void k_fill_i32(int* x, long long n, int v) {
 
 template <bool kPq, bool kOrd>
 __global__ void __launch_bounds__(256) k_mg_p2g_bu(DevParams P, Level L, const int* __restrict__ cellStart, double* q,
-                                                   const double* __restrict__ yv, const double* __restrict__ scal) {
+                                                   const double* __restrict__ yv, double* scal, const double* rho) {
     if (cr_halted(L.halt)) return;
     __shared__ double tb[kOrd ? 256 * kP2gK : 1];
-    mg_p2g_lanes<kPq, kOrd>(P, L, cellStart, q, yv, scal, blockIdx.x, tb);
+    __shared__ double sh[kPq ? 257 : 1];
+    auto beta = [&] {
+        if (!rho) return scal[kRHO] / scal[kRHOP];
+        const double v = dot_fold(rho, nblk(P.nf, kChunk), sh);
+        if (blockIdx.x == 0 && threadIdx.x == 0) scal[kRHON] = v;  // read by later launches only
+        return v / scal[kRHO];
+    };
+    mg_p2g_lanes<kPq, kOrd>(P, L, cellStart, q, yv, beta, blockIdx.x, tb);
 }
 
 // restriction into L, then begin + update of L on the same row
@@ -424,9 +431,11 @@ __global__ void __launch_bounds__(256) k_dot_partial(int nf, const double* __res
 }
 
 __global__ void __launch_bounds__(256) k_dot_final(const double* __restrict__ part, int nchunks, double* scal,
-                                                   int slot, int shift_slot, double* host, const int* halt) {
+                                                   int slot, int shift_slot, double* host, const int* halt,
+                                                   int shiftRho) {
     if (cr_halted(halt)) return;
     __shared__ double sh[256];
+    if (shiftRho && threadIdx.x == 0) dot_shift_rho(scal);
     dot_final_body(part, nchunks, scal, slot, shift_slot, sh, host);
 }
 
@@ -450,9 +459,10 @@ __global__ void __launch_bounds__(256) k_dot_final_record(const double* __restri
 // thread before thread 0 writes it, behind the reduction's barriers
 __global__ void __launch_bounds__(256) k_dot_final_stop(const double* __restrict__ part, int nchunks, double* scal,
                                                         int* ctl, int step, double tol, long long maxit, int* hctl,
-                                                        double* hrr) {
+                                                        double* hrr, int shiftRho) {
     if (ctl[kCtlHalt]) return;
     __shared__ double sh[256];
+    if (shiftRho && threadIdx.x == 0) dot_shift_rho(scal);
     dot_final_body(part, nchunks, scal, kRR, -1, sh, hrr);
     if (threadIdx.x != 0) return;
     const double rr = scal[kRR];
@@ -480,14 +490,20 @@ __global__ void k_pq_update(int nf, const double* __restrict__ scal, const doubl
 }
 
 template <bool kPq>
-__global__ void __launch_bounds__(256) k_xrs_update(int nf, const double* __restrict__ scal,
+__global__ void __launch_bounds__(256) k_xrs_update(int nf, const double* __restrict__ scal, const double* tmp,
                                                     double* __restrict__ p, const double* __restrict__ q,
                                                     const double* __restrict__ u, double* __restrict__ x,
                                                     double* __restrict__ r, double* __restrict__ s,
                                                     double* __restrict__ part, const int* halt) {
     if (cr_halted(halt)) return;
-    __shared__ double sh[256];
-    xrs_update_chunk<kPq>(nf, scal, p, q, u, x, r, s, part, blockIdx.x, sh);
+    __shared__ double sh[256], sf[kPq ? 257 : 1];
+    auto coef = [&](double& alpha, double& beta) {
+        const bool fold = kPq && tmp;
+        const double rho = scal[fold ? kRHON : kRHO], rhop = kPq ? scal[fold ? kRHO : kRHOP] : 1.0;
+        alpha = rho / (fold ? dot_fold(tmp, nblk(nf, kChunk), sf) : scal[kTMP]);
+        beta = kPq ? rho / rhop : 0.0;
+    };
+    xrs_update_chunk<kPq>(nf, coef, p, q, u, x, r, s, part, blockIdx.x, sh);
 }
 
 __global__ void k_store_velocity(int nf, const double* __restrict__ x, double* __restrict__ vel) {
@@ -722,17 +738,19 @@ void launch_mg_p2g_bu(hipStream_t st, const DevParams& P, Level& L, const int* c
     double* qw = const_cast<double*>(q);  // not written without kPq
     if (L.ordered)
         hipLaunchKernelGGL((k_mg_p2g_bu<false, true>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, qw,
-                           nullptr, nullptr);
+                           nullptr, nullptr, nullptr);
     else
         hipLaunchKernelGGL((k_mg_p2g_bu<false, false>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, qw,
-                           nullptr, nullptr);
+                           nullptr, nullptr, nullptr);
 }
 void launch_mg_p2g_bu_pq(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, double* q,
-                         const double* y, const double* scal) {
+                         const double* y, double* scal, const double* rho) {
     if (L.ordered)
-        hipLaunchKernelGGL((k_mg_p2g_bu<true, true>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, q, y, scal);
+        hipLaunchKernelGGL((k_mg_p2g_bu<true, true>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, q, y, scal,
+                           rho);
     else
-        hipLaunchKernelGGL((k_mg_p2g_bu<true, false>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, q, y, scal);
+        hipLaunchKernelGGL((k_mg_p2g_bu<true, false>), dim3(p2g_blocks(L)), dim3(256), 0, st, P, L, cellStart, q, y, scal,
+                           rho);
 }
 void launch_mg_restrict_bu(hipStream_t st, const Level& S, Level& L) {
     hipLaunchKernelGGL(k_mg_restrict_bu, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, S, L);
@@ -858,9 +876,9 @@ void launch_axpy(hipStream_t st, long long n, const double* x, double* y) {
 void launch_dot_partial(hipStream_t st, const DevParams& P, const double* x, const double* y, double* part) {
     hipLaunchKernelGGL(k_dot_partial, dim3(nblk(P.nf, kChunk)), dim3(kChunk), 0, st, P.nf, x, y, part, P.halt);
 }void launch_dot_final(hipStream_t st, const DevParams& P, const double* part, double* scal, int slot,
-                      int shift_slot, double* host) {
+                      int shift_slot, double* host, bool shiftRho) {
     hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(256), 0, st, part, nblk(P.nf, kChunk), scal, slot, shift_slot,
-                       host, P.halt);
+                       host, P.halt, shiftRho ? 1 : 0);
 }
 void launch_dot_final_record(hipStream_t st, const DevParams& P, const double* part, double* scal, const int* ctl,
                              long long it, double* rec, long long cap) {
@@ -868,21 +886,21 @@ void launch_dot_final_record(hipStream_t st, const DevParams& P, const double* p
                        cap, P.halt);
 }
 void launch_dot_final_stop(hipStream_t st, const DevParams& P, const double* part, double* scal, int* ctl, int step,
-                           double tol, long long maxit, int* hctl, double* hrr) {
+                           double tol, long long maxit, int* hctl, double* hrr, bool shiftRho) {
     hipLaunchKernelGGL(k_dot_final_stop, dim3(1), dim3(256), 0, st, part, nblk(P.nf, kChunk), scal, ctl, step, tol,
-                       maxit, hctl, hrr);
+                       maxit, hctl, hrr, shiftRho ? 1 : 0);
 }
 void launch_pq_update(hipStream_t st, const DevParams& P, const double* scal, const double* s, const double* y,
                       double* p, double* q) {
     hipLaunchKernelGGL(k_pq_update, dim3(nblk(3LL * P.nf, 256)), dim3(256), 0, st, P.nf, scal, s, y, p, q, P.halt);
 }
 void launch_xrs_update(hipStream_t st, const DevParams& P, const double* scal, double* p, const double* q,
-                       const double* u, double* x, double* r, double* s, double* part, bool pq) {
+                       const double* u, double* x, double* r, double* s, double* part, bool pq, const double* tmp) {
     if (pq)
-        hipLaunchKernelGGL(k_xrs_update<true>, dim3(nblk(P.nf, kChunk)), dim3(kChunk), 0, st, P.nf, scal, p, q, u, x,
+        hipLaunchKernelGGL(k_xrs_update<true>, dim3(nblk(P.nf, kChunk)), dim3(kChunk), 0, st, P.nf, scal, tmp, p, q, u, x,
                            r, s, part, P.halt);
     else
-        hipLaunchKernelGGL(k_xrs_update<false>, dim3(nblk(P.nf, kChunk)), dim3(kChunk), 0, st, P.nf, scal, p, q, u, x,
+        hipLaunchKernelGGL(k_xrs_update<false>, dim3(nblk(P.nf, kChunk)), dim3(kChunk), 0, st, P.nf, scal, nullptr, p, q, u, x,
                            r, s, part, P.halt);
 }
 void launch_store_velocity(hipStream_t st, const DevParams& P, const double* x, double* vel) {
