@@ -231,9 +231,9 @@ __device__ inline void sweep(const Level& L, int lb, double* tb) {
     }
     const long long t = (long long)lb * 256 + threadIdx.x;
     const bool s3 = L.cs[0] == 3 && L.cs[1] == 3;
-    if (s3 && L.cs[2] == 3) mg_sweep_lanes<VT, kUpdate, kOrd, 3, 3, 3>(L, t, tb);
-    else if (s3 && L.cs[2] == 1) mg_sweep_lanes<VT, kUpdate, kOrd, 3, 3, 1>(L, t, tb);
-    else mg_sweep_lanes<VT, kUpdate, kOrd, 0, 0, 0>(L, t, tb);
+    if (s3 && L.cs[2] == 3) mg_sweep_lanes<VT, kUpdate, kOrd, false, 3, 3, 3>(L, L, t, tb);
+    else if (s3 && L.cs[2] == 1) mg_sweep_lanes<VT, kUpdate, kOrd, false, 3, 3, 1>(L, L, t, tb);
+    else mg_sweep_lanes<VT, kUpdate, kOrd, false, 0, 0, 0>(L, L, t, tb);
 }
 template <bool kUpdate>
 __global__ void __launch_bounds__(256) kb_mg_sweep(const BScene* tab, const int* off, int ns, SceneSet on, int l,
@@ -290,8 +290,8 @@ __global__ void __launch_bounds__(T) kb_mg_coarse(const BScene* tab, int ns, Sce
     const double* in = B.fuse > 0 ? S.R : S.Q;
     double* io = lv_s(S, B.fuse > 0 ? c : c ^ 1);
     const int* halt = B.ctl ? B.ctl + kCtlHalt : nullptr;
-    if (K.ordered) mg_coarse_cycle<N, T, XB, true>(K, B.fuse, B.depth, in, io, S.nrow, halt, sh);
-    else mg_coarse_cycle<N, T, XB, false>(K, B.fuse, B.depth, in, io, S.nrow, halt, sh);
+    if (K.ordered) mg_coarse_cycle<N, T, XB, true>(K, B.fuse, B.depth, in, io, S.nrow, false, halt, sh);
+    else mg_coarse_cycle<N, T, XB, false>(K, B.fuse, B.depth, in, io, S.nrow, false, halt, sh);
 }
 
 #undef MPH_SCENE

@@ -285,12 +285,23 @@ __device__ inline void mg_residual_update_row(const Level& L, int row) {
 // workgroup (ordered only)
 constexpr int kRowLanes = 4, kRowQ = 7;  // kRowQ: stencil cells per lane (27 / 4, rounded up)
 constexpr int kRowTerms = 3 * kRowQ;
-template <class VT, bool kUpdate, bool kOrd, int C0, int C1, int C2>
-__device__ inline void mg_sweep_lanes(const Level& L, long long t, double* tb) {
+
+// the prolongation's value of level U for row rd of cell (gx, gy, gz) of level L (mg_prolong_row)
+__device__ inline double mg_parent_value(const Level& U, const Level& L, int gx, int gy, int gz, int rd) {
+    const int g = grid_id(U, ((gx + L.mn[0]) / 2) - U.mn[0], ((gy + L.mn[1]) / 2) - U.mn[1],
+                          ((gz + L.mn[2]) / 2) - U.mn[2]);
+    double sum = 0.0;
+    sum += 1.0 * 1.0 * lv_s(U, U.cur)[3 * g + rd];
+    return sum;
+}
+
+// lane u's part of the sum of `row`, for the four lanes of the row (on: it has one); the
+// whole sum in its first lane.  kUp: on the iterate after the prolongation from U, formed
+// as it is read (the same add as mg_prolong_row's); own: that of the row itself.
+template <class VT, bool kOrd, bool kUp, int C0, int C1, int C2>
+__device__ inline double mg_lanes_sum(const Level& L, const Level& U, int row, bool on, double* tb, double* own) {
     constexpr int T = kRowTerms;
     const int u = threadIdx.x & (kRowLanes - 1);
-    const int row = (int)(t / kRowLanes);
-    const bool on = row < L.nrow;
     const int cs1 = C0 ? C1 : L.cs[1], cs2 = C0 ? C2 : L.cs[2];
     const int N = (C0 ? C0 : L.cs[0]) * cs1 * cs2, Q = row_chain(N);  // N <= 27
     const VT* __restrict__ A = sizeof(VT) == 8 ? (const VT*)L.A : (const VT*)L.A32;
@@ -301,6 +312,7 @@ __device__ inline void mg_sweep_lanes(const Level& L, long long t, double* tb) {
         int gx, gy, gz;
         grid_xyz(L, row / 3, gx, gy, gz);
         const int c0 = L.cnt[0], c1 = L.cnt[1], c2 = L.cnt[2];
+        double up[kUp ? T : 1];
 #pragma unroll
         for (int k = 0; k < kRowQ; ++k) {
             const int q = u * Q + k;
@@ -313,11 +325,20 @@ __device__ inline void mg_sweep_lanes(const Level& L, long long t, double* tb) {
                 for (int sd = 0; sd < 3; ++sd) {
                     a[3 * k + sd] = (double)A[(3 * q + sd) * nrow + row];
                     xv[3 * k + sd] = xc[sd];
+                    if constexpr (kUp) up[3 * k + sd] = mg_parent_value(U, L, jx, jy, jz, sd);
                 }
             } else {
 #pragma unroll
-                for (int sd = 0; sd < 3; ++sd) a[3 * k + sd] = xv[3 * k + sd] = 0.0;
+                for (int sd = 0; sd < 3; ++sd) {
+                    a[3 * k + sd] = xv[3 * k + sd] = 0.0;
+                    if constexpr (kUp) up[3 * k + sd] = 0.0;
+                }
             }
+        }
+        if constexpr (kUp) {
+            *own = x[row] + mg_parent_value(U, L, gx, gy, gz, row % 3);
+#pragma unroll
+            for (int e = 0; e < T; ++e) xv[e] += up[e];
         }
     } else {
 #pragma unroll
@@ -328,28 +349,68 @@ __device__ inline void mg_sweep_lanes(const Level& L, long long t, double* tb) {
 #pragma unroll
         for (int e = 0; e < T; ++e) tb[T * threadIdx.x + e] = -1.0 * a[e] * xv[e];
         wave_sync();
-        if (u != 0 || !on) return;
-        for (int v = 0; v < kRowLanes; ++v)
-            for (int k = 0; k < Q && v * Q + k < N; ++k)
+        if (u == 0 && on)
+            for (int v = 0; v < kRowLanes; ++v)
+                for (int k = 0; k < Q && v * Q + k < N; ++k)
 #pragma unroll
-                for (int sd = 0; sd < 3; ++sd) sum += tb[T * (threadIdx.x + v) + 3 * k + sd];
+                    for (int sd = 0; sd < 3; ++sd) sum += tb[T * (threadIdx.x + v) + 3 * k + sd];
     } else {
 #pragma unroll
         for (int e = 0; e < T; ++e) sum = __builtin_fma(-a[e], xv[e], sum);
         sum += __shfl_xor(sum, 1, 64);
         sum += __shfl_xor(sum, 2, 64);
-        if (u != 0 || !on) return;
     }
+    return sum;
+}
+
+// kUp: the first sweep after the prolongation from U, whose launch it takes the place of
+template <class VT, bool kUpdate, bool kOrd, bool kUp, int C0, int C1, int C2>
+__device__ inline void mg_sweep_lanes(const Level& L, const Level& U, long long t, double* tb) {
+    const int row = (int)(t / kRowLanes);
+    const bool on = row < L.nrow;
+    double own = 0.0;
+    const double sum = mg_lanes_sum<VT, kOrd, kUp, C0, C1, C2>(L, U, row, on, tb, &own);
+    if ((threadIdx.x & (kRowLanes - 1)) != 0 || !on) return;
     double y = L.Q[row];
     y *= 1.0;
     y += sum;
     L.R[row] = y;
     if (kUpdate) {
-        double sv = x[row];
+        double sv = kUp ? own : lv_s(L, L.cur)[row];
         sv *= 1.0;
         sv += 1.0 * L.invD[row] * y;
         lv_s(L, L.cur ^ 1)[row] = sv;
     }
+}
+
+// The residual of S (mg_residual_row), its restriction into L (mg_restrict_row), then
+// begin and update of L: a group of 4 lanes per child (8, in 2D 4 children) forms a
+// coarse row's fine residuals, which are added in child order; a clipped child adds a
+// zero, which changes no bit.  S.R is read by nothing else then and is not written.  One
+// launch in the place of two of 3.8 and 4.6 us on the 64k drop.
+template <int C0, int C2>
+__host__ __device__ constexpr int restrict_lanes() { return kRowLanes * (C0 && C2 == 1 ? 4 : 8); }
+template <class VT, bool kOrd, int C0, int C1, int C2>
+__device__ inline void mg_residual_restrict_lanes(const Level& S, const Level& L, long long t, double* tb) {
+    constexpr int G = restrict_lanes<C0, C2>(), KC = G / kRowLanes, KZ = KC / 4;
+    const int lrow = (int)(t / G), c = (int)(t / kRowLanes) % KC, rd = lrow % 3;
+    const bool own = lrow < L.nrow;
+    int lx = 0, ly = 0, lz = 0;
+    if (own) grid_xyz(L, lrow / 3, lx, ly, lz);
+    const int fx = 2 * (lx + L.mn[0]) + c / (2 * KZ) - S.mn[0], fy = 2 * (ly + L.mn[1]) + (c / KZ) % 2 - S.mn[1];
+    const int fz = 2 * (lz + L.mn[2]) + c % KZ - S.mn[2];
+    const bool on = own && fx >= 0 && fx < S.cnt[0] && fy >= 0 && fy < S.cnt[1] && fz >= 0 && fz < S.cnt[2];
+    const int row = on ? 3 * grid_id(S, fx, fy, fz) + rd : 0;
+    const double q = on ? S.Q[row] : 0.0;
+    double y = mg_lanes_sum<VT, kOrd, false, C0, C1, C2>(S, S, row, on, tb, nullptr);
+    y = on ? q * 1.0 + y : 0.0;
+    double sum = 0.0;
+    const int l0 = (int)(threadIdx.x & 63) & ~(G - 1);
+#pragma unroll
+    for (int k = 0; k < KC; ++k) sum += 1.0 * 1.0 * __shfl(y, l0 + kRowLanes * k, 64);
+    if ((int)(threadIdx.x & 63) != l0 || !own) return;
+    L.Q[lrow] = sum;  // Q*0.0 is a zero, the sum never -0
+    mg_begin_update_row(L, lrow, sum);
 }
 
 // restriction (R of 3115-3175): Q_L = 0*Q_L + sum of the clipped 2x2x2 children of R_S,
@@ -515,11 +576,12 @@ struct CoarseShared {
 
 // K: the packed levels lc..D-1; in: R of level lc-1 (Q of level 0 when lc = 0); io: S of
 // level lc-1, which the prolongation updates (of level 0 when lc = 0, written); nio: its
-// rows.  XB: stencil cells whose LDS reads are in flight together.  halt: the CR stop
+// rows; plain: io is S of level lc, written in the place of that prolongation.
+// XB: stencil cells whose LDS reads are in flight together.  halt: the CR stop
 // flag or null, tested once the loads are under way.
 template <int N, int T, int XB, bool kOrd>
 __device__ inline void mg_coarse_cycle(const CoarsePack& K, int lc, int D, const double* __restrict__ in, double* io,
-                                       int nio, const int* halt, CoarseShared<T>& sh) {
+                                       int nio, bool plain, const int* halt, CoarseShared<T>& sh) {
     const int tid = threadIdx.x, st = K.stride;
     double a[3 * N], w, q = 0.0, s = 0.0;
     int po[(N + 1) / 2];  // pairs of LDS places
@@ -633,6 +695,10 @@ __device__ inline void mg_coarse_cycle(const CoarsePack& K, int lc, int D, const
         if (myl == 0) io[tid] = s;
     } else {
         const double* x = sh.S[lc == D - 1 ? 0 : 1];
+        if (plain) {
+            if (myl == lc) io[tid] = s;
+            return;
+        }
         for (int r = tid; r < nio; r += st) {
             double sum = 0.0;
             sum += 1.0 * 1.0 * x[K.up[r]];

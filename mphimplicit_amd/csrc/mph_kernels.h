@@ -264,7 +264,14 @@ void launch_mg_prolong(hipStream_t st, const Level& L, Level& S);
 // when lc = 0 (Q0 in, S0 out, three sweeps).  f32: pack the FP32 stencils where a level
 // has one.  lvs: device copy of the levels.
 void launch_mg_coarse_pack(hipStream_t st, const Level* lvs, int lc, int D, bool f32, const CoarsePack& K);
-void launch_mg_coarse(hipStream_t st, const DevParams& P, const CoarsePack& K, int lc, int D, const Level& S);
+// S: level lc-1 (0 when lc = 0), F: level lc.  Where S takes the lane-split sweeps, S of F is
+// written and the prolongation left to launch_mg_prolong_update
+void launch_mg_coarse(hipStream_t st, const DevParams& P, const CoarsePack& K, int lc, int D, const Level& S,
+                      const Level& F);
+// residual of S, restriction into L, begin, update
+void launch_mg_residual_restrict(hipStream_t st, Level& S, Level& L);
+// prolongation U -> L (unless launch_mg_coarse has done it: prolonged), then a residual-update sweep of L
+void launch_mg_prolong_update(hipStream_t st, const Level& U, Level& L, bool prolonged);
 void launch_mg_g2p(hipStream_t st, const DevParams& P, const Level& L0, const int* cellIndex,
                    const double* invDiagA, const double* q, double* u, double* part);
 // ---- conjugate residual ----

@@ -527,26 +527,19 @@ void precondition(mph_scene& S, const double* in, double* out, double* part, con
     Level& L0 = S.lv[0].L;
     if (pqy) launch_mg_p2g_bu_pq(st, S.P, L0, S.cellStart.p, S.q.p, pqy, S.scal.p, rho);
     else launch_mg_p2g_bu(st, S.P, L0, S.cellStart.p, in);  // P2G, S = 0, R = Q, S += invD R
-    if (F > 0) {
-        launch_mg_residual_update(st, L0);  // pre-smooth x2
-        launch_mg_residual(st, L0);
-    }
-    for (int l = 1; l < F; ++l) {
+    for (int l = 0; l < F; ++l) {  // pre-smooth x2 on level 0, x3 below
         Level& L = S.lv[l].L;
-        launch_mg_restrict_bu(st, S.lv[l - 1].L, L);  // pre-smooth x3
-        launch_mg_residual_update(st, L);
-        launch_mg_residual_update(st, L);
-        launch_mg_residual(st, L);
+        for (int k = 0; k < (l == 0 ? 1 : 2); ++k) launch_mg_residual_update(st, L);
+        if (l + 1 < F) launch_mg_residual_restrict(st, L, S.lv[l + 1].L);
+        else launch_mg_residual(st, L);
     }
-    launch_mg_coarse(st, S.P, S.pack, F, D, S.lv[F > 0 ? F - 1 : 0].L);
+    launch_mg_coarse(st, S.P, S.pack, F, D, S.lv[F > 0 ? F - 1 : 0].L, S.lv[F].L);
     if (F == 0) L0.cur ^= 1;
-    for (int l = F - 1; l > 0; --l) {
+    for (int l = F - 1; l >= 0; --l) {  // prolongation, post-smooth x3, x2 on level 0
         Level& L = S.lv[l].L;
-        for (int k = 0; k < 3; ++k) launch_mg_residual_update(st, L);  // post-smooth x3
-        launch_mg_prolong(st, L, S.lv[l - 1].L);
+        launch_mg_prolong_update(st, S.lv[l + 1].L, L, l == F - 1);
+        for (int k = 1; k < (l == 0 ? 2 : 3); ++k) launch_mg_residual_update(st, L);
     }
-    if (F > 0)
-        for (int k = 0; k < 2; ++k) launch_mg_residual_update(st, L0);  // post-smooth x2
     launch_mg_g2p(st, S.P, L0, S.cellIndex.p, S.invDiagA.p, in, out, part);
 }
 

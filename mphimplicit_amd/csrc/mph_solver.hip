@@ -339,33 +339,46 @@ __global__ void __launch_bounds__(256) k_mg_residual_update(Level L) {
 }
 
 constexpr int kRowBlock = 128;
-template <class VT, bool kUpdate, bool kOrd, int C0, int C1, int C2>
-__global__ void __launch_bounds__(kRowBlock) k_mg_sweep_lanes(Level L) {
+template <class VT, bool kUpdate, bool kOrd, bool kUp, int C0, int C1, int C2>
+__global__ void __launch_bounds__(kRowBlock) k_mg_sweep_lanes(Level L, Level U) {
     if (cr_halted(L.halt)) return;
     __shared__ double tb[kOrd ? kRowBlock * kRowTerms : 1];
-    mg_sweep_lanes<VT, kUpdate, kOrd, C0, C1, C2>(L, (long long)blockIdx.x * kRowBlock + threadIdx.x, tb);
+    mg_sweep_lanes<VT, kUpdate, kOrd, kUp, C0, C1, C2>(L, U, (long long)blockIdx.x * kRowBlock + threadIdx.x, tb);
 }
 
-// launches the lane-split sweep on a small level; false for a large one
-template <bool kUpdate>
-bool launch_sweep_lanes(hipStream_t st, const Level& L) {
-    if (!L.lanes || L.cs[0] * L.cs[1] * L.cs[2] > kRowLanes * kRowQ) return false;
-    const int nb = nblk((long long)kRowLanes * L.nrow, kRowBlock);
-    const bool s3 = L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 3, s2 = L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 1;
-#define MPH_SWEEP(VT, A, B, C)                                                                                       \
-    do {                                                                                                             \
-        if (L.ordered) hipLaunchKernelGGL((k_mg_sweep_lanes<VT, kUpdate, true, A, B, C>), dim3(nb), dim3(kRowBlock), 0, st, L); \
-        else hipLaunchKernelGGL((k_mg_sweep_lanes<VT, kUpdate, false, A, B, C>), dim3(nb), dim3(kRowBlock), 0, st, L);          \
+template <class VT, bool kOrd, int C0, int C1, int C2>
+__global__ void __launch_bounds__(kRowBlock) k_mg_residual_restrict(Level S, Level L) {
+    if (cr_halted(L.halt)) return;
+    __shared__ double tb[kOrd ? kRowBlock * kRowTerms : 1];
+    mg_residual_restrict_lanes<VT, kOrd, C0, C1, C2>(S, L, (long long)blockIdx.x * kRowBlock + threadIdx.x, tb);
+}
+
+// whether a level takes the lane-split kernels: a small one, a stencil that four lanes hold
+bool row_lanes(const Level& L) { return L.lanes && L.cs[0] * L.cs[1] * L.cs[2] <= kRowLanes * kRowQ; }
+
+// MPH_SHAPE(L, go): go(VT, ordered, C0, C1, C2) for the level's precision, order and stencil
+#define MPH_SHAPE3(L, go, VT, ORD)                                                                  \
+    do {                                                                                            \
+        if (L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 3) go(VT, ORD, 3, 3, 3);                      \
+        else if (L.cs[0] == 3 && L.cs[1] == 3 && L.cs[2] == 1) go(VT, ORD, 3, 3, 1);                 \
+        else go(VT, ORD, 0, 0, 0);                                                                  \
     } while (0)
-    if (L.f32) {
-        if (s3) MPH_SWEEP(float, 3, 3, 3);
-        else if (s2) MPH_SWEEP(float, 3, 3, 1);
-        else MPH_SWEEP(float, 0, 0, 0);
-    } else {
-        if (s3) MPH_SWEEP(double, 3, 3, 3);
-        else if (s2) MPH_SWEEP(double, 3, 3, 1);
-        else MPH_SWEEP(double, 0, 0, 0);
-    }
+#define MPH_SHAPE(L, go)                                                                            \
+    do {                                                                                            \
+        if (L.f32 && L.ordered) MPH_SHAPE3(L, go, float, true);                                     \
+        else if (L.f32) MPH_SHAPE3(L, go, float, false);                                            \
+        else if (L.ordered) MPH_SHAPE3(L, go, double, true);                                        \
+        else MPH_SHAPE3(L, go, double, false);                                                      \
+    } while (0)
+
+// launches the lane-split sweep on a small level; false for a large one
+template <bool kUpdate, bool kUp>
+bool launch_sweep_lanes(hipStream_t st, const Level& L, const Level& U) {
+    if (!row_lanes(L)) return false;
+    const int nb = nblk((long long)kRowLanes * L.nrow, kRowBlock);
+#define MPH_SWEEP(VT, ORD, A, B, C) \
+    hipLaunchKernelGGL((k_mg_sweep_lanes<VT, kUpdate, ORD, kUp, A, B, C>), dim3(nb), dim3(kRowBlock), 0, st, L, U)
+    MPH_SHAPE(L, MPH_SWEEP);
 #undef MPH_SWEEP
     return true;
 }
@@ -384,9 +397,9 @@ __global__ void k_mg_prolong(Level L, Level S) {
 // levels lc..D-1 in one workgroup (mg_coarse_cycle)
 template <int N, int T, int XB, bool kOrd>
 __global__ void __launch_bounds__(T) k_mg_coarse(CoarsePack K, int lc, int D, const double* __restrict__ in, double* io,
-                                                 int nio, const int* halt) {
+                                                 int nio, int plain, const int* halt) {
     __shared__ CoarseShared<T> sh;
-    mg_coarse_cycle<N, T, XB, kOrd>(K, lc, D, in, io, nio, halt, sh);
+    mg_coarse_cycle<N, T, XB, kOrd>(K, lc, D, in, io, nio, plain != 0, halt, sh);
 }
 
 __global__ void __launch_bounds__(64) k_mg_coarse_pack(const Level* __restrict__ lvs, int lc, int D, int f32, CoarsePack K) {
@@ -770,13 +783,33 @@ void launch_mg_update(hipStream_t st, Level& L) {
         else hipLaunchKernelGGL((KERNEL<double, false>), dim3(nb), dim3(256), 0, st, L);                           \
     } while (0)
 void launch_mg_residual(hipStream_t st, Level& L) {
-    if (!launch_sweep_lanes<false>(st, L)) MPH_ROWS(k_mg_residual);
+    if (!launch_sweep_lanes<false, false>(st, L, L)) MPH_ROWS(k_mg_residual);
 }
 void launch_mg_residual_update(hipStream_t st, Level& L) {
-    if (!launch_sweep_lanes<true>(st, L)) MPH_ROWS(k_mg_residual_update);
+    if (!launch_sweep_lanes<true, false>(st, L, L)) MPH_ROWS(k_mg_residual_update);
     L.cur ^= 1;
 }
 #undef MPH_ROWS
+void launch_mg_residual_restrict(hipStream_t st, Level& S, Level& L) {
+    if (!row_lanes(S)) {
+        launch_mg_residual(st, S);
+        launch_mg_restrict_bu(st, S, L);
+        return;
+    }
+#define MPH_RESTRICT(VT, ORD, A, B, C)                                                                              \
+    hipLaunchKernelGGL((k_mg_residual_restrict<VT, ORD, A, B, C>),                                                  \
+                       dim3(nblk((long long)restrict_lanes<A, C>() * L.nrow, kRowBlock)), dim3(kRowBlock), 0, st, S, L)
+    MPH_SHAPE(S, MPH_RESTRICT);
+#undef MPH_RESTRICT
+}
+void launch_mg_prolong_update(hipStream_t st, const Level& U, Level& L, bool prolonged) {
+    if (launch_sweep_lanes<true, true>(st, L, U)) {
+        L.cur ^= 1;
+        return;
+    }
+    if (!prolonged) launch_mg_prolong(st, U, L);
+    launch_mg_residual_update(st, L);
+}
 void launch_mg_restrict(hipStream_t st, const Level& S, Level& L) {
     hipLaunchKernelGGL(k_mg_restrict, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, S, L);
 }
@@ -786,15 +819,17 @@ void launch_mg_prolong(hipStream_t st, const Level& L, Level& S) {
 void launch_mg_coarse_pack(hipStream_t st, const Level* lvs, int lc, int D, bool f32, const CoarsePack& K) {
     hipLaunchKernelGGL(k_mg_coarse_pack, dim3(kCoarseRows2D / 64), dim3(64), 0, st, lvs, lc, D, f32 ? 1 : 0, K);
 }
-void launch_mg_coarse(hipStream_t st, const DevParams& P, const CoarsePack& K, int lc, int D, const Level& S) {
+void launch_mg_coarse(hipStream_t st, const DevParams& P, const CoarsePack& K, int lc, int D, const Level& S,
+                      const Level& F) {
     const double* in = lc == 0 ? S.Q : S.R;
-    double* io = S.S[lc == 0 ? S.cur ^ 1 : S.cur];
+    const int plain = lc > 0 && row_lanes(S) ? 1 : 0;  // the next sweep of S prolongs
+    double* io = plain ? F.S[F.cur] : S.S[lc == 0 ? S.cur ^ 1 : S.cur];
 #define MPH_COARSE(N, T, XB)                                                                                         \
     do {                                                                                                             \
         if (K.ordered)                                                                                               \
-            hipLaunchKernelGGL((k_mg_coarse<N, T, XB, true>), dim3(1), dim3(K.stride), 0, st, K, lc, D, in, io, S.nrow, P.halt); \
+            hipLaunchKernelGGL((k_mg_coarse<N, T, XB, true>), dim3(1), dim3(K.stride), 0, st, K, lc, D, in, io, S.nrow, plain, P.halt); \
         else                                                                                                         \
-            hipLaunchKernelGGL((k_mg_coarse<N, T, XB, false>), dim3(1), dim3(K.stride), 0, st, K, lc, D, in, io, S.nrow, P.halt); \
+            hipLaunchKernelGGL((k_mg_coarse<N, T, XB, false>), dim3(1), dim3(K.stride), 0, st, K, lc, D, in, io, S.nrow, plain, P.halt); \
     } while (0)
     if (K.cells == 9) MPH_COARSE(9, kCoarseRows2D, 4);
     else if (K.stride <= 256) MPH_COARSE(27, 256, 9);
