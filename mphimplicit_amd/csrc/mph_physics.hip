@@ -265,7 +265,10 @@ __global__ void __launch_bounds__(256) k_forces(DevParams P, const int* __restri
 // calculateMatrixA values (2251-2335): viscous blocks, inertia, wall terms of b.
 // kBlk: also the factored form's level-0 run sums (blk, from the run starts): lane q sums
 // the -alpha r r^T (the negated blocks; 0 beyond RadiusV and for the self entry) of the
-// fluid entries in visited cell q's run, all cells at a time
+// fluid entries in visited cell q's run, all cells at a time.  There the blocks are not
+// stored and the coefficients are alpha r r^T, six of them and three divisions an entry:
+// the nine of the reference, ((((visc mu) e_s) e_r) w'/d), take fourteen, and FP64 divisions
+// bound the kernel (3.7 ms on the 1M scene, of which 180M pairs' divisions about 2).
 template <bool kBlk>
 __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __restrict__ type,
                                                   const double* __restrict__ pos, const double* __restrict__ vel,
@@ -278,13 +281,14 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
                                                   double* __restrict__ fdiag, int* __restrict__ fwrap,
                                                   const unsigned short* __restrict__ runStart,
                                                   double* __restrict__ blk) {
-    constexpr int G = kLanes, K = 12;  // terms: the 3x3 coefficients, then a wall neighbour's velocity
+    // terms: the 3x3 coefficients (kBlk: 00 01 02 11 12 22), then a wall neighbour's velocity
+    constexpr int G = kLanes, C = kBlk ? 6 : 9, K = C + 3;
     __shared__ TermRows<K> T;
     __shared__ int wall[256];  // a wall neighbour inside RadiusV
     const int g = threadIdx.x & (G - 1), grp = threadIdx.x / G;
     const int i = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) / G);
     if (i >= P.nf) return;  // the whole group
-    double s = 0.0, sv = 0.0;  // lanes 0-8: the diagonal block; lanes 0-2: the wall terms of b
+    double s = 0.0, sv = 0.0;  // lanes 0..C-1: the diagonal block; lanes 0-2: the wall terms of b
     // lane g: the runs (upper triangles) of cells g, g + G
     constexpr int R = kBlk ? (kBlkRuns + G - 1) / G : 1;
     double run[R][6];
@@ -302,7 +306,7 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
     };
     // the 3x3 blocks are stored unless aval is null (a factored scene that builds its
     // multigrid level 0 from the factored form needs none)
-    const bool blocks = aval != nullptr;
+    const bool blocks = !kBlk && aval != nullptr;
     const int nv = (2 * P.range[0] + 1) * (2 * P.range[1] + 1) * (2 * P.range[2] + 1);
     int q0[R], q1[R];
     for (int c = 0; c < R; ++c) {
@@ -317,7 +321,8 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
         const int j = jnext;
         jnext = jn + G < nc ? nInd[b0 + jn + G] : 0;
         int f = 0;
-        double t[K] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        double t[K];
+        for (int e = 0; e < K; ++e) t[e] = 0.0;
         if (jn < nc) {
             if (i == j) {
                 iN = jn;
@@ -337,19 +342,29 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
                 if (inside) {
                     const double dij = sqrt(q.r2);
                     const double wdrij = -dwq_k(P.Kv, P.m2V, dij, P.radV);
-                    const double e[3] = {q.x[0] / dij, q.x[1] / dij, q.x[2] / dij};
                     const double muij = 2.0 * (mui * muj) / (mui + muj);
-                    if (falpha) {
+                    if (kBlk || falpha) {
                         alpha = P.visc * muij * wdrij / (dij * dij * dij);
                         if (jn < nfl && !(muij == P.mu0)) atomicOr(fwrap + 1, 1);
                     }
-                    for (int r = 0; r < 3; ++r)
-                        for (int sdim = 0; sdim < 3; ++sdim)
-                            t[3 * r + sdim] = +P.visc * muij * e[sdim] * e[r] * wdrij / dij;
+                    if constexpr (kBlk) {
+                        const double ax = alpha * q.x[0], ay = alpha * q.x[1], az = alpha * q.x[2];
+                        t[0] = ax * q.x[0];
+                        t[1] = ax * q.x[1];
+                        t[2] = ax * q.x[2];
+                        t[3] = ay * q.x[1];
+                        t[4] = ay * q.x[2];
+                        t[5] = az * q.x[2];
+                    } else {
+                        const double e[3] = {q.x[0] / dij, q.x[1] / dij, q.x[2] / dij};
+                        for (int r = 0; r < 3; ++r)
+                            for (int sdim = 0; sdim < 3; ++sdim)
+                                t[3 * r + sdim] = +P.visc * muij * e[sdim] * e[r] * wdrij / dij;
+                    }
                     if (is_wall(tj)) {
-                        t[9] = vel[3 * j];
-                        t[10] = vel[3 * j + 1];
-                        t[11] = vel[3 * j + 2];
+                        t[C] = vel[3 * j];
+                        t[C + 1] = vel[3 * j + 1];
+                        t[C + 2] = vel[3 * j + 2];
                         f = 1;
                     }
                 }
@@ -363,34 +378,32 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
             }
         }
         const bool walls = __ballot(f) != 0;
-        for (int e = 0; e < 9; ++e) T.at(e) = t[e];
+        for (int e = 0; e < C; ++e) T.at(e) = t[e];
         if (walls) {
-            for (int e = 9; e < K; ++e) T.at(e) = t[e];
+            for (int e = C; e < K; ++e) T.at(e) = t[e];
             wall[threadIdx.x] = f;
         }
         wave_sync();
-        if (g < 9) s = T.add(g, s);
+        if (g < C) s = T.add(g, s);
         if (walls && g < 3) {
             const double(&c)[K][G + 2] = T.v[grp];
+            const int c0 = kBlk ? g : 3 * g, c1 = kBlk ? (g == 0 ? 1 : g + 2) : 3 * g + 1;
+            const int c2 = kBlk ? (g == 0 ? 2 : g + 3) : 3 * g + 2;
             for (int o = 0; o < G; ++o)
                 if (wall[grp * G + o]) {
-                    sv += c[3 * g][o] * c[9][o];
-                    sv += c[3 * g + 1][o] * c[10][o];
-                    sv += c[3 * g + 2][o] * c[11][o];
+                    sv += c[c0][o] * c[C][o];
+                    sv += c[c1][o] * c[C + 1][o];
+                    sv += c[c2][o] * c[C + 2][o];
                 }
         }
-        if (kBlk) {
+        if constexpr (kBlk) {
             const double(&c)[K][G + 2] = T.v[grp];
 #pragma unroll
             for (int h = 0; h < R; ++h) {
                 const int lo = q0[h] > base ? q0[h] - base : 0, hi = q1[h] < base + G ? q1[h] - base : G;
                 for (int o = lo; o < hi; ++o) {
-                    run[h][0] += -c[0][o];
-                    run[h][1] += -c[1][o];
-                    run[h][2] += -c[2][o];
-                    run[h][3] += -c[4][o];
-                    run[h][4] += -c[5][o];
-                    run[h][5] += -c[8][o];
+#pragma unroll
+                    for (int e = 0; e < 6; ++e) run[h][e] += -c[e][o];
                 }
             }
         }
@@ -409,10 +422,14 @@ __global__ void __launch_bounds__(256, 4) k_matrix_a(DevParams P, const int* __r
             o[2] = dv2{run[h][4], run[h][5]};
         }
     const double coef = mass[i] / P.V / P.dt;
-    if (g < 9) {
-        if (g % 4 == 0) s += coef;
+    if (g < C) {
+        const int r = kBlk ? (g < 3 ? 0 : g < 5 ? 1 : 2) : g / 3, c = kBlk ? (g < 3 ? g : g < 5 ? g - 2 : 2) : g % 3;
+        if (r == c) s += coef;
         if (blocks) aval[a_val_index(sb, iN, g, lane)] = s;
-        if (fdiag) fdiag[9 * (long long)i + g] = s;
+        if (fdiag) {
+            fdiag[9 * (long long)i + 3 * r + c] = s;
+            if (kBlk) fdiag[9 * (long long)i + 3 * c + r] = s;
+        }
     }
     if (g == 0) selfIdx[i] = iN;
     if (g < 3) {
