@@ -229,7 +229,8 @@ struct VCycle {
     }
     // precondition (main.cpp:4122-4266) of in -> out for the multigrid scenes in `on`;
     // the scenes of pq update q = beta q + y on the way (in = kQ)
-    void apply(const Set& on, const Set& pq, int in, int out, bool part, bool f32) {
+    // fold: those of pq whose rho and tmp the kernels fold (fold_set)
+    void apply(const Set& on, const Set& pq, const Set& fold, int in, int out, bool part, bool f32) {
         if (on.empty()) return;
         auto F = [&](int s) { return sc[s]->fuse; };  // levels F..depth-1: one workgroup
         int maxF = 0;
@@ -241,7 +242,7 @@ struct VCycle {
                 if (on.has(s) && l < F(s)) m.add(s);
             return m;
         };
-        mg_p2g_bu(T, on.m, pq.m, in, curset(on, 0));  // P2G, S = 0, R = Q, S += invD R
+        mg_p2g_bu(T, on.m, pq.m, fold.m, in, curset(on, 0));  // P2G, S = 0, R = Q, S += invD R
         const Set top = above(0);
         ru(top, 0, f32);  // pre-smooth x2
         if (!top.empty()) mg_residual(T, top.m, 0, curset(top, 0), f32);
@@ -269,12 +270,13 @@ struct VCycle {
         }
         ru(top, 0, f32);  // post-smooth x2
         ru(top, 0, f32);
-        mg_g2p(T, on.m, curset(on, 0), in, out, part);
+        mg_g2p(T, on.m, curset(on, 0), in, out, part, fold.m);
     }
 };
 
 // apply_m of mph_scene.cpp for a set of scenes: the V-cycle, or a copy without it
-void apply_m(VCycle& V, const Set& on, int in, int out, bool part, bool f32, const Set& pq = Set{}) {
+void apply_m(VCycle& V, const Set& on, int in, int out, bool part, bool f32, const Set& pq = Set{},
+             const Set& fold = Set{}) {
     Set mg, plain;
     for (int s = 0; s < (int)V.sc.size(); ++s)
         if (on.has(s)) (V.sc[s]->prm.multigrid ? mg : plain).add(s);
@@ -282,7 +284,7 @@ void apply_m(VCycle& V, const Set& on, int in, int out, bool part, bool f32, con
         copy(V.T, plain.m, in, out);
         if (part) dot_partial(V.T, plain.m, in, out);
     }
-    V.apply(mg, pq, in, out, part, f32);
+    V.apply(mg, pq, fold, in, out, part, f32);
 }
 
 void solve_prologue(const Tables& T, const std::vector<mph_scene*>& sc, const Set& all) {
@@ -309,6 +311,13 @@ void finish_levels(const VCycle& V) {
 // once and is flagged in `failed`.
 bool nonfinite(double v) { return !std::isfinite(v); }
 
+// the scenes of pq that are small enough to fold rho and tmp, and those of `on` that are not
+// or not in pq
+void fold_set(const std::vector<mph_scene*>& sc, const Set& on, const Set& pq, Set& fold, Set& wide) {
+    for (int s = 0; s < (int)sc.size(); ++s)
+        if (on.has(s)) (pq.has(s) && (sc[s]->P.nf + kChunk - 1) / kChunk <= kFoldChunks ? fold : wide).add(s);
+}
+
 // one iteration of the CR loop body (4352-4378) for the scenes of `on`: y = A s
 // (the scenes of `first` also q = y, p = s; the others update p and q), rho = s.y,
 // u = M^-1 q, tmp = q.u, x, r and s updated, then r.r and the stop test on the device
@@ -318,12 +327,14 @@ void fp64_iteration(mph_batch& B, const Tables& T, VCycle& V, const Set& on, con
     for (int s = 0; s < T.ns; ++s)
         if (on.has(s) && !first.has(s)) (V.sc[s]->prm.multigrid ? pq : rest).add(s);
     bspmv(B, T, on.m, first.m, false, 1.0, kS, 0.0, kY, kY, kQ, kP, kS);
-    dot_final(T, on.m, kRHO, kRHOP);
+    Set fold, wide;
+    fold_set(V.sc, on, pq, fold, wide);
+    dot_final(T, wide.m, kRHO, kRHOP);
     pq_update(T, rest.m);
-    apply_m(V, on, kQ, kU, true, false, pq);
-    dot_final(T, on.m, kTMP, -1);
-    xrs_update(T, on.m, pq.m, kX);
-    dot_final_stop(T, on.m, 1);
+    apply_m(V, on, kQ, kU, true, false, pq, fold);
+    dot_final(T, wide.m, kTMP, -1);
+    xrs_update(T, on.m, pq.m, fold.m, kX);
+    dot_final_stop(T, on.m, 1, fold.m);
 }
 
 // solveWithConjugatedGradient (4270-4421) for every scene of `sc` in lockstep, with
@@ -507,15 +518,16 @@ int solve_mixed(mph_batch& B, const std::vector<mph_scene*>& sc, std::vector<cha
         }
         if (!inner.empty()) {
             bspmv(B, T, inner.m, restart.m, true, 1.0, kS, 0.0, kY, kY, kQ, kP, kS);
-            dot_final(T, inner.m, kRHO, kRHOP);
-            Set plain, pq;  // as fp64_iteration
+            Set plain, pq, fold, wide;  // as fp64_iteration
             for (int s = 0; s < ns; ++s)
                 if (rest.has(s)) (sc[s]->prm.multigrid ? pq : plain).add(s);
+            fold_set(sc, inner, pq, fold, wide);
+            dot_final(T, wide.m, kRHO, kRHOP);
             pq_update(T, plain.m);
-            apply_m(V, inner, kQ, kU, true, true, pq);
-            dot_final(T, inner.m, kTMP, -1);
-            xrs_update(T, inner.m, pq.m, kD);
-            dot_final(T, inner.m, kRR, -1);
+            apply_m(V, inner, kQ, kU, true, true, pq, fold);
+            dot_final(T, wide.m, kTMP, -1);
+            xrs_update(T, inner.m, pq.m, fold.m, kD);
+            dot_final(T, inner.m, kRR, -1, fold.m);
             for (int s = 0; s < ns; ++s)
                 if (inner.has(s)) z[s].it++, z[s].total++;
         }

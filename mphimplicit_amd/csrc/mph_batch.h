@@ -85,6 +85,8 @@ struct BScene {
     long long maxit;
 };
 
+__device__ inline double* part2(const BScene& B) { return B.part + B.P.nf / kChunk + 2; }
+
 // a scene's kernels return at once after its CR loop has stopped on the device
 __device__ inline bool halted(const BScene& B) { return B.ctl && B.ctl[kCtlHalt]; }
 
@@ -123,16 +125,21 @@ struct CellRanges {
 void spmv_fac_cells(const Tables& T, const SceneSet& on, const char* shapes, const SceneSet& first, double alpha,
                     int x, double beta, int yin, int y, int y2, int p_copy);
 void dot_partial(const Tables& T, const SceneSet& on, int a, int b);
-void dot_final(const Tables& T, const SceneSet& on, int slot, int shift_slot);
+// The scenes of `fold` have rho and tmp folded by the P2G and the x update (body::dot_fold):
+// the G2P leaves tmp's partials behind rho's (part2), the P2G rho in scal[kTMP] beside the
+// previous one in scal[kRHO], and the reduction of rr moves it there.
+void dot_final(const Tables& T, const SceneSet& on, int slot, int shift_slot, const SceneSet& fold = SceneSet{});
 // r.r and the stop test per scene, as launch_dot_final_stop (BScene::ctl, tol, maxit)
-void dot_final_stop(const Tables& T, const SceneSet& on, int step);
+void dot_final_stop(const Tables& T, const SceneSet& on, int step, const SceneSet& fold = SceneSet{});
 void ctl_reset(const Tables& T, const SceneSet& on);    // ctl = 0 (before the solve's first kernel)
 void ctl_release(const Tables& T, const SceneSet& on);  // ctl[kCtlHalt] = 0 (kernels after the loop run)
 void pq_update(const Tables& T, const SceneSet& on);
-void xrs_update(const Tables& T, const SceneSet& on, const SceneSet& pq, int x);  // pq: p = beta p + s first
+void xrs_update(const Tables& T, const SceneSet& on, const SceneSet& pq, const SceneSet& fold,
+                int x);  // pq: p = beta p + s first
 void store_velocity(const Tables& T, const SceneSet& on);
 // P2G, begin, update; the scenes of pq form q = beta q + y on the way (in = kQ)
-void mg_p2g_bu(const Tables& T, const SceneSet& on, const SceneSet& pq, int in, const SceneSet& cur);
+void mg_p2g_bu(const Tables& T, const SceneSet& on, const SceneSet& pq, const SceneSet& fold, int in,
+               const SceneSet& cur);
 void mg_restrict_bu(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);  // l-1 -> l, begin, update
 void mg_begin(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);
 void mg_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);
@@ -140,7 +147,8 @@ void mg_residual(const Tables& T, const SceneSet& on, int l, const SceneSet& cur
 void mg_residual_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur, bool f32);
 void mg_restrict(const Tables& T, const SceneSet& on, int l);  // level l-1 -> l
 void mg_prolong(const Tables& T, const SceneSet& on, int l, const SceneSet& curL, const SceneSet& curS);  // l -> l-1
-void mg_g2p(const Tables& T, const SceneSet& on, const SceneSet& cur0, int in, int out, bool part);
+void mg_g2p(const Tables& T, const SceneSet& on, const SceneSet& cur0, int in, int out, bool part,
+            const SceneSet& fold);
 // levels fuse..depth-1 of each scene in one workgroup; cur: the scenes whose level
 // fuse-1 (level 0 when fuse is 0) has its ping-pong bit set; dim: of the scenes in `on`
 void mg_coarse(const Tables& T, const SceneSet& on, const SceneSet& cur, int dim);

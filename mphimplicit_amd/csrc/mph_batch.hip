@@ -98,24 +98,32 @@ __global__ void __launch_bounds__(256) kb_dot_partial(const BScene* tab, const i
     dot_partial_chunk(B.P.nf, B.vec[a], B.vec[b], B.part, lb, sh);
 }
 
+__device__ inline void shift_rho(const BScene& B) {
+    B.scal[kRHOP] = B.scal[kRHO];
+    B.scal[kRHO] = B.scal[kTMP];
+}
+
 // one workgroup per scene
 __global__ void __launch_bounds__(256) kb_dot_final(const BScene* tab, int ns, SceneSet on, int slot,
-                                                    int shift_slot) {
+                                                    int shift_slot, SceneSet fold) {
     __shared__ double sh[256];
     const int s = blockIdx.x;
     if (s >= ns || !in_set(on, s)) return;
     const BScene& B = tab[s];
     if (halted(B)) return;
+    if (in_set(fold, s) && threadIdx.x == 0) shift_rho(B);
     dot_final_body(B.part, nblk(B.P.nf, 256), B.scal, slot, shift_slot, sh);
 }
 
 // r.r and the CR stop test of each scene (k_dot_final_stop of mph_solver.hip)
-__global__ void __launch_bounds__(256) kb_dot_final_stop(const BScene* tab, int ns, SceneSet on, int step) {
+__global__ void __launch_bounds__(256) kb_dot_final_stop(const BScene* tab, int ns, SceneSet on, int step,
+                                                         SceneSet fold) {
     __shared__ double sh[256];
     const int s = blockIdx.x;
     if (s >= ns || !in_set(on, s)) return;
     const BScene& B = tab[s];
     if (halted(B)) return;
+    if (in_set(fold, s) && threadIdx.x == 0) shift_rho(B);
     dot_final_body(B.part, nblk(B.P.nf, 256), B.scal, kRR, -1, sh);
     if (threadIdx.x != 0) return;
     const double rr = B.scal[kRR];
@@ -150,10 +158,16 @@ __global__ void kb_pq_update(const BScene* tab, const int* off, int ns, SceneSet
 }
 
 __global__ void __launch_bounds__(256) kb_xrs_update(const BScene* tab, const int* off, int ns, SceneSet on,
-                                                     SceneSet pq, int x) {
-    __shared__ double sh[256];
+                                                     SceneSet pq, SceneSet fold, int x) {
+    __shared__ double sh[256], sf[257];
     MPH_SCENE(kOffChunk)
     auto coef = [&](double& alpha, double& beta) {
+        if (in_set(fold, s)) {
+            const double rho = B.scal[kTMP], rhop = B.scal[kRHO];
+            alpha = rho / dot_fold(part2(B), nblk(B.P.nf, kChunk), sf);
+            beta = rho / rhop;
+            return;
+        }
         alpha = B.scal[kRHO] / B.scal[kTMP];
         beta = in_set(pq, s) ? B.scal[kRHO] / B.scal[kRHOP] : 0.0;
     };
@@ -180,12 +194,17 @@ __device__ inline Level level(const BScene& B, int l, const SceneSet& cur, int s
 }
 
 __global__ void __launch_bounds__(256) kb_mg_p2g_bu(const BScene* tab, const int* off, int ns, SceneSet on,
-                                                    SceneSet pq, int in, SceneSet cur) {
-    __shared__ double tb[256 * kP2gK];
+                                                    SceneSet pq, SceneSet fold, int in, SceneSet cur) {
+    __shared__ double tb[256 * kP2gK], sf[257];
     MPH_SCENE(kOffP2g)
     const Level L = level(B, 0, cur, s);
     const bool f = in_set(pq, s);
-    auto beta = [&] { return B.scal[kRHO] / B.scal[kRHOP]; };
+    auto beta = [&] {
+        if (!in_set(fold, s)) return B.scal[kRHO] / B.scal[kRHOP];
+        const double v = dot_fold(B.part, nblk(B.P.nf, kChunk), sf);
+        if (lb == 0 && threadIdx.x == 0) B.scal[kTMP] = v;  // read by later launches only
+        return v / B.scal[kRHO];
+    };
 #define MPH_P2G(PQ, ORD) mg_p2g_lanes<PQ, ORD>(B.P, L, B.cellStart, B.vec[in], B.vec[kY], beta, lb, tb)
     if (L.ordered) {
         if (f) MPH_P2G(true, true);
@@ -268,11 +287,12 @@ __global__ void kb_mg_prolong(const BScene* tab, const int* off, int ns, SceneSe
 }
 
 __global__ void __launch_bounds__(256) kb_mg_g2p(const BScene* tab, const int* off, int ns, SceneSet on,
-                                                 SceneSet cur0, int in, int out, int part) {
+                                                 SceneSet cur0, int in, int out, int part, SceneSet fold) {
     __shared__ double sh[256];
     MPH_SCENE(kOffChunk)
     const Level L = level(B, 0, cur0, s);
-    mg_g2p_chunk(B.P, L, B.cellIndex, B.invDiagA, B.vec[in], B.vec[out], part ? B.part : nullptr, lb, sh);
+    mg_g2p_chunk(B.P, L, B.cellIndex, B.invDiagA, B.vec[in], B.vec[out],
+                 part ? (in_set(fold, s) ? part2(B) : B.part) : nullptr, lb, sh);
 }
 
 // levels fuse..depth-1 of each scene in its own workgroup (mg_coarse_cycle; 2D and 3D
@@ -364,13 +384,13 @@ void spmv_fac(const Tables& T, const SceneSet& all, const SceneSet& first, const
     if (dot >= 0) MPH_LAUNCH(kb_dot_partial, kOffChunk, dot, y);
 }
 void dot_partial(const Tables& T, const SceneSet& on, int a, int b) { MPH_LAUNCH(kb_dot_partial, kOffChunk, a, b); }
-void dot_final(const Tables& T, const SceneSet& on, int slot, int shift_slot) {
+void dot_final(const Tables& T, const SceneSet& on, int slot, int shift_slot, const SceneSet& fold) {
     if (T.ns > 0 && any(on))
-        hipLaunchKernelGGL(kb_dot_final, dim3(T.ns), dim3(256), 0, T.st, T.tab, T.ns, on, slot, shift_slot);
+        hipLaunchKernelGGL(kb_dot_final, dim3(T.ns), dim3(256), 0, T.st, T.tab, T.ns, on, slot, shift_slot, fold);
 }
-void dot_final_stop(const Tables& T, const SceneSet& on, int step) {
+void dot_final_stop(const Tables& T, const SceneSet& on, int step, const SceneSet& fold) {
     if (T.ns > 0 && any(on))
-        hipLaunchKernelGGL(kb_dot_final_stop, dim3(T.ns), dim3(256), 0, T.st, T.tab, T.ns, on, step);
+        hipLaunchKernelGGL(kb_dot_final_stop, dim3(T.ns), dim3(256), 0, T.st, T.tab, T.ns, on, step, fold);
 }
 void ctl_reset(const Tables& T, const SceneSet& on) {
     if (T.ns > 0 && any(on)) hipLaunchKernelGGL(kb_ctl, dim3(T.ns), dim3(64), 0, T.st, T.tab, T.ns, on, 0);
@@ -382,16 +402,17 @@ void pq_update(const Tables& T, const SceneSet& on) {
     const int g = T.blocks(kOffElem);
     if (g > 0 && any(on)) hipLaunchKernelGGL(kb_pq_update, dim3(g), dim3(256), 0, T.st, T.tab, T.off, T.ns, on);
 }
-void xrs_update(const Tables& T, const SceneSet& on, const SceneSet& pq, int x) {
-    MPH_LAUNCH(kb_xrs_update, kOffChunk, pq, x);
+void xrs_update(const Tables& T, const SceneSet& on, const SceneSet& pq, const SceneSet& fold, int x) {
+    MPH_LAUNCH(kb_xrs_update, kOffChunk, pq, fold, x);
 }
 void store_velocity(const Tables& T, const SceneSet& on) {
     const int g = T.blocks(kOffElem);
     if (g > 0 && any(on))
         hipLaunchKernelGGL(kb_store_velocity, dim3(g), dim3(256), 0, T.st, T.tab, T.off, T.ns, on);
 }
-void mg_p2g_bu(const Tables& T, const SceneSet& on, const SceneSet& pq, int in, const SceneSet& cur) {
-    MPH_LAUNCH(kb_mg_p2g_bu, kOffP2g, pq, in, cur);
+void mg_p2g_bu(const Tables& T, const SceneSet& on, const SceneSet& pq, const SceneSet& fold, int in,
+               const SceneSet& cur) {
+    MPH_LAUNCH(kb_mg_p2g_bu, kOffP2g, pq, fold, in, cur);
 }
 void mg_restrict_bu(const Tables& T, const SceneSet& on, int l, const SceneSet& cur) {
     MPH_LAUNCH(kb_mg_restrict_bu, kOffLevel + l, l, cur);
@@ -412,8 +433,9 @@ void mg_restrict(const Tables& T, const SceneSet& on, int l) { MPH_LAUNCH(kb_mg_
 void mg_prolong(const Tables& T, const SceneSet& on, int l, const SceneSet& curL, const SceneSet& curS) {
     MPH_LAUNCH(kb_mg_prolong, kOffLevel + l - 1, l, curL, curS);
 }
-void mg_g2p(const Tables& T, const SceneSet& on, const SceneSet& cur0, int in, int out, bool part) {
-    MPH_LAUNCH(kb_mg_g2p, kOffChunk, cur0, in, out, part ? 1 : 0);
+void mg_g2p(const Tables& T, const SceneSet& on, const SceneSet& cur0, int in, int out, bool part,
+            const SceneSet& fold) {
+    MPH_LAUNCH(kb_mg_g2p, kOffChunk, cur0, in, out, part ? 1 : 0, fold);
 }
 
 void mg_coarse(const Tables& T, const SceneSet& on, const SceneSet& cur, int dim) {
