@@ -237,9 +237,9 @@ def run_gpu(args, precision="fp64", form=None):
         k32 = "k_spmv (particle matrix, sliced 3x3 blocks, FP32 values)"
     rf64 = roofline(k64, scene.scalar("SpmvMs"), l64_prev, b64, r64, traffic if precision == "fp64" else None)
     if factored:
-        rf64["note"] = ("the factored product moves ~2.8 GB of algorithmic HBM bytes where the assembled one moves "
-                        "13.2 GB; its limit is the cache traffic of gathering neighbours' x, position and t "
-                        "(three 16-byte pairs per entry) through L2 and the Infinity Cache, not HBM")
+        rf64["note"] = ("the factored product moves 0.7 GB of algorithmic HBM bytes where the assembled one moves "
+                        "13.2 GB; its limit is the FP64 issue (52% of the staged pass), the LDS reads and the waits of "
+                        "180M staged entries, not HBM")
     rf32 = roofline(k32, scene.scalar("SpmvMsF32"), l32_prev, b32, r32, None)
     for rf in (rf64, rf32):
         rf["measured_over"] = ("%d steps after the timed ones, every product bracketed by HIP events on the scene "
