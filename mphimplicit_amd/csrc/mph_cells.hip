@@ -3,7 +3,7 @@
 // Replaces calculateCellParticle (source/main.cpp:1164-1379) and calculateNeighbor
 // (1382-1667).  The particle order is the reference's bitonic network, emulated
 // exactly (it is not stable, so a radix sort would order ties differently): the
-// passes with distance < 2048 run inside LDS, the wider ones as global passes.
+// passes with distance < 8192 run inside a workgroup, the wider ones as global passes.
 // Neighbour lists come out ascending (fluid block, then wall block) because the
 // 27 (9 in 2D) cells are visited in ascending CellId, as in the reference.
 #include "mph_kernels.h"
@@ -12,8 +12,8 @@ namespace mph {
 
 namespace {
 
-constexpr int kSortBlock = 2048;  // keys per LDS block (16 KiB)
-constexpr int kSortThreads = 256;
+constexpr int kSortBlock = 8192;  // keys per workgroup (64 KB of LDS)
+constexpr int kSortThreads = 1024;
 constexpr int kScanShare = 32768;  // particles from which four share a wavefront of the neighbour search
 
 __device__ inline int cell_id(const DevParams& P, int cx, int cy, int cz) {  // CellId, main.cpp:109-113
@@ -54,43 +54,83 @@ __device__ inline int pair_lo(int t, int logd) {  // t-th pair (lo index) at dis
     return ((t >> logd) << (logd + 1)) | (t & ((1 << logd) - 1));
 }
 
-// all stages iMain < log2(n) inside one LDS block of n keys
-__global__ void __launch_bounds__(kSortThreads) k_bitonic_block_sort(uint64_t* keys, int n, int logn) {
-    __shared__ uint64_t sh[kSortBlock];
-    const int base = blockIdx.x * n;
-    for (int k = threadIdx.x; k < n; k += blockDim.x) sh[k] = keys[base + k];
-    __syncthreads();
-    for (int iMain = 0; iMain < logn; ++iMain) {
-        for (int iSub = 0; iSub <= iMain; ++iSub) {
-            const int logd = iMain - iSub;
-            for (int t = threadIdx.x; t < (n >> 1); t += blockDim.x) {
-                const int lo = pair_lo(t, logd);
-                const int gi = base + lo;
-                const bool up = ((gi >> iMain) & 2) == 0;
-                cmp_swap(sh[lo], sh[lo | (1 << logd)], up);
-            }
-            __syncthreads();
-        }
-    }
-    for (int k = threadIdx.x; k < n; k += blockDim.x) keys[base + k] = sh[k];
+// A block of n <= kSortBlock keys lives in registers, eight consecutive keys per thread: a
+// pass at distance 1, 2 or 4 stays inside a thread, at 8 to 256 inside a wavefront (DPP and
+// shuffles) and only from 512 on goes through LDS (10 of the 91 passes of 8192 keys).  The issue
+// of one CU bounds it: 36 us for 4096 keys, 60 for 8192, 16 per merge.  With every pass in LDS,
+// blocks of 2048 keys took 40 us and 10 per merge, and the passes from 2048 on a launch each: 36
+// launches per sort of the 64k drop, now 21.  Blocks of 2048 keys in registers take 29 and 8 us,
+// but their launches cost the smaller scenes more (batch of 12 scenes 20.3 against 19.6 ms).
+constexpr int kSortKeys = kSortBlock / kSortThreads;
+static_assert(kSortKeys == 8, "three distances inside a thread, six inside a wavefront");
+
+// the compare-exchange of all keys of a thread at distance 2^L < kSortKeys; gi: its first index
+template <int L>
+__device__ inline void pass_thread(uint64_t (&v)[kSortKeys], int gi, int iMain) {
+#pragma unroll
+    for (int k = 0; k < kSortKeys; ++k)
+        if (!(k & (1 << L))) cmp_swap(v[k], v[k | (1 << L)], (((gi + k) >> iMain) & 2) == 0);
 }
 
-// the passes of stage iMain with distance < n, inside one LDS block
-__global__ void __launch_bounds__(kSortThreads) k_bitonic_block_merge(uint64_t* keys, int n, int logn, int iMain) {
-    __shared__ uint64_t sh[kSortBlock];
-    const int base = blockIdx.x * n;
-    for (int k = threadIdx.x; k < n; k += blockDim.x) sh[k] = keys[base + k];
-    __syncthreads();
-    for (int logd = logn - 1; logd >= 0; --logd) {
-        for (int t = threadIdx.x; t < (n >> 1); t += blockDim.x) {
-            const int lo = pair_lo(t, logd);
-            const int gi = base + lo;
-            const bool up = ((gi >> iMain) & 2) == 0;
-            cmp_swap(sh[lo], sh[lo | (1 << logd)], up);
-        }
+// another lane's key without LDS: quad_perm [1,0,3,2] (0xB1, lane ^ 1) and [2,3,0,1] (0x4E,
+// lane ^ 2), row_ror:8 (0x128, lane ^ 8 within a row of 16)
+template <int kCtl>
+__device__ inline uint64_t lane_dpp(uint64_t v) {
+    const int lo = (int)(uint32_t)v, hi = (int)(uint32_t)(v >> 32);
+    const uint32_t a = (uint32_t)__builtin_amdgcn_update_dpp(lo, lo, kCtl, 0xf, 0xf, false);
+    const uint32_t b = (uint32_t)__builtin_amdgcn_update_dpp(hi, hi, kCtl, 0xf, 0xf, false);
+    return ((uint64_t)b << 32) | a;
+}
+
+// the pass of stage iMain at distance 2^logd < n; every thread of the workgroup calls it
+__device__ inline void block_pass(uint64_t (&v)[kSortKeys], int gi, int logd, int iMain, uint64_t* sh) {
+    if (logd == 0) return pass_thread<0>(v, gi, iMain);
+    if (logd == 1) return pass_thread<1>(v, gi, iMain);
+    if (logd == 2) return pass_thread<2>(v, gi, iMain);
+    const int t = threadIdx.x, td = 1 << (logd - 3);  // the partner is thread t ^ td
+    uint64_t o[kSortKeys];
+    if (td == 1) {
+#pragma unroll
+        for (int k = 0; k < kSortKeys; ++k) o[k] = lane_dpp<0xB1>(v[k]);
+    } else if (td == 2) {
+#pragma unroll
+        for (int k = 0; k < kSortKeys; ++k) o[k] = lane_dpp<0x4E>(v[k]);
+    } else if (td == 8) {
+#pragma unroll
+        for (int k = 0; k < kSortKeys; ++k) o[k] = lane_dpp<0x128>(v[k]);
+    } else if (td < 64) {
+#pragma unroll
+        for (int k = 0; k < kSortKeys; ++k) o[k] = __shfl_xor((unsigned long long)v[k], td, 64);
+    } else {
+        __syncthreads();  // the previous pass through LDS has been read
+#pragma unroll
+        for (int k = 0; k < kSortKeys; ++k) sh[k * kSortThreads + t] = v[k];
         __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kSortKeys; ++k) o[k] = sh[k * kSortThreads + (t ^ td)];
     }
-    for (int k = threadIdx.x; k < n; k += blockDim.x) keys[base + k] = sh[k];
+    const bool lo = !(t & td), up = ((gi >> iMain) & 2) == 0;
+#pragma unroll
+    for (int k = 0; k < kSortKeys; ++k) {
+        const uint32_t a = (uint32_t)((lo ? v[k] : o[k]) >> 32), b = (uint32_t)((lo ? o[k] : v[k]) >> 32);
+        if ((a > b) == up) v[k] = o[k];
+    }
+}
+
+// kMerge: the passes of stage iMain0 with distance < n; else all stages below log2(n).  Keys
+// past n (small sorts) take part in no exchange with the others: n is a power of two.
+template <bool kMerge>
+__global__ void __launch_bounds__(kSortThreads) k_bitonic_block(uint64_t* keys, int n, int logn, int iMain0) {
+    __shared__ uint64_t sh[kSortBlock];
+    const int base = blockIdx.x * n, at = kSortKeys * threadIdx.x, gi = base + at;
+    uint64_t v[kSortKeys];
+#pragma unroll
+    for (int k = 0; k < kSortKeys; ++k) v[k] = at + k < n ? keys[gi + k] : 0;
+    for (int iMain = kMerge ? iMain0 : 0; iMain < (kMerge ? iMain0 + 1 : logn); ++iMain)
+        for (int logd = kMerge ? logn - 1 : iMain; logd >= 0; --logd) block_pass(v, gi, logd, iMain, sh);
+#pragma unroll
+    for (int k = 0; k < kSortKeys; ++k)
+        if (at + k < n) keys[gi + k] = v[k];
 }
 
 // one pass at distance 2^logd >= block size
@@ -443,13 +483,13 @@ void launch_bitonic(hipStream_t st, const DevParams& P, uint64_t* keys) {
     const int n = P.p2 < kSortBlock ? P.p2 : kSortBlock;
     int logn = 0;
     while ((1 << logn) < n) ++logn;
-    const int nb = P.p2 / n;
-    hipLaunchKernelGGL(k_bitonic_block_sort, dim3(nb), dim3(kSortThreads), 0, st, keys, n, logn);
+    const int nb = P.p2 / n, nt = n / kSortKeys < 64 ? 64 : n / kSortKeys;
+    hipLaunchKernelGGL(k_bitonic_block<false>, dim3(nb), dim3(nt), 0, st, keys, n, logn, 0);
     for (int iMain = logn; iMain < P.p2pow; ++iMain) {
         for (int logd = iMain; logd >= logn; --logd)
             hipLaunchKernelGGL(k_bitonic_global, dim3(nblk(P.p2 / 2, 256)), dim3(256), 0, st, keys, P.p2 / 2, logd,
                                iMain);
-        hipLaunchKernelGGL(k_bitonic_block_merge, dim3(nb), dim3(kSortThreads), 0, st, keys, n, logn, iMain);
+        hipLaunchKernelGGL(k_bitonic_block<true>, dim3(nb), dim3(nt), 0, st, keys, n, logn, iMain);
     }
 }
 
