@@ -384,10 +384,11 @@ __device__ inline void mg_sweep_lanes(const Level& L, const Level& U, long long 
 }
 
 // The residual of S (mg_residual_row), its restriction into L (mg_restrict_row), then
-// begin and update of L: a group of 4 lanes per child (8, in 2D 4 children) forms a
-// coarse row's fine residuals, which are added in child order; a clipped child adds a
-// zero, which changes no bit.  S.R is read by nothing else then and is not written.  One
-// launch in the place of two of 3.8 and 4.6 us on the 64k drop.
+// begin and update of L: a group of 4 lanes per child (8 children, 4 where S is one cell
+// deep in z, as in 2D) forms a coarse row's fine residuals, which are added in child
+// order; a clipped child adds a zero, which changes no bit.  S.R is read by nothing else
+// then and is not written.  One launch in the place of two of 3.8 and 4.6 us on the 64k
+// drop.
 template <int C0, int C2>
 __host__ __device__ constexpr int restrict_lanes() { return kRowLanes * (C0 && C2 == 1 ? 4 : 8); }
 template <class VT, bool kOrd, int C0, int C1, int C2>
@@ -398,7 +399,8 @@ __device__ inline void mg_residual_restrict_lanes(const Level& S, const Level& L
     int lx = 0, ly = 0, lz = 0;
     if (own) grid_xyz(L, lrow / 3, lx, ly, lz);
     const int fx = 2 * (lx + L.mn[0]) + c / (2 * KZ) - S.mn[0], fy = 2 * (ly + L.mn[1]) + (c / KZ) % 2 - S.mn[1];
-    const int fz = 2 * (lz + L.mn[2]) + c % KZ - S.mn[2];
+    // KZ = 1: S is one cell deep in z, and that cell may be the coarse cell's second
+    const int fz = KZ == 1 ? 0 : 2 * (lz + L.mn[2]) + c % KZ - S.mn[2];
     const bool on = own && fx >= 0 && fx < S.cnt[0] && fy >= 0 && fy < S.cnt[1] && fz >= 0 && fz < S.cnt[2];
     const int row = on ? 3 * grid_id(S, fx, fy, fz) + rd : 0;
     const double q = on ? S.Q[row] : 0.0;
