@@ -184,9 +184,11 @@ int mph_scene_run_phase(mph_scene* s, int phase);
  * form only when its multigrid level 0 spans fewer than 3 cells along an axis,
  * otherwise level 0 and InvDiagA come from the factored scalars and CsrCofA is not
  * available), FactoredCellsUsed (1 when the FP64 second pass of the factored
- * product runs staged per cell, option FactoredCells), and NeighborOneScan (1 when
- * the last neighbour search built the lists in one scan, 0 when it ran the count and
- * fill passes: a scene's first search, or a list longer than the last search's
+ * product runs staged per cell with the last assembled matrix; 0 before there is
+ * one, and where the scene or option FactoredCells has it run as the chunk kernel),
+ * and NeighborOneScan (1 when the last neighbour search built the lists in one scan,
+ * 0 when it ran the count and fill passes: a scene's first search, or a list longer
+ * than the last search's
  * largest plus a margin; the lists are the same either way, alone or in a batch). */
 int mph_scene_field_size(mph_scene* s, const char* field, size_t* bytes, int* elem_bytes);
 int mph_scene_read(mph_scene* s, const char* field, void* host, size_t bytes);

@@ -1656,7 +1656,7 @@ int mph_scene_scalar(mph_scene* S, const char* name, double* v) {
     else if (n == "TunedCac") *v = 0;  // one variant
     else if (n == "TunedFuse") *v = 0;  // one variant: the levels that fit one workgroup are fused
     else if (n == "TunedGalerkin") *v = S->tuneGal.best;
-    else if (n == "FactoredCellsUsed") *v = factored(*S) && fac_cells(*S) ? 1.0 : 0.0;
+    else if (n == "FactoredCellsUsed") *v = factored(*S) && fac_cells(*S) && S->fslotValid ? 1.0 : 0.0;
     else if (n == "FactoredBytes" || n == "FactoredBytesF32") {
         // algorithmic bytes of one factored product, every array read or written once:
         // per list entry a column and the stored value (FP64: alpha or beta, 8 B;

@@ -1,0 +1,80 @@
+"""When the factored product's second pass runs staged per cell (GPU).
+
+FactoredCellsUsed tells which kernel the last assembled matrix has its FP64 second pass
+run as; either gives the same bits.  The cells take part only once the rows' staged
+places have been built, so switching the option on afterwards leaves the chunk kernel in
+place until the next step.  A cell whose visited cells hold more records than the staging
+does has its rows gathered inside the cell kernel.
+"""
+import numpy as np
+import pytest
+
+from mphimplicit_amd import abi, scenes
+from mphimplicit_amd.scene import Scene
+from test_gpu_coarse import L0, pool
+
+pytestmark = pytest.mark.gpu
+
+
+def assembled(p, g, cells):
+    """The scene with its matrix assembled, and a product."""
+    p.operator_form = abi.OPERATOR_FACTORED
+    s = Scene(p, g)
+    s.set_option("FactoredCells", cells)
+    for ph in range(abi.PHASE_KINEMATICS, abi.PHASE_MULTIPLY_C + 1):
+        s.run_phase(ph)
+    return s, product(s)
+
+
+def product(s):
+    x = np.random.default_rng(3).standard_normal(3 * int(s.scalar("FluidCount")))
+    return s.apply_matrix(x).view(np.int64)
+
+
+@pytest.mark.parametrize("n", [(23, 17), (13, 11, 9)], ids=lambda n: "x".join(map(str, n)))
+def test_cells_used(n):
+    print("[faccells] %s" % (n,), flush=True)
+    p, g = pool(n)
+    p.operator_form = abi.OPERATOR_FACTORED
+    p.end_time = 1.0e9
+    with Scene(p, g) as s:
+        assert s.scalar("FactoredCellsUsed") == 0  # no matrix yet
+        s.step(1)
+        assert s.scalar("FactoredCellsUsed") == 1
+        y = product(s)
+        s.set_option("FactoredCells", 0)
+        assert s.scalar("FactoredCellsUsed") == 0
+        assert np.array_equal(product(s), y)
+        s.step(1)
+        s.set_option("FactoredCells", 1)  # this matrix has no staged places
+        assert s.scalar("FactoredCellsUsed") == 0
+        y = product(s)
+        s.step(1)
+        assert s.scalar("FactoredCellsUsed") == 1
+    p.operator_form = abi.OPERATOR_ASSEMBLED
+    with Scene(p, g) as s:
+        s.step(1)
+        assert s.scalar("FactoredCellsUsed") == 0
+
+
+def wide(n, radius):
+    """A pool with a larger MaxRadius, in spacings, in a domain to match."""
+    p, g = pool(n)
+    p.radius_ratio_a = p.radius_ratio_v = radius
+    for d in range(len(n)):  # cells a little wider than the radius
+        w = g.domain_max[d] - g.domain_min[d]
+        g.domain_max[d] = g.domain_min[d] + np.ceil(w / (radius * L0)) * (radius + 0.1) * L0
+    return p, g
+
+
+# 9 cells of 8 spacings hold 576 particles and more, 27 cells of 5.5 hold 4492
+@pytest.mark.parametrize("n,radius", [((60, 50), 8.0), ((20, 19, 18), 5.5)], ids=["2d", "3d"])
+def test_more_records_than_staged(n, radius):
+    print("[faccells] %s radius %g" % (n, radius), flush=True)
+    out = []
+    for cells in (0, 1):
+        s, y = assembled(*wide(n, radius), cells)
+        with s:
+            assert s.scalar("FactoredCellsUsed") == cells
+        out.append(y)
+    assert np.array_equal(*out)
