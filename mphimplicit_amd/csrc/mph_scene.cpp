@@ -367,6 +367,31 @@ int phase_matrix_a(mph_scene& S) {
     return MPH_OK;
 }
 
+// The buffers of the cell-staged second pass, allocated if need be.  False where they
+// would take more than the pass is worth, or the allocation failed: they are optional,
+// the chunk kernel runs without them.  A row's places take as many blocks as the longest
+// row, so a clump of particles pads every row; a descriptor stands for every cell of the
+// bounding box, empty or not, so fluid that is scattered over a large domain has mostly
+// those of empty cells.  Either may take twice the bytes of the neighbour lists and 8 MiB.
+// (Pools take 0.5 to 1 times the lists for the places and 0.02 to 0.4 for the descriptors.
+// Sprays of 15% and 35% of a lattice are within the bound too; there a product takes 59 and
+// 62 us in cells, 89 and 87 when the cells staged through a table.)
+constexpr long long kCellSpare = 2 << 20;  // 4-byte words
+bool cell_places(mph_scene& S) {
+    const long long blk = 8 * kFacLanes, row = blk * ((S.hmaxW + blk - 1) / blk), cells = fac_bbox_cells(S);
+    const long long words = 2 * S.E + kCellSpare;
+    if (cells <= 0 || kFacDesc * cells > words || row * S.P.nf > 2 * words) return false;
+    if (S.fslot.ensure((size_t)(row * S.P.nf)) == MPH_OK && S.fdesc.ensure((size_t)(kFacDesc * cells)) == MPH_OK) {
+        S.fslotRow = (int)row;
+        return true;
+    }
+    (void)hipGetLastError();  // as search_scratch
+    S.fslot.release();
+    S.fdesc.release();
+    g_err.clear();
+    return false;
+}
+
 int phase_matrix_c(mph_scene& S) {
     int rc;
     // D = C Lambda is read only by C Lambda C^T, which a scene without blocks skips
@@ -391,14 +416,8 @@ int phase_matrix_c(mph_scene& S) {
         if (mixed(S))  // alpha was written by the matrix-A phase
             launch_fac_u(S.st, S.P, S.nFluid.p, S.nPtr.p, S.nInd.p, S.falpha.p, S.pos.p, S.fu32.p);
         // the cells' descriptors and the rows' staged places for the cell-staged FP64 pass
-        // (a scene alone and in a batch).  A row's places take as many blocks as the
-        // longest row: where that is far above the mean (a clump of particles), the pass
-        // is left to the chunk kernel
-        const long long blk = 8 * kFacLanes, row = blk * ((S.hmaxW + blk - 1) / blk), cells = fac_bbox_cells(S);
-        if (fac_cells(S) && row * S.P.nf <= 4 * S.E + (64 << 20) && cells > 0) {
-            if ((rc = S.fslot.ensure((size_t)(row * S.P.nf))) || (rc = S.fdesc.ensure((size_t)(kFacDesc * cells))))
-                return rc;
-            S.fslotRow = (int)row;
+        // (a scene alone and in a batch)
+        if (fac_cells(S) && cell_places(S)) {
             S.fslotValid = true;
             launch_fac_slots(S.st, S.P, fac_op(S, false));
         }

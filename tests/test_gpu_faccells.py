@@ -78,3 +78,42 @@ def test_more_records_than_staged(n, radius):
             assert s.scalar("FactoredCellsUsed") == cells
         out.append(y)
     assert np.array_equal(*out)
+
+
+def two_drops(n):
+    """Two drops at opposite corners of a domain of n cells per axis."""
+    side = 3.6 * n
+    at = [2.0, side - 8.0]
+    fluid = np.concatenate([scenes.lattice([a] * 3, [a + 6] * 3, L0, 3) for a in at])
+    walls = scenes.lattice([0, 0, 0], [4, 4, 2], L0, 3)
+    g = scenes.assemble(fluid, walls, 0.0, L0, [0.0] * 3, [side * L0] * 3, 5, 3)
+    p = scenes.base_params(3, 0.1, (0.0, 0.0, -9.8), 5.0e-4, 4)
+    p.multigrid = 0
+    return p, g
+
+
+def clump(n):
+    """n^3 particles two spacings apart, and 384 in one place."""
+    grid = scenes.lattice([0] * 3, [n] * 3, 2 * L0, 3)
+    u = np.stack(np.meshgrid(np.arange(8), np.arange(8), np.arange(6), indexing="ij"), axis=-1).reshape(-1, 3)
+    fluid = np.concatenate([grid, (n + 0.13 + 0.25 * u) * L0])
+    walls = scenes.lattice([0, 0, -4], [4, 4, -2], L0, 3)
+    g = scenes.assemble(fluid, walls, 0.0, L0, [-0.09] * 3, [(2 * n + 9.5) * L0] * 3, 5, 3, jitter=0)
+    return scenes.base_params(3, 0.1, (0.0, 0.0, -9.8), 5.0e-4, 4), g
+
+
+@pytest.mark.parametrize("make", [lambda: two_drops(100), lambda: clump(28)], ids=["two_drops", "clump"])
+def test_places_not_worth_their_memory(make):
+    """A million cells for 432 particles, one long row among 22 thousand: the chunk kernel,
+    and no buffers for the cells."""
+    p, g = make()
+    print("[faccells] np=%d" % g.np, flush=True)
+    out = []
+    for cells in (0, 1):
+        s, y = assembled(p, g, cells)
+        with s:
+            assert s.scalar("FactoredCellsUsed") == 0
+            out.append((y, s.device_bytes()))
+    assert np.array_equal(out[0][0], out[1][0])
+    assert np.isfinite(out[0][0].view(np.float64)).all()
+    assert out[0][1] == out[1][1]
