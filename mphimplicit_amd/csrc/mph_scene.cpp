@@ -668,10 +668,12 @@ FacOp fac_op(mph_scene& S, bool f32) {
         F.cellLo[d] = S.hbbox[3 + d];
         F.cellCnt[d] = cells ? S.hbbox[d] - S.hbbox[3 + d] + 1 : 0;
     }
-    // the records of 3x3x3 cells of a lattice decide how many are staged
+    // the records of a lattice in the visited cells decide how many are staged
     double most = 1;
-    for (int d = 0; d < 3; ++d) most *= std::ceil(3.0 * S.P.cw[d] / S.P.l);
-    F.cellShape = S.P.dim == 2 ? kFacCell2D : most <= kFacCellSlots[kFacCell3D] ? kFacCell3D : kFacCell3DWide;
+    for (int d = 0; d < S.P.dim; ++d) most *= std::ceil(3.0 * S.P.cw[d] / S.P.l);
+    F.cellShape = S.P.dim == 2 && most <= kFacCellSlots[kFacCell2D] ? kFacCell2D
+                  : most <= kFacCellSlots[kFacCell3D]               ? kFacCell3D
+                                                                    : kFacCell3DWide;
     return F;
 }
 

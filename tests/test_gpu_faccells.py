@@ -67,9 +67,12 @@ def wide(n, radius):
     return p, g
 
 
-# 9 cells of 8 spacings hold 576 particles and more, 27 cells of 5.5 hold 4492
-@pytest.mark.parametrize("n,radius", [((60, 50), 8.0), ((20, 19, 18), 5.5)], ids=["2d", "3d"])
-def test_more_records_than_staged(n, radius):
+# The launch shape follows the particles that a lattice has in the visited cells: up to 256
+# in 2D, up to 1408, and beyond.  9 cells of 5.5 spacings hold 273 and more, of 8 spacings
+# 576; of 18 spacings 2916, and 27 of 5.5 hold 4492, more than the largest staging (2816)
+@pytest.mark.parametrize("n,radius", [((30, 31), 5.0), ((60, 50), 5.5), ((60, 50), 8.0), ((70, 60), 13.0),
+                                      ((70, 60), 18.0), ((20, 19, 18), 5.5)], ids=str)
+def test_large_radii(n, radius):
     print("[faccells] %s radius %g" % (n, radius), flush=True)
     out = []
     for cells in (0, 1):
