@@ -145,16 +145,19 @@ constexpr int kFacLanes = 8;
 constexpr int kFacRowsT = 64, kFacRowsY = 32;
 // launch shapes of the cell-staged pass: threads per workgroup and staged records (56
 // bytes of LDS each).  The particles that a lattice has in the visited cells decide (fac_op).
-// 3D: 1408 records let two workgroups share a CU (27 cells of 3.51 spacings hold at most
-// 11^3 = 1331 lattice particles); domains of few cells have wider ones and take 2816, one
-// workgroup per CU.  2D: a cell holds about 12 rows and its 9 visited cells 110-144 records,
+// 3D: 1456 records (81,536 bytes) are the most that let two workgroups share a CU: 27 cells
+// of 3.51 spacings hold at most 11^3 = 1331 lattice particles, with one axis of up to 4
+// spacings 12 11 11 = 1452.  Domains of few cells have wider ones and take 2816, one
+// workgroup per CU.  (With 1408 a film of 150 x 150 x 3, whose cells are 3.86 spacings deep,
+// took the large shape: 78 us per product, now 63; a 34 x 38 x 42 pool 73, now 59.)  2D: a
+// cell holds about 12 rows and its 9 visited cells 110-144 records,
 // so 128 threads and 256 records keep many workgroups on a CU.  2D radii of more than 5
 // spacings have larger cells and take the 3D shapes: with 256 records their rows would be
 // gathered (us per product at radius 6, 8 and 12 spacings, 12k, 10k and 3.6k particles: 39,
 // 57 and 146 gathered, 29, 31 and 52 staged; 75 and 59 at radius 6 and 90k).
 enum { kFacCell3D = 0, kFacCell3DWide = 1, kFacCell2D = 2, kFacCellShapes = 3 };
 constexpr int kFacCellThreads[kFacCellShapes] = {512, 512, 128};
-constexpr int kFacCellSlots[kFacCellShapes] = {1408, 2816, 256};
+constexpr int kFacCellSlots[kFacCellShapes] = {1456, 2816, 256};
 
 constexpr int kSlice = 64;    // particles per A slice (one wavefront)
 

@@ -68,15 +68,16 @@ def wide(n, radius):
 
 
 # The launch shape follows the particles that a lattice has in the visited cells: up to 256
-# in 2D, up to 1408, and beyond.  9 cells of 5.5 spacings hold 273 and more, of 8 spacings
-# 576; of 18 spacings 2916, and 27 of 5.5 hold 4492, more than the largest staging (2816)
+# in 2D, up to 1456, and beyond.  9 cells of 5.5 spacings hold 273 and more, of 8 spacings
+# 576; of 18 spacings 2916, and 27 of 5.5 hold 4492, more than the largest staging (2816).
+# A pool 3 deep has cells of 3.86 spacings in z: 11 x 11 x 12 of a lattice
 @pytest.mark.parametrize("n,radius", [((30, 31), 5.0), ((60, 50), 5.5), ((60, 50), 8.0), ((70, 60), 13.0),
-                                      ((70, 60), 18.0), ((20, 19, 18), 5.5)], ids=str)
+                                      ((70, 60), 18.0), ((20, 19, 18), 5.5), ((38, 32, 3), 3.5)], ids=str)
 def test_large_radii(n, radius):
     print("[faccells] %s radius %g" % (n, radius), flush=True)
     out = []
     for cells in (0, 1):
-        s, y = assembled(*wide(n, radius), cells)
+        s, y = assembled(*(wide(n, radius) if radius > 3.5 else pool(n)), cells)
         with s:
             assert s.scalar("FactoredCellsUsed") == cells
         out.append(y)
