@@ -15,6 +15,15 @@ namespace body {
 
 __host__ __device__ inline int nblk(long long n, int bs) { return (int)((n + bs - 1) / bs); }
 
+// launch(g0, n) for stretches of `cells` workgroups.  A launch of 2^32 threads or more runs
+// only its remainder, without an error: 16.8 million workgroups of 256
+template <class F>
+inline void per_cell(int cells, F launch) {
+    constexpr int kMost = 1 << 22;
+    for (long long g0 = 0; g0 < cells; g0 += kMost)
+        launch((int)g0, cells - g0 < kMost ? (int)(cells - g0) : kMost);
+}
+
 // CR scalars: rr0, rs0, rr, rho, rho_prev, tmp (= q.u), rs
 enum { kRR0 = 0, kRS0 = 1, kRR = 2, kRHO = 3, kRHOP = 4, kTMP = 5, kRS = 6, kRSIter = 7, kNScal = 8,
        kRHON = 10 };

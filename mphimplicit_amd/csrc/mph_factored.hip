@@ -278,7 +278,7 @@ constexpr int kGal0Cells = 4096;
 template <int T>
 __global__ void __launch_bounds__(T) k_fac_gal0(DevParams P, Level L, FacOp F, const int* __restrict__ cellStart,
                                                 const double* __restrict__ blk, const double* __restrict__ gtab,
-                                                const int* __restrict__ gmask) {
+                                                const int* __restrict__ gmask, int g0) {
     typedef double dv2 __attribute__((ext_vector_type(2)));
     constexpr int kRanges = 54, kGal0List = 6 * T;  // ranges: fluid, then wall particles of 27 cells
     __shared__ double sbuf[T * 9];    // the list, then the partition sums
@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(T) k_fac_gal0(DevParams P, Level L, FacOp F, c
     __shared__ unsigned char rcell[64];
     const int ncs = L.cs[0] * L.cs[1] * L.cs[2];
     const int nparts = T / ncs;
-    const int g = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t / 64;
+    const int g = g0 + blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t / 64;
     const int c = t % ncs, part = t / ncs;
     const bool active = part < nparts;
     int gx, gy, gz;
@@ -924,9 +924,10 @@ void launch_fac_level0(hipStream_t st, const DevParams& P, const Level& L0, cons
     hipLaunchKernelGGL(k_fac_g, dim3(nblk(P.np, 128)), dim3(128), 0, st, P, cellIndex, F.runP, F.nPtrP, F.nIndP,
                        F.beta, F.pos, F.selfC, gtab, gmask);
     hipLaunchKernelGGL(k_fac_invdiag, dim3(nblk(8LL * P.nf, 256)), dim3(256), 0, st, P, F, invDiagA);
-    if (L0.cells <= 0) return;
-#define MPH_GAL0(T) \
-    hipLaunchKernelGGL(k_fac_gal0<T>, dim3(L0.cells), dim3(T), 0, st, P, L0, F, cellStart, blk, gtab, gmask)
+#define MPH_GAL0(T)                                                                                               \
+    body::per_cell(L0.cells, [&](int g0, int n) {                                                                 \
+        hipLaunchKernelGGL(k_fac_gal0<T>, dim3(n), dim3(T), 0, st, P, L0, F, cellStart, blk, gtab, gmask, g0);    \
+    })
     if (P.dim == 2) MPH_GAL0(64);
     else if (L0.cells < kGal0Cells) MPH_GAL0(512);
     else MPH_GAL0(256);

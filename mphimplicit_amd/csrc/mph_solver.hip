@@ -62,9 +62,9 @@ __global__ void k_inv_diag(DevParams P, const int* __restrict__ selfIdx, const l
 __global__ void __launch_bounds__(256) k_mg_galerkin0(DevParams P, Level L, const int* __restrict__ cellStart,
                                                       const unsigned short* __restrict__ runStart,
                                                       const long long* __restrict__ start,
-                                                      const double* __restrict__ aval) {
+                                                      const double* __restrict__ aval, int g0) {
     const int ncs = L.cs[0] * L.cs[1] * L.cs[2];
-    const int g = blockIdx.x;
+    const int g = g0 + blockIdx.x;
     if ((int)threadIdx.x >= 9 * ncs) return;
     const int c = threadIdx.x / 9, e = threadIdx.x % 9;
     int gx, gy, gz;
@@ -110,13 +110,13 @@ __global__ void __launch_bounds__(256) k_mg_galerkin0_lds(DevParams P, Level L, 
                                                           const unsigned short* __restrict__ runStart,
                                                           const int* __restrict__ nFluid,
                                                           const long long* __restrict__ start,
-                                                          const double* __restrict__ aval) {
+                                                          const double* __restrict__ aval, int g0) {
     typedef double d2 __attribute__((ext_vector_type(2)));
     constexpr int kTask = (kGalRow / 2 * 9 * kGalGroup + 255) / 256;  // block pairs' entries per thread
     __shared__ double row[kGalGroup * kGalRow * 9];
     __shared__ unsigned short rs[kGalGroup * kRuns];
     const int ncs = L.cs[0] * L.cs[1] * L.cs[2];
-    const int g = blockIdx.x, t = threadIdx.x;
+    const int g = g0 + blockIdx.x, t = threadIdx.x;
     const bool active = t < 9 * ncs;
     const int c = t / 9, e = t % 9;
     int gx, gy, gz;
@@ -191,9 +191,9 @@ __global__ void __launch_bounds__(256) k_mg_galerkin0_lds(DevParams P, Level L, 
 // cell, block entry); children in R order, then fine stencil entries in shift order.
 // (A thread per stencil cell that tested every entry and loaded the matching blocks one
 // after the other took 118 us per level at 64k particles, 20 in 2D; now 10 and 7.)
-__global__ void __launch_bounds__(256) k_mg_galerkinL(Level S, Level L) {
+__global__ void __launch_bounds__(256) k_mg_galerkinL(Level S, Level L, int g0) {
     __shared__ double sA[8 * 27 * 9];
-    const int g = blockIdx.x, t = threadIdx.x;
+    const int g = g0 + blockIdx.x, t = threadIdx.x;
     const int ncs = L.cs[0] * L.cs[1] * L.cs[2], scs = S.cs[0] * S.cs[1] * S.cs[2];
     int l[3];
     grid_xyz(L, g, l[0], l[1], l[2]);
@@ -732,16 +732,19 @@ void launch_inv_diag(hipStream_t st, const DevParams& P, const int* selfIdx, ASl
 void launch_mg_galerkin0(hipStream_t st, const DevParams& P, const Level& L, const int* cellStart,
                          const unsigned short* runStart, const int* nFluid, ASlices A, int variant) {
     const int threads = 9 * L.cs[0] * L.cs[1] * L.cs[2];  // <= 243
-    if (L.cells <= 0) return;
-    if (variant == 1)
-        hipLaunchKernelGGL(k_mg_galerkin0_lds, dim3(L.cells), dim3(256), 0, st, P, L, cellStart, runStart, nFluid,
-                           A.start, A.val);
-    else
-        hipLaunchKernelGGL(k_mg_galerkin0, dim3(L.cells), dim3((threads + 63) / 64 * 64), 0, st, P, L, cellStart,
-                           runStart, A.start, A.val);
+    per_cell(L.cells, [&](int g0, int n) {
+        if (variant == 1)
+            hipLaunchKernelGGL(k_mg_galerkin0_lds, dim3(n), dim3(256), 0, st, P, L, cellStart, runStart, nFluid,
+                               A.start, A.val, g0);
+        else
+            hipLaunchKernelGGL(k_mg_galerkin0, dim3(n), dim3((threads + 63) / 64 * 64), 0, st, P, L, cellStart,
+                               runStart, A.start, A.val, g0);
+    });
 }
 void launch_mg_galerkinL(hipStream_t st, const Level& S, const Level& L) {
-    hipLaunchKernelGGL(k_mg_galerkinL, dim3(L.cells), dim3(256), 0, st, S, L);
+    per_cell(L.cells, [&](int g0, int n) {
+        hipLaunchKernelGGL(k_mg_galerkinL, dim3(n), dim3(256), 0, st, S, L, g0);
+    });
 }
 void launch_mg_invd(hipStream_t st, const Level& L) {
     hipLaunchKernelGGL(k_mg_invd, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
