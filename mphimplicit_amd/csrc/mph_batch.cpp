@@ -98,6 +98,7 @@ int build_tables(mph_batch& B, const std::vector<mph_scene*>& sc, Tables& T, boo
     B.cell.assign(ns, 0);
     B.shape.assign(ns, 0);
     B.hoff.assign((size_t)kOffRows * (ns + 1), 0);
+    long long allCells = 0;
     for (int s = 0; s < ns; ++s) {
         mph_scene& S = *sc[s];
         if (S.depth > kMaxLevels) return fail(MPH_E_STATE, "multigrid depth above the batch limit");
@@ -142,10 +143,12 @@ int build_tables(mph_batch& B, const std::vector<mph_scene*>& sc, Tables& T, boo
             b.maxit = S.prm.max_iterations > 0 ? S.prm.max_iterations : 3LL * S.P.nf;
         }
         auto put = [&](int row, int blocks) { B.hoff[(size_t)row * (ns + 1) + s + 1] = blocks; };
-        // the cell-staged FP64 pass: one workgroup per cell of the fluid bounding box
+        // the cell-staged FP64 pass: one workgroup per cell of the fluid bounding box, for as
+        // many scenes as one launch holds
         const FacOp& F = b.fac[0];
         const long long cells = (long long)F.cellCnt[0] * F.cellCnt[1] * F.cellCnt[2];
-        B.cell[s] = b.factored && F.slot && cells > 0 ? 1 : 0;
+        B.cell[s] = b.factored && F.slot && cells > 0 && allCells + cells <= kFacCellsMost ? 1 : 0;
+        if (B.cell[s]) allCells += cells;
         B.shape[s] = (char)F.cellShape;
         put(kOffCell, B.cell[s] ? (int)cells : 0);
         put(kOffChunk, (S.P.nf + 255) / 256);

@@ -157,6 +157,8 @@ constexpr int kFacRowsT = 64, kFacRowsY = 32;
 // 57 and 146 gathered, 29, 31 and 52 staged; 75 and 59 at radius 6 and 90k).
 enum { kFacCell3D = 0, kFacCell3DWide = 1, kFacCell2D = 2, kFacCellShapes = 3 };
 constexpr int kFacCellThreads[kFacCellShapes] = {512, 512, 128};
+// a launch of 2^32 threads or more runs only the remainder, without an error
+constexpr long long kFacCellsMost = (1LL << 32) / 512 - 1;
 constexpr int kFacCellSlots[kFacCellShapes] = {1456, 2816, 256};
 
 constexpr int kSlice = 64;    // particles per A slice (one wavefront)

@@ -380,7 +380,7 @@ constexpr long long kCellSpare = 2 << 20;  // 4-byte words
 bool cell_places(mph_scene& S) {
     const long long blk = 8 * kFacLanes, row = blk * ((S.hmaxW + blk - 1) / blk), cells = fac_bbox_cells(S);
     const long long words = 2 * S.E + kCellSpare;
-    if (cells <= 0 || kFacDesc * cells > words || row * S.P.nf > 2 * words) return false;
+    if (cells <= 0 || cells > kFacCellsMost || kFacDesc * cells > words || row * S.P.nf > 2 * words) return false;
     if (S.fslot.ensure((size_t)(row * S.P.nf)) == MPH_OK && S.fdesc.ensure((size_t)(kFacDesc * cells)) == MPH_OK) {
         S.fslotRow = (int)row;
         return true;

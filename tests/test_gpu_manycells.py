@@ -1,19 +1,23 @@
-"""Multigrid levels of more cells than one launch has workgroups for (GPU).
+"""More cells than one launch has workgroups for (GPU).
 
 Two drops at opposite corners of the domain span 17.6 million level-0 cells in 3D (43 GB of
 level matrices) and 68 million in 2D (its level 1 has 17.0 million).  Every level's matrix
 is the sum of the finer one's blocks, so the entries of the coarsest add up to 1^T A 1, with
 the product A 1 from the particles (bound 1e-12 of the entries' magnitudes, as in
 test_gpu_level0.py).
+
+The cell-staged second pass runs a workgroup of 512 threads per cell of the bounding box.  A
+block of fluid and one drop far from it make that more than a launch holds, alone or as
+two members of a batch: the chunk kernel takes over, with the same bits.
 """
 import numpy as np
 import pytest
 import torch
 
 from mphimplicit_amd import abi, scenes
-from mphimplicit_amd.scene import Scene
+from mphimplicit_amd.scene import Batch, Scene
 from test_gpu_coarse import L0
-from test_gpu_faccells import two_drops
+from test_gpu_faccells import assembled, two_drops
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +47,48 @@ def test_levels_of_many_cells(make, gb, form):
         total = float(s.apply_matrix(np.ones(3 * int(s.scalar("FluidCount")))).sum())
     entries, most = float(a.sum()), float(np.abs(a).sum())
     assert abs(entries - total) <= 1e-12 * most, (entries, total)
+
+
+def block_and_drop(block, n):
+    """block^3 particles in one corner of a domain of n cells per axis, 27 in the other."""
+    side = 3.6 * n
+    fluid = np.concatenate([scenes.lattice([2.0] * 3, [2.0 + block] * 3, L0, 3),
+                            scenes.lattice([side - 5.0] * 3, [side - 2.0] * 3, L0, 3)])
+    walls = scenes.lattice([0, 0, 0], [4, 4, 2], L0, 3)
+    g = scenes.assemble(fluid, walls, 0.0, L0, [0.0] * 3, [side * L0] * 3, 5, 3)
+    p = scenes.base_params(3, 0.1, (0.0, 0.0, -9.8), 5.0e-4, 4)
+    p.operator_form = abi.OPERATOR_FACTORED
+    p.multigrid = 0
+    p.cr_tolerance = 1e-4
+    p.end_time = 1.0e9
+    return p, g
+
+
+def test_product_of_many_cells():
+    p, g = block_and_drop(162, 199)
+    print("[manycells] np=%d" % g.np, flush=True)
+    out = []
+    for cells in (0, 1):
+        s, y = assembled(p, g, cells)
+        with s:
+            assert s.scalar("FactoredCellsUsed") == 0
+        out.append(y)
+    assert np.array_equal(*out)
+
+
+def test_batch_of_many_cells():
+    p, g = block_and_drop(129, 158)
+    print("[manycells] 2 members of np=%d" % g.np, flush=True)
+    with Scene(p, g) as s:
+        st = s.step(1)
+        assert s.scalar("FactoredCellsUsed") == 1
+        v = s.read("Velocity").view(np.int64)
+    members = [Scene(p, g) for _ in range(2)]
+    with Batch() as b:
+        for m in members:
+            b.add(m)
+        for m, t in zip(members, b.step()):
+            assert (t.cr_iterations, t.rr) == (st.cr_iterations, st.rr)
+            assert np.array_equal(m.read("Velocity").view(np.int64), v)
+    for m in members:
+        m.close()
