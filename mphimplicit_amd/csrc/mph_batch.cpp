@@ -156,7 +156,7 @@ int build_tables(mph_batch& B, const std::vector<mph_scene*>& sc, Tables& T, boo
         put(kOffRowsT, (S.P.np + kFacRowsT - 1) / kFacRowsT);
         put(kOffRowsT32, (S.P.np + kFacRowsY - 1) / kFacRowsY);
         put(kOffRowsY, (S.P.nf + kFacRowsY - 1) / kFacRowsY);
-        put(kOffP2g, b.mg ? (8 * b.lv[0].nrow + 255) / 256 : 0);
+        put(kOffP2g, b.mg ? (int)((8LL * b.lv[0].nrow + 255) / 256) : 0);
         for (int l = 0; l < b.depth; ++l) {
             put(kOffLevel + l, (b.lv[l].nrow + 255) / 256);
             put(kOffSweep + l, ((b.lv[l].lanes ? 4 : 1) * b.lv[l].nrow + 255) / 256);

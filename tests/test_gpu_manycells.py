@@ -92,3 +92,25 @@ def test_batch_of_many_cells():
             assert np.array_equal(m.read("Velocity").view(np.int64), v)
     for m in members:
         m.close()
+
+
+def test_batch_level0_of_90_million_cells():
+    """The batch's P2G takes 8 lanes for each of 270 million level-0 rows."""
+    if torch.cuda.mem_get_info()[0] < 160 << 30:
+        pytest.skip("needs 160 GB of device memory")
+    p, g = two_drops_2d(9230)
+    p.operator_form = abi.OPERATOR_FACTORED
+    p.cr_tolerance = 1e-4
+    p.end_time = 1.0e9
+    print("[manycells] np=%d" % g.np, flush=True)
+    out = []
+    for batch in (False, True):
+        with Scene(p, g) as s:
+            if batch:
+                with Batch() as b:
+                    b.add(s)
+                    st = b.step()[0]
+            else:
+                st = s.step(1)
+            out.append((st.cr_iterations, st.rr, s.read("Velocity").tobytes()))
+    assert out[0] == out[1]
