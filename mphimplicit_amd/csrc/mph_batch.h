@@ -141,11 +141,8 @@ void store_velocity(const Tables& T, const SceneSet& on);
 void mg_p2g_bu(const Tables& T, const SceneSet& on, const SceneSet& pq, const SceneSet& fold, int in,
                const SceneSet& cur);
 void mg_restrict_bu(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);  // l-1 -> l, begin, update
-void mg_begin(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);
-void mg_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur);
 void mg_residual(const Tables& T, const SceneSet& on, int l, const SceneSet& cur, bool f32);
 void mg_residual_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur, bool f32);
-void mg_restrict(const Tables& T, const SceneSet& on, int l);  // level l-1 -> l
 void mg_prolong(const Tables& T, const SceneSet& on, int l, const SceneSet& curL, const SceneSet& curS);  // l -> l-1
 void mg_g2p(const Tables& T, const SceneSet& on, const SceneSet& cur0, int in, int out, bool part,
             const SceneSet& fold);

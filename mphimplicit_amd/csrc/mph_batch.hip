@@ -224,20 +224,6 @@ __global__ void kb_mg_restrict_bu(const BScene* tab, const int* off, int ns, Sce
     mg_begin_update_row(L, row, mg_restrict_row(B.lv[l - 1], L, row));
 }
 
-__global__ void kb_mg_begin(const BScene* tab, const int* off, int ns, SceneSet on, int l, SceneSet cur) {
-    MPH_SCENE(kOffLevel + l)
-    const int row = lb * 256 + threadIdx.x;
-    const Level L = level(B, l, cur, s);
-    if (row < L.nrow) mg_begin_row(L, row);
-}
-
-__global__ void kb_mg_update(const BScene* tab, const int* off, int ns, SceneSet on, int l, SceneSet cur) {
-    MPH_SCENE(kOffLevel + l)
-    const int row = lb * 256 + threadIdx.x;
-    const Level L = level(B, l, cur, s);
-    if (row < L.nrow) mg_update_row(L, row);
-}
-
 // FP32 stencil where the level has one and the launch asks for it (mixed inner solve)
 template <class VT, bool kUpdate, bool kOrd>
 __device__ inline void sweep(const Level& L, int lb, double* tb) {
@@ -268,13 +254,6 @@ __global__ void __launch_bounds__(256) kb_mg_sweep(const BScene* tab, const int*
         if (h) sweep<float, kUpdate, false>(L, lb, tb);
         else sweep<double, kUpdate, false>(L, lb, tb);
     }
-}
-
-__global__ void kb_mg_restrict(const BScene* tab, const int* off, int ns, SceneSet on, int l) {
-    MPH_SCENE(kOffLevel + l)
-    const int row = lb * 256 + threadIdx.x;
-    const Level& L = B.lv[l];
-    if (row < L.nrow) mg_restrict_row(B.lv[l - 1], L, row);
 }
 
 __global__ void kb_mg_prolong(const BScene* tab, const int* off, int ns, SceneSet on, int l, SceneSet curL,
@@ -417,19 +396,12 @@ void mg_p2g_bu(const Tables& T, const SceneSet& on, const SceneSet& pq, const Sc
 void mg_restrict_bu(const Tables& T, const SceneSet& on, int l, const SceneSet& cur) {
     MPH_LAUNCH(kb_mg_restrict_bu, kOffLevel + l, l, cur);
 }
-void mg_begin(const Tables& T, const SceneSet& on, int l, const SceneSet& cur) {
-    MPH_LAUNCH(kb_mg_begin, kOffLevel + l, l, cur);
-}
-void mg_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur) {
-    MPH_LAUNCH(kb_mg_update, kOffLevel + l, l, cur);
-}
 void mg_residual(const Tables& T, const SceneSet& on, int l, const SceneSet& cur, bool f32) {
     MPH_LAUNCH(kb_mg_sweep<false>, kOffSweep + l, l, cur, f32 ? 1 : 0);
 }
 void mg_residual_update(const Tables& T, const SceneSet& on, int l, const SceneSet& cur, bool f32) {
     MPH_LAUNCH(kb_mg_sweep<true>, kOffSweep + l, l, cur, f32 ? 1 : 0);
 }
-void mg_restrict(const Tables& T, const SceneSet& on, int l) { MPH_LAUNCH(kb_mg_restrict, kOffLevel + l, l); }
 void mg_prolong(const Tables& T, const SceneSet& on, int l, const SceneSet& curL, const SceneSet& curS) {
     MPH_LAUNCH(kb_mg_prolong, kOffLevel + l - 1, l, curL, curS);
 }

@@ -118,22 +118,8 @@ __device__ inline int galerkin_self(const DevParams& P, const Level& L, int g) {
 // ---------------------------------------------------------------------------
 // multigrid rows (preconditionWithMultiGrid)
 
-__device__ inline void mg_begin_row(const Level& L, int row) {  // myDscal(0.0, S); myDcopy(Q, R)
-    double* S = lv_s(L, L.cur);
-    S[row] *= 0.0;
-    L.R[row] = L.Q[row];
-}
-
-__device__ inline void mg_update_row(const Level& L, int row) {  // myDdmv(1.0, invD, R, 1.0, S)
-    double* S = lv_s(L, L.cur);
-    double y = S[row];
-    y *= 1.0;
-    y += 1.0 * L.invD[row] * L.R[row];
-    S[row] = y;
-}
-
-// mg_begin_row then mg_update_row on the same row (both touch that row only).  S*0.0 is a
-// zero and Q is never -0 (a sum from +0), so S = invD Q is formed without the old S.
+// myDscal(0.0, S), myDcopy(Q, R), then myDdmv(1.0, invD, R, 1.0, S) on the same row.  S*0.0
+// is a zero and Q is never -0 (a sum from +0), so S = invD Q is formed without the old S.
 __device__ inline void mg_begin_update_row(const Level& L, int row, double r) {
     L.R[row] = r;
     double y = 0.0;

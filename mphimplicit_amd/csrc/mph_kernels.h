@@ -261,11 +261,8 @@ void launch_mg_p2g_bu(hipStream_t st, const DevParams& P, Level& L, const int* c
 void launch_mg_p2g_bu_pq(hipStream_t st, const DevParams& P, Level& L, const int* cellStart, double* q,
                          const double* y, double* scal, const double* rho);  // rho: its partials, folded here, or null
 void launch_mg_restrict_bu(hipStream_t st, const Level& S, Level& L);  // restriction, begin, update
-void launch_mg_begin(hipStream_t st, Level& L);        // S *= 0; R = Q
-void launch_mg_update(hipStream_t st, Level& L);       // S += invD R
 void launch_mg_residual(hipStream_t st, Level& L);     // R = Q - A S
 void launch_mg_residual_update(hipStream_t st, Level& L);  // R = Q - A S; S += invD R
-void launch_mg_restrict(hipStream_t st, const Level& S, Level& L);
 void launch_mg_prolong(hipStream_t st, const Level& L, Level& S);
 // levels lc..D-1 of the V-cycle in one workgroup, from their packed rows.  S is level
 // lc-1 (its R is restricted, its current S takes the prolongation), or level 0 itself

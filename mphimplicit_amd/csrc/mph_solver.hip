@@ -314,16 +314,6 @@ __global__ void k_mg_restrict_bu(Level S, Level L) {
     mg_begin_update_row(L, row, mg_restrict_row(S, L, row));
 }
 
-__global__ void k_mg_begin(Level L) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row < L.nrow) mg_begin_row(L, row);
-}
-
-__global__ void k_mg_update(Level L) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row < L.nrow) mg_update_row(L, row);
-}
-
 // threads per workgroup of the kernels with a thread per multigrid row: 73k rows (1M scene)
 // are 1147 workgroups for 256 CUs, where workgroups of 256 threads left most CUs waiting for
 // the 30 with a second one.  Residual-update sweep 14.5 -> 12.6 us, residual 13.5 -> 12.1;
@@ -387,11 +377,6 @@ bool launch_sweep_lanes(hipStream_t st, const Level& L, const Level& U) {
     MPH_SHAPE(L, MPH_SWEEP);
 #undef MPH_SWEEP
     return true;
-}
-
-__global__ void k_mg_restrict(Level S, Level L) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row < L.nrow) mg_restrict_row(S, L, row);
 }
 
 __global__ void k_mg_prolong(Level L, Level S) {
@@ -777,12 +762,6 @@ void launch_mg_p2g_bu_pq(hipStream_t st, const DevParams& P, Level& L, const int
 void launch_mg_restrict_bu(hipStream_t st, const Level& S, Level& L) {
     hipLaunchKernelGGL(k_mg_restrict_bu, dim3(nblk(L.nrow, kRowThreads)), dim3(kRowThreads), 0, st, S, L);
 }
-void launch_mg_begin(hipStream_t st, Level& L) {
-    hipLaunchKernelGGL(k_mg_begin, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
-}
-void launch_mg_update(hipStream_t st, Level& L) {
-    hipLaunchKernelGGL(k_mg_update, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, L);
-}
 #define MPH_ROWS(KERNEL)                                                                                           \
     do {                                                                                                           \
         const int nb = nblk(L.nrow, kRowThreads);                                                                          \
@@ -818,9 +797,6 @@ void launch_mg_prolong_update(hipStream_t st, const Level& U, Level& L, bool pro
     }
     if (!prolonged) launch_mg_prolong(st, U, L);
     launch_mg_residual_update(st, L);
-}
-void launch_mg_restrict(hipStream_t st, const Level& S, Level& L) {
-    hipLaunchKernelGGL(k_mg_restrict, dim3(nblk(L.nrow, 256)), dim3(256), 0, st, S, L);
 }
 void launch_mg_prolong(hipStream_t st, const Level& L, Level& S) {
     hipLaunchKernelGGL(k_mg_prolong, dim3(nblk(S.nrow, kRowThreads)), dim3(kRowThreads), 0, st, L, S);
@@ -919,7 +895,8 @@ void launch_axpy(hipStream_t st, long long n, const double* x, double* y) {
 }
 void launch_dot_partial(hipStream_t st, const DevParams& P, const double* x, const double* y, double* part) {
     hipLaunchKernelGGL(k_dot_partial, dim3(nblk(P.nf, kChunk)), dim3(kChunk), 0, st, P.nf, x, y, part, P.halt);
-}void launch_dot_final(hipStream_t st, const DevParams& P, const double* part, double* scal, int slot,
+}
+void launch_dot_final(hipStream_t st, const DevParams& P, const double* part, double* scal, int slot,
                       int shift_slot, double* host, bool shiftRho) {
     hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(256), 0, st, part, nblk(P.nf, kChunk), scal, slot, shift_slot,
                        host, P.halt, shiftRho ? 1 : 0);
