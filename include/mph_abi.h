@@ -175,9 +175,9 @@ int mph_scene_run_phase(mph_scene* s, int phase);
  * R2g Swa Swg Swp Swv MaxRadius ParticleCount FluidCount PowerParticleCount
  * CellCount0..2 TotalCellCount NeighborIndCount NeighborIndCountP MultiGridDepth
  * CRIterations rr0 rr rs0 rs RefinementSteps ABlocks ASlots CBlocks, the timing
- * scalars of mph_scene_set_timing, TunedSpmv64 TunedSpmv32 TunedCac TunedGalerkin
- * (the variants the run-time tuner kept, -1 while still exploring), TunedFuse (0: one
- * variant of the fused coarse V-cycle),
+ * scalars of mph_scene_set_timing, TunedSpmv64 TunedSpmv32 TunedGalerkin (the variants
+ * the run-time tuner kept, -1 while still exploring), TunedCac TunedFuse (0: C Lambda
+ * C^T and the fused coarse V-cycle have one variant),
  * and for the factored operator FactoredBytes and FactoredBytesF32 (algorithmic
  * bytes of one product with FP64 / FP32 scalars) and AssembledBlocks (1 when the
  * step assembled the 3x3 blocks: always for the assembled form; for the factored
@@ -188,8 +188,8 @@ int mph_scene_run_phase(mph_scene* s, int phase);
  * one, and where the scene or option FactoredCells has it run as the chunk kernel),
  * and NeighborOneScan (1 when the last neighbour search built the lists in one scan,
  * 0 when it ran the count and fill passes: a scene's first search, or a list longer
- * than the last search's
- * largest plus a margin; the lists are the same either way, alone or in a batch). */
+ * than the last search's largest plus a margin; the lists are the same either way,
+ * alone or in a batch). */
 int mph_scene_field_size(mph_scene* s, const char* field, size_t* bytes, int* elem_bytes);
 int mph_scene_read(mph_scene* s, const char* field, void* host, size_t bytes);
 int mph_scene_write(mph_scene* s, const char* field, const void* host, size_t bytes);
@@ -238,8 +238,10 @@ int mph_scene_set_timing(mph_scene* s, int on);
  *   "FactoredCells"     1: the FP64 factored product's second pass runs one
  *                  workgroup per cell with the visited cells' records staged in
  *                  LDS; 0: the chunk kernel, every neighbour gathered through the
- *                  caches; 2 (default): the faster one, which is the cells wherever
- *                  they can be staged.  Alone and in a batch; the same bits either way.
+ *                  caches; 2 (default): the faster one, which is the cells as well.
+ *                  The chunk kernel also runs where the cells' buffers would outgrow
+ *                  twice the neighbour lists (FactoredCellsUsed).  Alone and in a
+ *                  batch; the same bits either way.
  *   "FactoredCellsXcd"  1 (default): the cells of that pass are dealt to the XCDs in
  *                  contiguous ranges; 0: round robin.
  *   "CrStop"       where the FP64 CR loop tests rr/rr0 < tol (main.cpp:4344-4346):

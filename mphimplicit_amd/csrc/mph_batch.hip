@@ -275,7 +275,9 @@ __global__ void __launch_bounds__(256) kb_mg_g2p(const BScene* tab, const int* o
 }
 
 // levels fuse..depth-1 of each scene in its own workgroup (mg_coarse_cycle; 2D and 3D
-// scenes take launches of their own)
+// scenes take launches of their own).  Both orders are in the kernel: 14 (3D) or 18 (2D) of
+// the values loaded before the branch reach the unordered cycle through scratch, once per
+// cycle; the sweeps have no scratch access.  Every 3D scene takes the 512-thread variant
 template <int N, int T, int XB>
 __global__ void __launch_bounds__(T) kb_mg_coarse(const BScene* tab, int ns, SceneSet on, SceneSet cur) {
     const int s = blockIdx.x;

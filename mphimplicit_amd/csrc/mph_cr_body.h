@@ -139,8 +139,8 @@ __device__ inline int wrap3(int v, int n) {
 // factored form, which keeps no bits of the reference): four chains over the stencil
 // cells [uQ, (u+1)Q), Q = cells/4 rounded up, with fused multiply-adds, combined as
 // (c0 + c1) + (c2 + c3); the lane-split sweeps give each lane one chain, so every kernel
-// that takes such a sum gets the same bits.  Per sweep of a level of 5k rows 4.2 us
-// against 4.75 us ordered, of the one-workgroup cycle 12.8 against 14.4 us (64k drop).
+// that takes such a sum gets the same bits.  Per sweep of a level of 4k rows 4.3 us
+// against 4.8 us ordered, of the one-workgroup cycle 12.0 against 13.4 us (64k drop).
 template <bool kOrd>
 struct RowSum {
     double c[kOrd ? 1 : 4];
@@ -271,11 +271,10 @@ __device__ inline void mg_residual_update_row(const Level& L, int row) {
 // row's first lane adds all terms in stencil order (the order of mg_row_sum), read back
 // through LDS.  Otherwise each lane sums its own, one of RowSum's four chains.  So the
 // sums are those of mg_residual_row and mg_residual_update_row either way.  Measured on
-// a level of 73k rows, one thread per row is faster (14.3 against 18.4 us per ordered
-// sweep, 14.5 against 15.6 us unordered); on levels of 10k rows and fewer the lanes take
-// 20-30% off.  C0 C1 C2 give the
-// stencil at compile time (3x3x3, 3x3x1); 0 0 0 reads it from the level (other shapes),
-// at the price of runtime index arithmetic.
+// a level of 73k rows, one thread per row is faster (12.4 against 18.6 us per ordered
+// sweep, 12.1 against 15.5 us unordered); on levels of 10k rows and fewer the lanes take
+// 20-30% off.  C0 C1 C2 give the stencil at compile time (3x3x3, 3x3x1); 0 0 0 reads it
+// from the level (other shapes), at the price of runtime index arithmetic.
 // t: the thread's number over the level's lanes; tb: kRowTerms doubles per thread of the
 // workgroup (ordered only)
 constexpr int kRowLanes = 4, kRowQ = 7;  // kRowQ: stencil cells per lane (27 / 4, rounded up)
@@ -460,10 +459,11 @@ __device__ inline void mg_prolong_row(const Level& L, const Level& S, int row) {
 // are laid out per thread once per multigrid build (coarse_pack), so the cycle starts
 // with one round of coalesced loads, all in flight together (2.3-3.4 us), and a sweep
 // is 27 LDS reads and a chain of 81 ordered adds per row (9 and 27 in 2D).  The chain
-// bounds it: about 24 cycles per add, 0.9 us per 3D sweep.  Measured per cycle: 14.2 us
-// on the 64k-particle drop (105 rows), 18.8 us on the 1M-particle scene (216 rows),
-// 14.0 us on a 2D pool of 4,100 (372 rows).  Re-reading the stencils through L2 in
-// every sweep, three dependent rounds of loads each, took 47.7, 63.9 and 60.4 us.
+// bounds it: about 24 cycles per add, 0.9 us per 3D sweep.  Measured per cycle, ordered
+// and in chains: 13.4 and 12.0 us on the 64k-particle drop (320 threads), 14.0 and 14.3 us
+// on the 1M-particle scene (256), 13.3 and 12.4 us on a 2D pool of 4,100 (448).
+// Re-reading the stencils through L2 in every sweep, three dependent rounds of loads
+// each, took 47.7, 63.9 and 60.4 us ordered.
 //
 // Invalid cells of a stencil narrower than 3 along an axis are padded with a zero
 // value and the row's own cell: they add a zero, which changes no bit of a sum that
@@ -1511,8 +1511,8 @@ __device__ inline double pq_elem(double beta, double v, double w) {
 // loop's q = beta q + y (4364-4366) is formed here as q is loaded and written back
 // (every fluid particle lies in exactly one level-0 cell, so each element is updated
 // once); q is written only then.  tb: 256 * kP2gK doubles of LDS (ordered only).
-// Unordered, with the update, 19.0 us on the 1M scene (72 MB, 3.8 TB/s) and 5.6 us on
-// the 64k drop; ordered 25.2 and 9.8 us, bound by the first lane's chain of adds.
+// Unordered, with the update, 19.5 us on the 1M scene (72 MB, 3.7 TB/s) and 6.1 us on
+// the 64k drop; ordered 21.5 and 9.4 us, bound by the first lane's chain of adds.
 constexpr int kP2gLanes = 8, kP2gK = 8;
 // coef(): beta, called by every thread of the workgroup (kPq only)
 template <bool kPq, bool kOrd, class F>

@@ -525,8 +525,9 @@ __global__ void __launch_bounds__(256, 4) k_fac_y(DevParams P, FacOp F, const do
 // the fluid neighbours, one walk forms both terms.  On the 1M-particle scene the pass
 // takes 428 us; it took 726 us when it streamed alpha beside the places and walked the P
 // lists on their own (10 bytes per entry at 4.3 TB/s, a dependent round of list loads
-// per 32 entries, and the P part's gathers).  The VALU issues 61% of the time, the rest
-// is a workgroup's waits for its loads at two workgroups per CU.
+// per 32 entries, and the P part's gathers).  The VALU issues 52% of the time, the rest
+// is LDS reads with their bank conflicts and a workgroup's waits for its loads at two
+// workgroups per CU.
 // A row's entries, lanes and order of summation are those of body::fac_row_gather, so
 // the results are the chunk kernel's.  The rows go straight to y; the dot partials of
 // the fused epilogue come from a dot-partial launch afterwards (the chunks of 256 rows
@@ -844,7 +845,9 @@ __device__ inline void fac_y_cell_any(const DevParams& P, const FacOp& F, const 
 #undef MPH_Y
 }
 
-// four waves per SIMD: two workgroups of 512 threads on a CU
+// four waves per SIMD: two workgroups of 512 threads on a CU.  The three bodies share one
+// kernel of 128 registers.  What spills (4 registers, 7 in the batch) does so in the body of
+// several viscosities alone; the others have no scratch access
 template <bool kNeg, int kShape>
 __global__ void __launch_bounds__(kFacCellThreads[kShape], kShape == kFacCell3DWide ? 2 : 4)
     k_fac_y_cell(DevParams P, FacOp F, const double* __restrict__ x, double beta, const double* yin, double* y,

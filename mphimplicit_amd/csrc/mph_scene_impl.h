@@ -187,7 +187,8 @@ struct mph_scene {
     bool blocks = true;  // this step assembles the 3x3 blocks (see blocks_wanted)
     mph::host::DBuf<double> falpha, fdiag, selfC, fbeta, frec;  // FacOp::alpha, diag, selfC, beta, rec
     mph::host::DBuf<float> fu32, fv32, frec32;  // FP32 form (mixed precision): FacOp::u32, v32, rec32
-    // FP64 second pass staged per cell in LDS (0: the chunk kernel; 1, 2: the cells).
+    // FP64 second pass staged per cell in LDS (0: the chunk kernel; 1, 2: the cells, where
+    // their buffers are worth it: cell_places).
     // Measured per second pass, chunk kernel against cells (with their dot partials): 2D
     // 160k fluid 49 against 37 us; 3D 1M about 1150 against 438 us.
     int facCells = 2;
@@ -273,7 +274,7 @@ bool mixed(const mph_scene& S);
 bool factored(const mph_scene& S);
 // rows of the convergence record (16 bytes each): iterations past this are not kept
 constexpr long long kConvRowsMax = 1LL << 22;
-bool fac_cells(const mph_scene& S);  // the FP64 second pass is the cell-staged one (facCells)
+bool fac_cells(const mph_scene& S);  // the FP64 second pass may be the cell-staged one (facCells)
 // whether the step assembles the 3x3 blocks: always for the assembled form; for the
 // factored form only when the multigrid's level 0 cannot be built from the factored
 // scalars (a level-0 grid under 3 cells along an active axis)
